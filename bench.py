@@ -570,6 +570,8 @@ def time_gemm_any(type_id, n_tok, n_rows, n_cols, steps, warmup):
 def gemm_route(type_id, n_tok, n_rows, n_cols):
     """what qlin_gemm_bf16_any_dev does with this shape when it is handed a workspace"""
     r = qlinear.load().qlin_probe_gemm_route(type_id, n_rows, n_cols, n_tok, n_cols, 1)
+    if r == 3:
+        return "few-token kernel, no workspace"
     if r:
         return "decoded inside the product (%s tiles), no workspace" % ("256-token x 128-row" if r == 1 else "128-token x 64-row")
     return "dense library product" if type_id == synth.GGML_BF16 else "decode to bf16 + dense library product"

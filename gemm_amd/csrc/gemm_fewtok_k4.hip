@@ -1,0 +1,8 @@
+/* gemm_fewtok_k4.hip - the few-token product (Q4_K, Q5_K, Q2_K): instances of gemm_fewtok.h */
+#include "gemm_fewtok.h"
+
+namespace qlin {
+hipError_t fewtok_q4k(const FewtokCall &c) { return fewtok_format<TQ4K, 32>(c); }
+hipError_t fewtok_q5k(const FewtokCall &c) { return fewtok_format<TQ5K, 24>(c); }
+hipError_t fewtok_q2k(const FewtokCall &c) { return fewtok_format<TQ2K, 24>(c); }
+}  // namespace qlin

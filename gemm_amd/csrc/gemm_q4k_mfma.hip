@@ -371,9 +371,9 @@ hipError_t launch_tiled(const void *W, const uint16_t *X, float *Y, int n_rows, 
 
 hipError_t launch_gemm_q4k_bf16(const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                                 int n_tok, int ldx, int ldy, hipStream_t stream) {
-    /* up to 48 tokens the weights are better streamed once per 16 tokens with exact codes (13-39 us at
-     * 14336 x 4096) than pushed through a 256-token tile (54 us whatever the count) */
-    if (n_tok <= kFewTokens) return launch_gemm_q4k_fewtok(W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
+    const FewtokCall few = {1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream};
+    if (fewtok_takes(T_Q4_K, n_rows, n_cols, n_tok, ldx)) return launch_gemm_fewtok(T_Q4_K, few);
+    if (n_tok <= fewtok_unrounded(T_Q4_K)) return launch_gemm_fewtok_one_by_one(T_Q4_K, few);
     /* the four-wave kernels, large or small tiles by how many there are (their 32-bit offsets hold 256 rows of X) */
     const FusedTile tile = choose_fused_tile(T_Q4_K, n_rows, n_cols, n_tok, ldx, false);
     if (tile != kFusedNone) return launch_fused_tile(tile, T_Q4_K, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);

@@ -753,8 +753,8 @@ int qlin_gemm_tokenmajor(float *Y, const void *W, uint32_t type, int n_cols, con
         const uint16_t *Xb = (const uint16_t *)g.tmp[2].p;
         float *Yd = (float *)g.tmp[1].p;
         const FusedTile tile = choose_fused_tile(type, n_rows, n_cols, n_tok, n_cols, true);
-        if (type == T_Q4_K && n_tok <= kFewTokens) {
-            HIP_TRY(launch_gemm_q4k_bf16(dW, Xb, Yd, n_rows, n_cols, n_tok, n_cols, n_rows, g.stream));
+        if (fewtok_takes(type, n_rows, n_cols, n_tok, n_cols)) {
+            HIP_TRY(launch_gemm_fewtok(type, {1, &dW, Xb, &Yd, &n_rows, n_cols, n_tok, n_cols, &n_rows, g.stream}));
         } else if (tile != kFusedNone) {
             HIP_TRY(launch_fused_tile(tile, type, dW, Xb, Yd, n_rows, n_cols, n_tok, n_cols, n_rows, g.stream));
         } else {
@@ -1048,6 +1048,12 @@ size_t qlin_gemm_bf16_any_workspace_bytes(int n_rows, int n_cols) {
     return dense_gemm_weight_bytes(n_rows, n_cols) + kDenseLibWorkspace;
 }
 
+/* the few-token kernel; the formats without a tile kernel keep to what they ask of the caller (a workspace) and to the
+ * dense product that was chosen */
+static bool takes_fewtok(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool ws_ok) {
+    return fewtok_takes(type, n_rows, n_cols, n_tok, ldx) && (gemm_kq_wave4_covers(type) || (ws_ok && g.dense_gemm_mode == 0));
+}
+
 int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                            int n_tok, int ldx, int ldy, void *workspace, size_t workspace_bytes, void *stream) {
     if (int rc = check_linear_shape(type, n_rows, n_cols)) return rc;
@@ -1056,28 +1062,22 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
     if (!W || !X || !Y) return fail(QLIN_ERR_ARG, "null pointer");
     if (!aligned(W, 16) || !aligned(X, 16) || !aligned(Y, 4) || ldx % 8)
         return fail(QLIN_ERR_ARG, "W and X need 16-byte alignment, Y 4-byte, ldx %% 8 == 0");
-    /* Q4_K, a few tokens: its few-token kernel (exact codes, no workspace) */
     const bool ws_ok = workspace && aligned(workspace, 256) && workspace_bytes >= qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols);
-    if (type == T_Q4_K && n_tok <= kFewTokens)
-        return qlin_gemm_bf16_dev(type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    /* a few tokens of a Q6_K, Q5_K, Q3_K, Q2_K or Q8_0 tensor: streamed once per eight tokens with exact codes
-     * (14336 x 4096 Q6_K, 8 tokens: decode + library GEMM about 75 us) */
-    {
-        hipError_t e = hipSuccess;
-        if (launch_gemm_kq_fewtok(type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream, &e)) {
-            if (e != hipSuccess) return fail(QLIN_ERR_DEVICE, "few-token GEMM launch failed: %s", hipGetErrorString(e));
-            return QLIN_OK;
-        }
-    }
     {
         std::lock_guard<std::mutex> lk(g.mu);
         if (int rc = ensure_init_locked(0)) return rc;
     }
     /* the formats with a tile kernel (gemm_kq_formats.h): decoded into the matrix operand inside the product, no workspace, in large or small
      * tiles by the shape - except where decoding once into the caller's workspace measured faster */
-    /* (up to four tokens of the formats without a few-token kernel are faster one by one through the matvec below) */
-    const bool matvec_first = (type == T_IQ4_NL || type == T_IQ4_XS || type == T_Q4_0) && n_tok <= kMatvecTokens && ws_ok;
-    if (const FusedTile tile = matvec_first ? kFusedNone : choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok);
+    if (takes_fewtok(type, n_rows, n_cols, n_tok, ldx, ws_ok)) {
+        HIP_TRY(launch_gemm_fewtok(type, {1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, (hipStream_t)stream}));
+        return QLIN_OK;
+    }
+    if (ldx >= (1 << 22) && n_cols % 256 == 0 && fewtok_has(type) && n_tok <= fewtok_unrounded(type) && fewtok_unrounded(type) > kMatvecTokens) {
+        HIP_TRY(launch_gemm_fewtok_one_by_one(type, {1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, (hipStream_t)stream}));
+        return QLIN_OK;
+    }
+    if (const FusedTile tile = choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok);
         tile != kFusedNone) {
         HIP_TRY(launch_fused_tile(tile, type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
         return QLIN_OK;
@@ -1139,24 +1139,30 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
     if (!W || !Y || !n_rows || !ldy) return fail(QLIN_ERR_ARG, "null pointer");
     /* one launch where every tensor on its own would take the same tile kernel; the checks are those of the
      * single-tensor call, which a tensor that fails them goes through below to report it */
-    bool together = n_mat > 1 && n_tok > 0 && X && aligned(X, 16) && ldx % 8 == 0 && ldx >= n_cols && n_tok > kFewTokens;
+    bool together = n_mat > 1 && n_tok > 0 && X && aligned(X, 16) && ldx % 8 == 0 && ldx >= n_cols;
     FusedTile tile = kFusedNone;
+    bool few = false;
     for (int i = 0; i < n_mat && together; i++) {
         const bool ws_ok = workspace && aligned(workspace, 256) &&
                            workspace_bytes >= qlin_gemm_bf16_any_workspace_bytes(n_rows[i], n_cols);
         together = n_rows[i] > 0 && W[i] && Y[i] && aligned(W[i], 16) && aligned(Y[i], 4) && ldy[i] >= n_rows[i] &&
                    n_cols > 0; /* the chooser checks format and row length */
         if (!together) break;
-        const FusedTile mine = choose_fused_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
-        together = mine != kFusedNone && (i == 0 || mine == tile);
+        const bool mine_few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
+        const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(T_Q4_K) ? kFusedNone : choose_fused_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        together = (mine_few || mine != kFusedNone) && (i == 0 || (mine == tile && mine_few == few));
         tile = mine;
+        few = mine_few;
     }
     if (together) {
         {
             std::lock_guard<std::mutex> lk(g.mu);
             if (int rc = ensure_init_locked(0)) return rc;
         }
-        if (tile == kFusedLarge)
+        if (few)
+            HIP_TRY(launch_gemm_fewtok(type, {n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream}));
+        else if (tile == kFusedLarge)
             HIP_TRY(launch_gemm_kq_bf16_wave4_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
         else
             HIP_TRY(launch_gemm_kq_bf16_wave4s_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
@@ -1312,6 +1318,7 @@ int qlin_probe_clocks(void *stream, double *shader_mhz) {
 }
 
 int qlin_probe_gemm_route(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, int have_workspace) {
+    if (takes_fewtok(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0)) return 3;
     return (int)choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0);
 }
 

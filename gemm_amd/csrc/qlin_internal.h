@@ -103,9 +103,6 @@ hipError_t launch_gemv_q4k(const GemvJob &job, const float *x, int n_cols, hipSt
 hipError_t launch_gemm_f32(uint32_t type, const void *W, const float *X, float *Y, int n_rows,
                            int n_cols, int n_tok, int ldx, int ldy, hipStream_t stream);
 
-/* Q4_K x bf16 on the matrix cores */
-/* the same contraction for a handful of tokens: exact 4-bit codes through the matrix instruction, block
- * scales in fp32, weights streamed once per 16 tokens (moe_ffn_q4k.hip) */
 /* any format: decode to bf16 (dequant.hip), then the dense library GEMM (gemm_dense_lt.hip) */
 hipError_t launch_dequant_bf16(uint32_t type, const void *W, uint16_t *out, int n_rows, int n_cols, size_t row_bytes,
                                hipStream_t stream);
@@ -119,16 +116,34 @@ const char *launch_gemm_dense_bf16(const uint16_t *Wd, const uint16_t *X, float 
  * aligned, ldx % 8 == 0 */
 hipError_t launch_gemm_dense_own(const uint16_t *Wd, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
                                  int ldx, int ldy, hipStream_t stream);
-constexpr int kKqFewTokens = 24; /* up to this many tokens Q6_K, Q5_K, Q3_K, Q2_K and Q8_0 tensors are streamed once per
-                                    eight tokens with exact codes instead of decoded to bf16 for the library's GEMM */
-/* false: not a shape for this kernel (the caller takes another route); true: launched, *err says how it went */
-bool launch_gemm_kq_fewtok(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
-                           int ldx, int ldy, hipStream_t stream, hipError_t *err);
+/* the few-token kernel (gemm_fewtok.h): up to three tensors of one format and row length against the same activations */
+struct FewtokCall {
+    int n_mat; /* 1..3 */
+    const void *const *W;
+    const uint16_t *X;
+    float *const *Y;
+    const int *n_rows;
+    int n_cols, n_tok, ldx;
+    const int *ldy;
+    hipStream_t stream;
+};
+bool fewtok_has(uint32_t type);
+int fewtok_unrounded(uint32_t type); /* token count up to which the codes stay unrounded */
+bool fewtok_takes(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx);
+hipError_t launch_gemm_fewtok(uint32_t type, const FewtokCall &c);
+hipError_t launch_gemm_fewtok_one_by_one(uint32_t type, const FewtokCall &c); /* any ldx */
+hipError_t fewtok_q4k(const FewtokCall &c);
+hipError_t fewtok_q5k(const FewtokCall &c);
+hipError_t fewtok_q6k(const FewtokCall &c);
+hipError_t fewtok_q2k(const FewtokCall &c);
+hipError_t fewtok_q3k(const FewtokCall &c);
+hipError_t fewtok_q8_0(const FewtokCall &c);
+hipError_t fewtok_q4_0(const FewtokCall &c);
+hipError_t fewtok_iq4nl(const FewtokCall &c);
+hipError_t fewtok_iq4xs(const FewtokCall &c);
+hipError_t fewtok_iq3s(const FewtokCall &c);
+hipError_t fewtok_iq2xxs(const FewtokCall &c);
 constexpr int kMatvecTokens = 4; /* qlin_gemm_bf16_any_dev: up to this many tokens of a format without a few-token kernel go through the matvec */
-constexpr int kFewTokens = 32; /* launch_gemm_q4k_bf16 hands token counts up to this to the few-token kernel (14336 x 4096:
-                                  24 us at 32 tokens, 34 at 48; the small-tile kernel 26 for up to 128) */
-hipError_t launch_gemm_q4k_fewtok(const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
-                                  int ldx, int ldy, hipStream_t stream);
 /* 256-token x 128-row tiles on four waves, one per SIMD, weights decoded from their blocks into the matrix operand
  * (gemm_kq_wave4.hip): the formats of gemm_kq_wave4_covers, n_cols % 256 == 0, ldx < 2^22 */
 bool gemm_kq_wave4_covers(uint32_t type);

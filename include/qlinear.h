@@ -235,10 +235,11 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * 513..1024, ...), 128-token x 64-row tiles for smaller shapes (4096-row projections at 512 tokens, any row count at
  * 33..256 tokens). Given a workspace, the decode + dense route still takes the shapes where decoding once measured
  * faster: large-tile shapes above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512 (Q6_K, Q8_0), small-tile
- * shapes of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024. Q4_K up to 32 tokens: the few-token kernel of qlin_gemm_bf16_dev.
- * Up to 24 tokens of a Q6_K, Q5_K, Q3_K, Q2_K or
- * Q8_0 tensor (n_cols % 256 == 0, the tensor's bytes a multiple of 16) also run in one fused kernel with
- * unrounded weights (~1e-6) and leave the workspace alone (it may be NULL then). Up to 4 tokens of any other
+ * shapes of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024.
+ * Up to 64 tokens of these formats (and, given a workspace, of IQ3_S and IQ2_XXS), and up to 128 where a tensor has at most
+ * 5120 rows, run in the few-token kernel (n_cols % 256 == 0, no workspace used), which streams the blocks once: with unrounded
+ * codes (~1e-6) up to 32 tokens of Q4_K, 24 of Q5_K, Q6_K, Q2_K, Q3_K and Q8_0 and 4 of the others, beyond that with the
+ * same single rounding to bf16. Up to 4 tokens of any other
  * block format go one by one through the matvec kernels (exact weights, ~1e-6; the workspace holds their
  * activations as fp32, and when ldx is so wide that (n_tok - 1) * ldx + n_cols floats do not fit it they take the
  * decode + dense route). workspace: device memory, 256-byte aligned, at least
@@ -259,7 +260,7 @@ int qlin_gemm_bf16_any_dev(uint32_t ggml_type, const void *W, const uint16_t *X,
 /* qlin_gemm_bf16_any_dev for one to three weight tensors of ONE format and row length against the same activations:
  * the Q, K and V projections of a prefill chunk, which the reference multiplies tensor by tensor
  * (tf_gemm_f16_mt_tokenmajor per projection, common/transformer.h:5256-5258). Y[i][t * ldy[i] + r] is tensor i's
- * product. Where every tensor on its own would take the same tile kernel (more than 32 tokens of a format with one)
+ * product. Where every tensor on its own would take the same kernel of this library (few-token, small or large tiles)
  * they share one launch, their row tiles numbered through, with the results of one call per tensor bit for bit: a
  * 1024-row K or V projection alone is 64 workgroups of 128 tokens x 64 rows at 512 tokens on 256 compute units (Q4_K
  * 4096 + 1024 + 1024 rows x 4096 at 512 tokens: 36 us in one launch against 24 + 22 + 22). Every other case is one

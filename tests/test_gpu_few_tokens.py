@@ -1,0 +1,85 @@
+"""GPU parity of the few-token product (up to 128 tokens) at the sizes where it can go wrong: every capacity of its
+instances and one token past it, fewer super-blocks than waves, an uneven number per wave, ragged last row tiles, one and
+two row tiles per workgroup, padded X and Y, several tensors in one launch. Unrounded codes are held to 2e-6 (fp32 sums of
+at most 2304 products and their block scales: a few units of 2^-24 each), rounded weights to 2e-5 against weights rounded
+once to bf16, as for the tile kernels."""
+import numpy as np
+import pytest
+
+from gemm_amd import qlinear
+import synth
+from tests.conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+EXACT_MAX = {synth.GGML_Q4_K: 32, synth.GGML_Q5_K: 24, synth.GGML_Q6_K: 24, synth.GGML_Q2_K: 24, synth.GGML_Q3_K: 24,
+             synth.GGML_Q8_0: 24, synth.GGML_Q4_0: 4, synth.GGML_IQ4_NL: 4, synth.GGML_IQ4_XS: 4, synth.GGML_IQ3_S: 4,
+             synth.GGML_IQ2_XXS: 4}
+NAME = synth.TYPE_NAMES
+
+
+GRID = (synth.GGML_IQ3_S, synth.GGML_IQ2_XXS)  # up to 64 tokens
+
+
+def check(oracle, tid, rows_list, n_cols, n_tok, sample=None, pad=8):
+    rng = np.random.default_rng(tid * 1000 + n_tok)
+    Ws = [synth.make_weights(tid, r, n_cols, seed=tid + 7 * i + n_tok) for i, r in enumerate(rows_list)]
+    Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_tok, tokens=n_tok))
+    ldx = n_cols + pad
+    Xpad = np.full((n_tok, ldx), 0x7FC0, np.uint16)  # NaN between the rows: it must not be read into a sum
+    Xpad[:, :n_cols] = Xb
+    dX = qlinear.DevBuf.from_numpy(Xpad)
+    dWs = [qlinear.DevBuf.from_numpy(w) for w in Ws]
+    ldys = [r + 3 for r in rows_list]
+    dYs = [qlinear.DevBuf.from_numpy(np.full((n_tok, ld), -3.0, np.float32)) for ld in ldys]
+    ws = qlinear.DevBuf(max(qlinear.gemm_bf16_any_workspace_bytes(r, n_cols) for r in rows_list))
+    assert qlinear.load().qlin_probe_gemm_route(tid, rows_list[0], n_cols, n_tok, ldx, 1) == 3
+    qlinear.gemm_bf16_multi_dev(tid, dWs, dX, dYs, rows_list, n_cols, n_tok, ldx, ldys, ws)
+    qlinear.sync()
+    Xf = synth.bf16_bits_to_f32(Xb).astype(np.float64)
+    for W, dY, r, ld in zip(Ws, dYs, rows_list, ldys):
+        Y = dY.to_numpy(np.float32, (n_tok, ld))
+        assert np.all(Y[:, r:] == -3.0)
+        at = np.arange(r) if sample is None or r <= 200 else np.unique(np.concatenate([rng.choice(r, sample, replace=False), np.arange(r - 40, r)]))
+        dec = oracle.dequant_matrix(tid, W[at], n_cols)
+        if n_tok > EXACT_MAX[tid]:
+            dec = synth.bf16_bits_to_f32(synth.to_bf16_bits(dec))
+        want = Xf @ dec.astype(np.float64).T
+        assert rel_l2(Y[:, at], want) <= (2e-5 if n_tok > EXACT_MAX[tid] else 2e-6), (NAME[tid], n_tok, r)
+    for b in dWs + dYs + [dX, ws]:
+        b.free()
+
+
+@pytest.mark.parametrize("n_tok", [1, 4, 5, 8, 9, 16, 17, 24, 25, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 128])
+@pytest.mark.parametrize("tid", sorted(EXACT_MAX), ids=lambda t: NAME[t])
+def test_every_capacity(oracle, tid, n_tok):
+    if n_tok <= 64 or tid not in GRID:
+        check(oracle, tid, [37], 2304, n_tok)  # nine super-blocks over eight waves, three row tiles, the last of five rows
+
+
+@pytest.mark.parametrize("n_tok", [3, 8, 16, 24, 32, 48, 64])
+@pytest.mark.parametrize("tid", sorted(EXACT_MAX), ids=lambda t: NAME[t])
+def test_two_row_tiles_per_workgroup(oracle, tid, n_tok):
+    rows, n_cols = ([4663], 768) if n_tok % 16 == 0 else ([4627, 130, 33], 256)
+    check(oracle, tid, rows, n_cols, n_tok, sample=60)
+
+
+@pytest.mark.parametrize("n_tok", [7, 40, 100])
+@pytest.mark.parametrize("tid", sorted(EXACT_MAX), ids=lambda t: NAME[t])
+def test_tensors_of_one_launch_equal_a_call_each(tid, n_tok):
+    """bit for bit, though the joint launch puts two row tiles in a workgroup and a call of its own one"""
+    rows, n_cols = [2500, 2300, 48], 512
+    Ws = [synth.make_weights(tid, r, n_cols, seed=r) for r in rows]
+    dX = qlinear.DevBuf.from_numpy(synth.to_bf16_bits(synth.make_activation(n_cols, seed=3, tokens=n_tok)))
+    ws = qlinear.DevBuf(qlinear.gemm_bf16_any_workspace_bytes(max(rows), n_cols))
+    dWs, got = [qlinear.DevBuf.from_numpy(w) for w in Ws], []
+    for together in (True, False):
+        dYs = [qlinear.DevBuf(n_tok * r * 4) for r in rows]
+        if together:
+            qlinear.gemm_bf16_multi_dev(tid, dWs, dX, dYs, rows, n_cols, n_tok, n_cols, rows, ws)
+        else:
+            for w, y, r in zip(dWs, dYs, rows):
+                qlinear.gemm_bf16_any_dev(tid, w, dX, y, r, n_cols, n_tok, n_cols, r, ws)
+        qlinear.sync()
+        got.append([y.to_numpy(np.uint32, (n_tok, r)) for y, r in zip(dYs, rows)])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
