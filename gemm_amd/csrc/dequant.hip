@@ -1,42 +1,100 @@
 /*
  * dequant.hip - block decoders: raw GGML blocks -> fp32, bit-identical to the reference's
- * scalar decoders (common/ggml_dequant.h:1479-1687, :2793-3058, type switch :3177-3265).
+ * scalar decoders (common/ggml_dequant.h:1479-1687, :2793-3058, type switch :3177-3265),
+ * and the same rounded once to bf16.
  *
- * One thread decodes eight consecutive elements and writes 32 contiguous bytes, so a
- * wavefront writes 2 KiB of contiguous fp32 per store pair. The kernel is bound by that
- * write stream (4 B out per 0.26..1.06 B in).
+ * One thread decodes groups of eight consecutive elements. What bounds the kernels is the stream of stores (4 or 2 B out
+ * per 0.26..1.06 B in) as long as a group costs few instructions: whole rows one after another are taken as one run of
+ * blocks, whose block and place in it are shifts of the thread's index, the codes come in by dword loads and are masked
+ * four at a time. 14336 x 4096, with 64-bit divisions and byte loads before: Q5_K to bf16 52 -> 38 us (158 MB, 4.2 TB/s),
+ * Q6_K to bf16 39 -> 34.5 (165 MB, 4.8 TB/s), to fp32 Q4_K 67 -> 54 (268 MB, 5.0 TB/s), Q6_K 70 -> 46 (5.8 TB/s).
  */
 #include "qlin_device.h"
 #include "qlin_internal.h"
 
 namespace qlin {
 
-template <uint32_t T, bool VEC>
+__device__ __forceinline__ void store8(float *o, const float (&y)[8]) {
+    reinterpret_cast<float4 *>(o)[0] = make_float4(y[0], y[1], y[2], y[3]);
+    reinterpret_cast<float4 *>(o)[1] = make_float4(y[4], y[5], y[6], y[7]);
+}
+__device__ __forceinline__ void store8(uint16_t *o, const float (&y)[8]) {
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+    uint4 v;
+    uint32_t *vp = &v.x;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        bf16x2 r;
+        r[0] = (__bf16)y[2 * i];
+        r[1] = (__bf16)y[2 * i + 1];
+        vp[i] = __builtin_bit_cast(uint32_t, r);
+    }
+    *reinterpret_cast<uint4 *>(o) = v;
+}
+
+/* n_groups groups of eight of one run of blocks; out 16-byte aligned. A workgroup takes 512 groups, a thread two of them
+ * 256 apart, so that each store of the workgroup is part of a contiguous stretch.
+ * fp32: the two float4 of a thread lie 32 bytes from the next thread's, so a wave would write every second 16 bytes of
+ * 2 KB per store; it turns them through its own part of LDS and writes 1 KB in one piece (Q6_K 70 us -> 46, Q4_K 66 -> 54
+ * by that alone). */
+template <uint32_t T, class OUT>
 __global__ void __launch_bounds__(256)
-dequant_kernel(const uint8_t *__restrict__ W, const int32_t *__restrict__ row_ids, int n_src_rows,
-               float *__restrict__ out, int n_rows, int n_cols, size_t row_bytes, int blocks_per_row) {
+dequant_run_kernel(const uint8_t *__restrict__ W, OUT *__restrict__ out, unsigned long long n_groups) {
     using C = Codec<T>;
-    constexpr int GPB = C::BE / 8; /* 8-element groups per block */
-    const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long groups_per_row = (long long)blocks_per_row * GPB;
-    if (gid >= groups_per_row * n_rows) return;
-    const int row = (int)(gid / groups_per_row);
-    const int g = (int)(gid - (long long)row * groups_per_row);
-    const int blk = g / GPB, k0 = (g - blk * GPB) * 8;
+    constexpr unsigned GPB = C::BE / 8; /* groups per block, a power of two */
+    static_assert((GPB & (GPB - 1)) == 0 && 256 % GPB == 0, "blocks do not divide a workgroup's groups");
+    const unsigned long long first = (unsigned long long)blockIdx.x * 512;
+    const uint8_t *w = W + first / GPB * C::BB;
+    OUT *o = out + first * 8;
+    const unsigned left = (unsigned)min(n_groups - first, 512ull);
+#pragma unroll
+    for (unsigned h = 0; h < 2; h++) {
+        const unsigned lane = threadIdx.x & 63u, g0 = threadIdx.x - lane + 256 * h, g = g0 + lane;
+        if (g0 >= left) return;
+        float y[8];
+        if (g < left) C::decode8(w + g / GPB * C::BB, (int)(g % GPB) * 8, y);
+        if constexpr (sizeof(OUT) == 2) {
+            if (g < left) store8(o + g * 8, y);
+        } else {
+            __shared__ float4 turn[256 * 2];
+            float4 *t = turn + (threadIdx.x - lane) * 2;
+            t[2 * lane] = make_float4(y[0], y[1], y[2], y[3]);
+            t[2 * lane + 1] = make_float4(y[4], y[5], y[6], y[7]);
+            __builtin_amdgcn_wave_barrier();
+            float4 *ow = reinterpret_cast<float4 *>(o + g0 * 8);
+            const unsigned n = 2 * min(64u, left - g0);
+            if (lane < n) ow[lane] = t[lane];
+            if (lane + 64 < n) ow[lane + 64] = t[lane + 64];
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+/* row by row: gathered rows, rows that end inside a block, rows at a distance, outputs that are not aligned. `chunks`
+ * workgroups to a row, or several short rows to a workgroup. */
+template <uint32_t T, class OUT, bool VEC>
+__global__ void __launch_bounds__(256)
+dequant_rows_kernel(const uint8_t *__restrict__ W, const int32_t *__restrict__ row_ids, int n_src_rows,
+                    OUT *__restrict__ out, int n_rows, int n_cols, size_t row_bytes, unsigned groups_per_row, unsigned chunks) {
+    using C = Codec<T>;
+    constexpr unsigned GPB = C::BE / 8;
+    const unsigned set = blockIdx.x / chunks, g = (blockIdx.x - set * chunks) * blockDim.x + threadIdx.x;
+    const unsigned row = set * blockDim.y + threadIdx.y;
+    if (row >= (unsigned)n_rows || g >= groups_per_row) return;
+    const unsigned blk = g / GPB, k0 = g % GPB * 8;
     float y[8];
     /* output row `row` is source row row_ids[row] when a list is given (embedding lookup); an id
      * outside the table yields a row of zeros */
-    const int src_row = row_ids ? row_ids[row] : row;
+    const int src_row = row_ids ? row_ids[row] : (int)row;
     if (src_row >= 0 && src_row < n_src_rows) {
-        C::decode8(W + (size_t)src_row * row_bytes + (size_t)blk * C::BB, k0, y);
+        C::decode8(W + (size_t)src_row * row_bytes + (size_t)blk * C::BB, (int)k0, y);
     } else {
 #pragma unroll
         for (int i = 0; i < 8; i++) y[i] = 0.0f;
     }
-    float *o = out + (size_t)row * n_cols + (size_t)blk * C::BE + k0;
-    if (VEC) {
-        reinterpret_cast<float4 *>(o)[0] = make_float4(y[0], y[1], y[2], y[3]);
-        reinterpret_cast<float4 *>(o)[1] = make_float4(y[4], y[5], y[6], y[7]);
+    OUT *o = out + (size_t)row * n_cols + (size_t)blk * C::BE + k0;
+    if constexpr (VEC) {
+        store8(o, y);
     } else {
 #pragma unroll
         for (int i = 0; i < 8; i++) o[i] = y[i];
@@ -68,67 +126,30 @@ convert_plain_kernel(uint32_t type, const uint8_t *__restrict__ src, const int32
     }
 }
 
-/* the same decode with the result rounded once to bf16 (nearest even) and stored 8 values = 16 bytes per
- * thread: the weight operand of the dense matrix-core GEMM */
-template <uint32_t T>
-__global__ void __launch_bounds__(256)
-dequant_bf16_kernel(const uint8_t *__restrict__ W, uint16_t *__restrict__ out, int n_rows, int n_cols,
-                    size_t row_bytes, int blocks_per_row) {
-    using C = Codec<T>;
-    constexpr int GPB = C::BE / 8;
-    /* a thread decodes two 8-element groups half a workgroup's span apart, so that each of its two
-     * 16-byte stores is part of a contiguous 4 KB of the workgroup */
-    const long long groups_per_row = (long long)blocks_per_row * GPB;
-    const long long n_groups = groups_per_row * n_rows;
-    const long long base = (long long)blockIdx.x * 512 + threadIdx.x;
-    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const long long gid = base + 256 * h;
-        if (gid >= n_groups) return;
-        const int row = (int)(gid / groups_per_row);
-        const int g = (int)(gid - (long long)row * groups_per_row);
-        const int blk = g / GPB, k0 = (g - blk * GPB) * 8;
-        float y[8];
-        C::decode8(W + (size_t)row * row_bytes + (size_t)blk * C::BB, k0, y);
-        uint4 v;
-        uint32_t *vp = &v.x;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            bf16x2 r;
-            r[0] = (__bf16)y[2 * i];
-            r[1] = (__bf16)y[2 * i + 1];
-            vp[i] = __builtin_bit_cast(uint32_t, r);
-        }
-        *reinterpret_cast<uint4 *>(out + (size_t)row * n_cols + (size_t)blk * C::BE + k0) = v;
-    }
-}
-
-template <uint32_t T>
-static hipError_t launch_bf16_typed(const void *W, uint16_t *out, int n_rows, int n_cols, size_t row_bytes,
-                                    hipStream_t stream) {
-    const int bpr = n_cols / Codec<T>::BE;
-    const long long groups = (long long)bpr * (Codec<T>::BE / 8) * n_rows;
-    if (groups == 0) return hipSuccess;
-    hipLaunchKernelGGL((dequant_bf16_kernel<T>), dim3((unsigned)((groups + 511) / 512)), dim3(256), 0, stream,
-                       (const uint8_t *)W, out, n_rows, n_cols, row_bytes, bpr);
-    return hipGetLastError();
-}
-
-template <uint32_t T>
-static hipError_t launch_typed(const void *W, const int32_t *row_ids, int n_src_rows, float *out, int n_rows,
+template <uint32_t T, class OUT>
+static hipError_t launch_typed(const void *W, const int32_t *row_ids, int n_src_rows, OUT *out, int n_rows,
                                int n_cols, size_t row_bytes, hipStream_t stream) {
-    const int bpr = n_cols / Codec<T>::BE;
-    const long long groups = (long long)bpr * (Codec<T>::BE / 8) * n_rows;
-    if (groups == 0) return hipSuccess;
-    const unsigned grid = (unsigned)((groups + 255) / 256);
-    const bool vec = (n_cols % 4 == 0) && ((reinterpret_cast<uintptr_t>(out) & 15u) == 0);
-    if (vec)
-        hipLaunchKernelGGL((dequant_kernel<T, true>), dim3(grid), dim3(256), 0, stream,
-                           (const uint8_t *)W, row_ids, n_src_rows, out, n_rows, n_cols, row_bytes, bpr);
-    else
-        hipLaunchKernelGGL((dequant_kernel<T, false>), dim3(grid), dim3(256), 0, stream,
-                           (const uint8_t *)W, row_ids, n_src_rows, out, n_rows, n_cols, row_bytes, bpr);
+    using C = Codec<T>;
+    const size_t bpr = n_cols / C::BE, groups_per_row = bpr * (C::BE / 8);
+    if (groups_per_row == 0 || n_rows == 0) return hipSuccess;
+    const bool aligned = (reinterpret_cast<uintptr_t>(out) & 15u) == 0;
+    if (!row_ids && aligned && (n_rows == 1 || ((size_t)n_cols == bpr * C::BE && row_bytes == bpr * C::BB))) {
+        const unsigned long long n = (unsigned long long)groups_per_row * n_rows;
+        hipLaunchKernelGGL((dequant_run_kernel<T, OUT>), dim3((unsigned)((n + 511) / 512)), dim3(256), 0, stream,
+                           (const uint8_t *)W, out, n);
+        return hipGetLastError();
+    }
+    unsigned wide = 1;
+    while (wide < 256 && wide < groups_per_row) wide *= 2;
+    const unsigned tall = 256 / wide, chunks = (unsigned)((groups_per_row + wide - 1) / wide);
+    const dim3 grid(chunks * (((unsigned)n_rows + tall - 1) / tall)), wg(wide, tall);
+    if (sizeof(OUT) == 2 || (n_cols % 4 == 0 && aligned)) {
+        hipLaunchKernelGGL((dequant_rows_kernel<T, OUT, true>), grid, wg, 0, stream, (const uint8_t *)W, row_ids,
+                           n_src_rows, out, n_rows, n_cols, row_bytes, (unsigned)groups_per_row, chunks);
+    } else if constexpr (sizeof(OUT) == 4) {
+        hipLaunchKernelGGL((dequant_rows_kernel<T, OUT, false>), grid, wg, 0, stream, (const uint8_t *)W, row_ids,
+                           n_src_rows, out, n_rows, n_cols, row_bytes, (unsigned)groups_per_row, chunks);
+    }
     return hipGetLastError();
 }
 
@@ -154,7 +175,7 @@ hipError_t launch_dequant(uint32_t type, const void *W, const int32_t *row_ids, 
 hipError_t launch_dequant_bf16(uint32_t type, const void *W, uint16_t *out, int n_rows, int n_cols, size_t row_bytes,
                                hipStream_t stream) {
     switch (type) {
-#define QLIN_CASE(TT) case TT: return launch_bf16_typed<TT>(W, out, n_rows, n_cols, row_bytes, stream);
+#define QLIN_CASE(TT) case TT: return launch_typed<TT>(W, nullptr, n_rows, out, n_rows, n_cols, row_bytes, stream);
     QLIN_FOR_EACH_BLOCK_TYPE(QLIN_CASE)
     QLIN_FOR_EACH_DENSE_TYPE(QLIN_CASE)
 #undef QLIN_CASE

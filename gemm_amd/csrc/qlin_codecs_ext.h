@@ -39,10 +39,9 @@ __device__ __forceinline__ float sign_pm1(uint32_t bit) { return bit ? -1.0f : 1
 template <> struct Codec<T_Q4_0> : Geom<T_Q4_0> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk));
-        const uint8_t *q = blk + 2 + (k0 & 15);
-        const int sh = (k0 >> 4) * 4;
+        const Dwords2 q = bytes_at(ld_2xu32(blk + 2 + (k0 & 15)), (k0 >> 4) * 4, 15u);
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = (float)((int)((q[i] >> sh) & 15) - 8) * d;
+        for (int i = 0; i < 8; i++) y[i] = (byte_f32(q, i) - 8.0f) * d;
     }
 };
 
@@ -50,10 +49,9 @@ template <> struct Codec<T_Q4_0> : Geom<T_Q4_0> {
 template <> struct Codec<T_Q4_1> : Geom<T_Q4_1> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk)), m = half_bits_exact(ld_u16(blk + 2));
-        const uint8_t *q = blk + 4 + (k0 & 15);
-        const int sh = (k0 >> 4) * 4;
+        const Dwords2 q = bytes_at(ld_2xu32(blk + 4 + (k0 & 15)), (k0 >> 4) * 4, 15u);
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = (float)((q[i] >> sh) & 15) * d + m;
+        for (int i = 0; i < 8; i++) y[i] = byte_f32(q, i) * d + m;
     }
 };
 
@@ -62,13 +60,9 @@ template <> struct Codec<T_Q5_0> : Geom<T_Q5_0> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk));
         const uint32_t hb = blk[2 + (k0 >> 3)]; /* the eight fifth bits of this group */
-        const uint8_t *q = blk + 6 + (k0 & 15);
-        const int sh = (k0 >> 4) * 4;
+        const Dwords2 q = bytes_at(ld_2xu32(blk + 6 + (k0 & 15)), (k0 >> 4) * 4, 15u);
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int v = (int)(((q[i] >> sh) & 15) | (((hb >> i) & 1u) << 4));
-            y[i] = (float)(v - 16) * d;
-        }
+        for (int i = 0; i < 8; i++) y[i] = (byte_f32(q, i) - (((hb >> i) & 1u) ? 0.0f : 16.0f)) * d;
     }
 };
 
@@ -77,13 +71,9 @@ template <> struct Codec<T_Q5_1> : Geom<T_Q5_1> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk)), m = half_bits_exact(ld_u16(blk + 2));
         const uint32_t hb = blk[4 + (k0 >> 3)];
-        const uint8_t *q = blk + 8 + (k0 & 15);
-        const int sh = (k0 >> 4) * 4;
+        const Dwords2 q = bytes_at(ld_2xu32(blk + 8 + (k0 & 15)), (k0 >> 4) * 4, 15u);
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int v = (int)(((q[i] >> sh) & 15) | (((hb >> i) & 1u) << 4));
-            y[i] = (float)v * d + m;
-        }
+        for (int i = 0; i < 8; i++) y[i] = (byte_f32(q, i) + (((hb >> i) & 1u) ? 16.0f : 0.0f)) * d + m;
     }
 };
 
@@ -139,13 +129,14 @@ template <> struct Codec<T_Q1_0> : Geom<T_Q1_0> {
 /* Q2_K [scales 16][qs 64][d][dmin]: (d*(sc&15))*q2 - dmin*(sc>>4)   (:1505-1534) */
 template <> struct Codec<T_Q2_K> : Geom<T_Q2_K> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
-        const float d = half_bits_exact(ld_u16(blk + 80)), dmin = half_bits_exact(ld_u16(blk + 82));
+        const uint32_t dd = ld_u32(blk + 80);
+        const float d = half_bits_exact(dd & 0xFFFFu), dmin = half_bits_exact(dd >> 16);
         const int half = k0 >> 7, j = (k0 >> 5) & 3, sub = (k0 >> 4) & 1, l0 = k0 & 15;
         const uint32_t sc = blk[8 * half + 2 * j + sub];
         const float dl = d * (float)(sc & 15u), ml = dmin * (float)(sc >> 4);
-        const uint8_t *q = blk + 16 + 32 * half + 16 * sub + l0;
+        const Dwords2 q = bytes_at(ld_2xu32(blk + 16 + 32 * half + 16 * sub + l0), 2 * j, 3u);
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = dl * (float)((q[i] >> (2 * j)) & 3) - ml;
+        for (int i = 0; i < 8; i++) y[i] = dl * byte_f32(q, i) - ml;
     }
 };
 
@@ -158,17 +149,15 @@ template <> struct Codec<T_Q3_K> : Geom<T_Q3_K> {
         const int half = k0 >> 7, j = (k0 >> 5) & 3, sub = (k0 >> 4) & 1, l0 = k0 & 15;
         const int is = 8 * half + 2 * j + sub;
         const uint8_t *s = blk + 96;
-        const int lo4 = is < 8 ? (s[is] & 15) : (s[is - 8] >> 4);
+        const int lo4 = (s[is & 7] >> (is < 8 ? 0 : 4)) & 15;
         const int hi2 = (s[8 + (is & 3)] >> (2 * (is >> 2))) & 3;
         const float dl = d * (float)((lo4 | (hi2 << 4)) - 32);
-        const uint8_t *q = blk + 32 + 32 * half + 16 * sub + l0;
-        const uint8_t *hm = blk + 16 * sub + l0;
-        const int hsh = 4 * half + j;
+        const Dwords2 h = bytes_at(ld_2xu32(blk + 16 * sub + l0), 4 * half + j, 1u);
+        Dwords2 q = bytes_at(ld_2xu32(blk + 32 + 32 * half + 16 * sub + l0), 2 * j, 3u);
+        q.x |= h.x << 2;
+        q.y |= h.y << 2;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int v = (int)((q[i] >> (2 * j)) & 3) - (((hm[i] >> hsh) & 1) ? 0 : 4);
-            y[i] = dl * (float)v;
-        }
+        for (int i = 0; i < 8; i++) y[i] = dl * (byte_f32(q, i) - 4.0f);
     }
 };
 
@@ -196,14 +185,15 @@ template <> struct Codec<T_IQ3_XXS> : Geom<T_IQ3_XXS> {
  * bits 2g,2g+1 of scales_h; (d*(ls-32)) * iq4nl[nibble]   (:2956-2973) */
 template <> struct Codec<T_IQ4_XS> : Geom<T_IQ4_XS> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
-        const float d = half_bits_exact(ld_u16(blk));
         const int g = k0 >> 5, r = k0 & 31;
-        const int ls = (int)(((blk[4 + (g >> 1)] >> (4 * (g & 1))) & 15) | (((ld_u16(blk + 2) >> (2 * g)) & 3u) << 4));
+        const Dwords2 hd = ld_2xu32(blk);
+        const float d = half_bits_exact(hd.x & 0xFFFFu);
+        const int ls = (int)(((hd.y >> (4 * g)) & 15u) | (((hd.x >> (16 + 2 * g)) & 3u) << 4));
         const float dl = d * (float)(ls - 32);
-        const uint8_t *q = blk + 8 + 16 * g + (r & 15);
-        const int sh = (r >> 4) * 4;
+        const Dwords2 n = bytes_at(ld_2xu32(blk + 8 + 16 * g + (r & 15)), (r >> 4) * 4, 15u);
+        const Dwords2 q = {iq4_table_bytes(n.x), iq4_table_bytes(n.y)};
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = dl * (float)qlin_iq4nl_values[(q[i] >> sh) & 15];
+        for (int i = 0; i < 8; i++) y[i] = dl * (byte_f32(q, i) - 128.0f);
     }
 };
 
@@ -304,10 +294,9 @@ template <> struct Codec<T_TQ1_0> : Geom<T_TQ1_0> {
 template <> struct Codec<T_TQ2_0> : Geom<T_TQ2_0> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk + 64));
-        const uint8_t *q = blk + 32 * (k0 >> 7) + (k0 & 31);
-        const int sh = 2 * ((k0 >> 5) & 3);
+        const Dwords2 q = bytes_at(ld_2xu32(blk + 32 * (k0 >> 7) + (k0 & 31)), 2 * ((k0 >> 5) & 3), 3u);
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = (float)((int)((q[i] >> sh) & 3) - 1) * d;
+        for (int i = 0; i < 8; i++) y[i] = (byte_f32(q, i) - 1.0f) * d;
     }
 };
 

@@ -79,6 +79,38 @@ __device__ __forceinline__ uint32_t ld_u16(const uint8_t *p) {
 __device__ __forceinline__ uint32_t ld_u32_a2(const uint8_t *p) { /* 2-byte aligned dword */
     return ld_u16(p) | (ld_u16(p + 2) << 16);
 }
+/* dwords from any address, one load instruction each: a decoder that loads its codes by the byte issues eight times the
+ * loads, and masks and converts each by itself (dequant.hip has the figures) */
+struct Dwords2 { uint32_t x, y; };
+struct Dwords4 { uint32_t x, y, z, w; };
+__device__ __forceinline__ uint32_t ld_u32(const uint8_t *p) {
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+__device__ __forceinline__ Dwords2 ld_2xu32(const uint8_t *p) {
+    Dwords2 v;
+    __builtin_memcpy(&v, p, 8);
+    return v;
+}
+__device__ __forceinline__ Dwords4 ld_4xu32(const uint8_t *p) {
+    Dwords4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+/* byte i (0..7) of two dwords, as a float */
+__device__ __forceinline__ float byte_f32(const Dwords2 &v, int i) { return (float)(((i < 4 ? v.x : v.y) >> (8 * (i & 3))) & 255u); }
+/* bits `mask` (of every byte) of the bytes shifted right by sh */
+__device__ __forceinline__ Dwords2 bytes_at(const Dwords2 &v, int sh, uint32_t mask) {
+    return Dwords2{(v.x >> sh) & (mask * 0x01010101u), (v.y >> sh) & (mask * 0x01010101u)};
+}
+/* the 16-entry table of IQ4_NL and IQ4_XS for four nibbles, with 128 added */
+__device__ __forceinline__ uint32_t iq4_table_bytes(uint32_t nib) {
+    const uint32_t i7 = nib & 0x07070707u;
+    const uint32_t lo = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, i7), hi = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, i7);
+    const uint32_t m = ((nib >> 3) & 0x01010101u) * 255u;
+    return (m & hi) | (~m & lo);
+}
 
 /* hardware conversion: exact for every finite input (subnormals included) and for infinities;
  * quiets a signalling NaN */
@@ -104,16 +136,15 @@ __device__ __forceinline__ uint32_t iq_sign_byte(uint32_t i7) {
     return i7 | ((__popc(i7) & 1u) << 7);
 }
 
-/* 6-bit scale and min of sub-block g from the 12 packed bytes of a Q4_K/Q5_K super-block
- * (get_scale_min_k4, common/ggml_dequant.h:1582-1590) */
-__device__ __forceinline__ void k4_scale_min(const uint8_t *s, int g, uint32_t &sc, uint32_t &mn) {
-    if (g < 4) {
-        sc = s[g] & 63u;
-        mn = s[g + 4] & 63u;
-    } else {
-        sc = (s[g + 4] & 15u) | ((uint32_t)(s[g - 4] >> 6) << 4);
-        mn = ((uint32_t)s[g + 4] >> 4) | ((uint32_t)(s[g] >> 6) << 4);
-    }
+/* d * scale and dmin * min of sub-block g from the 16-byte header of a Q4_K/Q5_K super-block (get_scale_min_k4,
+ * common/ggml_dequant.h:1582-1590): [d][dmin][12 packed bytes] */
+__device__ __forceinline__ void k4_scales(const Dwords4 &h, int g, float &dl, float &ml) {
+    const int at = 8 * (g & 3);
+    const uint32_t top_sc = (h.y >> (at + 6)) & 3u, top_mn = (h.z >> (at + 6)) & 3u, both = h.w >> at;
+    const uint32_t sc = g < 4 ? (h.y >> at) & 63u : (both & 15u) | (top_sc << 4);
+    const uint32_t mn = g < 4 ? (h.z >> at) & 63u : ((both >> 4) & 15u) | (top_mn << 4);
+    dl = half_bits_exact(h.x & 0xFFFFu) * (float)sc;
+    ml = half_bits_exact(h.x >> 16) * (float)mn;
 }
 
 /*
@@ -133,43 +164,34 @@ template <uint32_t T> struct Codec;
 template <> struct Codec<T_Q8_0> : Geom<T_Q8_0> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk));
-        const int8_t *q = reinterpret_cast<const int8_t *>(blk + 2 + k0);
+        const Dwords2 q = ld_2xu32(blk + 2 + k0);
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = d * (float)q[i];
+        for (int i = 0; i < 8; i++) y[i] = d * (float)(int)(int8_t)((i < 4 ? q.x : q.y) >> (8 * (i & 3)));
     }
 };
 
 template <> struct Codec<T_Q4_K> : Geom<T_Q4_K> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
-        const float d = half_bits_exact(ld_u16(blk));
-        const float dmin = half_bits_exact(ld_u16(blk + 2));
         const int g = k0 >> 5, l0 = k0 & 31;
-        uint32_t sc, mn;
-        k4_scale_min(blk + 4, g, sc, mn);
-        const float dl = d * (float)sc, ml = dmin * (float)mn;
-        const uint8_t *q = blk + 16 + (g >> 1) * 32 + l0;
-        const int sh = (g & 1) * 4;
+        float dl, ml;
+        k4_scales(ld_4xu32(blk), g, dl, ml);
+        const Dwords2 q = bytes_at(ld_2xu32(blk + 16 + (g >> 1) * 32 + l0), (g & 1) * 4, 15u);
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = dl * (float)((q[i] >> sh) & 15) - ml;
+        for (int i = 0; i < 8; i++) y[i] = dl * byte_f32(q, i) - ml;
     }
 };
 
 template <> struct Codec<T_Q5_K> : Geom<T_Q5_K> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
-        const float d = half_bits_exact(ld_u16(blk));
-        const float dmin = half_bits_exact(ld_u16(blk + 2));
         const int g = k0 >> 5, l0 = k0 & 31;
-        uint32_t sc, mn;
-        k4_scale_min(blk + 4, g, sc, mn);
-        const float dl = d * (float)sc, ml = dmin * (float)mn;
-        const uint8_t *qh = blk + 16 + l0;
-        const uint8_t *q = blk + 48 + (g >> 1) * 32 + l0;
-        const int sh = (g & 1) * 4;
+        float dl, ml;
+        k4_scales(ld_4xu32(blk), g, dl, ml);
+        const Dwords2 h = bytes_at(ld_2xu32(blk + 16 + l0), g, 1u);
+        Dwords2 q = bytes_at(ld_2xu32(blk + 48 + (g >> 1) * 32 + l0), (g & 1) * 4, 15u);
+        q.x |= h.x << 4;
+        q.y |= h.y << 4;
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int v = ((q[i] >> sh) & 15) + (((qh[i] >> g) & 1) << 4);
-            y[i] = dl * (float)v - ml;
-        }
+        for (int i = 0; i < 8; i++) y[i] = dl * byte_f32(q, i) - ml;
     }
 };
 
@@ -180,28 +202,24 @@ template <> struct Codec<T_Q6_K> : Geom<T_Q6_K> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk + 208));
         const int half = k0 >> 7, r = k0 & 127, seg = r >> 5, l0 = r & 31;
-        const uint8_t *ql = blk + 64 * half + 32 * (seg & 1) + l0;
-        const uint8_t *qh = blk + 128 + 32 * half + l0;
         const int8_t sc = reinterpret_cast<const int8_t *>(blk + 192)[8 * half + 2 * seg + (l0 >> 4)];
         const float dl = d * (float)sc;
-        const int nsh = (seg >> 1) * 4, hsh = 2 * seg;
+        const Dwords2 h = bytes_at(ld_2xu32(blk + 128 + 32 * half + l0), 2 * seg, 3u);
+        Dwords2 q = bytes_at(ld_2xu32(blk + 64 * half + 32 * (seg & 1) + l0), (seg >> 1) * 4, 15u);
+        q.x |= h.x << 4;
+        q.y |= h.y << 4;
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const uint32_t lo = ld_u32_a2(ql + 4 * j), hi = ld_u32_a2(qh + 4 * j);
-            const uint32_t q4 = ((lo >> nsh) & 0x0F0F0F0Fu) | (((hi >> hsh) & 0x03030303u) << 4);
-#pragma unroll
-            for (int i = 0; i < 4; i++) y[4 * j + i] = dl * ((float)((q4 >> (8 * i)) & 255u) - 32.0f);
-        }
+        for (int i = 0; i < 8; i++) y[i] = dl * (byte_f32(q, i) - 32.0f);
     }
 };
 
 template <> struct Codec<T_IQ4_NL> : Geom<T_IQ4_NL> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk));
-        const uint8_t *q = blk + 2 + (k0 & 15);
-        const int sh = (k0 >> 4) * 4;
+        const Dwords2 n = bytes_at(ld_2xu32(blk + 2 + (k0 & 15)), (k0 >> 4) * 4, 15u);
+        const Dwords2 q = {iq4_table_bytes(n.x), iq4_table_bytes(n.y)};
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = d * (float)qlin_iq4nl_values[(q[i] >> sh) & 15];
+        for (int i = 0; i < 8; i++) y[i] = d * (byte_f32(q, i) - 128.0f);
     }
 };
 
@@ -209,7 +227,8 @@ template <> struct Codec<T_IQ2_XXS> : Geom<T_IQ2_XXS> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = half_bits_exact(ld_u16(blk));
         const int g = k0 >> 5, l = (k0 & 31) >> 3;
-        const uint32_t a0 = ld_u32_a2(blk + 2 + 8 * g), a1 = ld_u32_a2(blk + 6 + 8 * g);
+        const Dwords2 a = ld_2xu32(blk + 2 + 8 * g);
+        const uint32_t a0 = a.x, a1 = a.y;
         const float db = d * (0.5f + (float)(a1 >> 28)) * 0.25f;
         const uint64_t cell = qlin_iq2xxs_grid[(a0 >> (8 * l)) & 255u];
         const uint32_t sg = iq_sign_byte((a1 >> (7 * l)) & 127u);
@@ -228,8 +247,9 @@ template <> struct Codec<T_IQ3_S> : Geom<T_IQ3_S> {
         const uint32_t nib = (blk[106 + (g >> 1)] >> (4 * (g & 1))) & 15u;
         const float db = d * (float)(1u + 2u * nib);
         const uint32_t qh = blk[66 + g];
-        const uint32_t i0 = blk[2 + 8 * g + 2 * l] | (((qh >> (2 * l)) & 1u) << 8);
-        const uint32_t i1 = blk[2 + 8 * g + 2 * l + 1] | (((qh >> (2 * l + 1)) & 1u) << 8);
+        const uint32_t ix = ld_u16(blk + 2 + 8 * g + 2 * l);
+        const uint32_t i0 = (ix & 255u) | (((qh >> (2 * l)) & 1u) << 8);
+        const uint32_t i1 = (ix >> 8) | (((qh >> (2 * l + 1)) & 1u) << 8);
         const uint32_t c0 = qlin_iq3s_grid[i0], c1 = qlin_iq3s_grid[i1];
         const uint32_t sb = blk[74 + 4 * g + l];
 #pragma unroll
