@@ -1197,6 +1197,11 @@ int qlin_gemm_f32_any_dev(uint32_t type, const void *W, const float *X, float *Y
     }
     if (!workspace || !aligned(workspace, 256) || workspace_bytes < qlin_gemm_f32_any_workspace_bytes(n_rows, n_cols))
         return fail(QLIN_ERR_ARG, "workspace must be 256-byte aligned and hold qlin_gemm_f32_any_workspace_bytes(n_rows, n_cols) bytes");
+    if (f32_split_takes(type, n_rows, n_cols, n_tok, workspace_bytes)) {
+        const F32SplitCall c = {W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, workspace, workspace_bytes, (hipStream_t)stream};
+        HIP_TRY(launch_gemm_f32_split(type, c));
+        return QLIN_OK;
+    }
     const float *Wd = (const float *)W; /* fp32 weights are used where they are */
     if (type != T_F32) {
         HIP_TRY(launch_dequant(type, W, nullptr, n_rows, (float *)workspace, n_rows, n_cols, row_size(type, n_cols),

@@ -143,6 +143,38 @@ hipError_t fewtok_iq4nl(const FewtokCall &c);
 hipError_t fewtok_iq4xs(const FewtokCall &c);
 hipError_t fewtok_iq3s(const FewtokCall &c);
 hipError_t fewtok_iq2xxs(const FewtokCall &c);
+/* fp32 products without rounding on the matrix cores, activations as two fp16 numbers (gemm_f32_split.h) */
+constexpr int kF32NotFinite = 1 << 20; /* in place of a token's power of two */
+struct F32SplitCall {
+    const void *W;
+    const float *X;
+    float *Y;
+    int n_rows, n_cols, n_tok, ldx, ldy;
+    void *workspace;
+    size_t workspace_bytes;
+    hipStream_t stream;
+};
+/* token tiles of 32 token_blocks tokens, K in `parts` parts, and where the workspace holds what (fragments first) */
+struct F32SplitPlan {
+    bool fits;
+    int token_blocks, token_tiles, parts;
+    size_t sums_at, exp_at, parts_at;
+};
+F32SplitPlan f32_split_plan(uint32_t type, int n_rows, int n_cols, int n_tok, size_t workspace_bytes);
+bool f32_split_takes(uint32_t type, int n_rows, int n_cols, int n_tok, size_t workspace_bytes);
+hipError_t launch_gemm_f32_split(uint32_t type, const F32SplitCall &c);
+hipError_t launch_f32_split(const F32SplitCall &c, const F32SplitPlan &p, int sum_group);
+hipError_t f32_split_q4k(const F32SplitCall &c);
+hipError_t f32_split_q5k(const F32SplitCall &c);
+hipError_t f32_split_q6k(const F32SplitCall &c);
+hipError_t f32_split_q2k(const F32SplitCall &c);
+hipError_t f32_split_q3k(const F32SplitCall &c);
+hipError_t f32_split_q8_0(const F32SplitCall &c);
+hipError_t f32_split_q4_0(const F32SplitCall &c);
+hipError_t f32_split_iq4nl(const F32SplitCall &c);
+hipError_t f32_split_iq4xs(const F32SplitCall &c);
+hipError_t f32_split_iq3s(const F32SplitCall &c);
+hipError_t f32_split_iq2xxs(const F32SplitCall &c);
 constexpr int kMatvecTokens = 4; /* qlin_gemm_bf16_any_dev: up to this many tokens of a format without a few-token kernel go through the matvec */
 /* 256-token x 128-row tiles on four waves, one per SIMD, weights decoded from their blocks into the matrix operand
  * (gemm_kq_wave4.hip): the formats of gemm_kq_wave4_covers, n_cols % 256 == 0, ldx < 2^22 */

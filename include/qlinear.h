@@ -273,10 +273,12 @@ int qlin_gemm_bf16_multi_dev(uint32_t ggml_type, int n_mat, const void *const *W
  * Vector-ALU kernel, no workspace: the choice for a few tokens. */
 int qlin_gemm_f32_dev(uint32_t ggml_type, const void *W, const float *X, float *Y, int n_rows,
                       int n_cols, int n_tok, int ldx, int ldy, void *stream);
-/* The fp32 contraction for many tokens, any supported type: W is decoded once to fp32 (bit-exact, as
- * qlin_dequant_dev) into `workspace` and multiplied by the vendor library's dense fp32 GEMM (fp32 operands,
- * fp32 accumulation on the matrix cores) -- what tf_gemm_f16_mt_tokenmajor (common/transformer.h:4487)
- * computes for fp32 activations, without the 16-bit rounding of its fast paths. Relative L2 against a
+/* The fp32 contraction for many tokens, any supported type: what tf_gemm_f16_mt_tokenmajor (common/transformer.h:4487)
+ * computes for fp32 activations, without the 16-bit rounding of its fast paths. Q4_K, Q5_K, Q6_K, Q2_K, Q3_K, Q8_0, Q4_0,
+ * IQ4_NL, IQ4_XS, IQ3_S and IQ2_XXS with n_cols a multiple of 256, from about 2 M weights on, multiply their codes as they
+ * are with activations carried as two fp16 numbers (24 bits) on the matrix cores; everything else is decoded once to fp32
+ * (bit-exact, as qlin_dequant_dev) into `workspace` and multiplied by the vendor library's dense fp32 GEMM. fp32
+ * accumulation either way; the same call takes the same route each time. Relative L2 against a
  * double-precision reference <= 1e-5. Fewer than 8 tokens run the kernel of qlin_gemm_f32_dev and leave the
  * workspace alone (it may then be NULL). workspace: device memory, 256-byte aligned, at least
  * qlin_gemm_f32_any_workspace_bytes(n_rows, n_cols) bytes (4 bytes per weight + 32 MiB for the library);

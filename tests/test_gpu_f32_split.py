@@ -1,0 +1,80 @@
+"""GPU parity of the fp32 product on the matrix cores (activations as two fp16 numbers, codes unrounded) at the sizes where
+it can go wrong: one and two blocks of 32 tokens and one token past them, ragged row tiles, one super-block and more than
+there are parts, K in one part and in several, workspaces that hold only some of the tokens, rows of X at any alignment,
+tokens of very different magnitude, infinities and NaN; and one shape just too small for it. Bar 1e-6: an activation keeps 2^-24 of itself (6e-8), the sums are
+fp32 sums over at most 256 products and 64 super-blocks."""
+import numpy as np
+import pytest
+
+from gemm_amd import qlinear
+import synth
+from tests.conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+TYPES = (synth.GGML_Q4_K, synth.GGML_Q5_K, synth.GGML_Q6_K, synth.GGML_Q2_K, synth.GGML_Q3_K, synth.GGML_Q8_0, synth.GGML_Q4_0,
+         synth.GGML_IQ4_NL, synth.GGML_IQ4_XS, synth.GGML_IQ3_S, synth.GGML_IQ2_XXS)
+NAME = synth.TYPE_NAMES
+TOL = 1e-6
+
+
+def product(tid, W, X, n_rows, n_cols, pad=0, ldy=None):
+    n_tok, ldx, ldy = X.shape[0], n_cols + pad, ldy or n_rows
+    Xpad = np.full((n_tok, ldx), np.nan, np.float32)  # NaN between the rows: it must not be read into a sum
+    Xpad[:, :n_cols] = X
+    dW, dX = qlinear.DevBuf.from_numpy(W), qlinear.DevBuf.from_numpy(Xpad)
+    dY = qlinear.DevBuf.from_numpy(np.full((n_tok, ldy), -3.0, np.float32))
+    ws = qlinear.DevBuf(qlinear.gemm_f32_any_workspace_bytes(n_rows, n_cols))
+    qlinear.gemm_f32_any_dev(tid, dW, dX, dY, n_rows, n_cols, n_tok, ldx, ldy, ws)
+    qlinear.sync()
+    Y = dY.to_numpy(np.float32, (n_tok, ldy))
+    for b in (dW, dX, dY, ws):
+        b.free()
+    assert np.all(Y[:, n_rows:] == -3.0)
+    return Y[:, :n_rows]
+
+
+def check(oracle, tid, n_tok, n_rows, n_cols, pad=0):
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid + n_tok + n_rows)
+    X = synth.make_activation(n_cols, seed=n_tok + n_cols, tokens=n_tok)
+    Y = product(tid, W, X, n_rows, n_cols, pad, n_rows + 3)
+    want = X.astype(np.float64) @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T
+    assert rel_l2(Y, want) <= TOL, (NAME[tid], n_tok, n_rows, n_cols, rel_l2(Y, want))
+
+
+@pytest.mark.parametrize("n_tok,n_rows,n_cols,pad", [(8, 8229, 256, 0), (32, 1025, 2304, 4), (33, 3077, 768, 1), (65, 2305, 1024, 6),
+                                                     (64, 2303, 1024, 0)])
+@pytest.mark.parametrize("tid", TYPES, ids=lambda t: NAME[t])
+def test_edges(oracle, tid, n_tok, n_rows, n_cols, pad):
+    check(oracle, tid, n_tok, n_rows, n_cols, pad)
+
+
+@pytest.mark.parametrize("tid", (synth.GGML_Q4_K, synth.GGML_Q6_K), ids=lambda t: NAME[t])
+@pytest.mark.parametrize("n_tok,n_rows,n_cols", [(1000, 147, 16384), (64, 16384, 512), (1025, 9300, 256)])
+def test_divisions(oracle, tid, n_tok, n_rows, n_cols):
+    """tokens in chunks (three quarters of the first shape's workspace hold 460); enough tiles for one part; many token tiles"""
+    check(oracle, tid, n_tok, n_rows, n_cols)
+
+
+@pytest.mark.parametrize("tid", (synth.GGML_Q5_K, synth.GGML_Q8_0, synth.GGML_Q2_K), ids=lambda t: NAME[t])
+@pytest.mark.parametrize("n_rows", (4700, 70000))
+def test_magnitudes_and_not_finite(oracle, tid, n_rows):
+    """each token keeps its own precision whatever its size, up to the largest floats and down to subnormals; one that holds
+    an infinity or a NaN gives what the plain sum gives and leaves its neighbours alone (few and many rows: K in parts, in one)"""
+    n_cols, n_tok = 512, 40
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid)
+    X = synth.make_activation(n_cols, seed=9, tokens=n_tok)
+    sizes = {0: 1e30, 1: 1e-30, 2: 3e-42, 3: 65504.0, 4: 0.0, 5: 1e-4, 38: 2e33}
+    for t, s in sizes.items():
+        X[t] *= np.float32(s)
+    X[10, 100], X[11, 7], X[39, 511] = np.inf, np.nan, -np.inf
+    Y = product(tid, W, X, n_rows, n_cols)
+    at = np.r_[0:50, n_rows - 50:n_rows]
+    with np.errstate(invalid="ignore"):
+        want = X.astype(np.float64) @ oracle.dequant_matrix(tid, W[at], n_cols).astype(np.float64).T
+    Y = Y[:, at]
+    for t in range(n_tok):
+        if np.all(np.isfinite(X[t])):
+            bar = TOL * np.linalg.norm(want[t]) + np.sqrt(len(at)) * 2.0 ** -149  # (a result cannot be finer than a subnormal)
+            assert np.linalg.norm(Y[t] - want[t]) <= bar, t
+        else:
+            assert np.array_equal(np.isnan(Y[t]), np.isnan(want[t])) and np.array_equal(np.isposinf(Y[t]), np.isposinf(want[t])), t
