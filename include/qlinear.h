@@ -233,7 +233,7 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * decoded inside the product by this library's tile kernels, with the same single rounding to bf16, and leave the workspace alone (it may be NULL
  * for them): 256-token x 128-row tiles where 200 or more of them fill the chip (12800 rows at 257..512 tokens, 6400 at
  * 513..1024, ...), 128-token x 64-row tiles for smaller shapes (4096-row projections at 512 tokens, any row count at
- * 33..256 tokens). Given a workspace, the decode + dense route still takes the shapes where decoding once measured
+ * 65..256 tokens). Given a workspace, the decode + dense route still takes the shapes where decoding once measured
  * faster: large-tile shapes above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512 (Q6_K, Q8_0), small-tile
  * shapes of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024.
  * Up to 64 tokens of these formats (and, given a workspace, of IQ3_S and IQ2_XXS), and up to 128 where a tensor has at most

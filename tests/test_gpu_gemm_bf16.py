@@ -17,7 +17,7 @@ from tests.conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
 Q4K = synth.GGML_Q4_K
-FEW_TOKENS = 32  # kFewTokens of the library: up to here the weights stay exact
+FEW_TOKENS = 32  # fewtok_unrounded of the library for Q4_K: up to here the weights stay exact
 
 
 def run_gemm(W, Xb, n_rows, n_cols, n_tok, ldx=None, ldy=None):
