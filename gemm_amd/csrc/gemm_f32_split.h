@@ -177,7 +177,9 @@ gemm_f32_split_kernel(SplitArgs p) {
                    img_at = (uint32_t)(uintptr_t)(lds_void *)img;
 
     /* weights: as in the few-token kernel, piece 64 q + lane of the image is part id % kPieces of row id / kPieces */
-    auto w_rsrc = [&](bool any) { /* past the last super-block the requests are made all the same, and touch no memory */
+    /* Past the part's last super-block the requests are made all the same, so that they stay countable, and touch no memory: a
+     * buffer of no bytes, read from its start - every offset is past its end, whichever way a scalar offset is counted */
+    auto w_rsrc = [&](bool any) {
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(p.W) + (size_t)(rows_here ? row0 : 0) * row_bytes, 0,
                                                  any ? (int)(rows_here * row_bytes) : 0, 0x00020000);
     };
@@ -189,9 +191,10 @@ gemm_f32_split_kernel(SplitArgs p) {
     }
     const bool w_last = 64 * (S::kWReq - 1) + lane < S::kImage / 16;
     auto request_w = [&](int sb) {
+        const uint32_t at = sb < sb1 ? (uint32_t)sb * (uint32_t)F::kBlock : 0u;
 #pragma unroll
         for (int q = 0; q < S::kWReq; q++)
-            if (q + 1 < S::kWReq || w_last) request16(img_at + 1024u * q, w_off[q], w_rsrc(sb < sb1), (uint32_t)sb * (uint32_t)F::kBlock);
+            if (q + 1 < S::kWReq || w_last) request16(img_at + 1024u * q, w_off[q], w_rsrc(sb < sb1), at);
     };
     /* fragments: wave w brings the w-th KB of each 32 tokens' stage; the last stage is asked for again past the end */
     const int n_groups = 8 * p.n_sb, last_group = 8 * sb1 - 1;

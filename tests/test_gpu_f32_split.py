@@ -78,3 +78,25 @@ def test_magnitudes_and_not_finite(oracle, tid, n_rows):
             assert np.linalg.norm(Y[t] - want[t]) <= bar, t
         else:
             assert np.array_equal(np.isnan(Y[t]), np.isnan(want[t])) and np.array_equal(np.isposinf(Y[t]), np.isposinf(want[t])), t
+
+
+@pytest.mark.parametrize("tid", TYPES, ids=lambda t: NAME[t])
+@pytest.mark.parametrize("n_tok,n_rows,n_cols", [(9, 8193, 256), (40, 1030, 2304)])
+def test_tensor_anywhere_in_its_buffer(oracle, tid, n_tok, n_rows, n_cols):
+    """a tensor that starts 2 bytes into a buffer and ends with it: blocks are read from any even address, and the requests
+    that a wave makes past its last super-block read nothing"""
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid + n_rows)
+    X = synth.make_activation(n_cols, seed=n_tok, tokens=n_tok)
+    want = product(tid, W, X, n_rows, n_cols)
+    dW = qlinear.DevBuf.from_numpy(np.concatenate([np.zeros(2, np.uint8), W.view(np.uint8).reshape(-1)]))
+    dX, dY = qlinear.DevBuf.from_numpy(X), qlinear.DevBuf(n_tok * n_rows * 4)
+    ws = qlinear.DevBuf(qlinear.gemm_f32_any_workspace_bytes(n_rows, n_cols))
+    qlinear.check(qlinear.load().qlin_gemm_f32_any_dev(tid, dW.ptr + 2, dX.ptr, dY.ptr, n_rows, n_cols, n_tok, n_cols, n_rows, ws.ptr,
+                                                       ws.nbytes, None))
+    qlinear.sync()
+    got = dY.to_numpy(np.float32, (n_tok, n_rows))
+    for b in (dW, dX, dY, ws):
+        b.free()
+    assert np.array_equal(got, want)
+    exact = X.astype(np.float64) @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T
+    assert rel_l2(got, exact) <= TOL
