@@ -16,12 +16,13 @@
  * Two forms of the arithmetic:
  *   exact    the codes go through the matrix instruction as they are - integers of up to 8 bits are exact in bf16 - and
  *            the block scales are applied to the 32-element sums in fp32 (formats with a scale per 16 elements: the
- *            token operand holds zeros in the lanes of the other 16, eight tokens per instruction). A constant that the
- *            format subtracts from its codes goes in as the instruction's C operand (a product of the activations with
- *            that constant), a minimum as a second sum. 4-bit codes become bf16 two at a time through the fp8
- *            conversion; 5- and 6-bit codes by a byte permute that puts a fixed high byte on top (32 + q and 64 + q have
- *            all their low bits in the low byte; the 32 or 64 is subtracted with the format's own constant); 8-bit ones
- *            through the byte-to-float conversion.
+ *            token operand holds zeros in the lanes of the other 16, eight tokens per instruction). A minimum goes in as a
+ *            second sum. 4-bit codes become bf16 two at a time through the fp8 conversion; 5- and 6-bit codes by a byte
+ *            permute that puts a fixed high byte on top (32 + q and 64 + q have all their low bits in the low byte). Such
+ *            a 32 or 64, and what the format itself subtracts from its codes, comes off as the instruction's C operand, a
+ *            product of the activations with that constant, or (Q5_K) with the minimum.
+ *            8-bit codes go through the byte-to-float conversion signed (as unsigned numbers with 128 taken off, the
+ *            magnitudes of IQ3_S, at most 15, drowned in it: 1.8e-7, now 6.5e-8).
  *   rounded  the weights are decoded in fp32 as the codec does and rounded once to bf16: the vector work per weight then
  *            does not depend on the number of tokens.
  *
@@ -57,6 +58,7 @@ template <int V> QLIN_INL bf16x8 const_bf16() {
     const u32x4 v = {w, w, w, w};
     return __builtin_bit_cast(bf16x8, v);
 }
+QLIN_INL uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
 /* eight codes (unsigned bytes) as bf16, exact */
 template <bool SMALL> QLIN_INL bf16x8 codes_bf16(uint32_t a, uint32_t b) {
     u32x4 r;
@@ -66,12 +68,19 @@ template <bool SMALL> QLIN_INL bf16x8 codes_bf16(uint32_t a, uint32_t b) {
         r.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, false));
         r.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, true));
     } else { /* integers up to 255 have no bits below bf16's */
-        auto pair = [](float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); };
-        r.x = pair(ubyte_f32<0>(a), ubyte_f32<1>(a));
-        r.y = pair(ubyte_f32<2>(a), ubyte_f32<3>(a));
-        r.z = pair(ubyte_f32<0>(b), ubyte_f32<1>(b));
-        r.w = pair(ubyte_f32<2>(b), ubyte_f32<3>(b));
+        r.x = upper_halves(ubyte_f32<0>(a), ubyte_f32<1>(a));
+        r.y = upper_halves(ubyte_f32<2>(a), ubyte_f32<3>(a));
+        r.z = upper_halves(ubyte_f32<0>(b), ubyte_f32<1>(b));
+        r.w = upper_halves(ubyte_f32<2>(b), ubyte_f32<3>(b));
     }
+    return __builtin_bit_cast(bf16x8, r);
+}
+/* eight codes less 128 as bf16, exact */
+QLIN_INL bf16x8 signed_bf16(uint32_t a, uint32_t b) {
+    a ^= 0x80808080u;
+    b ^= 0x80808080u;
+    const u32x4 r = {upper_halves(signed_byte(a, 0), signed_byte(a, 8)), upper_halves(signed_byte(a, 16), signed_byte(a, 24)),
+                     upper_halves(signed_byte(b, 0), signed_byte(b, 8)), upper_halves(signed_byte(b, 16), signed_byte(b, 24))};
     return __builtin_bit_cast(bf16x8, r);
 }
 template <int HI> QLIN_INL bf16x8 ready_bf16(uint32_t a, uint32_t b) {
@@ -112,9 +121,15 @@ template <class F, int NT, int TT, bool EXACT> struct Shape {
     static constexpr int kWaveLds = kXChunk + kImage > kPart ? kXChunk + kImage : kPart;
     /* the same for every NT, so that a row's sum does not depend on how many rows a launch has */
     static constexpr int kWaves = 8 * (TT * 1024 + 16 * F::kPieces * 16) + 4 * F::kTable <= 160 * 1024 ? 8 : 7;
+    /* Chains of fp32 sums that a wave's share of K is divided over. The formats with few unrounded tokens come from the
+     * matvec, which sums 64 short shares; their error at K = 14336, 3 tokens, against 64 bits with one chain / four 1.5e-7 /
+     * 9.7e-8 (the matvec 8.4e-8). Q4_0 has registers for two without giving up a workgroup per compute unit (151936 x 4096
+     * 71 us, with four 87). The other formats keep one (the kernel they come from had half as many waves: Q4_K 2.7e-7,
+     * now 2.0e-7). */
+    static constexpr int kChains = EXACT && F::kUnrounded <= 4 ? (F::kSmall ? 2 : 4) : 1;
     /* four waves per SIMD - a wave alone issues a vector instruction every five cycles, four together one every 2.4 to
      * 4.3 - where the registers allow; two otherwise */
-    static constexpr int kPerSimd = TT <= 2 ? 4 : EXACT ? (NT == 1 || kDiag ? 2 : 4) : TT <= 6 ? 4 : 2;
+    static constexpr int kPerSimd = kChains > 2 && NT > 1 ? 6 : TT <= 2 ? 4 : EXACT ? (NT == 1 || kDiag ? 2 : 4) : TT <= 6 ? 4 : 2;
     static constexpr bool kStepwise = NT > 1 || (TT >= 4 && !EXACT) || (kDiag && F::kHasMin); /* see the end of a step */
     static_assert(TT * kXSteps % 2 == 0 && kWaves * kWaveLds + 4 * F::kTable <= 160 * 1024, "whole requests; LDS");
 };
@@ -125,6 +140,8 @@ __global__ void __launch_bounds__((64 * Shape<F, NT, TT, EXACT>::kWaves))
 gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_tok, int ldx) {
     using S = Shape<F, NT, TT, EXACT>;
     constexpr int kOps = S::kOps, kRow = F::kPieces * 16, XS = S::kXSteps;
+    /* codes of eight bits go in signed; the other formats' constants as the instruction's C operand */
+    constexpr bool kSigned = F::kOffset == 128, kAsC = F::kOffset != 0 && !kSigned;
     constexpr uint32_t kPastEnd = 0xFFFFFFF0u; /* an offset outside every buffer: the request returns zeros */
     extern __shared__ __attribute__((aligned(1024))) uint8_t fewtok_lds[];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n_waves = blockDim.x >> 6;
@@ -180,11 +197,14 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
     const int tok0 = S::kDiag || TT == 1 ? j & 7 : j; /* operand o holds token 16 o (8 o) + tok0 */
     const uint32_t x_rd = (uint32_t)(tok0 * (64 * XS) + ((kg ^ swizzle(tok0)) << 4));
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    f32x4 acc[NT][kOps];
+    constexpr int CH = S::kChains;
+    f32x4 acc[NT][kOps][CH];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-        for (int o = 0; o < kOps; o++) acc[nt][o] = zero;
+        for (int o = 0; o < kOps; o++)
+#pragma unroll
+            for (int i = 0; i < CH; i++) acc[nt][o][i] = zero;
 
     for (int sb = wv; sb < n_sb; sb += n_waves) {
         typename F::Hdr hdr[NT];
@@ -212,7 +232,7 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
             each<XS>([&](auto step) {
                 constexpr int u = decltype(step)::value, U = u0 + u;
                 f32x4 xs[kOps]; /* sums of the activations, or their products with the constant to be subtracted */
-                if constexpr (EXACT && (F::kHasMin || F::kOffset != 0)) {
+                if constexpr (EXACT && (F::kHasMin || kAsC)) {
 #pragma unroll
                     for (int o = 0; o < kOps; o++)
                         xs[o] = mma(__builtin_bit_cast(bf16x8, xa[o][u]), const_bf16<(F::kHasMin ? 1 : -F::kOffset - F::kBase)>(), zero);
@@ -226,26 +246,27 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
                     const float s = F::template scale<U>(hdr[nt], kg);
                     if constexpr (EXACT) {
                         bf16x8 w;
-                        if constexpr (F::kReady != 0) w = ready_bf16<F::kReady>(a, b);
+                        if constexpr (kSigned) w = signed_bf16(a, b);
+                        else if constexpr (F::kReady != 0) w = ready_bf16<F::kReady>(a, b);
                         else w = codes_bf16<F::kSmall>(a, b);
 #pragma unroll
                         for (int o = 0; o < kOps; o++) {
-                            const f32x4 c = mma(__builtin_bit_cast(bf16x8, xa[o][u]), w, F::kOffset != 0 ? xs[o] : zero);
+                            const f32x4 c = mma(__builtin_bit_cast(bf16x8, xa[o][u]), w, kAsC ? xs[o] : zero);
 #pragma unroll
-                            for (int v = 0; v < 4; v++) acc[nt][o][v] = fmaf(s, c[v], acc[nt][o][v]);
+                            for (int v = 0; v < 4; v++) acc[nt][o][U % CH][v] = fmaf(s, c[v], acc[nt][o][U % CH][v]);
                         }
                         if constexpr (F::kHasMin) {
                             const float m = fmaf((float)F::kBase, s, F::template minimum<U>(hdr[nt], kg));
 #pragma unroll
                             for (int o = 0; o < kOps; o++)
 #pragma unroll
-                                for (int v = 0; v < 4; v++) acc[nt][o][v] = fmaf(-m, xs[o][v], acc[nt][o][v]);
+                                for (int v = 0; v < 4; v++) acc[nt][o][U % CH][v] = fmaf(-m, xs[o][v], acc[nt][o][U % CH][v]);
                         }
                     } else {
                         const float off = F::kHasMin ? F::template minimum<U>(hdr[nt], kg) : s * (float)F::kOffset;
                         const bf16x8 w = weights_bf16<F::kSmall>(a, b, s, off);
 #pragma unroll
-                        for (int o = 0; o < kOps; o++) acc[nt][o] = mma(__builtin_bit_cast(bf16x8, xa[o][u]), w, acc[nt][o]);
+                        for (int o = 0; o < kOps; o++) acc[nt][o][0] = mma(__builtin_bit_cast(bf16x8, xa[o][u]), w, acc[nt][o][0]);
                     }
                 }
                 /* no further ahead than the steps that share loads: left alone the compiler fetches the whole image first,
@@ -255,7 +276,7 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
 #pragma unroll
                     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-                        for (int o = 0; o < kOps; o++) asm volatile("" : "+v"(acc[nt][o]));
+                        for (int o = 0; o < kOps; o++) asm volatile("" : "+v"(acc[nt][o][U % CH]));
                     asm volatile("" ::: "memory");
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -272,7 +293,11 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
     for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int o = 0; o < kOps; o++) {
-            f32x4 v = acc[nt][o];
+#pragma unroll
+            for (int n = CH / 2; n > 0; n /= 2)
+#pragma unroll
+                for (int i = 0; i < n; i++) acc[nt][o][i] += acc[nt][o][i + n];
+            f32x4 v = acc[nt][o][0];
             if constexpr (S::kDiag) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) v[i] = add_lane32(v[i]); /* the two scale groups */
@@ -320,8 +345,8 @@ template <class F, int TT, bool EXACT> hipError_t fewtok_rows(const FewtokCall &
     return fewtok_launch<F, 1, TT, EXACT>(c);
 }
 
-/* EXACT_MAX: token count up to which a format's codes stay unrounded */
-template <class F, int EXACT_MAX> hipError_t fewtok_format(const FewtokCall &c) {
+template <class F> hipError_t fewtok_format(const FewtokCall &c) {
+    constexpr int EXACT_MAX = F::kUnrounded;
     const int n = c.n_tok;
     if (n <= EXACT_MAX) {
         if constexpr (EXACT_MAX <= 8) return fewtok_rows<F, 1, true>(c);

@@ -2,7 +2,7 @@
 #include "gemm_fewtok.h"
 
 namespace qlin {
-hipError_t fewtok_q8_0(const FewtokCall &c) { return fewtok_format<TQ8_0, 24>(c); }
-hipError_t fewtok_q4_0(const FewtokCall &c) { return fewtok_format<TQ4_0, 4>(c); }
-hipError_t fewtok_iq4nl(const FewtokCall &c) { return fewtok_format<TIQ4NL, 4>(c); }
+hipError_t fewtok_q8_0(const FewtokCall &c) { return fewtok_format<TQ8_0>(c); }
+hipError_t fewtok_q4_0(const FewtokCall &c) { return fewtok_format<TQ4_0>(c); }
+hipError_t fewtok_iq4nl(const FewtokCall &c) { return fewtok_format<TIQ4NL>(c); }
 }  // namespace qlin

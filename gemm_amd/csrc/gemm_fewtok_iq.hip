@@ -2,7 +2,7 @@
 #include "gemm_fewtok.h"
 
 namespace qlin {
-hipError_t fewtok_iq4xs(const FewtokCall &c) { return fewtok_format<TIQ4XS, 4>(c); }
-hipError_t fewtok_iq3s(const FewtokCall &c) { return fewtok_format<TIQ3S, 4>(c); }
-hipError_t fewtok_iq2xxs(const FewtokCall &c) { return fewtok_format<TIQ2XXS, 4>(c); }
+hipError_t fewtok_iq4xs(const FewtokCall &c) { return fewtok_format<TIQ4XS>(c); }
+hipError_t fewtok_iq3s(const FewtokCall &c) { return fewtok_format<TIQ3S>(c); }
+hipError_t fewtok_iq2xxs(const FewtokCall &c) { return fewtok_format<TIQ2XXS>(c); }
 }  // namespace qlin

@@ -2,7 +2,7 @@
 #include "gemm_fewtok.h"
 
 namespace qlin {
-hipError_t fewtok_q4k(const FewtokCall &c) { return fewtok_format<TQ4K, 32>(c); }
-hipError_t fewtok_q5k(const FewtokCall &c) { return fewtok_format<TQ5K, 24>(c); }
-hipError_t fewtok_q2k(const FewtokCall &c) { return fewtok_format<TQ2K, 24>(c); }
+hipError_t fewtok_q4k(const FewtokCall &c) { return fewtok_format<TQ4K>(c); }
+hipError_t fewtok_q5k(const FewtokCall &c) { return fewtok_format<TQ5K>(c); }
+hipError_t fewtok_q2k(const FewtokCall &c) { return fewtok_format<TQ2K>(c); }
 }  // namespace qlin

@@ -2,6 +2,6 @@
 #include "gemm_fewtok.h"
 
 namespace qlin {
-hipError_t fewtok_q6k(const FewtokCall &c) { return fewtok_format<TQ6K, 24>(c); }
-hipError_t fewtok_q3k(const FewtokCall &c) { return fewtok_format<TQ3K, 24>(c); }
+hipError_t fewtok_q6k(const FewtokCall &c) { return fewtok_format<TQ6K>(c); }
+hipError_t fewtok_q3k(const FewtokCall &c) { return fewtok_format<TQ3K>(c); }
 }  // namespace qlin

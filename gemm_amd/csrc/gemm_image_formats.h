@@ -55,7 +55,8 @@ QLIN_INL float signed_byte(uint32_t w, int at) { return (float)(int)(int8_t)(w >
  *   kOffset     what the format subtracts from a code
  *   scale<u>    the factor of the lane's elements; minimum<u> (kHasMin): what is subtracted after that
  *   kGroup16    the factor belongs to 16 elements, not 32
- *   kShare      steps u that are scheduled together */
+ *   kShare      steps u that are scheduled together
+ *   kUnrounded  token count up to which the few-token kernel leaves the codes unrounded */
 constexpr uint32_t kNoPiece = 0xFFFFFFFFu;
 
 struct HdrK4 { float d, dmin; uint32_t sc_lo, sc_hi, mn_lo, mn_hi; };
@@ -71,7 +72,7 @@ QLIN_INL HdrK4 k4_header(const uint8_t *row) {
     return r;
 }
 struct TQ4K {
-    static constexpr int kBlock = 144, kPieces = 9, kOffset = 0, kTable = 0, kReady = 0, kBase = 0, kShare = 2;
+    static constexpr int kBlock = 144, kPieces = 9, kOffset = 0, kTable = 0, kReady = 0, kBase = 0, kShare = 2, kUnrounded = 32;
     static constexpr bool kSmall = true, kHasMin = true, kGroup16 = false;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return 16u * p; }
     typedef HdrK4 Hdr;
@@ -85,7 +86,7 @@ struct TQ4K {
     template <int U> static QLIN_INL float minimum(const Hdr &h, int) { return h.dmin * ubyte_f32<U & 3>(U < 4 ? h.mn_lo : h.mn_hi); }
 };
 struct TQ5K {
-    static constexpr int kBlock = 176, kPieces = 11, kOffset = 0, kTable = 0, kReady = 0x42, kBase = 32, kShare = 2;
+    static constexpr int kBlock = 176, kPieces = 11, kOffset = 0, kTable = 0, kReady = 0x42, kBase = 32, kShare = 2, kUnrounded = 24;
     static constexpr bool kSmall = false, kHasMin = true, kGroup16 = false;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return 16u * p; }
     typedef HdrK4 Hdr;
@@ -109,7 +110,7 @@ struct TQ5K {
     template <int U> static QLIN_INL float minimum(const Hdr &h, int kg) { return TQ4K::minimum<U>(h, kg); }
 };
 struct TQ6K {
-    static constexpr int kBlock = 210, kPieces = 15, kOffset = 32, kTable = 0, kReady = 0x42, kBase = 64, kShare = 2;
+    static constexpr int kBlock = 210, kPieces = 15, kOffset = 32, kTable = 0, kReady = 0x42, kBase = 64, kShare = 2, kUnrounded = 24;
     static constexpr bool kSmall = false, kHasMin = false, kGroup16 = true;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return p < 13 ? 16u * p : p == 13 ? 194u : kNoPiece; }
     struct Hdr { float d; u32x4 sc; }; /* the scales shifted so that the lane's are bytes 0 and 2 of a dword */
@@ -140,7 +141,7 @@ struct TQ6K {
     template <int U> static QLIN_INL float minimum(const Hdr &, int) { return 0.0f; }
 };
 struct TQ8_0 {
-    static constexpr int kBlock = 272, kPieces = 17, kOffset = 128, kTable = 0, kReady = 0, kBase = 0, kShare = 1;
+    static constexpr int kBlock = 272, kPieces = 17, kOffset = 128, kTable = 0, kReady = 0, kBase = 0, kShare = 1, kUnrounded = 24;
     static constexpr bool kSmall = false, kHasMin = false, kGroup16 = false;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return 16u * p; }
     struct Hdr { const uint8_t *row; };
@@ -154,7 +155,7 @@ struct TQ8_0 {
     template <int U> static QLIN_INL float minimum(const Hdr &, int) { return 0.0f; }
 };
 struct TQ2K {
-    static constexpr int kBlock = 84, kPieces = 7, kOffset = 0, kTable = 0, kReady = 0, kBase = 0, kShare = 2;
+    static constexpr int kBlock = 84, kPieces = 7, kOffset = 0, kTable = 0, kReady = 0, kBase = 0, kShare = 2, kUnrounded = 24;
     static constexpr bool kSmall = true, kHasMin = true, kGroup16 = true;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return p < 5 ? 16u * p : p == 5 ? 68u : kNoPiece; }
     struct Hdr { float d, dmin; u32x4 sc; };
@@ -175,7 +176,7 @@ struct TQ2K {
     template <int U> static QLIN_INL float minimum(const Hdr &h, int) { return h.dmin * (float)((h.sc[U >> 1] >> (16 * (U & 1) + 4)) & 15u); }
 };
 struct TQ3K {
-    static constexpr int kBlock = 110, kPieces = 7, kOffset = 4, kTable = 0, kReady = 0, kBase = 0, kShare = 2;
+    static constexpr int kBlock = 110, kPieces = 7, kOffset = 4, kTable = 0, kReady = 0, kBase = 0, kShare = 2, kUnrounded = 24;
     static constexpr bool kSmall = true, kHasMin = false, kGroup16 = true;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return p < 6 ? 16u * p : 94u; }
     struct Hdr { float d; uint32_t sc[4]; }; /* byte u of the eight in sc[0..1] / sc[2..3]: 6-bit scales 2 u (+ 1: the lane's) */
@@ -206,7 +207,7 @@ struct TQ3K {
     template <int U> static QLIN_INL float minimum(const Hdr &, int) { return 0.0f; }
 };
 struct TQ4_0 {
-    static constexpr int kBlock = 144, kPieces = 9, kOffset = 8, kTable = 0, kReady = 0, kBase = 0, kShare = 1;
+    static constexpr int kBlock = 144, kPieces = 9, kOffset = 8, kTable = 0, kReady = 0, kBase = 0, kShare = 1, kUnrounded = 4;
     static constexpr bool kSmall = true, kHasMin = false, kGroup16 = false;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return 16u * p; }
     struct Hdr { const uint8_t *row; };
@@ -221,7 +222,7 @@ struct TQ4_0 {
     template <int U> static QLIN_INL float minimum(const Hdr &, int) { return 0.0f; }
 };
 struct TIQ4NL {
-    static constexpr int kBlock = 144, kPieces = 9, kOffset = 128, kTable = 0, kReady = 0, kBase = 0, kShare = 1;
+    static constexpr int kBlock = 144, kPieces = 9, kOffset = 128, kTable = 0, kReady = 0, kBase = 0, kShare = 1, kUnrounded = 4;
     static constexpr bool kSmall = false, kHasMin = false, kGroup16 = false;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return 16u * p; }
     typedef TQ4_0::Hdr Hdr;
@@ -235,7 +236,7 @@ struct TIQ4NL {
     template <int U> static QLIN_INL float minimum(const Hdr &, int) { return 0.0f; }
 };
 struct TIQ4XS {
-    static constexpr int kBlock = 136, kPieces = 9, kOffset = 128, kTable = 0, kReady = 0, kBase = 0, kShare = 1;
+    static constexpr int kBlock = 136, kPieces = 9, kOffset = 128, kTable = 0, kReady = 0, kBase = 0, kShare = 1, kUnrounded = 4;
     static constexpr bool kSmall = false, kHasMin = false, kGroup16 = false;
     static QLIN_INL uint32_t piece_src(uint32_t p) { return p < 8 ? 16u * p : 120u; }
     struct Hdr { float d; uint32_t hi, lo; };
@@ -261,7 +262,7 @@ struct TIQ4XS {
 };
 /* the grid formats look their magnitudes up in a table that the workgroup stages in LDS */
 struct TIQ3S {
-    static constexpr int kBlock = 110, kPieces = 7, kOffset = 128, kTable = 512, kReady = 0, kBase = 0, kShare = 1;
+    static constexpr int kBlock = 110, kPieces = 7, kOffset = 128, kTable = 512, kReady = 0, kBase = 0, kShare = 1, kUnrounded = 4;
     static constexpr bool kSmall = false, kHasMin = false, kGroup16 = false;
     static QLIN_INL const uint32_t *table() { return qlin_iq3s_grid; }
     static QLIN_INL uint32_t piece_src(uint32_t p) { return p < 6 ? 16u * p : 94u; }
@@ -277,7 +278,7 @@ struct TIQ3S {
     template <int U> static QLIN_INL float minimum(const Hdr &, int) { return 0.0f; }
 };
 struct TIQ2XXS {
-    static constexpr int kBlock = 66, kPieces = 5, kOffset = 128, kTable = 512, kReady = 0, kBase = 0, kShare = 1;
+    static constexpr int kBlock = 66, kPieces = 5, kOffset = 128, kTable = 512, kReady = 0, kBase = 0, kShare = 1, kUnrounded = 4;
     static constexpr bool kSmall = false, kHasMin = false, kGroup16 = false;
     static QLIN_INL const uint32_t *table() { return reinterpret_cast<const uint32_t *>(qlin_iq2xxs_grid); }
     static QLIN_INL uint32_t piece_src(uint32_t p) { return p < 4 ? 16u * p : 50u; }

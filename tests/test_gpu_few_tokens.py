@@ -83,3 +83,27 @@ def test_tensors_of_one_launch_equal_a_call_each(tid, n_tok):
         got.append([y.to_numpy(np.uint32, (n_tok, r)) for y, r in zip(dYs, rows)])
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+# K = 1024: four waves with a super-block each, and in it eight sums of 32 exact products that the matrix instruction adds,
+# scaled and added in fp32. That is about a dozen roundings of half a unit of 2^-24 at most, of partial sums that grow to
+# the result, and their root mean square stays below 1.5 units; a code that goes in with a constant which comes off after a
+# rounding shows as more.
+UNROUNDED_BAR = 1.75 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("tid,n_tok", [(t, n) for t in sorted(EXACT_MAX) for n in (3, 8, 16, 24) if n <= EXACT_MAX[t] and t != synth.GGML_Q5_K],
+                         ids=str)
+def test_unrounded_codes_keep_fp32_precision(oracle, tid, n_tok):
+    n_rows, n_cols = 1024, 1024
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid)
+    Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_tok, tokens=n_tok))
+    dW, dX, dY = qlinear.DevBuf.from_numpy(W), qlinear.DevBuf.from_numpy(Xb), qlinear.DevBuf(n_tok * n_rows * 4)
+    ws = qlinear.DevBuf(qlinear.gemm_bf16_any_workspace_bytes(n_rows, n_cols))
+    qlinear.gemm_bf16_any_dev(tid, dW, dX, dY, n_rows, n_cols, n_tok, n_cols, n_rows, ws)
+    qlinear.sync()
+    Y = dY.to_numpy(np.float32, (n_tok, n_rows))
+    for b in (dW, dX, dY, ws):
+        b.free()
+    want = synth.bf16_bits_to_f32(Xb).astype(np.float64) @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T
+    assert rel_l2(Y, want) <= UNROUNDED_BAR, (NAME[tid], n_tok, rel_l2(Y, want) * 2.0 ** 24)
