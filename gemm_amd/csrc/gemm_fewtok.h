@@ -20,7 +20,8 @@
  *            second sum. 4-bit codes become bf16 two at a time through the fp8 conversion; 5- and 6-bit codes by a byte
  *            permute that puts a fixed high byte on top (32 + q and 64 + q have all their low bits in the low byte). Such
  *            a 32 or 64, and what the format itself subtracts from its codes, comes off as the instruction's C operand, a
- *            product of the activations with that constant, or (Q5_K) with the minimum.
+ *            product of the activations with that constant: before the scale, where the sum is as long as its terms
+ *            (Q5_K's 32 taken off with the minimum, after 32 s had been rounded: error 1.2e-7 at K = 1024, now 8.8e-8).
  *            8-bit codes go through the byte-to-float conversion signed (as unsigned numbers with 128 taken off, the
  *            magnitudes of IQ3_S, at most 15, drowned in it: 1.8e-7, now 6.5e-8).
  *   rounded  the weights are decoded in fp32 as the codec does and rounded once to bf16: the vector work per weight then
@@ -237,6 +238,14 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
                     for (int o = 0; o < kOps; o++)
                         xs[o] = mma(__builtin_bit_cast(bf16x8, xa[o][u]), const_bf16<(F::kHasMin ? 1 : -F::kOffset - F::kBase)>(), zero);
                 }
+                f32x4 c0[kOps]; /* where the instruction starts */
+#pragma unroll
+                for (int o = 0; o < kOps; o++) {
+                    if constexpr (EXACT && kAsC) c0[o] = xs[o];
+                    else if constexpr (EXACT && F::kHasMin && F::kBase != 0 && TT == 1) c0[o] = mma(__builtin_bit_cast(bf16x8, xa[o][u]), const_bf16<-F::kBase>(), zero);
+                    else if constexpr (EXACT && F::kHasMin && F::kBase != 0) c0[o] = xs[o] * (float)-F::kBase; /* (the same numbers) */
+                    else c0[o] = zero;
+                }
 #pragma unroll
                 for (int nt = 0; nt < NT; nt++) {
                     const uint8_t *row = img + (16 * nt + j) * kRow;
@@ -251,12 +260,12 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
                         else w = codes_bf16<F::kSmall>(a, b);
 #pragma unroll
                         for (int o = 0; o < kOps; o++) {
-                            const f32x4 c = mma(__builtin_bit_cast(bf16x8, xa[o][u]), w, kAsC ? xs[o] : zero);
+                            const f32x4 c = mma(__builtin_bit_cast(bf16x8, xa[o][u]), w, c0[o]);
 #pragma unroll
                             for (int v = 0; v < 4; v++) acc[nt][o][U % CH][v] = fmaf(s, c[v], acc[nt][o][U % CH][v]);
                         }
                         if constexpr (F::kHasMin) {
-                            const float m = fmaf((float)F::kBase, s, F::template minimum<U>(hdr[nt], kg));
+                            const float m = F::template minimum<U>(hdr[nt], kg);
 #pragma unroll
                             for (int o = 0; o < kOps; o++)
 #pragma unroll
