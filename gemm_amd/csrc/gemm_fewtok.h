@@ -6,7 +6,7 @@
  *
  * With this few tokens the weights' own bytes are what a launch cannot do without, so the kernel has the structure of
  * the matvec (gemv_q4k.hip) and not that of a tile product: a workgroup owns NT * 16 rows, its eight waves split K - wave
- * w takes super-blocks w, w + 8, ... - and meet once, in LDS, for the sum over K. A wave copies a super-block of all its
+ * w takes super-blocks w, w + 8, ... (seven waves where LDS is short) - and meet once, in LDS, for the sum over K. A wave copies a super-block of all its
  * rows by load-to-LDS requests into an image of its own (whole blocks, consecutive lanes consecutive 16-byte pieces,
  * source addresses of any alignment) and the activations of those 256 elements the same way, chunk by chunk, the next
  * chunk on its way while one is multiplied; it waits by counting its own requests and needs no barrier before the final
@@ -110,11 +110,12 @@ template <bool SMALL> QLIN_INL bf16x8 weights_bf16(uint32_t a, uint32_t b, float
 /* Shape of an instance: NT 16-row tiles, up to 8 TT tokens. kXSteps: 32-element steps whose activations are fetched and
  * held at a time - short chunks leave LDS for a second workgroup per compute unit, which measured more than longer ones
  * (Q4_K, 32 tokens, 14336 x 4096: chunks of two steps 16.3 us, of four 18.8); with eight tokens and one row tile whole
- * super-blocks (4096 x 14336, 8 tokens: 11.5 against 12.9). A second chunk or image ahead measured no gain. */
+ * super-blocks (4096 x 14336, 8 tokens: 11.5 against 12.9); single steps where two row tiles and more than 96 tokens fill
+ * the LDS. A second chunk or image ahead measured no gain. */
 template <class F, int NT, int TT, bool EXACT> struct Shape {
     static constexpr bool kDiag = EXACT && F::kGroup16;      /* eight tokens per instruction */
     static constexpr int kOps = kDiag ? TT : (TT + 1) / 2;   /* token operands */
-    static constexpr int kXSteps = TT == 1 ? (NT == 1 ? 8 : 4) : TT == 2 ? (NT == 1 ? 4 : 2) : kDiag && NT == 2 ? 4 : 2;
+    static constexpr int kXSteps = NT == 2 && TT > 12 ? 1 : TT == 1 ? (NT == 1 ? 8 : 4) : TT == 2 ? (NT == 1 ? 4 : 2) : kDiag && NT == 2 ? 4 : 2;
     static constexpr int kParts = 8 / kXSteps;               /* chunks per super-block */
     static constexpr int kXReq = TT * kXSteps / 2, kXChunk = kXReq * 1024; /* requests and bytes of a chunk of activations */
     static constexpr int kImage = NT * 16 * F::kPieces * 16, kWReq = (kImage + 1023) / 1024; /* of a wave's image */
@@ -169,7 +170,7 @@ gemm_fewtok_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_
      * that the 16 tokens of an operand read fall into 16 bank groups; tokens past the end arrive as zeros */
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(X), 0,
                                                                             ((n_tok - 1) * ldx + n_sb * 256) * 2, 0x00020000);
-    auto swizzle = [](int tok) { return XS == 2 ? (tok >> 1) & 7 : S::kDiag || TT == 1 ? tok & 7 : tok & 15; };
+    auto swizzle = [](int tok) { return XS == 1 ? (tok >> 2) & 3 : XS == 2 ? (tok >> 1) & 7 : S::kDiag || TT == 1 ? tok & 7 : tok & 15; };
     uint32_t x_off[S::kXReq];
 #pragma unroll
     for (int q = 0; q < S::kXReq; q++) {
@@ -343,13 +344,19 @@ template <class F, int NT, int TT, bool EXACT> hipError_t fewtok_launch(const Fe
 
 /* One row tile per workgroup up to a tile for every compute unit and a few over; two beyond, which read the activations
  * once for both (us, 16 tokens, one / two: Q4_K 256 tiles 5.6 / 6.8, 384 tiles 8.4 / 7.6, 864 tiles 12.4 / 9.9; Q6_K 7.8 /
- * 11.4, 11.6 / 11.9, 16.8 / 14.4). Q8_0 with eight tokens: two images leave no room for a second workgroup (13.3 / 16).
- * More than 64 tokens: one. */
+ * 11.4, 11.6 / 11.9, 16.8 / 14.4). Q8_0 with eight tokens: two images leave no room for a second workgroup (13.3 / 16), and
+ * from 65 tokens on they do not fit at all. Rows of up to four super-blocks have as many waves, and a compute unit holds
+ * more of those workgroups, so that one tile reaches further (24 tokens 9216 x 1024 Q6_K, one / two: 7.1 / 8.9, 64 tokens
+ * 14336 x 256 Q4_K 6.2 / 9.1) - except 17 and more unrounded tokens of Q4_K and Q5_K, whose waves want many registers
+ * (32 tokens 9216 x 1024 Q4_K 7.1 / 6.2). From 65 tokens on a workgroup of eight waves fills a compute unit (320 tiles x
+ * 4096, one / two: 96 tokens Q4_K 18.4 / 12.5, 128 tokens 23.4 / 18.2; 288 tiles x 2048 at 128 15.1 / 11.1). */
 template <class F, int TT, bool EXACT> hipError_t fewtok_rows(const FewtokCall &c) {
-    if constexpr (TT <= 8) {
-        int tiles = 0;
+    if constexpr (TT <= 8 || F::kPieces < 17) {
+        constexpr bool kSmallGroups = !(EXACT && TT >= 3 && F::kHasMin && !F::kGroup16);
+        const int n_sb = c.n_cols / 256, waves = kSmallGroups && n_sb <= 4 ? n_sb : 8;
+        long long tiles = 0;
         for (int i = 0; i < c.n_mat; i++) tiles += (c.n_rows[i] + 15) / 16;
-        if (tiles > 288 && !(F::kPieces >= 17 && TT == 1 && tiles > 512)) return fewtok_launch<F, 2, TT, EXACT>(c);
+        if (tiles * waves > (TT <= 8 ? 288 : 256) * 8 && !(F::kPieces >= 17 && TT == 1 && tiles > 512)) return fewtok_launch<F, 2, TT, EXACT>(c);
     }
     return fewtok_launch<F, 1, TT, EXACT>(c);
 }

@@ -21,15 +21,29 @@ int fewtok_unrounded(uint32_t type) {
     }
 }
 
-/* Up to 64 tokens always; up to 128 while there are few row tiles (320 of 16 rows): the kernel reads the activations once
- * per 16 rows then, where the small-tile kernel, whose workgroup takes 64 rows, fills the chip from about 14000 rows on
- * (us, this kernel / small tiles, 77 tokens: Q4_K 3840 x 2560 8.6 / 12.5, 4096 x 4096 10.2 / 17.5, 2560 x 6912
- * 13.6 / 25.8, but 13824 x 2560 19.6 / 16.8; Q6_K 9.5 / 16.3, 12.9 / 26.5, 18 / 41, 24 / 21; 128 tokens Q4_K 11.4 / 13,
- * 15.2 / 18, 19.9 / 26.6, 40 / 17). The grid formats, which have no tile kernel, end at 64 (IQ3_S 13824 x 2560 at 64
- * tokens 23 us, decode + dense product 63): beyond, their product is that of a cached bf16 copy bit for bit. */
+/* Unrounded tokens always. With rounded weights the small-tile kernel, whose workgroup takes 64 rows, computes the same;
+ * it is the faster one where this kernel's workgroups no longer run in one go (us, this kernel / small tiles):
+ *   49 to 64 tokens, more than 512 row tiles: 64 tokens 8192 x 2048 Q4_K 7.1 / 10.7, but 8704 x 2048 11.9 / 10.9, 9216 x
+ *     2560 Q5_K 15.8 / 13.3 (14336 x 4096 Q4_K 19.9 / 20.9). Not Q8_0, whose decode costs the tile kernel more (9216 x 2048
+ *     14.2 / 17.1), and not very many rows of 1024 elements (24576 x 1024 Q4_K 11.1 / 11.8, but 14336 x 1024 8.3 / 8.0)
+ *   65 to 128 tokens, more than 320: 80 tokens Q4_K 4096 x 4096 9.2 / 17.3, 5120 x 4096 11.2 / 17.6, but 77 tokens
+ *     13824 x 2560 19.6 / 16.8; past 96 tokens, rows below 2048 (Q8_0: 4096) elements: 256 (128 tokens 5120 x 1024 Q4_K 9.5 / 7.9)
+ *   rows so short that one or two waves do all of K: 256 elements from 49 tokens on (64 tokens 4096 x 256 5.6 / 5.1), 512
+ *     from 97 on (128 tokens 4096 x 512 Q4_K 7.0 / 6.1; with more than 256 row tiles from 81 on)
+ * The grid formats, which have no tile kernel, end at 64 (IQ3_S 13824 x 2560 at 64 tokens 23 us, decode + dense product
+ * 63): beyond, their product is that of a cached bf16 copy bit for bit. */
 bool fewtok_takes(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx) {
     if (!fewtok_has(type) || n_cols % 256 != 0 || n_tok > 128 || ldx >= (1 << 22)) return false;
-    return n_tok <= 64 || ((n_rows + 15) / 16 <= 320 && gemm_kq_wave4_covers(type));
+    if (n_tok <= fewtok_unrounded(type)) return true;
+    if (!gemm_kq_wave4_covers(type)) return n_tok <= 64;
+    const int tiles = n_rows / 16 + (n_rows % 16 != 0), n_sb = n_cols / 256;
+    if (n_tok <= 48) return true;
+    if (n_sb == 1) return false;
+    if (n_tok <= 64) return tiles <= 512 || type == T_Q8_0 || (n_sb == 4 && tiles >= 1200);
+    if (n_tok <= 80) return tiles <= 320;
+    if (n_tok <= 96) return tiles <= (n_sb == 2 ? 256 : 320);
+    if (type == T_Q8_0) return tiles <= (n_sb < 16 ? 256 : 320);
+    return n_sb > 2 && tiles <= (n_sb < 8 ? 256 : 320);
 }
 
 hipError_t launch_gemm_fewtok(uint32_t type, const FewtokCall &c) {

@@ -1150,7 +1150,7 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
         if (!together) break;
         const bool mine_few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
-        const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(T_Q4_K) ? kFusedNone : choose_fused_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(type) ? kFusedNone : choose_fused_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         together = (mine_few || mine != kFusedNone) && (i == 0 || (mine == tile && mine_few == few));
         tile = mine;
         few = mine_few;

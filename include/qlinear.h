@@ -236,10 +236,12 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * 65..256 tokens). Given a workspace, the decode + dense route still takes the shapes where decoding once measured
  * faster: large-tile shapes above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512 (Q6_K, Q8_0), small-tile
  * shapes of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024.
- * Up to 64 tokens of these formats (and, given a workspace, of IQ3_S and IQ2_XXS), and up to 128 where a tensor has at most
- * 5120 rows, run in the few-token kernel (n_cols % 256 == 0, no workspace used), which streams the blocks once: with unrounded
- * codes (~1e-6) up to 32 tokens of Q4_K, 24 of Q5_K, Q6_K, Q2_K, Q3_K and Q8_0 and 4 of the others, beyond that with the
- * same single rounding to bf16. Up to 4 tokens of any other
+ * A few tokens of these formats (and, given a workspace, up to 64 of IQ3_S and IQ2_XXS) run in the few-token kernel
+ * (n_cols % 256 == 0, no workspace used), which streams the blocks once: with unrounded codes (~1e-6) up to 32 tokens of
+ * Q4_K, 24 of Q5_K, Q6_K, Q2_K, Q3_K and Q8_0 and 4 of the others; beyond that, with the same single rounding to bf16, up
+ * to 48 tokens, up to 64 where a tensor has at most 8192 rows and up to 128 where it has at most 5120 (somewhat less
+ * for rows of fewer than 2048 elements). A token with an infinity or a NaN leaves the others alone; with unrounded codes
+ * its own results may be NaN where exact arithmetic gives an infinity. Up to 4 tokens of any other
  * block format go one by one through the matvec kernels (exact weights, ~1e-6; the workspace holds their
  * activations as fp32, and when ldx is so wide that (n_tok - 1) * ldx + n_cols floats do not fit it they take the
  * decode + dense route). workspace: device memory, 256-byte aligned, at least

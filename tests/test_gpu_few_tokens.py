@@ -63,11 +63,17 @@ def test_two_row_tiles_per_workgroup(oracle, tid, n_tok):
     check(oracle, tid, rows, n_cols, n_tok, sample=60)
 
 
-@pytest.mark.parametrize("n_tok", [7, 40, 100])
+@pytest.mark.parametrize("n_tok", [65, 81, 97, 128])
+@pytest.mark.parametrize("tid", sorted(set(EXACT_MAX) - set(GRID)), ids=lambda t: NAME[t])
+def test_two_row_tiles_of_many_tokens(oracle, tid, n_tok):
+    check(oracle, tid, [4663], 2048 if n_tok <= 96 else 4096, n_tok, sample=40)
+
+
+@pytest.mark.parametrize("n_tok,n_cols", [(7, 512), (40, 512), (100, 512), (40, 2048), (90, 2048), (100, 2048)])
 @pytest.mark.parametrize("tid", sorted(EXACT_MAX), ids=lambda t: NAME[t])
-def test_tensors_of_one_launch_equal_a_call_each(tid, n_tok):
+def test_tensors_of_one_launch_equal_a_call_each(tid, n_tok, n_cols):
     """bit for bit, though the joint launch puts two row tiles in a workgroup and a call of its own one"""
-    rows, n_cols = [2500, 2300, 48], 512
+    rows = [2500, 2300, 48]
     Ws = [synth.make_weights(tid, r, n_cols, seed=r) for r in rows]
     dX = qlinear.DevBuf.from_numpy(synth.to_bf16_bits(synth.make_activation(n_cols, seed=3, tokens=n_tok)))
     ws = qlinear.DevBuf(qlinear.gemm_bf16_any_workspace_bytes(max(rows), n_cols))

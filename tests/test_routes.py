@@ -1,0 +1,33 @@
+"""Which kernel qlin_gemm_bf16_any_dev chooses, at both sides of every limit of the few-token kernel. CPU only: the choice
+is a function of format and shape (qlin_probe_gemm_route: 0 matvec or decode + dense, 1 and 2 the tile kernels, 3 few tokens)."""
+import pytest
+
+from gemm_amd import qlinear
+import synth
+
+ALL = (synth.GGML_Q4_K, synth.GGML_Q5_K, synth.GGML_Q6_K, synth.GGML_Q2_K, synth.GGML_Q3_K, synth.GGML_Q8_0, synth.GGML_Q4_0,
+       synth.GGML_IQ4_NL, synth.GGML_IQ4_XS)
+FEW, MATVEC = 3, 0
+
+
+def route(tid, n_rows, n_cols, n_tok, have_workspace=1):
+    return qlinear.load().qlin_probe_gemm_route(tid, n_rows, n_cols, n_tok, n_cols, have_workspace)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: synth.TYPE_NAMES[t])
+def test_rounded_weights_go_to_the_faster_of_the_few_token_and_tile_kernels(tid):
+    q8 = tid == synth.GGML_Q8_0
+    for n_rows, n_cols, n_tok, few in [
+            (8192, 2048, 64, True), (8193, 2048, 64, q8), (8193, 2048, 48, True), (20000, 1024, 64, True), (16000, 1024, 64, q8),
+            (5120, 2048, 80, True), (5121, 2048, 80, False), (5120, 2048, 128, not q8), (5120, 4096, 128, True), (4096, 2048, 128, True),
+            (5120, 1536, 128, False), (4096, 1536, 128, True), (5120, 512, 80, True), (5120, 512, 81, False), (4096, 512, 96, True),
+            (4096, 512, 97, q8), (64, 256, 48, True), (64, 256, 49, False), (64, 4096, 129, False)]:
+        assert (route(tid, n_rows, n_cols, n_tok) == FEW) == few, (n_rows, n_cols, n_tok)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: synth.TYPE_NAMES[t])
+def test_unrounded_tokens_stay_unrounded(tid):
+    """whatever the shape: a tile kernel would round their weights"""
+    n = 32 if tid == synth.GGML_Q4_K else 4 if tid in (synth.GGML_Q4_0, synth.GGML_IQ4_NL, synth.GGML_IQ4_XS) else 24
+    for n_rows, n_cols in [(16, 256), (50000, 256), (50000, 4096), (300, 16384)]:
+        assert route(tid, n_rows, n_cols, n) == FEW
