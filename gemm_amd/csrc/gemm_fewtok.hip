@@ -46,6 +46,32 @@ bool fewtok_takes(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx) {
     return n_sb > 2 && tiles <= (n_sb < 8 ? 256 : 320);
 }
 
+/* Tokens that go one by one through the matvec instead (whose bar is the same, exact weights): the formats that multiply up
+ * to four tokens unrounded, where the tensor is so large that the matvec's own launch is cheaper by size (us, this kernel /
+ * widening x and a matvec per token; long: rows of 12288 elements and more, of which a wave here walks an eighth alone).
+ *   one token   IQ4_NL, IQ4_XS from 32 M weights (4096 x 4096 5.3 / 7.0, 9216 x 4096 12.4 / 9.6, 14336 x 4096 13.1 / 11.0) and
+ *               long rows (2048 x 14336 12.5 / 11.3); IQ3_S from 16 M and 4608 rows (5120 x 2048 6.6 / 7.2, 9216 x 4096 15.3 / 11.1)
+ *               and long rows; Q4_0 above 64 M (9216 x 8192 13.7 / 13.2, 28672 x 4096 15.1 / 14.1); IQ2_XXS, whose table
+ *               every workgroup fills, from 3072 elements or 4608 rows (4096 x 2048 6.0 / 6.7, 4096 x 4096 8.9 / 7.0,
+ *               28672 x 4096 36.3 / 13.1)
+ *   two         IQ2_XXS above 32 M (4096 x 4096 8.7 / 10.9, 9216 x 4096 20.3 / 14.6) and long rows (4096 x 14336 22.1 / 17.8)
+ *   three       IQ2_XXS above 64 M and 8192 rows (8192 x 8192 21.5 / 25.6, 9216 x 14336 60.2 / 47.5)
+ * Rows of up to 1024 elements stay (28672 x 1024 IQ4_NL 8.3 / 14.5). */
+bool fewtok_leaves_to_matvec(uint32_t type, int n_rows, int n_cols, int n_tok) {
+    const long long weights = (long long)n_rows * n_cols, M = 1 << 20;
+    if (n_cols <= 1024) return false;
+    const bool long_rows = n_cols >= 12288;
+    switch (type) {
+    case T_IQ4_NL: case T_IQ4_XS: return n_tok == 1 && (long_rows || weights >= 32 * M);
+    case T_IQ3_S: return n_tok == 1 && (long_rows || (weights > 16 * M && n_rows >= 4608));
+    case T_Q4_0: return n_tok == 1 && weights > 64 * M;
+    case T_IQ2_XXS:
+        return (n_tok == 1 && (n_cols >= 3072 || n_rows >= 4608)) || (n_tok == 2 && (long_rows || weights > 32 * M)) ||
+               (n_tok == 3 && weights > 64 * M && n_rows > 8192);
+    default: return false;
+    }
+}
+
 hipError_t launch_gemm_fewtok(uint32_t type, const FewtokCall &c) {
     switch (type) {
     case T_Q4_K: return fewtok_q4k(c);

@@ -1048,10 +1048,18 @@ size_t qlin_gemm_bf16_any_workspace_bytes(int n_rows, int n_cols) {
     return dense_gemm_weight_bytes(n_rows, n_cols) + kDenseLibWorkspace;
 }
 
+/* one to three tokens of a large tensor that the matvec serves better; it widens them into the workspace */
+static bool takes_matvec(uint32_t type, int n_rows, int n_cols, int n_tok, bool ws_ok) {
+    return ws_ok && n_cols % 256 == 0 && fewtok_leaves_to_matvec(type, n_rows, n_cols, n_tok);
+}
 /* the few-token kernel; the formats without a tile kernel keep to what they ask of the caller (a workspace) and to the
  * dense product that was chosen */
 static bool takes_fewtok(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool ws_ok) {
-    return fewtok_takes(type, n_rows, n_cols, n_tok, ldx) && (gemm_kq_wave4_covers(type) || (ws_ok && g.dense_gemm_mode == 0));
+    return fewtok_takes(type, n_rows, n_cols, n_tok, ldx) && (gemm_kq_wave4_covers(type) || (ws_ok && g.dense_gemm_mode == 0)) &&
+           !takes_matvec(type, n_rows, n_cols, n_tok, ws_ok);
+}
+static FusedTile takes_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool ws_ok) {
+    return takes_matvec(type, n_rows, n_cols, n_tok, ws_ok) ? kFusedNone : choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok);
 }
 
 int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
@@ -1067,8 +1075,6 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
         std::lock_guard<std::mutex> lk(g.mu);
         if (int rc = ensure_init_locked(0)) return rc;
     }
-    /* the formats with a tile kernel (gemm_kq_formats.h): decoded into the matrix operand inside the product, no workspace, in large or small
-     * tiles by the shape - except where decoding once into the caller's workspace measured faster */
     if (takes_fewtok(type, n_rows, n_cols, n_tok, ldx, ws_ok)) {
         HIP_TRY(launch_gemm_fewtok(type, {1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, (hipStream_t)stream}));
         return QLIN_OK;
@@ -1077,15 +1083,16 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
         HIP_TRY(launch_gemm_fewtok_one_by_one(type, {1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, (hipStream_t)stream}));
         return QLIN_OK;
     }
-    if (const FusedTile tile = choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok);
-        tile != kFusedNone) {
+    /* the formats with a tile kernel (gemm_kq_formats.h): decoded into the matrix operand inside the product, no workspace,
+     * in large or small tiles by the shape - except where decoding once into the caller's workspace measured faster */
+    if (const FusedTile tile = takes_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok); tile != kFusedNone) {
         HIP_TRY(launch_fused_tile(tile, type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
         return QLIN_OK;
     }
     if (!ws_ok)
         return fail(QLIN_ERR_ARG, "workspace must be 256-byte aligned and hold qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols) bytes");
-    /* up to four tokens of any other block format: each through the matvec (exact weights; 14336 x 4096 IQ4_XS, four
-     * tokens: 44 us against 95 us for decode + dense product), x widened to fp32 at the start of the workspace */
+    /* up to four tokens of any other block format, and what takes_matvec says: each through the matvec (exact weights;
+     * 14336 x 4096 IQ2_XXS, two tokens: 17 us, in the few-token kernel 20), x widened to fp32 at the start of the workspace */
     const size_t x_span = (size_t)(n_tok - 1) * ldx + n_cols; /* elements of X from the first token's to the last's */
     if (n_tok <= kMatvecTokens && type != T_F32 && type != T_F16 && type != T_BF16 && x_span <= (size_t)INT_MAX &&
         x_span * sizeof(float) <= workspace_bytes) { /* a very wide ldx: the dense route below */
@@ -1150,7 +1157,7 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
         if (!together) break;
         const bool mine_few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
-        const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(type) ? kFusedNone : choose_fused_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         together = (mine_few || mine != kFusedNone) && (i == 0 || (mine == tile && mine_few == few));
         tile = mine;
         few = mine_few;
@@ -1324,7 +1331,7 @@ int qlin_probe_clocks(void *stream, double *shader_mhz) {
 
 int qlin_probe_gemm_route(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, int have_workspace) {
     if (takes_fewtok(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0)) return 3;
-    return (int)choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0);
+    return (int)takes_tile(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0);
 }
 
 int qlin_probe_gemm_tile(int tile, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,

@@ -130,6 +130,7 @@ struct FewtokCall {
 bool fewtok_has(uint32_t type);
 int fewtok_unrounded(uint32_t type); /* token count up to which the codes stay unrounded */
 bool fewtok_takes(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx);
+bool fewtok_leaves_to_matvec(uint32_t type, int n_rows, int n_cols, int n_tok);
 hipError_t launch_gemm_fewtok(uint32_t type, const FewtokCall &c);
 hipError_t launch_gemm_fewtok_one_by_one(uint32_t type, const FewtokCall &c); /* any ldx */
 hipError_t fewtok_q4k(const FewtokCall &c);

@@ -242,7 +242,8 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * to 48 tokens, up to 64 where a tensor has at most 8192 rows and up to 128 where it has at most 5120 (somewhat less
  * for rows of fewer than 2048 elements). A token with an infinity or a NaN leaves the others alone; with unrounded codes
  * its own results may be NaN where exact arithmetic gives an infinity. Up to 4 tokens of any other
- * block format go one by one through the matvec kernels (exact weights, ~1e-6; the workspace holds their
+ * block format and, given a workspace, one token of a large IQ4_NL, IQ4_XS, IQ3_S or Q4_0 tensor and one to three of an
+ * IQ2_XXS tensor go one by one through the matvec kernels (exact weights, ~1e-6; the workspace holds their
  * activations as fp32, and when ldx is so wide that (n_tok - 1) * ldx + n_cols floats do not fit it they take the
  * decode + dense route). workspace: device memory, 256-byte aligned, at least
  * qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols) bytes (2 bytes per weight + 32 MiB for the library);

@@ -113,3 +113,26 @@ def test_unrounded_codes_keep_fp32_precision(oracle, tid, n_tok):
         b.free()
     want = synth.bf16_bits_to_f32(Xb).astype(np.float64) @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T
     assert rel_l2(Y, want) <= UNROUNDED_BAR, (NAME[tid], n_tok, rel_l2(Y, want) * 2.0 ** 24)
+
+
+@pytest.mark.parametrize("tid,n_rows,n_cols,n_tok", [
+    (synth.GGML_IQ4_NL, 70, 12288, 1), (synth.GGML_IQ4_XS, 70, 12288, 1), (synth.GGML_IQ3_S, 70, 12288, 1), (synth.GGML_IQ2_XXS, 70, 3072, 1),
+    (synth.GGML_IQ2_XXS, 4610, 1280, 1), (synth.GGML_IQ2_XXS, 70, 12288, 2)], ids=str)
+def test_tokens_that_go_to_the_matvec(oracle, tid, n_rows, n_cols, n_tok):
+    """exact weights as in the few-token kernel, rows of X and Y at a distance, nothing written between them"""
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid)
+    Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_tok, tokens=n_tok))
+    ldx, ldy = n_cols + 8, n_rows + 3
+    Xpad = np.full((n_tok, ldx), 0x7FC0, np.uint16)
+    Xpad[:, :n_cols] = Xb
+    assert qlinear.load().qlin_probe_gemm_route(tid, n_rows, n_cols, n_tok, ldx, 1) == 0
+    dW, dX, dY = qlinear.DevBuf.from_numpy(W), qlinear.DevBuf.from_numpy(Xpad), qlinear.DevBuf.from_numpy(np.full((n_tok, ldy), -3.0, np.float32))
+    ws = qlinear.DevBuf(qlinear.gemm_bf16_any_workspace_bytes(n_rows, n_cols))
+    qlinear.gemm_bf16_any_dev(tid, dW, dX, dY, n_rows, n_cols, n_tok, ldx, ldy, ws)
+    qlinear.sync()
+    Y = dY.to_numpy(np.float32, (n_tok, ldy))
+    for b in (dW, dX, dY, ws):
+        b.free()
+    assert np.all(Y[:, n_rows:] == -3.0)
+    want = synth.bf16_bits_to_f32(Xb).astype(np.float64) @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T
+    assert rel_l2(Y[:, :n_rows], want) <= 2e-6

@@ -31,3 +31,18 @@ def test_unrounded_tokens_stay_unrounded(tid):
     n = 32 if tid == synth.GGML_Q4_K else 4 if tid in (synth.GGML_Q4_0, synth.GGML_IQ4_NL, synth.GGML_IQ4_XS) else 24
     for n_rows, n_cols in [(16, 256), (50000, 256), (50000, 4096), (300, 16384)]:
         assert route(tid, n_rows, n_cols, n) == FEW
+
+
+@pytest.mark.parametrize("tid,n_rows,n_cols,n_tok,matvec", [
+    (synth.GGML_IQ4_NL, 4096, 4096, 1, False), (synth.GGML_IQ4_NL, 8192, 4096, 1, True), (synth.GGML_IQ4_NL, 8192, 4096, 2, False),
+    (synth.GGML_IQ4_NL, 40000, 1024, 1, False), (synth.GGML_IQ4_XS, 64, 12288, 1, True), (synth.GGML_IQ4_XS, 64, 12032, 1, False),
+    (synth.GGML_IQ3_S, 4607, 4096, 1, False), (synth.GGML_IQ3_S, 4608, 4096, 1, True), (synth.GGML_IQ3_S, 8192, 2048, 1, False),
+    (synth.GGML_Q4_0, 16384, 4096, 1, False), (synth.GGML_Q4_0, 16385, 4096, 1, True),
+    (synth.GGML_IQ2_XXS, 64, 2816, 1, False), (synth.GGML_IQ2_XXS, 64, 3072, 1, True), (synth.GGML_IQ2_XXS, 4608, 2048, 1, True),
+    (synth.GGML_IQ2_XXS, 4096, 4096, 2, False), (synth.GGML_IQ2_XXS, 8193, 4096, 2, True), (synth.GGML_IQ2_XXS, 64, 12288, 2, True),
+    (synth.GGML_IQ2_XXS, 8192, 14336, 3, False), (synth.GGML_IQ2_XXS, 8193, 14336, 3, True), (synth.GGML_IQ2_XXS, 8193, 14336, 4, False),
+    (synth.GGML_Q4_K, 151936, 4096, 1, False), (synth.GGML_Q8_0, 151936, 4096, 1, False)])
+def test_single_tokens_of_large_tensors_go_to_the_matvec(tid, n_rows, n_cols, n_tok, matvec):
+    assert route(tid, n_rows, n_cols, n_tok) == (MATVEC if matvec else FEW)
+    if tid not in (synth.GGML_IQ3_S, synth.GGML_IQ2_XXS):
+        assert route(tid, n_rows, n_cols, n_tok, have_workspace=0) == FEW  # nowhere to widen the activations
