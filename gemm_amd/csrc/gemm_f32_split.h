@@ -20,8 +20,8 @@
  *                   an image of its own by load-to-LDS requests, the fragments of 32 elements come into a ring of
  *                   stages that the waves share, one barrier per stage. K is divided over workgroups where the tiles alone
  *                   do not fill the chip; every part writes its sums to the workspace
- *   f32_finish      adds the parts in order, takes the power of two back; tokens that are not finite are computed as
- *                   the plain fp32 sum
+ *   f32_finish      adds the parts in order, takes the power of two back; tokens that are not finite get what
+ *                   the plain fp32 sum gives: infinities and NaN
  *
  * What bounds it: a wave multiplies for a third of its time, the rest are waits at the stage barrier and for the matrix
  * unit's results, with two waves per SIMD to fill them (Q4_K 512 tokens 14336 x 4096: 438 TFLOP/s counted once, 876 of
@@ -370,9 +370,12 @@ gemm_f32_split_kernel(SplitArgs p) {
         }
 }
 
-/* Adds the parts of K in order (one part: the product has written Y itself) and computes the tokens that hold an infinity
- * or a NaN, whose fragments are zeros, as the plain fp32 sum. A thread has R rows: four where rows of Y and of the parts
- * allow 16-byte accesses. */
+/* Adds the parts of K in order (one part: the product has written Y itself) and completes the tokens that hold an infinity
+ * or a NaN, whose fragments are zeros. Only those elements decide such a result - an infinity, or a NaN where the products
+ * with them do not agree - so a workgroup collects them a stretch of K at a time and decodes no more than their weights, a
+ * row only until it is NaN (64 tokens 4096 x 4096, one token not finite: a thread walking whole rows 845 us, now 38). Rows with
+ * weights that are not finite have a NaN from the product. A thread has R rows: four where rows of Y and of the parts allow
+ * 16-byte accesses. */
 template <uint32_t T, int R>
 __global__ void __launch_bounds__(256) f32_finish_kernel(const uint8_t *__restrict__ W, const float *__restrict__ X, const float *__restrict__ part,
                                                         const int *__restrict__ token_exp, float *__restrict__ Y, int n_rows, int n_cols, int n_tok,
@@ -381,28 +384,48 @@ __global__ void __launch_bounds__(256) f32_finish_kernel(const uint8_t *__restri
     typedef float vec __attribute__((ext_vector_type(R)));
     const int row = (blockIdx.x * 256 + threadIdx.x) * R, t = blockIdx.y;
     const int e = token_exp[t];
-    if (row >= n_rows || (parts == 1 && e != kF32NotFinite)) return;
+    if (parts == 1 && e != kF32NotFinite) return;
+    vec *out = reinterpret_cast<vec *>(Y + (size_t)t * ldy + row);
     vec sum = 0.0f;
-    if (e != kF32NotFinite) {
+    if (row < n_rows) {
+        if (parts == 1) sum = *out;
         const float *at = part + (size_t)t * n_rows + row;
+        if (parts > 1) {
 #pragma unroll 4
-        for (int s = 0; s < parts; s++) sum += *reinterpret_cast<const vec *>(at + (size_t)s * n_tok * n_rows);
-#pragma unroll
-        for (int i = 0; i < R; i++) sum[i] = __builtin_ldexpf(sum[i], -e);
-    } else {
-        const float *x = X + (size_t)t * ldx;
-        for (int i = 0; i < R; i++) {
-            const uint8_t *w = W + (size_t)(row + i) * ((size_t)(n_cols / C::BE) * C::BB);
-            float one = 0.0f;
-            for (int k = 0; k < n_cols; k += 8) {
-                float v[8];
-                C::decode8(w + (size_t)(k / C::BE) * C::BB, k % C::BE, v);
-                for (int l = 0; l < 8; l++) one += v[l] * x[k + l];
-            }
-            sum[i] = one;
+            for (int s = 0; s < parts; s++) sum += *reinterpret_cast<const vec *>(at + (size_t)s * n_tok * n_rows);
         }
     }
-    *reinterpret_cast<vec *>(Y + (size_t)t * ldy + row) = sum;
+    if (e != kF32NotFinite) {
+#pragma unroll
+        for (int i = 0; i < R; i++) sum[i] = __builtin_ldexpf(sum[i], -e);
+    } else { /* the same for the whole workgroup */
+        constexpr int kStretch = 1024;
+        __shared__ int found[kStretch], n_found;
+        const uint32_t *x = reinterpret_cast<const uint32_t *>(X + (size_t)t * ldx);
+        for (int k0 = 0; k0 < n_cols; k0 += kStretch) {
+            if (threadIdx.x == 0) n_found = 0;
+            __syncthreads();
+            for (int k = k0 + threadIdx.x; k < min(k0 + kStretch, n_cols); k += 256)
+                if ((x[k] & 0x7F800000u) == 0x7F800000u) found[atomicAdd(&n_found, 1)] = k;
+            __syncthreads();
+            bool open = row < n_rows; /* a result that is not NaN yet */
+            for (int n = 0; n < n_found && open; n++) {
+                const int k = found[n];
+                open = false;
+                for (int i = 0; i < R; i++) {
+                    if (sum[i] != sum[i]) continue;
+                    open = true;
+                    float v[8], w = 0.0f;
+                    C::decode8(W + (size_t)(row + i) * ((size_t)(n_cols / C::BE) * C::BB) + (size_t)(k / C::BE) * C::BB, k % C::BE & ~7, v);
+#pragma unroll
+                    for (int l = 0; l < 8; l++) w = (k & 7) == l ? v[l] : w;
+                    sum[i] += w * __uint_as_float(x[k]);
+                }
+            }
+            if (!__syncthreads_or(open)) break;
+        }
+    }
+    if (row < n_rows) *out = sum;
 }
 
 template <class F, int TM> hipError_t split_launch(const F32SplitCall &c, const SplitArgs &base) {

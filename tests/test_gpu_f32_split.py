@@ -81,6 +81,37 @@ def test_magnitudes_and_not_finite(oracle, tid, n_rows):
 
 
 @pytest.mark.parametrize("tid", TYPES, ids=lambda t: NAME[t])
+@pytest.mark.parametrize("n_tok,n_rows,n_cols", [(9, 1030, 2304), (33, 24003, 256), (66, 65540, 256)])
+def test_tokens_that_are_not_finite(oracle, tid, n_tok, n_rows, n_cols):
+    """what the sum over K gives them, wherever and however many their infinities and NaN are, at the ends of the stretches
+    of K that are searched together too; K in parts and in one, rows one and four to a thread; neighbours bit for bit as
+    without them"""
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid + 1)
+    X = synth.make_activation(n_cols, seed=n_tok, tokens=n_tok)
+    clean = product(tid, W, X, n_rows, n_cols)
+    last = n_cols - 1
+    X[0, last] = np.inf
+    X[1, [0, last]] = np.inf, np.inf
+    X[2, [3, last]] = -np.inf, np.inf
+    X[3, :] = np.inf
+    X[4, :] = np.nan
+    X[5, last // 2:] = -np.inf
+    X[7, [min(1023, last), min(1024, last - 1)]] = -np.inf, -np.inf
+    X[8, 5] = np.nan
+    bad = [0, 1, 2, 3, 4, 5, 7, 8]
+    Y = product(tid, W, X, n_rows, n_cols)
+    good = np.setdiff1d(np.arange(n_tok), bad)
+    assert np.array_equal(Y[good].view(np.uint32), clean[good].view(np.uint32))
+    at = np.unique(np.r_[0:60, n_rows // 2:n_rows // 2 + 60, n_rows - 60:n_rows])
+    dec = oracle.dequant_matrix(tid, W[at], n_cols).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = np.stack([(X[t].astype(np.float64) * dec).sum(axis=1) for t in bad])
+    got = Y[bad][:, at]
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
+
+
+@pytest.mark.parametrize("tid", TYPES, ids=lambda t: NAME[t])
 @pytest.mark.parametrize("n_tok,n_rows,n_cols", [(9, 8193, 256), (40, 1030, 2304)])
 def test_tensor_anywhere_in_its_buffer(oracle, tid, n_tok, n_rows, n_cols):
     """a tensor that starts 2 bytes into a buffer and ends with it: blocks are read from any even address, and the requests
