@@ -183,17 +183,11 @@ F32SplitPlan f32_split_plan(uint32_t type, int n_rows, int n_cols, int n_tok, si
 /* Whole super-blocks of the formats whose codes an image gives up, in a workspace that holds the fragments of 32 tokens, from
  * 2.25 M weights on (2 M up to 32 tokens): below, four launches cost more than decoding and the library's product do (us,
  * this route / that one, Q4_K: 64 tokens 1536 x 1536 17.8 / 19.4 but 2048 x 1024 16.6 / 16.1 and 512 x 4096 19.5 / 17.2; 512
- * tokens 1024 x 1024 21.5 / 18.3; 32 tokens 512 x 4096 16.1 / 19.7 but 512 x 2048 14.4 / 13.2; Q6_K the same). From 3 M for
- * 33 to 128 tokens of rows of one or two super-blocks, which leave few parts to divide K into (128 tokens 4608 x 512
- * IQ4_NL 24.1 / 20.9, but 16384 x 256 at 64 18.1 / 23.2). The grid formats, whose tables cost them more, from 2.25 M at any
- * token count and from 3 M for 33 to 64 tokens (IQ2_XXS 16 tokens 512 x 4096 18.6 / 17.2 but 2304 x 1024 16.2 / 16.7; 64
- * tokens 640 x 4096 23.1 / 19.7 but 3072 x 1024 20.5 / 21.0). The 32-bit offsets of a request hold a wave's 64 rows and a
- * token tile's fragments. */
+ * tokens 1024 x 1024 21.5 / 18.3; 32 tokens 512 x 4096 16.1 / 19.7 but 512 x 2048 14.4 / 13.2; Q6_K the same). The 32-bit
+ * offsets of a request hold a wave's 64 rows and a token tile's fragments. */
 bool f32_split_takes(uint32_t type, int n_rows, int n_cols, int n_tok, size_t workspace_bytes) {
     const long long weights = (long long)n_rows * n_cols;
-    const bool grid = type == T_IQ3_S || type == T_IQ2_XXS;
-    const bool three = n_tok > 32 && ((n_cols <= 512 && n_tok <= 128) || (grid && n_tok <= 64));
-    if (weights < (three ? 12LL << 18 : n_tok <= 32 && !grid ? 8LL << 18 : 9LL << 18)) return false;
+    if (weights < (n_tok <= 32 ? 8LL << 18 : 9LL << 18)) return false;
     return fewtok_has(type) && n_cols % 256 == 0 && n_cols <= (1 << 22) && f32_split_plan(type, n_rows, n_cols, 32, workspace_bytes).fits;
 }
 

@@ -1,6 +1,5 @@
-"""Which kernel qlin_gemm_bf16_any_dev and qlin_gemm_f32_any_dev choose, at both sides of every limit of the few-token kernel
-and of the split fp32 product. CPU only: the choice is a function of format and shape (qlin_probe_gemm_route: 0 matvec or
-decode + dense, 1 and 2 the tile kernels, 3 few tokens; qlin_probe_gemm_f32_route: 1 the split product)."""
+"""Which kernel qlin_gemm_bf16_any_dev chooses, at both sides of every limit of the few-token kernel. CPU only: the choice
+is a function of format and shape (qlin_probe_gemm_route: 0 matvec or decode + dense, 1 and 2 the tile kernels, 3 few tokens)."""
 import pytest
 
 from gemm_amd import qlinear
@@ -47,15 +46,3 @@ def test_single_tokens_of_large_tensors_go_to_the_matvec(tid, n_rows, n_cols, n_
     assert route(tid, n_rows, n_cols, n_tok) == (MATVEC if matvec else FEW)
     if tid not in (synth.GGML_IQ3_S, synth.GGML_IQ2_XXS):
         assert route(tid, n_rows, n_cols, n_tok, have_workspace=0) == FEW  # nowhere to widen the activations
-
-
-@pytest.mark.parametrize("tid", ALL + (synth.GGML_IQ3_S, synth.GGML_IQ2_XXS), ids=lambda t: synth.TYPE_NAMES[t])
-def test_fp32_products_that_multiply_codes(tid):
-    grid = tid in (synth.GGML_IQ3_S, synth.GGML_IQ2_XXS)
-    for n_rows, n_cols, n_tok, split in [
-            (8192, 4096, 7, False), (8192, 4096, 8, True), (8192, 4128, 64, False), (2048, 1024, 8, not grid), (2047, 1024, 8, False),
-            (2304, 1024, 32, True), (2303, 1024, 33, False), (2304, 1024, 33, not grid), (3072, 1024, 64, True), (2304, 1024, 65, True),
-            (4608, 512, 33, False), (6144, 512, 33, True), (6143, 512, 128, False), (4608, 512, 129, True), (9216, 256, 32, True),
-            (12287, 256, 128, False), (12288, 256, 128, True)]:
-        assert qlinear.load().qlin_probe_gemm_f32_route(tid, n_rows, n_cols, n_tok) == split, (n_rows, n_cols, n_tok)
-    assert not qlinear.load().qlin_probe_gemm_f32_route(synth.GGML_Q4_1, 8192, 4096, 64)
