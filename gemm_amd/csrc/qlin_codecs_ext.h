@@ -90,14 +90,23 @@ __device__ __forceinline__ float ue4m3_half(uint32_t x) {
     return (float)(8u + man) * __uint_as_float((e + 116u) << 23); /* (8+man) * 2^(e-11) */
 }
 
-/* MXFP4 [e][qs 16]: E2M1x2[nibble] * 2^(e-128); blocks are 17 bytes, so only byte loads (:2818-2830) */
+/* four E2M1x2 values (0 1 2 3 4 6 8 12, negated from nibble 8 on) with 12 added: byte_f32 - 12 is +0 for both zeros */
+__device__ __forceinline__ uint32_t e2m1_bytes(uint32_t nib) {
+    const uint32_t i7 = nib & 0x07070707u;
+    const uint32_t pos = __builtin_amdgcn_perm(0x18141210u, 0x0F0E0D0Cu, i7), neg = __builtin_amdgcn_perm(0x00040608u, 0x090A0B0Cu, i7);
+    const uint32_t m = ((nib >> 3) & 0x01010101u) * 255u;
+    return (m & neg) | (~m & pos);
+}
+
+/* MXFP4 [e][qs 16]: E2M1x2[nibble] * 2^(e-128); 17-byte blocks, so loads at any address (:2818-2830). 14336 x 4096 to
+ * fp32, with a table lookup per element before: 76 -> 48.5 us */
 template <> struct Codec<T_MXFP4> : Geom<T_MXFP4> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const float d = e8m0_half(blk[0]);
-        const uint8_t *q = blk + 1 + (k0 & 15);
-        const int sh = (k0 >> 4) * 4;
+        const Dwords2 n = bytes_at(ld_2xu32(blk + 1 + (k0 & 15)), (k0 >> 4) * 4, 15u);
+        const Dwords2 q = {e2m1_bytes(n.x), e2m1_bytes(n.y)};
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = (float)qlin_mxfp4_values[(q[i] >> sh) & 15] * d;
+        for (int i = 0; i < 8; i++) y[i] = (byte_f32(q, i) - 12.0f) * d;
     }
 };
 
@@ -106,10 +115,10 @@ template <> struct Codec<T_NVFP4> : Geom<T_NVFP4> {
     __device__ static void decode8(const uint8_t *blk, int k0, float (&y)[8]) {
         const int s = k0 >> 4;
         const float d = ue4m3_half(blk[s]);
-        const uint8_t *q = blk + 4 + 8 * s;
-        const int sh = ((k0 >> 3) & 1) * 4;
+        const Dwords2 n = bytes_at(ld_2xu32(blk + 4 + 8 * s), ((k0 >> 3) & 1) * 4, 15u);
+        const Dwords2 q = {e2m1_bytes(n.x), e2m1_bytes(n.y)};
 #pragma unroll
-        for (int i = 0; i < 8; i++) y[i] = (float)qlin_mxfp4_values[(q[i] >> sh) & 15] * d;
+        for (int i = 0; i < 8; i++) y[i] = (byte_f32(q, i) - 12.0f) * d;
     }
 };
 
