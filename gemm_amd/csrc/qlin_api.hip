@@ -1334,6 +1334,10 @@ int qlin_probe_gemm_route(uint32_t type, int n_rows, int n_cols, int n_tok, int 
     return (int)takes_tile(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0);
 }
 
+int qlin_probe_gemm_f32_route(uint32_t type, int n_rows, int n_cols, int n_tok) {
+    return n_tok >= kDenseMinTokens && f32_split_takes(type, n_rows, n_cols, n_tok, qlin_gemm_f32_any_workspace_bytes(n_rows, n_cols));
+}
+
 int qlin_probe_gemm_tile(int tile, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                          int n_tok, int ldx, int ldy, void *stream) {
     if (tile < 0 || tile > 1) return fail(QLIN_ERR_ARG, "tile: 0 (256 x 128) or 1 (128 x 64)");

@@ -29,8 +29,11 @@ int qlin_probe_hbm_read(const void *buf, size_t n_bytes, void *stream);
  * workspace; Q4_K, Q5_K, Q6_K, Q8_0, IQ4_NL, IQ4_XS, Q4_0; n_cols % 256 == 0. For timing one against the other and for the parity tests of
  * each on small shapes. */
 /* which kernel qlin_gemm_bf16_any_dev picks for a shape: 1 = the 256 x 128 tile kernel, 2 = the 128 x 64 one, 3 = the
- * few-token kernel, 0 = none of them (decode to bf16 + dense product) */
+ * few-token kernel, 0 = none of them (a matvec per token, or decode to bf16 + dense product) */
 int qlin_probe_gemm_route(uint32_t ggml_type, int n_rows, int n_cols, int n_tok, int ldx, int have_workspace);
+/* whether qlin_gemm_f32_any_dev multiplies a shape's codes on the matrix cores (1) or decodes to fp32 for the library's
+ * product, or takes the few-token fp32 kernel (0), given a workspace of qlin_gemm_f32_any_workspace_bytes bytes */
+int qlin_probe_gemm_f32_route(uint32_t ggml_type, int n_rows, int n_cols, int n_tok);
 int qlin_probe_gemm_tile(int tile, uint32_t ggml_type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                          int n_tok, int ldx, int ldy, void *stream);
 

@@ -1,8 +1,9 @@
 """GPU parity of the fp32 product on the matrix cores (activations as two fp16 numbers, codes unrounded) at the sizes where
 it can go wrong: one and two blocks of 32 tokens and one token past them, ragged row tiles, one super-block and more than
 there are parts, K in one part and in several, workspaces that hold only some of the tokens, rows of X at any alignment,
-tokens of very different magnitude, infinities and NaN; and one shape just too small for it. Bar 1e-6: an activation keeps 2^-24 of itself (6e-8), the sums are
-fp32 sums over at most 256 products and 64 super-blocks."""
+tokens of very different magnitude, magnitudes that differ within a token, infinities and NaN; and one shape just too small
+for it. Bar 1e-6: an activation keeps 23 bits (2^-23 = 1.2e-7 of itself at most), the sums are fp32 sums over at most 256
+products and 64 super-blocks."""
 import numpy as np
 import pytest
 
@@ -33,7 +34,12 @@ def product(tid, W, X, n_rows, n_cols, pad=0, ldy=None):
     return Y[:, :n_rows]
 
 
+def takes_codes(tid, n_rows, n_cols, n_tok):
+    return qlinear.load().qlin_probe_gemm_f32_route(tid, n_rows, n_cols, n_tok) == 1
+
+
 def check(oracle, tid, n_tok, n_rows, n_cols, pad=0):
+    assert takes_codes(tid, n_rows, n_cols, n_tok) == ((n_tok, n_rows, n_cols) != (64, 2303, 1024))
     W = synth.make_weights(tid, n_rows, n_cols, seed=tid + n_tok + n_rows)
     X = synth.make_activation(n_cols, seed=n_tok + n_cols, tokens=n_tok)
     Y = product(tid, W, X, n_rows, n_cols, pad, n_rows + 3)
@@ -131,3 +137,45 @@ def test_tensor_anywhere_in_its_buffer(oracle, tid, n_tok, n_rows, n_cols):
     assert np.array_equal(got, want)
     exact = X.astype(np.float64) @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T
     assert rel_l2(got, exact) <= TOL
+
+
+@pytest.mark.parametrize("n_tok,n_rows,n_cols", [(9, 8229, 256), (40, 1030, 2304)])
+@pytest.mark.parametrize("tid", [t for t in TYPES if t not in (synth.GGML_Q4_K, synth.GGML_Q5_K, synth.GGML_Q2_K)], ids=lambda t: NAME[t])
+def test_one_hot_activations_return_the_codec_values(oracle, tid, n_tok, n_rows, n_cols):
+    """bit for bit where a format subtracts no minimum: code times scales has at most 24 bits, in whatever order"""
+    assert takes_codes(tid, n_rows, n_cols, n_tok)
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid)
+    ks = ([0, 1, 15, 16, 31, 32, 127, 128, n_cols - 1] + list(range(2, n_cols, 97)))[:n_tok]
+    X = np.zeros((n_tok, n_cols), np.float32)
+    X[np.arange(len(ks)), ks] = 1.0
+    Y = product(tid, W, X, n_rows, n_cols)
+    assert np.array_equal(Y[:len(ks)], oracle.dequant_matrix(tid, W, n_cols)[:, ks].T)
+    assert not Y[len(ks):].any()
+
+
+@pytest.mark.parametrize("apart", [10, 15, 22, 30])
+@pytest.mark.parametrize("n_rows,n_cols", [(8229, 256), (1030, 2304)])
+def test_magnitudes_that_differ_within_a_token(oracle, n_rows, n_cols, apart):
+    """one element 2^apart above the others. Rows whose weight of it is not zero are as precise as ever. Rows where it is
+    zero show what the others keep: 2^-23 of themselves, and no less than 2^-39 of the largest (half a unit of the second
+    fp16 number's subnormals, 2^-25, in a token scaled to [2^14, 2^15))"""
+    tid, n_tok, big = synth.GGML_Q8_0, 12, 70
+    W = np.ascontiguousarray(synth.make_weights(tid, n_rows, n_cols, seed=apart)).view(np.uint8).reshape(n_rows, -1)
+    code = 34 * (big // 32) + 2 + big % 32
+    zero = np.arange(n_rows) % 2 == 1
+    W[zero, code] = 0
+    W[~zero, code] |= 1
+    X = synth.make_activation(n_cols, seed=3, tokens=n_tok)
+    X[:, big] = np.ldexp(np.abs(X).max(axis=1), apart)
+    assert takes_codes(tid, n_rows, n_cols, n_tok)
+    Y = product(tid, W, X, n_rows, n_cols)
+    dec = oracle.dequant_matrix(tid, W, n_cols).astype(np.float64)
+    want = X.astype(np.float64) @ dec.T
+    assert rel_l2(Y[:, ~zero], want[:, ~zero]) <= TOL
+    kept = np.maximum(2.0 ** -23 * np.abs(X), 2.0 ** -39 * np.abs(X[:, [big]])).astype(np.float64)
+    kept[:, big] = 0.0
+    small = np.abs(X).astype(np.float64)
+    small[:, big] = 0.0
+    assert np.all(np.abs(Y - want)[:, zero] <= (kept + TOL * small) @ np.abs(dec[zero]).T)
+    if apart <= 15:  # an ordinary outlier: the rows that do not see it keep the bar too
+        assert rel_l2(Y[:, zero], want[:, zero]) <= TOL

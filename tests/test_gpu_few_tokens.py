@@ -136,3 +136,29 @@ def test_tokens_that_go_to_the_matvec(oracle, tid, n_rows, n_cols, n_tok):
     assert np.all(Y[:, n_rows:] == -3.0)
     want = synth.bf16_bits_to_f32(Xb).astype(np.float64) @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T
     assert rel_l2(Y[:, :n_rows], want) <= 2e-6
+
+
+@pytest.mark.parametrize("n_tok", [3, 8, 16, 24, 40])
+@pytest.mark.parametrize("tid", sorted(EXACT_MAX), ids=lambda t: NAME[t])
+def test_a_token_that_is_not_finite_leaves_the_others_alone(tid, n_tok):
+    """also where two tokens share an operand of zeros and eight-token halves"""
+    n_rows, n_cols = 70, 2304
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid)
+    Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_tok, tokens=n_tok))
+    bad = np.unique([1, n_tok // 2 + 1, n_tok - 1])
+    got = []
+    for spoil in (False, True):
+        X = Xb.copy()
+        if spoil:
+            X[bad[0], 5], X[bad[-1], 700], X[bad[0], n_cols - 1] = 0x7F80, 0x7FC0, 0xFF80
+        dW, dX, dY = qlinear.DevBuf.from_numpy(W), qlinear.DevBuf.from_numpy(X), qlinear.DevBuf(n_tok * n_rows * 4)
+        ws = qlinear.DevBuf(qlinear.gemm_bf16_any_workspace_bytes(n_rows, n_cols))
+        qlinear.gemm_bf16_any_dev(tid, dW, dX, dY, n_rows, n_cols, n_tok, n_cols, n_rows, ws)
+        qlinear.sync()
+        got.append(dY.to_numpy(np.uint32, (n_tok, n_rows)))
+        for b in (dW, dX, dY, ws):
+            b.free()
+    rest = np.setdiff1d(np.arange(n_tok), [bad[0], bad[-1]])
+    assert np.array_equal(got[0][rest], got[1][rest])
+    spoiled = got[1][[bad[0], bad[-1]]].view(np.float32)
+    assert not np.isfinite(spoiled).any()

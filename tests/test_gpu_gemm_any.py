@@ -50,7 +50,7 @@ KQ = {synth.GGML_Q6_K, synth.GGML_Q5_K, synth.GGML_Q3_K, synth.GGML_Q2_K, synth.
 def streams_exact_weights(tid, n_tok, n_rows, n_cols):
     """few tokens of these formats go through a kernel that multiplies the unrounded weights; up to four tokens of any
     other block format (Q4_K has its own route) go through the matvec"""
-    if tid in KQ and n_tok <= 24 and n_cols % 256 == 0 and n_rows * synth.row_bytes(tid, n_cols) % 16 == 0:
+    if tid in KQ and n_tok <= 24 and n_cols % 256 == 0:
         return True
     return n_tok <= 4 and tid not in synth.DENSE_TYPES and tid != synth.GGML_Q4_K
 
@@ -181,13 +181,18 @@ def run_multi(tid, Ws, Xpad, rows, n_cols, n_tok, ldx, ldys, together, ws_bytes=
     ((256, 64, 70), 512, 130),   # ragged last tiles of the second and third tensor, two token tiles
     ((130, 129), 1280, 64),      # two tensors, neither a whole number of tiles
     ((64, 64, 64), 256, 33),     # one tile each, one super-block
+    ((130, 129), 1280, 129),     # the same three in the small-tile kernel
+    ((64, 64, 64), 256, 200),
+    ((70, 1, 300), 768, 100),    # and in the few-token kernel
     ((6400, 6500), 256, 1024),   # 200 and more 256-token x 128-row tiles each: the large-tile kernel
 ])
 def test_several_tensors_in_one_launch_equal_one_call_each(oracle, tid, rows, n_cols, n_tok):
-    """qlin_gemm_bf16_multi_dev on shapes where every tensor takes the same tile kernel: bit for bit what one call per
+    """qlin_gemm_bf16_multi_dev on shapes where every tensor takes the same kernel: bit for bit what one call per
     tensor gives (the same workgroups run, numbered through the tensors), right against the oracle, and nothing written
     past a tensor's rows"""
     rows = list(rows)
+    routes = [qlinear.load().qlin_probe_gemm_route(tid, r, n_cols, n_tok, n_cols + 8, 0) for r in rows]
+    assert routes == [1 if rows[0] == 6400 else 2 if n_tok > 128 else 3] * len(rows)
     Ws, Xb, Xpad, ldx, ldys = multi_case(tid, rows, n_cols, n_tok, seed=500 + tid)
     one_by_one = run_multi(tid, Ws, Xpad, rows, n_cols, n_tok, ldx, ldys, together=False)
     together = run_multi(tid, Ws, Xpad, rows, n_cols, n_tok, ldx, ldys, together=True)

@@ -4,9 +4,8 @@ Two bars per case:
   * the contract: relative L2 <= 2e-3 against a double-precision-accumulated reference that
     uses the EXACT fp32 decoded weights (the CPU oracle) and the same bf16-rounded activations;
   * the arithmetic: relative L2 <= 2e-5 against a double-precision reference of what the kernel
-    is designed to compute, so that only fp32 accumulation order is left: from 49 tokens on
-    the decoded weights rounded to bf16 (nearest even), up to FEW_TOKENS = 32 tokens the exact
-    weights (the few-token kernel does not round them).
+    is designed to compute, so that only fp32 accumulation order is left: up to FEW_TOKENS = 32
+    tokens the exact weights, beyond them the decoded weights rounded to bf16 (nearest even).
 """
 import numpy as np
 import pytest
@@ -33,6 +32,13 @@ def run_gemm(W, Xb, n_rows, n_cols, n_tok, ldx=None, ldy=None):
     return dY.to_numpy(np.float32, (n_tok, ldy))
 
 
+TILES = (1, 2)
+
+
+def route(n_rows, n_cols, n_tok):
+    return qlinear.load().qlin_probe_gemm_route(Q4K, n_rows, n_cols, n_tok, n_cols, 0)
+
+
 def references(oracle, W, Xb, n_cols):
     dec = oracle.dequant_matrix(Q4K, W, n_cols)
     Xf = synth.bf16_bits_to_f32(Xb).astype(np.float64)
@@ -47,10 +53,14 @@ def references(oracle, W, Xb, n_cols):
     (300, 257, 2048), (512, 1024, 4096), (33, 1000, 768), (16, 14336, 256), (17, 48, 512), (48, 100, 256),
     (49, 100, 256), (3, 16, 2560),
     (260, 12805, 256), (1030, 5130, 512),  # enough tiles for the 128-row variant of the kernel
-    # 49..128 tokens: 128-token tiles; more than a chip's worth of them (K stays whole), an odd super-block count
+    # 49..128 tokens: the few-token kernel where it has few row tiles; more than a chip's worth of 128-token tiles
     (128, 16500, 1024), (100, 20000, 512), (90, 130, 768), (65, 70, 2048),
+    # more tokens than the few-token kernel takes: small tiles of one and two token blocks, one super-block, an odd count
+    (129, 130, 768), (140, 70, 2048), (129, 100, 256), (257, 300, 1280),
 ])
 def test_gemm_bf16_shapes(oracle, n_tok, n_rows, n_cols):
+    if n_tok > 128:
+        assert route(n_rows, n_cols, n_tok) in TILES
     W = synth.make_weights(Q4K, n_rows, n_cols, seed=n_rows + n_tok)
     Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_cols + n_tok, tokens=n_tok))
     Y = run_gemm(W, Xb, n_rows, n_cols, n_tok)
@@ -59,9 +69,10 @@ def test_gemm_bf16_shapes(oracle, n_tok, n_rows, n_cols):
     assert rel_l2(Y, exact) <= 2e-3, (n_tok, n_rows, n_cols)
 
 
-@pytest.mark.parametrize("n_tok", [30, 72])  # few-token kernel, tile kernel
-def test_gemm_bf16_strides_and_untouched_padding(oracle, n_tok):
+@pytest.mark.parametrize("n_tok,tiles", [(30, False), (72, False), (160, True)])  # few-token kernel unrounded, rounded; tile kernel
+def test_gemm_bf16_strides_and_untouched_padding(oracle, n_tok, tiles):
     n_rows, n_cols = 200, 1024
+    assert (route(n_rows, n_cols, n_tok) in TILES) == tiles
     W = synth.make_weights(Q4K, n_rows, n_cols, seed=3)
     Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=4, tokens=n_tok))
     Y = run_gemm(W, Xb, n_rows, n_cols, n_tok, ldx=n_cols + 64, ldy=n_rows + 12)
@@ -82,13 +93,16 @@ def test_gemm_bf16_equals_per_token_matvec(oracle):
     Y = run_gemm(W, synth.to_bf16_bits(X), n_rows, n_cols, len(ks))
     dec = oracle.dequant_matrix(Q4K, W, n_cols)
     assert np.array_equal(Y, dec[:, ks].T)  # ten tokens: exact weights, bit for bit the codec's values
-    # the same probes inside a batch that takes the tile kernel: the bf16 rounding of those values
-    Xbig = np.zeros((FEW_TOKENS + 16, n_cols), np.float32)
-    Xbig[:len(ks)] = X
-    Ybig = run_gemm(W, synth.to_bf16_bits(Xbig), n_rows, n_cols, Xbig.shape[0])
+    # the same probes inside batches with rounded weights, of the few-token kernel and of the tile kernel: the bf16
+    # rounding of those values
     want = synth.bf16_bits_to_f32(synth.to_bf16_bits(dec[:, ks].T.copy()))
-    assert np.array_equal(Ybig[:len(ks)], want)
-    assert not Ybig[len(ks):].any()
+    for n_tok, tiles in ((FEW_TOKENS + 16, False), (144, True)):
+        assert (route(n_rows, n_cols, n_tok) in TILES) == tiles
+        Xbig = np.zeros((n_tok, n_cols), np.float32)
+        Xbig[:len(ks)] = X
+        Ybig = run_gemm(W, synth.to_bf16_bits(Xbig), n_rows, n_cols, n_tok)
+        assert np.array_equal(Ybig[:len(ks)], want)
+        assert not Ybig[len(ks):].any()
 
 
 def test_gemm_bf16_argument_checks():

@@ -1,7 +1,7 @@
-"""GPU parity of the exact prefill GEMM for every weight format (decode once to fp32, bit-exact, then the
-vendor library's dense fp32 GEMM with fp32 accumulation), through the C ABI: what
-tf_gemm_f16_mt_tokenmajor (common/transformer.h:4487) computes for fp32 activations. Nothing is rounded
-to 16 bits, so the bar is the matvec's: relative L2 <= 1e-5 against a double-precision contraction of the
+"""GPU parity of the exact prefill GEMM for every weight format, through the C ABI: what
+tf_gemm_f16_mt_tokenmajor (common/transformer.h:4487) computes for fp32 activations. Tensors below 2 M weights and the
+formats whose codes no kernel multiplies are decoded once to fp32, bit-exact, and multiplied by the vendor library's
+dense fp32 GEMM; the product that multiplies codes has its own tests. Weights are not rounded, so the bar is the matvec's: relative L2 <= 1e-5 against a double-precision contraction of the
 oracle's decoded weights with the same activations."""
 import numpy as np
 import pytest

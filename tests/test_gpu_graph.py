@@ -146,3 +146,48 @@ def test_prefill_sequence_in_a_graph(oracle):
     assert hip.hipStreamDestroy(stream) == 0
     for b in W + Y + [dX] + qkv_W + qkv_Y:
         b.free()
+
+
+def test_fp32_product_in_a_graph(oracle):
+    """The fp32 product on codes only enqueues, too: its launches (K in parts, and in one; a token that holds an infinity)
+    are captured with the caller's workspace and replayed bit-identically."""
+    hip = C.CDLL("libamdhip64.so")
+    lib = qlinear.load()
+    calls, stream, graph, gexec = [], C.c_void_p(), C.c_void_p(), C.c_void_p()
+    for i, (t, r, k, m) in enumerate([(Q4K, 1030, 2304, 40), (Q6K, 70000, 256, 70)]):
+        assert lib.qlin_probe_gemm_f32_route(t, r, k, m) == 1
+        W, X = synth.make_weights(t, r, k, seed=50 + i), synth.make_activation(k, seed=60 + i, tokens=m)
+        X[3, k - 1] = np.inf
+        dW, dX, dY = qlinear.DevBuf.from_numpy(W), qlinear.DevBuf.from_numpy(X), qlinear.DevBuf(m * r * 4)
+        ws = qlinear.DevBuf(qlinear.gemm_f32_any_workspace_bytes(r, k))
+        calls.append((t, r, k, m, W, X, dW, dX, dY, ws))
+
+    def enqueue(s):
+        for t, r, k, m, _, _, dW, dX, dY, ws in calls:
+            assert lib.qlin_gemm_f32_any_dev(t, dW.ptr, dX.ptr, dY.ptr, r, k, m, k, r, ws.ptr, ws.nbytes, s) == 0, lib.qlin_last_error()
+
+    enqueue(None)  # eager run: the reference for the replays, itself checked against the oracle
+    qlinear.sync()
+    want = [c[8].to_numpy(np.float32, (c[3], c[1])) for c in calls]
+    for (t, r, k, m, W, X, *_), got in zip(calls, want):
+        at, fine = np.arange(0, r, r // 300), np.arange(m) != 3
+        dec = oracle.dequant_matrix(t, W[at], k).astype(np.float64)
+        assert rel_l2(got[fine][:, at], X[fine].astype(np.float64) @ dec.T) <= 1e-6
+        assert not np.isfinite(got[3]).any()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+    assert hip.hipStreamBeginCapture(stream, 0) == 0  # hipStreamCaptureModeGlobal
+    enqueue(stream)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, C.c_size_t(0)) == 0
+    for replay in range(3):
+        for c in calls:
+            z = np.full(c[3] * c[1], -3.0, np.float32)
+            assert lib.qlin_dev_upload(c[8].ptr, z.ctypes.data, z.nbytes) == 0
+        assert hip.hipGraphLaunch(gexec, stream) == 0
+        assert hip.hipStreamSynchronize(stream) == 0
+        for c, w in zip(calls, want):
+            assert np.array_equal(c[8].to_numpy(np.uint32, (c[3], c[1])), w.view(np.uint32)), replay
+        enqueue(None)  # eager work between replays
+        qlinear.sync()
+    assert hip.hipGraphExecDestroy(gexec) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(stream) == 0

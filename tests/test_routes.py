@@ -1,5 +1,6 @@
-"""Which kernel qlin_gemm_bf16_any_dev chooses, at both sides of every limit of the few-token kernel. CPU only: the choice
-is a function of format and shape (qlin_probe_gemm_route: 0 matvec or decode + dense, 1 and 2 the tile kernels, 3 few tokens)."""
+"""Which kernel qlin_gemm_bf16_any_dev and qlin_gemm_f32_any_dev choose, at both sides of every limit of the few-token kernel
+and of the fp32 product on codes. CPU only: the choice is a function of format and shape (qlin_probe_gemm_route: 0 matvec or
+decode + dense, 1 and 2 the tile kernels, 3 few tokens; qlin_probe_gemm_f32_route: 1 the product on codes)."""
 import pytest
 
 from gemm_amd import qlinear
@@ -46,3 +47,12 @@ def test_single_tokens_of_large_tensors_go_to_the_matvec(tid, n_rows, n_cols, n_
     assert route(tid, n_rows, n_cols, n_tok) == (MATVEC if matvec else FEW)
     if tid not in (synth.GGML_IQ3_S, synth.GGML_IQ2_XXS):
         assert route(tid, n_rows, n_cols, n_tok, have_workspace=0) == FEW  # nowhere to widen the activations
+
+
+@pytest.mark.parametrize("tid", ALL + (synth.GGML_IQ3_S, synth.GGML_IQ2_XXS), ids=lambda t: synth.TYPE_NAMES[t])
+def test_fp32_products_that_multiply_codes(tid):
+    for n_rows, n_cols, n_tok, codes in [
+            (8192, 4096, 7, False), (8192, 4096, 8, True), (8192, 4128, 64, False), (2048, 1024, 32, True), (2047, 1024, 32, False),
+            (2304, 1024, 33, True), (2303, 1024, 33, False), (9216, 256, 2000, True)]:
+        assert qlinear.load().qlin_probe_gemm_f32_route(tid, n_rows, n_cols, n_tok) == codes, (n_rows, n_cols, n_tok)
+    assert not qlinear.load().qlin_probe_gemm_f32_route(synth.GGML_Q4_1, 8192, 4096, 64)
