@@ -6,10 +6,11 @@
  * The weights are never decoded to memory and never rounded: their codes are integers of at most 8 bits, exact in fp16,
  * and where code * sub-block scale is an integer of at most 11 bits (kFold) that product is exact too. An activation goes
  * in as two fp16 numbers: with the token scaled by a power of two so that its largest element lies in [2^14, 2^15),
- * hi = fp16(x) and lo = fp16(x - hi) leave 2^-24 of x (half a unit of fp32), for elements below 2^-15 of the token's
- * largest 2^-39 of that. v_mfma_f32_32x32x16_f16 then does the work twice, at sixteen times the rate of the fp32 matrix
+ * hi = fp16(x) and lo = fp16(x - hi) are within 2^-23 of x (23 bits; three quarters of all fp32 numbers are kept whole), for
+ * elements below 2^-16 of the token's largest within 2^-39 of that: lo's subnormals end there. v_mfma_f32_32x32x16_f16 then does the work twice, at sixteen times the rate of the fp32 matrix
  * instructions; block scales are applied to the sums in fp32. A minimum (Q4_K, Q5_K, Q2_K) is a product of its 6-bit
- * integers with the sub-blocks' sums of activations, one more instruction per 32 x 32 x 256.
+ * integers with the sub-blocks' sums of activations (summed in 64 bits, two fp16 numbers as well), one more instruction per
+ * 32 x 32 x 256.
  *
  * Launches of a call:
  *   f32_token_exp   the power of two of every token (kF32NotFinite for one that holds an infinity or a NaN); rows of up to

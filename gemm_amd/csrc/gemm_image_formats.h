@@ -32,13 +32,6 @@ template <int AT> QLIN_INL void lds_bytes8(const uint8_t *row, int var, uint32_t
 /* byte 0xFF for every set bit of the low four bits of v */
 QLIN_INL uint32_t mask_bytes(uint32_t v) { return (((v & 15u) * 0x00204081u) & 0x01010101u) * 255u; }
 QLIN_INL uint32_t with_signs(uint32_t mag, uint32_t m) { return ((mag ^ m) + (m & 0x01010101u)) ^ 0x80808080u; } /* + 128 */
-/* table of IQ4_NL / IQ4_XS, + 128 */
-QLIN_INL uint32_t iq4_bytes(uint32_t nib) {
-    const uint32_t i7 = nib & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, i7), hi = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, i7);
-    const uint32_t m = ((nib >> 3) & 0x01010101u) * 255u;
-    return (m & hi) | (~m & lo);
-}
 template <int N> QLIN_INL uint32_t shifted(uint32_t v) { /* v >> N, v << -N */
     if constexpr (N >= 0) return v >> N;
     else return v << -N;
@@ -229,8 +222,8 @@ struct TIQ4NL {
     static QLIN_INL Hdr header(const uint8_t *row, int) { return Hdr{row}; }
     template <int U> static QLIN_INL void codes(const uint8_t *row, int kg, const uint32_t *t, uint32_t &a, uint32_t &b) {
         TQ4_0::codes<U>(row, kg, t, a, b);
-        a = iq4_bytes(a);
-        b = iq4_bytes(b);
+        a = iq4_table_bytes(a);
+        b = iq4_table_bytes(b);
     }
     template <int U> static QLIN_INL float scale(const Hdr &h, int kg) { return TQ4_0::scale<U>(h, kg); }
     template <int U> static QLIN_INL float minimum(const Hdr &, int) { return 0.0f; }
@@ -251,8 +244,8 @@ struct TIQ4XS {
     template <int U> static QLIN_INL void codes(const uint8_t *row, int kg, const uint32_t *, uint32_t &a, uint32_t &b) {
         lds_bytes8<(U < 7 ? 8 + 16 * U : 128)>(row, 8 * (kg & 1), a, b);
         const uint32_t sh = 4u * (uint32_t)(kg >> 1);
-        a = iq4_bytes((a >> sh) & 0x0F0F0F0Fu);
-        b = iq4_bytes((b >> sh) & 0x0F0F0F0Fu);
+        a = iq4_table_bytes((a >> sh) & 0x0F0F0F0Fu);
+        b = iq4_table_bytes((b >> sh) & 0x0F0F0F0Fu);
     }
     template <int U> static QLIN_INL float scale(const Hdr &h, int) {
         const uint32_t ls = ((h.lo >> (4 * U)) & 15u) | (((h.hi >> (2 * U)) & 3u) << 4);
@@ -300,6 +293,8 @@ struct TIQ2XXS {
 template <class Fn, int... I> QLIN_INL void each_impl(Fn &&fn, std::integer_sequence<int, I...>) { (fn(std::integral_constant<int, I>{}), ...); }
 template <int N, class Fn> QLIN_INL void each(Fn &&fn) { each_impl(fn, std::make_integer_sequence<int, N>{}); }
 
+/* kq::dma16 in inline asm: around the builtin the compiler waits for every outstanding request before an LDS read that it
+ * cannot tell apart from its target (52 waits more in the instances of Q4_K and Q5_K), where these kernels count their own */
 QLIN_INL void request16(uint32_t lds_at, uint32_t voff, __amdgpu_buffer_rsrc_t rsrc, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
