@@ -279,10 +279,14 @@ int qlin_gemm_f32_dev(uint32_t ggml_type, const void *W, const float *X, float *
 /* The fp32 contraction for many tokens, any supported type: what tf_gemm_f16_mt_tokenmajor (common/transformer.h:4487)
  * computes for fp32 activations, without the 16-bit rounding of its fast paths. Q4_K, Q5_K, Q6_K, Q2_K, Q3_K, Q8_0, Q4_0,
  * IQ4_NL, IQ4_XS, IQ3_S and IQ2_XXS with n_cols a multiple of 256, from about 2 M weights on, multiply their codes as they
- * are with activations carried as two fp16 numbers (24 bits) on the matrix cores; everything else is decoded once to fp32
- * (bit-exact, as qlin_dequant_dev) into `workspace` and multiplied by the vendor library's dense fp32 GEMM. fp32
- * accumulation either way; the same call takes the same route each time. Relative L2 against a
- * double-precision reference <= 1e-5. Fewer than 8 tokens run the kernel of qlin_gemm_f32_dev and leave the
+ * are on the matrix cores, with activations carried as two fp16 numbers: an element keeps 23 bits of itself, but none
+ * below 2^-39 of the largest of its token. Everything else is decoded once to fp32 (bit-exact, as qlin_dequant_dev) into
+ * `workspace` and multiplied by the vendor library's dense fp32 GEMM. fp32 accumulation either way; the same call takes
+ * the same route each time. Relative L2 against a double-precision reference <= 1e-5 (about 3e-7 with codes, 1e-6
+ * without) - with codes, unless outputs rest on elements more than 2^20 below their token's largest alone. A token with
+ * infinities or NaN gets the infinities and NaN of its sums and leaves the others alone. A one-hot activation returns
+ * decoded weights bit for bit, except those of Q4_K, Q5_K and Q2_K multiplied as codes (whose minimum is subtracted after
+ * the products). Fewer than 8 tokens run the kernel of qlin_gemm_f32_dev and leave the
  * workspace alone (it may then be NULL). workspace: device memory, 256-byte aligned, at least
  * qlin_gemm_f32_any_workspace_bytes(n_rows, n_cols) bytes (4 bytes per weight + 32 MiB for the library);
  * calls that share a workspace must be ordered on one stream. */
