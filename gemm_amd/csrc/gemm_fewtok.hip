@@ -23,9 +23,12 @@ int fewtok_unrounded(uint32_t type) {
 
 /* Unrounded tokens always. With rounded weights the small-tile kernel, whose workgroup takes 64 rows, computes the same;
  * it is the faster one where this kernel's workgroups no longer run in one go (us, this kernel / small tiles):
- *   49 to 64 tokens, more than 512 row tiles: 64 tokens 8192 x 2048 Q4_K 7.1 / 10.7, but 8704 x 2048 11.9 / 10.9, 9216 x
- *     2560 Q5_K 15.8 / 13.3 (14336 x 4096 Q4_K 19.9 / 20.9). Not Q8_0, whose decode costs the tile kernel more (9216 x 2048
- *     14.2 / 17.1), and not very many rows of 1024 elements (24576 x 1024 Q4_K 11.1 / 11.8, but 14336 x 1024 8.3 / 8.0)
+ *   49 to 64 tokens, more than 512 row tiles of rows below 4096 elements: 64 tokens 8192 x 2048 Q4_K 7.1 / 10.7, but 8704 x
+ *     2048 11.9 / 10.9, 9216 x 2560 Q5_K 15.8 / 13.3; longer rows are even or better here (16384 x 4096 Q4_K 20.0 / 21.0). Not
+ *     Q8_0, whose decode costs the tile kernel more (9216 x 2048 14.2 / 17.1), and not from 1593 row tiles on, where 200
+ *     large tiles would be chosen, a quarter full (32000 x 2048 Q4_K 26 / 30; 1024 elements from 1200 on, 24576 x 1024 11.1 /
+ *     11.8; five to seven super-blocks, a wave for each, from 3000 on, 32000 x 1536 Q4_K 24.2 / 22.4, but 50000 x 1536
+ *     31.9 / 36.9)
  *   65 to 128 tokens, more than 320: 80 tokens Q4_K 4096 x 4096 9.2 / 17.3, 5120 x 4096 11.2 / 17.6, but 77 tokens
  *     13824 x 2560 19.6 / 16.8; past 96 tokens, rows below 2048 (Q8_0: 4096) elements: 256 (128 tokens 5120 x 1024 Q4_K 9.5 / 7.9)
  *   rows so short that one or two waves do all of K: 256 elements from 49 tokens on (64 tokens 4096 x 256 5.6 / 5.1), 512
@@ -39,7 +42,7 @@ bool fewtok_takes(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx) {
     const int tiles = n_rows / 16 + (n_rows % 16 != 0), n_sb = n_cols / 256;
     if (n_tok <= 48) return true;
     if (n_sb == 1) return false;
-    if (n_tok <= 64) return tiles <= 512 || type == T_Q8_0 || (n_sb == 4 && tiles >= 1200);
+    if (n_tok <= 64) return tiles <= 512 || type == T_Q8_0 || n_sb >= 16 || tiles >= (n_sb < 4 || n_sb > 7 ? 1593 : n_sb == 4 ? 1200 : 3000);
     if (n_tok <= 80) return tiles <= 320;
     if (n_tok <= 96) return tiles <= (n_sb == 2 ? 256 : 320);
     if (type == T_Q8_0) return tiles <= (n_sb < 16 ? 256 : 320);

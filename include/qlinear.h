@@ -239,8 +239,8 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * A few tokens of these formats (and, given a workspace, up to 64 of IQ3_S and IQ2_XXS) run in the few-token kernel
  * (n_cols % 256 == 0, no workspace used), which streams the blocks once: with unrounded codes (~1e-6) up to 32 tokens of
  * Q4_K, 24 of Q5_K, Q6_K, Q2_K, Q3_K and Q8_0 and 4 of the others; beyond that, with the same single rounding to bf16, up
- * to 48 tokens, up to 64 where a tensor has at most 8192 rows and up to 128 where it has at most 5120 (somewhat less
- * for rows of fewer than 2048 elements). A token with an infinity or a NaN leaves the others alone; with unrounded codes
+ * to 48 tokens, up to 64 where a tensor has at most 8192 rows or rows of 4096 elements and up to 128 where it has at
+ * most 5120 rows (somewhat less for rows of fewer than 2048 elements). A token with an infinity or a NaN leaves the others alone; with unrounded codes
  * its own results may be NaN where exact arithmetic gives an infinity. Up to 4 tokens of any other
  * block format and, given a workspace, one token of a large IQ4_NL, IQ4_XS, IQ3_S or Q4_0 tensor and one to three of an
  * IQ2_XXS tensor go one by one through the matvec kernels (exact weights, ~1e-6; the workspace holds their

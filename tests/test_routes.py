@@ -19,7 +19,9 @@ def route(tid, n_rows, n_cols, n_tok, have_workspace=1):
 def test_rounded_weights_go_to_the_faster_of_the_few_token_and_tile_kernels(tid):
     q8 = tid == synth.GGML_Q8_0
     for n_rows, n_cols, n_tok, few in [
-            (8192, 2048, 64, True), (8193, 2048, 64, q8), (8193, 2048, 48, True), (20000, 1024, 64, True), (16000, 1024, 64, q8),
+            (8192, 2048, 64, True), (8193, 2048, 64, q8), (8193, 2048, 48, True), (14336, 4096, 64, True), (14336, 3840, 64, q8),
+            (25472, 2048, 64, q8), (25473, 2048, 64, True), (32000, 512, 64, True), (32000, 1536, 64, q8), (48000, 1792, 64, True),
+            (19200, 1024, 64, True), (19184, 1024, 64, q8),
             (5120, 2048, 80, True), (5121, 2048, 80, False), (5120, 2048, 128, not q8), (5120, 4096, 128, True), (4096, 2048, 128, True),
             (5120, 1536, 128, False), (4096, 1536, 128, True), (5120, 512, 80, True), (5120, 512, 81, False), (4096, 512, 96, True),
             (4096, 512, 97, q8), (64, 256, 48, True), (64, 256, 49, False), (64, 4096, 129, False)]:
