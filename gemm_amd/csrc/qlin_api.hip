@@ -1062,6 +1062,17 @@ static FusedTile takes_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     return takes_matvec(type, n_rows, n_cols, n_tok, ws_ok) ? kFusedNone : choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok);
 }
 
+/* a matvec per token and tensor, on activations widened to fp32 in xf: x_span elements, from the first token's to the last's */
+static int matvec_tokens(uint32_t type, int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows,
+                         int n_cols, int n_tok, int ldx, const int *ldy, size_t x_span, float *xf, hipStream_t stream) {
+    HIP_TRY(launch_dequant(T_BF16, X, nullptr, 0, xf, 1, (int)x_span, 0, stream));
+    for (int i = 0; i < n_mat; i++)
+        for (int t = 0; t < n_tok; t++)
+            HIP_TRY(dispatch_gemv_job(type, single_job(W[i], Y[i] + (size_t)t * ldy[i], n_rows[i]), xf + (size_t)t * ldx, n_cols, stream));
+    return QLIN_OK;
+}
+static bool x_fits(size_t x_span, size_t workspace_bytes) { return x_span <= (size_t)INT_MAX && x_span * sizeof(float) <= workspace_bytes; }
+
 int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                            int n_tok, int ldx, int ldy, void *workspace, size_t workspace_bytes, void *stream) {
     if (int rc = check_linear_shape(type, n_rows, n_cols)) return rc;
@@ -1093,16 +1104,10 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
         return fail(QLIN_ERR_ARG, "workspace must be 256-byte aligned and hold qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols) bytes");
     /* up to four tokens of any other block format, and what takes_matvec says: each through the matvec (exact weights;
      * 14336 x 4096 IQ2_XXS, two tokens: 17 us, in the few-token kernel 20), x widened to fp32 at the start of the workspace */
-    const size_t x_span = (size_t)(n_tok - 1) * ldx + n_cols; /* elements of X from the first token's to the last's */
-    if (n_tok <= kMatvecTokens && type != T_F32 && type != T_F16 && type != T_BF16 && x_span <= (size_t)INT_MAX &&
-        x_span * sizeof(float) <= workspace_bytes) { /* a very wide ldx: the dense route below */
-        float *xf = (float *)workspace;
-        HIP_TRY(launch_dequant(T_BF16, X, nullptr, 0, xf, 1, (int)x_span, 0, (hipStream_t)stream));
-        for (int t = 0; t < n_tok; t++)
-            HIP_TRY(dispatch_gemv_job(type, single_job(W, Y + (size_t)t * ldy, n_rows), xf + (size_t)t * ldx, n_cols,
-                                      (hipStream_t)stream));
-        return QLIN_OK;
-    }
+    const size_t x_span = (size_t)(n_tok - 1) * ldx + n_cols;
+    if (n_tok <= kMatvecTokens && type != T_F32 && type != T_F16 && type != T_BF16 &&
+        x_fits(x_span, workspace_bytes)) /* a very wide ldx: the dense route below */
+        return matvec_tokens(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, x_span, (float *)workspace, (hipStream_t)stream);
     const uint16_t *Wd = (const uint16_t *)W; /* bf16 weights are used where they are */
     if (type != T_BF16) {
         HIP_TRY(launch_dequant_bf16(type, W, (uint16_t *)workspace, n_rows, n_cols, row_size(type, n_cols), (hipStream_t)stream));
@@ -1148,13 +1153,16 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
      * single-tensor call, which a tensor that fails them goes through below to report it */
     bool together = n_mat > 1 && n_tok > 0 && X && aligned(X, 16) && ldx % 8 == 0 && ldx >= n_cols;
     FusedTile tile = kFusedNone;
-    bool few = false;
+    bool few = false, matvecs = true; /* matvecs: widened once for all (IQ2_XXS 4096 + 1024 + 1024 rows x 4096, one token: 17.9 -> 13.8 us) */
+    const size_t x_span = n_tok > 0 ? (size_t)(n_tok - 1) * ldx + n_cols : 0;
     for (int i = 0; i < n_mat && together; i++) {
         const bool ws_ok = workspace && aligned(workspace, 256) &&
                            workspace_bytes >= qlin_gemm_bf16_any_workspace_bytes(n_rows[i], n_cols);
         together = n_rows[i] > 0 && W[i] && Y[i] && aligned(W[i], 16) && aligned(Y[i], 4) && ldy[i] >= n_rows[i] &&
                    n_cols > 0; /* the chooser checks format and row length */
         if (!together) break;
+        matvecs = matvecs && takes_matvec(type, n_rows[i], n_cols, n_tok, ws_ok) && x_fits(x_span, workspace_bytes);
+        if (matvecs) continue;
         const bool mine_few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
         const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
@@ -1167,6 +1175,8 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
             std::lock_guard<std::mutex> lk(g.mu);
             if (int rc = ensure_init_locked(0)) return rc;
         }
+        if (matvecs)
+            return matvec_tokens(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, x_span, (float *)workspace, (hipStream_t)stream);
         if (few)
             HIP_TRY(launch_gemm_fewtok(type, {n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream}));
         else if (tile == kFusedLarge)

@@ -162,3 +162,35 @@ def test_a_token_that_is_not_finite_leaves_the_others_alone(tid, n_tok):
     assert np.array_equal(got[0][rest], got[1][rest])
     spoiled = got[1][[bad[0], bad[-1]]].view(np.float32)
     assert not np.isfinite(spoiled).any()
+
+
+@pytest.mark.parametrize("rows,n_cols,n_tok", [((70, 33, 5), 3072, 1), ((70, 33), 12288, 2), ((4610, 33), 2048, 1)])
+def test_tensors_that_all_go_to_the_matvec(oracle, rows, n_cols, n_tok):
+    """what a call per tensor gives, bit for bit, from one widening of X; a tensor that does not go there (the last case's
+    second) changes nothing about that"""
+    tid, rows = synth.GGML_IQ2_XXS, list(rows)
+    Ws = [synth.make_weights(tid, r, n_cols, seed=r) for r in rows]
+    ldx = n_cols + 8
+    X = np.full((n_tok, ldx), 0x7FC0, np.uint16)
+    X[:, :n_cols] = synth.to_bf16_bits(synth.make_activation(n_cols, seed=5, tokens=n_tok))
+    ldys = [r + 2 for r in rows]
+    dWs, dX = [qlinear.DevBuf.from_numpy(w) for w in Ws], qlinear.DevBuf.from_numpy(X)
+    ws = qlinear.DevBuf(qlinear.gemm_bf16_any_workspace_bytes(max(rows), n_cols))
+    got = []
+    for together in (True, False):
+        dYs = [qlinear.DevBuf.from_numpy(np.full((n_tok, ld), -3.0, np.float32)) for ld in ldys]
+        if together:
+            qlinear.gemm_bf16_multi_dev(tid, dWs, dX, dYs, rows, n_cols, n_tok, ldx, ldys, ws)
+        else:
+            for w, y, r, ld in zip(dWs, dYs, rows, ldys):
+                qlinear.gemm_bf16_any_dev(tid, w, dX, y, r, n_cols, n_tok, ldx, ld, ws)
+        qlinear.sync()
+        got.append([y.to_numpy(np.float32, (n_tok, ld)) for y, ld in zip(dYs, ldys)])
+        for b in dYs:
+            b.free()
+    for b in dWs + [dX, ws]:
+        b.free()
+    Xf = synth.bf16_bits_to_f32(X[:, :n_cols]).astype(np.float64)
+    for W, a, b, r in zip(Ws, *got, rows):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)) and np.all(a[:, r:] == -3.0)
+        assert rel_l2(a[:, :r], Xf @ oracle.dequant_matrix(tid, W, n_cols).astype(np.float64).T) <= 2e-6
