@@ -279,6 +279,7 @@ static bool launch_gemv_tuned(uint32_t type, const GemvJob &job, const float *x,
                               hipStream_t s, hipError_t *err) {
     bool w_aligned = true;
     for (int m = 0; m < job.n_mat; m++) w_aligned = w_aligned && aligned(job.W[m], 16);
+    if (launch_gemv_dma(type, job, x, n_cols, g.n_cu, s, err, row_stride)) return true;
     if (type == T_Q4_K && n_cols % 256 == 0 && n_cols <= 16384 && w_aligned && aligned(x, 16)) {
         *err = launch_gemv_q4k(job, x, n_cols, s, g.n_cu, row_stride);
         return true;
