@@ -8,7 +8,7 @@
 #ifndef QLIN_GEMM_KQ_FORMATS_H
 #define QLIN_GEMM_KQ_FORMATS_H
 
-#include "qlin_device.h"
+#include "qlin_internal.h"
 
 namespace qlin {
 namespace kq {
@@ -553,6 +553,24 @@ QLIN_INL TileOf tile_of(const TileSet &set, int tile_all) {
     else if (tile_all < set.end1) { t.W = set.W1; t.Y = set.Y1; t.n_rows = set.n_rows1; t.ldy = set.ldy1; t.tile = tile_all - set.end0; }
     else { t.W = set.W2; t.Y = set.Y2; t.n_rows = set.n_rows2; t.ldy = set.ldy2; t.tile = tile_all - set.end1; }
     return t;
+}
+
+/* A workgroup's share of K (KSplit, qlin_internal.h): every tile is `parts` items, and the ends of the TileSet count items */
+struct KPart { const uint8_t *W; float *out; int n_rows, ld, tile, sb0, n_sb; };
+QLIN_INL KPart k_part(const TileSet &set, const KSplit &split, int item, int n_sb, int n_tok) {
+    const TileOf t = tile_of(set, item);
+    KPart p = {t.W, t.Y, t.n_rows, t.ldy, t.tile, 0, n_sb};
+    if (split.parts > 1) {
+        auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); }; /* (divisions run in vector registers) */
+        const unsigned parts = (unsigned)split.parts;
+        p.tile = uniform((int)((unsigned)t.tile / parts));
+        const unsigned part = (unsigned)(t.tile - p.tile * split.parts);
+        p.sb0 = uniform((int)((unsigned)n_sb * part / parts));
+        p.n_sb = uniform((int)((unsigned)n_sb * (part + 1) / parts)) - p.sb0;
+        p.out = split.buf + (size_t)part * n_tok * t.n_rows;
+        p.ld = t.n_rows;
+    }
+    return p;
 }
 
 /* one load-to-LDS request: lane l's 16 bytes from voff + soff of the buffer land at lds + 16 l */

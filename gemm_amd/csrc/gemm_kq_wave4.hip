@@ -54,6 +54,8 @@
 #include "gemm_kq_formats.h"
 #include "qlin_internal.h"
 
+#include <algorithm>
+
 namespace qlin {
 
 using namespace kq;
@@ -171,7 +173,7 @@ template <class F, int... J> QLIN_INL void load_cur_extra(Ctx<F> &c, std::intege
 
 template <class F>
 __global__ void __launch_bounds__(256)
-gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_tok, int ldx, int m_tiles) {
+gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles, KSplit split) {
     /* raw blocks of one super-block of each wave's 32 weight rows (32 x kPieces pieces, rounded up to whole requests) */
     __shared__ __attribute__((aligned(1024))) uint8_t w4_raw[4 * F::kReq * 1024];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -180,19 +182,21 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb,
      * that share one weight tile get ids 8 apart and meet in the same L2 */
     const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
     const int tile_m = slot_id % m_tiles;
-    const int tile_all = (slot_id / m_tiles) * 8 + xcd;
-    if (tile_all >= set.end2) return;
-    const TileOf t = tile_of(set, tile_all);
-    const uint8_t *W = t.W;
-    float *Y = t.Y;
-    const int n_rows = t.n_rows, ldy = t.ldy, tile_n = t.tile;
+    const int item = (slot_id / m_tiles) * 8 + xcd;
+    if (item >= set.end2) return;
+    /* this workgroup's super-blocks, and where its sums go */
+    const KPart part = k_part(set, split, item, n_sb_all, n_tok);
+    const int n_sb = part.n_sb, n_rows = part.n_rows, ldy = part.ld, tile_n = part.tile;
+    const uint8_t *W = part.W + (size_t)part.sb0 * F::kBlockBytes;
+    float *Y = part.out;
+    X += part.sb0 * 256;
 
     Ctx<F> c;
     c.raw = w4_raw;
     c.wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     c.n_sb = n_sb;
     c.unit = 1.0f / fp8_pair_lo(1u).x;
-    const uint32_t row_bytes = (uint32_t)n_sb * F::kBlockBytes;
+    const uint32_t row_bytes = (uint32_t)n_sb_all * F::kBlockBytes;
     /* Global loads are buffer loads: a descriptor of this workgroup's weight rows / token rows in scalar
      * registers, a 32-bit offset per lane that never changes, and a scalar offset that moves along K.
      * Weight role: lane (i = lane % 32, kg = lane / 32) owns row 32 wv + i; rows past the end re-read the last one
@@ -200,7 +204,7 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb,
     const int li = lane & 31, kg = lane >> 5;
     const int w_rows = min(kBN, n_rows - tile_n * kBN);
     c.w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W) + (size_t)tile_n * kBN * row_bytes, 0,
-                                                 w_rows * row_bytes, 0x00020000);
+                                                 (w_rows - 1) * row_bytes + (uint32_t)n_sb * F::kBlockBytes, 0x00020000);
     c.kg = kg;
 #pragma unroll
     for (int q = 0; q < F::kReq; q++) {
@@ -284,23 +288,49 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb,
 }
 
 namespace {
+
+/* adds the parts of K in order; a thread has R rows of a token */
+template <int R>
+__global__ void __launch_bounds__(256) k_join_kernel(const float *__restrict__ buf, float *__restrict__ Y, int parts, int n_rows, int n_tok, int ldy) {
+    typedef float vec __attribute__((ext_vector_type(R)));
+    const int row = (blockIdx.x * 256 + threadIdx.x) * R, t = blockIdx.y;
+    if (row >= n_rows) return;
+    const float *at = buf + (size_t)t * n_rows + row;
+    vec sum = *reinterpret_cast<const vec *>(at);
+#pragma unroll 4
+    for (int p = 1; p < parts; p++) sum += *reinterpret_cast<const vec *>(at + (size_t)p * n_tok * n_rows);
+    *reinterpret_cast<vec *>(Y + (size_t)t * ldy + row) = sum;
+}
+
+}  // namespace
+
+void launch_k_join(const KSplit &split, float *Y, int n_rows, int n_tok, int ldy, hipStream_t stream) {
+    const bool wide = n_rows % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0; /* (the workspace is 256-byte aligned) */
+    const int per = 256 * (wide ? 4 : 1);
+    hipLaunchKernelGGL(wide ? k_join_kernel<4> : k_join_kernel<1>, dim3((n_rows + per - 1) / per, n_tok), dim3(256), 0, stream, split.buf, Y,
+                       split.parts, n_rows, n_tok, ldy);
+}
+
+namespace {
 template <class F>
 hipError_t launch_wave4(int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows, int n_cols,
-                        int n_tok, int ldx, const int *ldy, hipStream_t stream) {
+                        int n_tok, int ldx, const int *ldy, KSplit split, hipStream_t stream) {
     const int n_sb = n_cols / 256;
     const int m_tiles = (n_tok + kBM - 1) / kBM;
     TileSet set;
-    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN);
+    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN) * split.parts;
+    if (split.parts > 1) set.end0 = set.end1 = set.end2 = n_tiles; /* (one tensor) */
     /* ids are dealt to 8 XCDs; pad the n-tile count to a multiple of 8 (surplus groups exit) */
     const int n_tiles_pad = (n_tiles + 7) / 8 * 8;
     hipLaunchKernelGGL(gemm_kq_bf16_wave4_kernel<F>, dim3(n_tiles_pad * m_tiles), dim3(256), 0, stream, set, X, n_sb,
-                       n_tok, ldx, m_tiles);
+                       n_tok, ldx, m_tiles, split);
+    if (split.parts > 1) launch_k_join(split, Y[0], n_rows[0], n_tok, ldy[0], stream);
     return hipGetLastError();
 }
 template <class F>
 hipError_t launch_wave4(const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok, int ldx, int ldy,
                         hipStream_t stream) {
-    return launch_wave4<F>(1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream);
+    return launch_wave4<F>(1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, KSplit(), stream);
 }
 }  // namespace
 
@@ -342,6 +372,60 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     return (n_tok <= small_max || !have_workspace) ? kFusedSmall : kFusedNone;
 }
 
+/* Long rows on few tiles: K divided over workgroups, the parts added by a second launch (k_join_kernel). A chip of 256 compute
+ * units with 64 tiles of a 4096 x 14336 product works through 56 super-blocks four times slower than it could; the tile
+ * kernels' parts read no activation and no weight twice, but their sums go through memory (8 bytes per part and result) and
+ * the second launch costs 3.5 us. Measured, us, one piece (few-token kernel to 128 tokens, then tiles, or decode + library) / divided, Q4_K:
+ * 4096 x 14336 with 77, 128, 160, 256, 384, 512, 768 tokens 31.8 / 26.4, 45 / 29.4, 67 / 39, 69 / 44, 71 / 63, 81 / 68, 121 / 97; 2560 x 6912
+ * with 128, 160, 256 19.5 / 15.8, 28 / 18, 31 / 19.5; 2048 x 5632 18.6 / 14.2, 23.5 / 15.4, 25 / 17.3; Q6_K 4096 x 14336 with 256, 768 83 / 47, 133 /
+ * 106. Not below 17 super-blocks: 4096 x 4096 gains nothing (160 tokens 18.9 / 17.9, 512 23.6 / 32), and K and V of 1024 rows, which would,
+ * share a launch with Q that fills the chip as it is. The estimates, in us, are fitted to such figures;
+ * they err by a tenth, so that a gain of less than 13 % is left alone. */
+FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, size_t workspace_bytes, FusedTile tile, bool few) {
+    const int n_sb = n_cols / 256;
+    if (!gemm_kq_wave4_covers(type) || n_cols % 256 != 0 || n_sb < 17 || ldx >= (1 << 22) || n_tok < 65 || n_tok > 1024) return {tile, 1};
+    double small = 1.0, large = 1.0, fewf = 1.0; /* the formats' times against Q4_K's */
+    switch (type) {
+    case T_Q5_K: small = 1.03; large = 1.02; break;
+    case T_Q6_K: small = 1.2; large = 1.1; fewf = 1.08; break;
+    case T_Q8_0: small = 1.65; large = 1.2; fewf = 1.1; break;
+    case T_IQ4_NL: small = 1.15; large = 1.03; break;
+    case T_IQ4_XS: small = 1.13; large = 1.13; break;
+    case T_Q3_K: small = 1.06; large = 1.03; break;
+    default: break;
+    }
+    const double results = (double)n_rows * n_tok, weights = (double)n_rows * n_cols;
+    const auto joined = [&](int parts) { return parts > 1 ? 3.5 + parts * results * 8.0 / 4e6 : 0.0; };
+    const auto small_us = [&](int parts) {
+        const int items = (n_rows + 63) / 64 * ((n_tok + 127) / 128) * parts;
+        return 4.5 + (n_sb + parts - 1) / parts * (parts > 1 ? (double)((items + 255) / 256) : std::max(1.0, items / 256.0)) * small * (0.65 + 0.008 * n_sb + 0.3 * std::min(1.0, items / 256.0)) + joined(parts);
+    };
+    const auto large_us = [&](int parts) {
+        const int items = (n_rows + 127) / 128 * ((n_tok + 255) / 256) * parts;
+        return 9.0 + (n_sb + parts - 1) / parts * ((items + 255) / 256) * large * (2.1 + 0.7 * std::min(1.0, items / 224.0)) + joined(parts);
+    };
+    const double one = few ? 4.0 + fewf * n_sb * (0.1 + 0.0048 * (n_tok <= 80 ? 80 : n_tok <= 96 ? 96 : 128)) * (0.7 + 0.3 * std::min(1.0, n_rows / 4096.0))
+                       : tile == kFusedSmall ? small_us(1)
+                       : tile == kFusedLarge ? large_us(1)
+                                             : 5.0 + weights * 2.8 / 4.2e6 + 2.0 * weights * n_tok / (1.25e9 * (0.4 + 0.6 * std::min(1.0, results / 6e6)));
+    FusedSplit best = {tile, 1};
+    double best_us = 0.87 * one;
+    for (int parts = 2; parts <= 16 && parts <= n_sb / 2 && parts * results * sizeof(float) <= (double)workspace_bytes; parts++) {
+        if (const double t = small_us(parts); t < best_us) { best_us = t; best = {kFusedSmall, parts}; }
+        if (const double t = large_us(parts); n_tok > 128 && t < best_us) { best_us = t; best = {kFusedLarge, parts}; }
+    }
+    return best;
+}
+
+hipError_t launch_fused_split(FusedSplit s, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
+                              int ldx, int ldy, void *workspace, hipStream_t stream) {
+    KSplit split;
+    split.buf = (float *)workspace;
+    split.parts = s.parts;
+    return s.tile == kFusedLarge ? launch_gemm_kq_bf16_wave4_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split)
+                                 : launch_gemm_kq_bf16_wave4s_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split);
+}
+
 hipError_t launch_fused_tile(FusedTile tile, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows,
                              int n_cols, int n_tok, int ldx, int ldy, hipStream_t stream) {
     if (tile == kFusedLarge) return launch_gemm_kq_bf16_wave4(type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
@@ -351,18 +435,18 @@ hipError_t launch_fused_tile(FusedTile tile, uint32_t type, const void *W, const
 
 hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
-                                           const int *ldy, hipStream_t stream) {
+                                           const int *ldy, hipStream_t stream, KSplit split) {
     if (n_mat < 1 || n_mat > 3) return hipErrorInvalidValue;
     switch (type) {
-    case T_Q4_K: return launch_wave4<FQ4K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q5_K: return launch_wave4<FQ5K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q6_K: return launch_wave4<FQ6K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q8_0: return launch_wave4<FQ8_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_IQ4_NL: return launch_wave4<FIQ4NL>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_IQ4_XS: return launch_wave4<FIQ4XS>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q4_0: return launch_wave4<FQ4_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q2_K: return launch_wave4<FQ2K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q3_K: return launch_wave4<FQ3K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
+    case T_Q4_K: return launch_wave4<FQ4K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q5_K: return launch_wave4<FQ5K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q6_K: return launch_wave4<FQ6K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q8_0: return launch_wave4<FQ8_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_IQ4_NL: return launch_wave4<FIQ4NL>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_IQ4_XS: return launch_wave4<FIQ4XS>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q4_0: return launch_wave4<FQ4_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q2_K: return launch_wave4<FQ2K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q3_K: return launch_wave4<FQ3K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -216,7 +216,7 @@ QLIN_INL void run_half(Ctx<F> &c, float *__restrict__ Y, int n_rows, int n_tok, 
 
 template <class F>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb, int n_tok, int ldx, int m_tiles) {
+gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles, KSplit split) {
     /* raw blocks of one super-block of the two row halves (32 x kPieces pieces each, rounded up to whole requests) */
     __shared__ __attribute__((aligned(1024))) uint8_t w4s_raw[2 * F::kReq * 1024];
     constexpr int nW = Ctx<F>::kMyReq;
@@ -226,12 +226,14 @@ gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb
      * that share one weight tile get ids 8 apart and meet in the same L2 */
     const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
     const int tile_m = slot_id % m_tiles;
-    const int tile_all = (slot_id / m_tiles) * 8 + xcd;
-    if (tile_all >= set.end2) return;
-    const TileOf t = tile_of(set, tile_all);
-    const uint8_t *W = t.W;
-    float *Y = t.Y;
-    const int n_rows = t.n_rows, ldy = t.ldy, tile_n = t.tile;
+    const int item = (slot_id / m_tiles) * 8 + xcd;
+    if (item >= set.end2) return;
+    /* this workgroup's super-blocks, and where its sums go */
+    const KPart part = k_part(set, split, item, n_sb_all, n_tok);
+    const int n_sb = part.n_sb, n_rows = part.n_rows, ldy = part.ld, tile_n = part.tile;
+    const uint8_t *W = part.W + (size_t)part.sb0 * F::kBlockBytes;
+    float *Y = part.out;
+    X += part.sb0 * 256;
 
     Ctx<F> c;
     c.raw = w4s_raw;
@@ -239,7 +241,7 @@ gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb
     const int wr = c.wv & 1, wk = c.wv >> 1;
     c.n_sb = n_sb;
     c.unit = 1.0f / fp8_pair_lo(1u).x;
-    const uint32_t row_bytes = (uint32_t)n_sb * F::kBlockBytes;
+    const uint32_t row_bytes = (uint32_t)n_sb_all * F::kBlockBytes;
     const int li = lane & 31, kg = lane >> 5;
     c.kg = kg;
     /* weights: lane (li, kg) owns row 32 wr + li of the tile; rows past the end re-read the last one (decoded, never
@@ -247,7 +249,7 @@ gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb
      * issues Q = wk, wk + 2, ... (one past the last: the last again, into the same place) */
     const int w_rows = min(kBN, n_rows - tile_n * kBN);
     c.w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(W) + (size_t)tile_n * kBN * row_bytes, 0,
-                                                 w_rows * row_bytes, 0x00020000);
+                                                 (w_rows - 1) * row_bytes + (uint32_t)n_sb * F::kBlockBytes, 0x00020000);
 #pragma unroll
     for (int q = 0; q < nW; q++) {
         const int Q = min(2 * q + wk, F::kReq - 1);
@@ -305,32 +307,34 @@ gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb
 namespace {
 template <class F>
 hipError_t launch_wave4s(int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows, int n_cols,
-                         int n_tok, int ldx, const int *ldy, hipStream_t stream) {
+                         int n_tok, int ldx, const int *ldy, KSplit split, hipStream_t stream) {
     const int n_sb = n_cols / 256;
     const int m_tiles = (n_tok + kBM - 1) / kBM;
     TileSet set;
-    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN);
+    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN) * split.parts;
+    if (split.parts > 1) set.end0 = set.end1 = set.end2 = n_tiles; /* (one tensor) */
     const int n_tiles_pad = (n_tiles + 7) / 8 * 8; /* ids are dealt to 8 XCDs; surplus groups exit */
     hipLaunchKernelGGL(gemm_kq_bf16_wave4s_kernel<F>, dim3(n_tiles_pad * m_tiles), dim3(256), 0, stream, set, X, n_sb,
-                       n_tok, ldx, m_tiles);
+                       n_tok, ldx, m_tiles, split);
+    if (split.parts > 1) launch_k_join(split, Y[0], n_rows[0], n_tok, ldy[0], stream);
     return hipGetLastError();
 }
 }  // namespace
 
 hipError_t launch_gemm_kq_bf16_wave4s_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
                                             float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
-                                            const int *ldy, hipStream_t stream) {
+                                            const int *ldy, hipStream_t stream, KSplit split) {
     if (n_mat < 1 || n_mat > 3) return hipErrorInvalidValue;
     switch (type) {
-    case T_Q4_K: return launch_wave4s<FQ4K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q5_K: return launch_wave4s<FQ5K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q6_K: return launch_wave4s<FQ6K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q8_0: return launch_wave4s<FQ8_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_IQ4_NL: return launch_wave4s<FIQ4NL>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_IQ4_XS: return launch_wave4s<FIQ4XS>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q4_0: return launch_wave4s<FQ4_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q2_K: return launch_wave4s<FQ2K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    case T_Q3_K: return launch_wave4s<FQ3K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
+    case T_Q4_K: return launch_wave4s<FQ4K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q5_K: return launch_wave4s<FQ5K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q6_K: return launch_wave4s<FQ6K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q8_0: return launch_wave4s<FQ8_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_IQ4_NL: return launch_wave4s<FIQ4NL>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_IQ4_XS: return launch_wave4s<FIQ4XS>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q4_0: return launch_wave4s<FQ4_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q2_K: return launch_wave4s<FQ2K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q3_K: return launch_wave4s<FQ3K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -1063,6 +1063,13 @@ static FusedTile takes_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     return takes_matvec(type, n_rows, n_cols, n_tok, ws_ok) ? kFusedNone : choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok);
 }
 
+/* long rows on few tiles: K over several workgroups (parts of 1: not this shape) */
+static FusedSplit takes_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool ws_ok, size_t workspace_bytes) {
+    if (!ws_ok) return {kFusedNone, 1};
+    return choose_fused_split(type, n_rows, n_cols, n_tok, ldx, workspace_bytes, takes_tile(type, n_rows, n_cols, n_tok, ldx, true),
+                              takes_fewtok(type, n_rows, n_cols, n_tok, ldx, true));
+}
+
 /* a matvec per token and tensor, on activations widened to fp32 in xf: x_span elements, from the first token's to the last's */
 static int matvec_tokens(uint32_t type, int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows,
                          int n_cols, int n_tok, int ldx, const int *ldy, size_t x_span, float *xf, hipStream_t stream) {
@@ -1086,6 +1093,10 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
     {
         std::lock_guard<std::mutex> lk(g.mu);
         if (int rc = ensure_init_locked(0)) return rc;
+    }
+    if (const FusedSplit split = takes_split(type, n_rows, n_cols, n_tok, ldx, ws_ok, workspace_bytes); split.parts > 1) {
+        HIP_TRY(launch_fused_split(split, type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, workspace, (hipStream_t)stream));
+        return QLIN_OK;
     }
     if (takes_fewtok(type, n_rows, n_cols, n_tok, ldx, ws_ok)) {
         HIP_TRY(launch_gemm_fewtok(type, {1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, (hipStream_t)stream}));
@@ -1164,6 +1175,10 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
         if (!together) break;
         matvecs = matvecs && takes_matvec(type, n_rows[i], n_cols, n_tok, ws_ok) && x_fits(x_span, workspace_bytes);
         if (matvecs) continue;
+        if (takes_split(type, n_rows[i], n_cols, n_tok, ldx, ws_ok, workspace_bytes).parts > 1) { /* the parts' place holds one tensor's */
+            together = false;
+            break;
+        }
         const bool mine_few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
         const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
@@ -1341,6 +1356,8 @@ int qlin_probe_clocks(void *stream, double *shader_mhz) {
 }
 
 int qlin_probe_gemm_route(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, int have_workspace) {
+    const FusedSplit split = takes_split(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0, qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols));
+    if (split.parts > 1) return (int)split.tile;
     if (takes_fewtok(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0)) return 3;
     return (int)takes_tile(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0);
 }

@@ -58,3 +58,12 @@ def test_fp32_products_that_multiply_codes(tid):
             (2304, 1024, 33, True), (2303, 1024, 33, False), (9216, 256, 2000, True)]:
         assert qlinear.load().qlin_probe_gemm_f32_route(tid, n_rows, n_cols, n_tok) == codes, (n_rows, n_cols, n_tok)
     assert not qlinear.load().qlin_probe_gemm_f32_route(synth.GGML_Q4_1, 8192, 4096, 64)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: synth.TYPE_NAMES[t])
+def test_long_rows_on_few_tiles_divide_k_where_there_is_a_workspace(tid):
+    """the route then is a tile kernel where one piece would take the few-token kernel; rows of up to 16 super-blocks, 64 tokens and
+    a call without a workspace keep theirs"""
+    assert route(tid, 4096, 14336, 128) == 2 and route(tid, 4096, 14336, 128, have_workspace=0) == FEW
+    assert route(tid, 4096, 14336, 64) == FEW and route(tid, 4096, 4096, 128) == FEW and route(tid, 1024, 4096, 128) == FEW
+    assert tid not in (synth.GGML_Q4_K, synth.GGML_Q6_K) or route(tid, 4096, 14336, 768) == 1
