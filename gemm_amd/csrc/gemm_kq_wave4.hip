@@ -291,7 +291,8 @@ namespace {
 
 /* adds the parts of K in order; a thread has R rows of a token */
 template <int R>
-__global__ void __launch_bounds__(256) k_join_kernel(const float *__restrict__ buf, float *__restrict__ Y, int parts, int n_rows, int n_tok, int ldy) {
+__global__ void __launch_bounds__(256)
+k_join_kernel(const float *__restrict__ buf, float *__restrict__ Y, int parts, int n_rows, int n_tok, int ldy) {
     typedef float vec __attribute__((ext_vector_type(R)));
     const int row = (blockIdx.x * 256 + threadIdx.x) * R, t = blockIdx.y;
     if (row >= n_rows) return;
@@ -398,16 +399,18 @@ FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, 
     const auto joined = [&](int parts) { return parts > 1 ? 3.5 + parts * results * 8.0 / 4e6 : 0.0; };
     const auto small_us = [&](int parts) {
         const int items = (n_rows + 63) / 64 * ((n_tok + 127) / 128) * parts;
-        return 4.5 + (n_sb + parts - 1) / parts * (parts > 1 ? (double)((items + 255) / 256) : std::max(1.0, items / 256.0)) * small * (0.65 + 0.008 * n_sb + 0.3 * std::min(1.0, items / 256.0)) + joined(parts);
+        const double rounds = parts > 1 ? (double)((items + 255) / 256) : std::max(1.0, items / 256.0);
+        return 4.5 + (n_sb + parts - 1) / parts * rounds * small * (0.65 + 0.008 * n_sb + 0.3 * std::min(1.0, items / 256.0)) + joined(parts);
     };
     const auto large_us = [&](int parts) {
         const int items = (n_rows + 127) / 128 * ((n_tok + 255) / 256) * parts;
         return 9.0 + (n_sb + parts - 1) / parts * ((items + 255) / 256) * large * (2.1 + 0.7 * std::min(1.0, items / 224.0)) + joined(parts);
     };
-    const double one = few ? 4.0 + fewf * n_sb * (0.1 + 0.0048 * (n_tok <= 80 ? 80 : n_tok <= 96 ? 96 : 128)) * (0.7 + 0.3 * std::min(1.0, n_rows / 4096.0))
-                       : tile == kFusedSmall ? small_us(1)
-                       : tile == kFusedLarge ? large_us(1)
-                                             : 5.0 + weights * 2.8 / 4.2e6 + 2.0 * weights * n_tok / (1.25e9 * (0.4 + 0.6 * std::min(1.0, results / 6e6)));
+    double one; /* in one piece */
+    if (few) one = 4.0 + fewf * n_sb * (0.1 + 0.0048 * (n_tok <= 80 ? 80 : n_tok <= 96 ? 96 : 128)) * (0.7 + 0.3 * std::min(1.0, n_rows / 4096.0));
+    else if (tile == kFusedSmall) one = small_us(1);
+    else if (tile == kFusedLarge) one = large_us(1);
+    else one = 5.0 + weights * 2.8 / 4.2e6 + 2.0 * weights * n_tok / (1.25e9 * (0.4 + 0.6 * std::min(1.0, results / 6e6)));
     FusedSplit best = {tile, 1};
     double best_us = 0.87 * one;
     for (int parts = 2; parts <= 16 && parts <= n_sb / 2 && parts * results * sizeof(float) <= (double)workspace_bytes; parts++) {

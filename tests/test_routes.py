@@ -64,6 +64,6 @@ def test_fp32_products_that_multiply_codes(tid):
 def test_long_rows_on_few_tiles_divide_k_where_there_is_a_workspace(tid):
     """the route then is a tile kernel where one piece would take the few-token kernel; rows of up to 16 super-blocks, 64 tokens and
     a call without a workspace keep theirs"""
-    assert route(tid, 4096, 14336, 128) == 2 and route(tid, 4096, 14336, 128, have_workspace=0) == FEW
+    assert route(tid, 4096, 14336, 128) == (FEW if tid == synth.GGML_Q8_0 else 2) and route(tid, 4096, 14336, 128, have_workspace=0) == FEW
     assert route(tid, 4096, 14336, 64) == FEW and route(tid, 4096, 4096, 128) == FEW and route(tid, 1024, 4096, 128) == FEW
     assert tid not in (synth.GGML_Q4_K, synth.GGML_Q6_K) or route(tid, 4096, 14336, 768) == 1
