@@ -14,7 +14,7 @@
  *
  * Launches of a call:
  *   f32_token_exp   the power of two of every token (kF32NotFinite for one that holds an infinity or a NaN); rows of up to
- *                   2048 elements: part of the next
+ *                   2048 elements, or up to 4096 in a small X: one launch for both
  *   f32_split       X -> operand fragments of 1 KB (lane l: token l & 31, elements 8 (l >> 5) ..), so that the product's
  *                   requests and LDS reads are linear; the sub-block sums the same way
  *   gemm_f32_split  four waves per workgroup, each 32 TN rows x 32 TM tokens; a wave copies a super-block of its rows to

@@ -35,30 +35,12 @@ __global__ void __launch_bounds__(256) f32_token_exp_kernel(const float *__restr
 
 /* A workgroup lays out 256 elements of 32 tokens: thread (token, 32 elements). The order of its stores is the fragments'
  * (gemm_f32_split.h); tokens past the end are zeros. SUM: elements per sum of activations (0: none). WIDE: 16-byte
- * loads, where X's rows allow them. OWN_EXP: finds the powers of two itself, every workgroup those of its tokens over all
- * of K, which costs less than a launch for short rows. */
-template <int SUM, bool WIDE, bool OWN_EXP>
-__global__ void __launch_bounds__(256) f32_split_kernel(const float *__restrict__ X, int *__restrict__ token_exp, uint8_t *__restrict__ frags,
+ * loads, where X's rows allow them. */
+template <int SUM, bool WIDE>
+__global__ void __launch_bounds__(256) f32_split_kernel(const float *__restrict__ X, const int *__restrict__ token_exp, uint8_t *__restrict__ frags,
                                                        uint8_t *__restrict__ sums, int n_sb, int n_tok, int ldx) {
     const int j = threadIdx.x >> 3, u = threadIdx.x & 7, sb = blockIdx.x, tb = blockIdx.y, t = 32 * tb + j;
-    int e = kF32NotFinite;
-    if constexpr (OWN_EXP) {
-        static_assert(WIDE, "16-byte loads");
-        uint32_t largest = 0;
-        if (t < n_tok) {
-            const uint4 *row = reinterpret_cast<const uint4 *>(X + (size_t)t * ldx);
-#pragma unroll 8
-            for (int k = u; k < 64 * n_sb; k += 8) {
-                const uint4 q = row[k];
-                largest = max(max(largest, max(q.x & 0x7FFFFFFFu, q.y & 0x7FFFFFFFu)), max(q.z & 0x7FFFFFFFu, q.w & 0x7FFFFFFFu));
-            }
-        }
-        for (int d = 4; d > 0; d >>= 1) largest = max(largest, (uint32_t)__shfl_xor((int)largest, d, 64));
-        if (t < n_tok) {
-            e = token_exp_of(largest);
-            if (sb == 0 && u == 0) token_exp[t] = e;
-        }
-    } else if (t < n_tok) e = token_exp[t];
+    const int e = t < n_tok ? token_exp[t] : kF32NotFinite;
     const bool live = e != kF32NotFinite;
     const float *x = X + (size_t)(live ? t : 0) * ldx + 256 * sb + 32 * u;
     float v[32];
@@ -105,16 +87,107 @@ __global__ void __launch_bounds__(256) f32_split_kernel(const float *__restrict_
     }
 }
 
-constexpr int kOwnExpCols = 2048; /* 512 tokens x 1024: 2 us less than with a launch for the powers of two */
+/* The same for short rows in one launch: a workgroup finds the powers of two of two tokens and lays their rows out, 256 threads
+ * a token. Thread i takes pieces i and i + 256 of eight elements, which wait in registers for the largest element, so that X
+ * is read once. What bounds it is the launches of a short call: one in place of two, 320 tokens x 4096 into 4096 rows 46.1
+ * -> 43.5 us, 8 tokens 17.0 -> 15.4; with four tokens a workgroup 45.2 and 17.0 (too few workgroups), with one 43.6 and 15.5
+ * (single 16-byte pieces of a line). */
+constexpr int kTokensPer = 2, kHeld = 2;
+template <int SUM, bool WIDE>
+__global__ void __launch_bounds__(256 * kTokensPer)
+f32_split_rows_kernel(const float *__restrict__ X, int *__restrict__ token_exp, uint8_t *__restrict__ frags, uint8_t *__restrict__ sums, int n_sb,
+                 int n_tok, int ldx) {
+    __shared__ uint32_t per_wave[4 * kTokensPer];
+    const int mine = threadIdx.x >> 8, i = threadIdx.x & 255, t = kTokensPer * blockIdx.x + mine, pieces = 32 * n_sb;
+    const float *x = X + (size_t)(t < n_tok ? t : 0) * ldx;
+    auto load = [&](int p, float (&v)[8]) {
+        if constexpr (WIDE) {
+            const float4 a = *reinterpret_cast<const float4 *>(x + 8 * p), b = *reinterpret_cast<const float4 *>(x + 8 * p + 4);
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; k++) v[k] = x[8 * p + k];
+        }
+    };
+    uint32_t largest = 0;
+    auto look = [&](const float (&v)[8]) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) largest = max(largest, __float_as_uint(v[k]) & 0x7FFFFFFFu);
+    };
+    float held[kHeld][8];
+    if (t < n_tok) {
+#pragma unroll
+        for (int k = 0; k < kHeld; k++)
+            if (i + 256 * k < pieces) load(i + 256 * k, held[k]);
+#pragma unroll
+        for (int k = 0; k < kHeld; k++)
+            if (i + 256 * k < pieces) look(held[k]);
+    }
+    for (int d = 32; d > 0; d >>= 1) largest = max(largest, (uint32_t)__shfl_xor((int)largest, d, 64));
+    if ((threadIdx.x & 63) == 0) per_wave[threadIdx.x >> 6] = largest;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 4; w++) largest = max(largest, per_wave[4 * mine + w]);
+    const int e = t < n_tok ? token_exp_of(largest) : kF32NotFinite;
+    if (i == 0 && t < n_tok) token_exp[t] = e;
+    const bool live = e != kF32NotFinite;
+    const int j = t & 31, tb = t >> 5;
+    auto lay_out = [&](int p, const float (&in)[8]) {
+        half8 hi, lo;
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float v = live ? __builtin_ldexpf(in[k], e) : 0.0f;
+            hi[k] = (_Float16)v;
+            lo[k] = (_Float16)(v - (float)hi[k]);
+            if (SUM != 0) s += (double)v;
+        }
+        const int group = p >> 2, c = p & 3; /* 32 elements; step c >> 1, lane half c & 1 */
+        uint8_t *at = frags + ((size_t)tb * (8 * n_sb) + group) * 4096 + 16 * j + 1024 * (c >> 1) + 512 * (c & 1);
+        *reinterpret_cast<half8 *>(at) = hi;
+        *reinterpret_cast<half8 *>(at + 2048) = lo;
+        if constexpr (SUM != 0) { /* two or four neighbours have the rest of the sum */
+            s += __shfl_xor(s, 1, 64);
+            if (SUM == 32) s += __shfl_xor(s, 2, 64);
+            s *= 1.0 / 32; /* 32 elements below 2^15 */
+            const _Float16 head = (_Float16)(float)s, tail = (_Float16)(float)(s - (double)(float)head);
+            /* 32: lanes 0 .. 31 hold the eight heads, 32 .. 63 the tails; 16: lane half h sums 8 h .. + 7, heads then tails */
+            constexpr int kPer = SUM == 16 ? 2048 : 1024;
+            const int of = SUM == 16 ? 2 * (group & 7) + (c >> 1) : group & 7;
+            uint8_t *to = sums + ((size_t)tb * n_sb + (group >> 3)) * kPer + 16 * j + (SUM == 16 ? 512 * (of >> 3) + 2 * (of & 7) : 2 * of);
+            if ((c & (SUM / 8 - 1)) == 0) {
+                *reinterpret_cast<_Float16 *>(to) = head;
+                *reinterpret_cast<_Float16 *>(to + kPer / 2) = tail;
+            }
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < kHeld; k++)
+        if (i + 256 * k < pieces) lay_out(i + 256 * k, held[k]);
+}
+
+/* One launch for rows of up to 2048 elements; of up to 4096 where 16-byte loads read them and X holds at most 3 * 2^19 elements.
+ * Beyond, the pieces of lines that its workgroups store from different compute units cost more than the launch. A call of
+ * two launches against one, of n tokens into 1024 rows: 320 x 4096 29.3 us, 27.2; 400 x 4096 29.2, 29.3; 512 x 4096 30.0, 32.8;
+ * 600 x 3072 30.0, 30.8; 512 x 4096 with single loads 30.5, 33.4; the layout of 512 x 14336 alone 18.5, 31. */
+bool one_launch(int n_cols, int n_tok, bool wide) {
+    return n_cols <= 2048 || (n_cols <= 4096 && wide && (size_t)n_tok * n_cols <= (size_t)3 << 19);
+}
+static_assert(4096 <= 256 * kHeld * 8, "a row waits in registers");
 
 template <int SUM> void launch_split(const F32SplitCall &c, const F32SplitPlan &p) {
     uint8_t *ws = (uint8_t *)c.workspace;
     int *e = (int *)(ws + p.exp_at);
-    const bool wide = ((uintptr_t)c.X & 15) == 0 && c.ldx % 4 == 0, own = wide && c.n_cols <= kOwnExpCols;
-    if (!own) hipLaunchKernelGGL(f32_token_exp_kernel, dim3(c.n_tok), dim3(256), 0, c.stream, c.X, e, c.n_cols, c.ldx);
-    const auto kernel = own ? f32_split_kernel<SUM, true, true> : wide ? f32_split_kernel<SUM, true, false> : f32_split_kernel<SUM, false, false>;
-    hipLaunchKernelGGL(kernel, dim3(c.n_cols / 256, p.token_tiles * p.token_blocks), dim3(256), 0, c.stream, c.X, e, ws, ws + p.sums_at,
-                       c.n_cols / 256, c.n_tok, c.ldx);
+    const int n_sb = c.n_cols / 256, blocks = p.token_tiles * p.token_blocks;
+    const bool wide = ((uintptr_t)c.X & 15) == 0 && c.ldx % 4 == 0;
+    if (one_launch(c.n_cols, c.n_tok, wide)) {
+        const auto kernel = wide ? f32_split_rows_kernel<SUM, true> : f32_split_rows_kernel<SUM, false>;
+        hipLaunchKernelGGL(kernel, dim3(blocks * 32 / kTokensPer), dim3(256 * kTokensPer), 0, c.stream, c.X, e, ws, ws + p.sums_at, n_sb, c.n_tok, c.ldx);
+        return;
+    }
+    hipLaunchKernelGGL(f32_token_exp_kernel, dim3(c.n_tok), dim3(256), 0, c.stream, c.X, e, c.n_cols, c.ldx);
+    const auto kernel = wide ? f32_split_kernel<SUM, true> : f32_split_kernel<SUM, false>;
+    hipLaunchKernelGGL(kernel, dim3(n_sb, blocks), dim3(256), 0, c.stream, c.X, e, ws, ws + p.sums_at, n_sb, c.n_tok, c.ldx);
 }
 
 size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }

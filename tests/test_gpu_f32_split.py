@@ -61,6 +61,21 @@ def test_divisions(oracle, tid, n_tok, n_rows, n_cols):
     check(oracle, tid, n_tok, n_rows, n_cols)
 
 
+@pytest.mark.parametrize("tid", (synth.GGML_Q4_K, synth.GGML_Q6_K, synth.GGML_Q8_0), ids=lambda t: NAME[t])
+@pytest.mark.parametrize("n_tok,n_cols", [(9, 2304), (33, 3840), (63, 4096), (384, 4096), (385, 4096), (40, 4352)])
+def test_one_launch_and_two_lay_out_the_same(tid, n_tok, n_cols):
+    """rows with an odd stride are read singly and laid out by a second launch, aligned ones of up to 4096 elements in the
+    first: the product's operand is the same, so its results are, bit for bit"""
+    n_rows = 2100
+    assert takes_codes(tid, n_rows, n_cols, n_tok)
+    W = synth.make_weights(tid, n_rows, n_cols, seed=tid + n_cols)
+    X = synth.make_activation(n_cols, seed=n_tok, tokens=n_tok)
+    X[n_tok // 2, n_cols - 1] = np.inf
+    X[n_tok - 1] *= np.float32(1e-20)
+    one, two = (product(tid, W, X, n_rows, n_cols, pad) for pad in (4, 1))
+    assert np.array_equal(one, two, equal_nan=True)
+
+
 @pytest.mark.parametrize("tid", (synth.GGML_Q5_K, synth.GGML_Q8_0, synth.GGML_Q2_K), ids=lambda t: NAME[t])
 @pytest.mark.parametrize("n_rows", (4700, 70000))
 def test_magnitudes_and_not_finite(oracle, tid, n_rows):
