@@ -355,10 +355,17 @@ bool gemm_kq_wave4_covers(uint32_t type) {
  * IQ4_NL 27 / 45, 80 / 108, 46 / 55, 148 / 161, 63 / 63, 44 / 88; IQ4_XS 27 / 45, 82 / 110, 47 / 55, 154 / 162, 64 / 63,
  * 45 / 80; Q4_0 24 / 41, 72 / 91, 41 / 50, 133 / 144, 57 / 56, 39 / 72; Q2_K 24 / 42, 70 / 94, 41 / 52, 132 / 149, 55 / 58,
  * 38 / 74; Q3_K 26 / 45, 75 / 102, 44 / 54, 144 / 160, 61 / 61, 42 / 82).
- * Without a workspace there is no decode + dense route to prefer. */
+ * Without a workspace there is no decode + dense route to prefer.
+ * Up to 128 tokens half of a large tile is empty: small tiles whatever their number (77 tokens 28672 x 4096 large / small: Q4_K
+ * 51 / 38, Q5_K 52 / 41, Q6_K 57 / 48; 128 tokens 65536 x 1024 Q4_K 1.26 times, IQ4_XS 1.27, Q3_K 1.30; Q8_0 even). Past 128
+ * tokens by how often the chip has to go round: 256 large tiles (their row tiles are padded to eights) run at a time, 512 small
+ * ones, and a small round costs 0.82 of a large one, its last part less the less there is of it (time of small tiles over large,
+ * Q4_K ... Q6_K at 4096 columns: one round of large tiles, 512 small ones 0.82 - 0.89, 576 to 768 1.08 - 1.24, 1000 1.24 - 1.37;
+ * two rounds, 792 to 960 small ones 0.71 - 0.81, 1160 0.92 - 0.98, 1400 1.06 - 1.14, 1840 1.31 - 1.46; three, 1560 0.81 - 0.87,
+ * 2080 1.04 - 1.13, 2800 1.27 - 1.42; Q8_0's small tiles cost 1.2 times as much). */
 FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool have_workspace) {
     if (!gemm_kq_wave4_covers(type) || n_cols % 256 != 0 || ldx >= (1 << 22)) return kFusedNone;
-    const long long large_tiles = (long long)((n_rows + 127) / 128) * ((n_tok + 255) / 256);
+    const long long large_tiles = ((long long)n_rows + 127) / 128 * ((n_tok + 255) / 256), small_tiles = ((long long)n_rows + 63) / 64 * ((n_tok + 127) / 128);
     /* token counts up to which the large-tile and the small-tile kernel measured faster than decode + dense */
     int large_max = 512, small_max = 256; /* Q8_0 */
     switch (type) {
@@ -369,8 +376,14 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     case T_Q6_K: small_max = 512; break;
     default: break;
     }
-    if (large_tiles >= 200) return (n_tok <= large_max || !have_workspace) ? kFusedLarge : kFusedNone;
-    return (n_tok <= small_max || !have_workspace) ? kFusedSmall : kFusedNone;
+    const bool large_ok = n_tok <= large_max || !have_workspace, small_ok = n_tok <= small_max || !have_workspace;
+    if (large_tiles >= 200 && !large_ok) return kFusedNone;
+    if (n_tok > 128 && large_ok && small_ok) {
+        const long long padded = (((long long)n_rows + 127) / 128 + 7) / 8 * 8 * ((n_tok + 255) / 256), rounds = (padded + 255) / 256;
+        return small_tiles > (rounds == 1 || type == T_Q8_0 ? 512 : 650) * rounds ? kFusedLarge : kFusedSmall;
+    }
+    if (large_tiles >= 200 && (n_tok > 128 || type == T_Q8_0)) return kFusedLarge;
+    return small_ok ? kFusedSmall : kFusedNone;
 }
 
 /* Long rows on few tiles: K divided over workgroups, the parts added by a second launch (k_join_kernel). A chip of 256 compute
@@ -407,7 +420,10 @@ FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, 
         return 9.0 + (n_sb + parts - 1) / parts * ((items + 255) / 256) * large * (2.1 + 0.7 * std::min(1.0, items / 224.0)) + joined(parts);
     };
     double one; /* in one piece */
-    if (few) one = 4.0 + fewf * n_sb * (0.1 + 0.0048 * (n_tok <= 80 ? 80 : n_tok <= 96 ? 96 : 128)) * (0.7 + 0.3 * std::min(1.0, n_rows / 4096.0));
+    if (few) {
+        one = 4.0 + fewf * n_sb * (0.1 + 0.0048 * (n_tok <= 80 ? 80 : n_tok <= 96 ? 96 : 128)) * (0.7 + 0.3 * std::min(1.0, n_rows / 4096.0));
+        if (n_rows > 5120) one *= type == T_Q8_0 ? 1.75 : n_tok <= 96 ? 1.25 + n_rows / 50000.0 : 1.25 + n_rows / 20000.0; /* two workgroups a unit */
+    }
     else if (tile == kFusedSmall) one = small_us(1);
     else if (tile == kFusedLarge) one = large_us(1);
     else one = 5.0 + weights * 2.8 / 4.2e6 + 2.0 * weights * n_tok / (1.25e9 * (0.4 + 0.6 * std::min(1.0, results / 6e6)));
