@@ -32,12 +32,10 @@ int fewtok_unrounded(uint32_t type) {
  *     Rows of 2304 to 4864 elements from 1400 tiles on: the chip takes the small tiles in few enough goes (us, 64 tokens,
  *     this kernel / small tiles, 26624 x 2560 Q4_K 33 / 25, 28672 x 4096 42.8 / 38.4, Q6_K 53.9 / 48.7; at 1280 tiles even;
  *     8192 elements even everywhere)
- *   65 to 96 tokens, more than 512 row tiles, two workgroups a compute unit (rows of up to 2048 elements: 320): 80 tokens Q4_K
- *     8192 x 4096 13.7 / 22.0, 6144 x 4096 13.6 / 20.8, 8192 x 2560 10.2 / 13.3, but 8448 x 2560 17.4 / 13.4 and 8448 x 4096
- *     even; the other formats gain 1.2 to 1.8 times up to there
- *   97 to 128 tokens, more than 320: 128 tokens 8192 x 4096 Q4_K 24 / 22.4. Q6_K, whose codes cost the tiles more, from 4096
- *     elements on 512: 6144 x 4096 24 / 29, 8192 x 4096 28 / 30; Q8_0 the same, 6144 x 4096 32 / 35.6. Rows below 2048
- *     (Q8_0: 4096) elements: 256 (128 tokens 5120 x 1024 Q4_K 9.5 / 7.9)
+ *   65 to 128 tokens, more than 320: 80 tokens Q4_K 4096 x 4096 9.2 / 17.3, 5120 x 4096 11.2 / 17.6, but 77 tokens
+ *     13824 x 2560 19.6 / 16.8. (A tensor alone gains up to 512: 80 tokens Q4_K 8192 x 4096 12.7 / 20.3. Pairs of such tensors, gate
+ *     and up, which share a launch and whose results are those of a call each, lose: 2 x 6144 x 2560 at 96 18.7 / 13.8.) Past 96 tokens,
+ *     rows below 2048 (Q8_0: 4096) elements: 256 (128 tokens 5120 x 1024 Q4_K 9.5 / 7.9)
  *   rows so short that one or two waves do all of K: 256 elements from 49 tokens on (64 tokens 4096 x 256 5.6 / 5.1), 512
  *     from 97 on (128 tokens 4096 x 512 Q4_K 7.0 / 6.1; with more than 256 row tiles from 81 on)
  * The grid formats, which have no tile kernel, end at 64 (IQ3_S 13824 x 2560 at 64 tokens 23 us, decode + dense product
@@ -54,9 +52,9 @@ bool fewtok_takes(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx) {
         if (n_sb > 8) return n_sb >= 20 || (n_sb >= 16 && tiles < 1400);
         return tiles >= (n_sb < 4 || n_sb > 7 ? 1593 : n_sb == 4 ? 1200 : 3000);
     }
-    if (n_tok <= 96) return tiles <= (n_sb > 8 ? 512 : n_sb == 2 && n_tok > 80 ? 256 : 320);
-    if (n_sb >= 16 && (type == T_Q6_K || type == T_Q8_0)) return tiles <= 512;
-    if (type == T_Q8_0) return tiles <= 256;
+    if (n_tok <= 80) return tiles <= 320;
+    if (n_tok <= 96) return tiles <= (n_sb == 2 ? 256 : 320);
+    if (type == T_Q8_0) return tiles <= (n_sb < 16 ? 256 : 320);
     return n_sb > 2 && tiles <= (n_sb < 8 ? 256 : 320);
 }
 

@@ -420,10 +420,7 @@ FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, 
         return 9.0 + (n_sb + parts - 1) / parts * ((items + 255) / 256) * large * (2.1 + 0.7 * std::min(1.0, items / 224.0)) + joined(parts);
     };
     double one; /* in one piece */
-    if (few) {
-        one = 4.0 + fewf * n_sb * (0.1 + 0.0048 * (n_tok <= 80 ? 80 : n_tok <= 96 ? 96 : 128)) * (0.7 + 0.3 * std::min(1.0, n_rows / 4096.0));
-        if (n_rows > 5120) one *= type == T_Q8_0 ? 1.75 : n_tok <= 96 ? 1.25 + n_rows / 50000.0 : 1.25 + n_rows / 20000.0; /* two workgroups a unit */
-    }
+    if (few) one = 4.0 + fewf * n_sb * (0.1 + 0.0048 * (n_tok <= 80 ? 80 : n_tok <= 96 ? 96 : 128)) * (0.7 + 0.3 * std::min(1.0, n_rows / 4096.0));
     else if (tile == kFusedSmall) one = small_us(1);
     else if (tile == kFusedLarge) one = large_us(1);
     else one = 5.0 + weights * 2.8 / 4.2e6 + 2.0 * weights * n_tok / (1.25e9 * (0.4 + 0.6 * std::min(1.0, results / 6e6)));

@@ -1232,8 +1232,7 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
      * single-tensor call, which a tensor that fails them goes through below to report it */
     bool together = n_mat > 1 && n_tok > 0 && X && aligned(X, 16) && ldx % 8 == 0 && ldx >= n_cols;
     FusedTile tile = kFusedNone;
-    long long total = 0, most = 0;
-    bool few = false, same = true, matvecs = true; /* matvecs: widened once for all (IQ2_XXS 4096 + 1024 + 1024 rows x 4096, one token: 17.9 -> 13.8 us) */
+    bool few = false, matvecs = true; /* matvecs: widened once for all (IQ2_XXS 4096 + 1024 + 1024 rows x 4096, one token: 17.9 -> 13.8 us) */
     const size_t x_span = n_tok > 0 ? (size_t)(n_tok - 1) * ldx + n_cols : 0;
     for (int i = 0; i < n_mat && together; i++) {
         const bool ws_ok = workspace && aligned(workspace, 256) &&
@@ -1250,28 +1249,10 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
         const bool mine_few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
         const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
-        together = mine_few || mine != kFusedNone;
-        same = same && (i == 0 || (mine == tile && mine_few == few));
+        together = (mine_few || mine != kFusedNone) && (i == 0 || (mine == tile && mine_few == few));
         tile = mine;
         few = mine_few;
-        total += n_rows[i];
-        most = std::max(most, (long long)n_rows[i]);
     }
-    /* Rounded weights: the kernel that the launch's rows ask for, all tensors' together (past 512 row tiles the few-token kernel's
-     * workgroups, past 512 small tiles these, no longer run in one go). Q8_0's few-token kernel stays ahead for longer: to 128
-     * tokens only where a tensor alone has more than 320 tiles (2 x 4224 x 5376 at 66 tokens few-token 37 us, tiles 43; 2 x 7808 x
-     * 2304 at 88 33, 24). Over 265 pairs and triples whose kernel this and the lines for one tensor change, 49 to 700 tokens,
-     * 1.46 times as fast as by each tensor's rows, and a launch each where these asked for different kernels. */
-    if (together && !matvecs && n_tok > 64 && (type != T_Q8_0 || n_tok > 128 || most > 320 * 16) && total <= INT_MAX) {
-        const bool sum_few = takes_fewtok(type, (int)total, n_cols, n_tok, ldx, true);
-        const FusedTile sum_tile = sum_few ? kFusedNone : takes_tile(type, (int)total, n_cols, n_tok, ldx, true);
-        if ((!same || !few || total > 512 * 16) && (sum_few || sum_tile != kFusedNone)) {
-            few = sum_few;
-            tile = sum_tile;
-            same = true;
-        }
-    }
-    together = together && same;
     if (together) {
         {
             std::lock_guard<std::mutex> lk(g.mu);

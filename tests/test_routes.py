@@ -71,12 +71,10 @@ def test_long_rows_on_few_tiles_divide_k_where_there_is_a_workspace(tid):
 
 @pytest.mark.parametrize("tid", ALL, ids=lambda t: synth.TYPE_NAMES[t])
 def test_the_lines_between_the_kernels_past_48_tokens(tid):
-    """how often the chip has to go round: 512 workgroups of the few-token kernel and of small tiles at a time, 256 large tiles"""
-    q8, codes_cost = tid == synth.GGML_Q8_0, tid in (synth.GGML_Q6_K, synth.GGML_Q8_0)
-    small, large = 2, 1
+    """how often the chip has to go round: 512 small tiles at a time, 256 large ones"""
+    q8, small, large = tid == synth.GGML_Q8_0, 2, 1
     for n_rows, n_cols, n_tok, want in [
-            (8192, 2560, 65, FEW), (8192, 2560, 96, FEW), (8193, 2560, 96, small), (8192, 4096, 128, FEW if codes_cost else small),
-            (8193, 4096, 128, small), (26624, 2560, 64, FEW if q8 else small), (28672, 4096, 64, FEW if q8 else small),
-            (28672, 4096, 128, large if q8 else small), (16384, 2048, 256, small), (16385, 2048, 256, large), (16384, 2048, 129, small),
-            (16385, 2048, 130, large), (10880, 2048, 200, small), (41984, 2048, 256, large), (32896, 2048, 256, large if q8 else small)]:
+            (26624, 2560, 64, FEW if q8 else small), (28672, 4096, 64, FEW if q8 else small), (28672, 4096, 128, large if q8 else small),
+            (16384, 2048, 256, small), (16385, 2048, 256, large), (16384, 2048, 129, small), (16385, 2048, 130, large),
+            (10880, 2048, 200, small), (41984, 2048, 256, large), (32896, 2048, 256, large if q8 else small)]:
         assert route(tid, n_rows, n_cols, n_tok) == want, (n_rows, n_cols, n_tok)
