@@ -230,16 +230,18 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * tf_gemm_f16_mt_tokenmajor for the formats it re-decodes once per token (common/transformer.h:4535-4572):
  * W is decoded once to bf16 (nearest even) into `workspace` and multiplied by the dense matrix-core GEMM of
  * the vendor library. Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, IQ4_NL, IQ4_XS and Q4_0 tensors (n_cols % 256 == 0) are instead
- * decoded inside the product by this library's tile kernels, with the same single rounding to bf16, and leave the workspace alone (it may be NULL
- * for them): 256-token x 128-row tiles where 200 or more of them fill the chip (12800 rows at 257..512 tokens, 6400 at
- * 513..1024, ...), 128-token x 64-row tiles for smaller shapes (4096-row projections at 512 tokens, any row count at
- * 65..256 tokens). Given a workspace, the decode + dense route still takes the shapes where decoding once measured
+ * decoded inside the product by this library's tile kernels, with the same single rounding to bf16 and no workspace (it may be NULL
+ * for them): 128-token x 64-row tiles up to 128 tokens (Q8_0: up to 25472 rows) and beyond where 512 of them or fewer hold the
+ * product, 256-token x 128-row tiles above that wherever they take the chip fewer rounds. Given a workspace, rows of 4352
+ * elements and more on few tiles (65 to 1024 tokens) divide K over workgroups, whose sums go through the workspace to a second
+ * launch (the order of the fp32 sums differs from a call without one).
+ * Given a workspace, the decode + dense route still takes the shapes where decoding once measured
  * faster: large-tile shapes above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512 (Q6_K, Q8_0), small-tile
  * shapes of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024.
  * A few tokens of these formats (and, given a workspace, up to 64 of IQ3_S and IQ2_XXS) run in the few-token kernel
  * (n_cols % 256 == 0, no workspace used), which streams the blocks once: with unrounded codes (~1e-6) up to 32 tokens of
  * Q4_K, 24 of Q5_K, Q6_K, Q2_K, Q3_K and Q8_0 and 4 of the others; beyond that, with the same single rounding to bf16, up
- * to 48 tokens, up to 64 where a tensor has at most 8192 rows or rows of 4096 elements and up to 128 where it has at
+ * to 48 tokens, up to 64 where a tensor has at most 8192 rows or rows of 4096 elements (at most 22384 rows of up to 4864) and up to 128 where it has at
  * most 5120 rows (somewhat less for rows of fewer than 2048 elements). A token with an infinity or a NaN leaves the others alone; with unrounded codes
  * its own results may be NaN where exact arithmetic gives an infinity. Up to 4 tokens of any other
  * block format and, given a workspace, one token of a large IQ4_NL, IQ4_XS, IQ3_S or Q4_0 tensor and one to three of an
