@@ -20,6 +20,7 @@
 #include <array>
 #include <map>
 #include <mutex>
+#include <vector>
 
 #include "qlin_device.h"
 #include "qlin_internal.h"
@@ -66,15 +67,26 @@ const char *make_plan(Plan &p, bool fp32, long long n_rows, long long n_cols, lo
     if (hipblasLtMatmulPreferenceCreate(&pref) != HIPBLAS_STATUS_SUCCESS) return "hipblasLtMatmulPreferenceCreate failed";
     /* The library's kernels that split K over workgroups and reduce through the workspace write a padded
      * output (ldy > n_rows) as if it were dense (measured: K = 8192 and up with few output tiles, relative
-     * error 1.4). Offering no workspace leaves only kernels that write Y themselves. */
+     * error 1.4). Kernels without a workspace write Y themselves. */
     if (ldy != n_rows) lib_ws_bytes = 0;
     hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &lib_ws_bytes, sizeof(lib_ws_bytes));
-    hipblasLtMatmulHeuristicResult_t res[1];
-    int n = 0;
-    const hipblasStatus_t st = hipblasLtMatmulAlgoGetHeuristic(g_handle, p.desc, p.a, p.b, p.c, p.c, pref, 1, res, &n);
+    /* The limit above is no promise: the heuristic's first answer may need more (35536 x 2560 at 664 tokens 53 MiB, offered 32 or
+     * nothing; 94 of 744 random products of 256 to 160000 rows and 65 to 4096 tokens, up to 64 MiB), and the product then runs
+     * and writes past the end. So an answer counts only if what it needs fits: the first one, else the first of a longer list (the
+     * second answer nearly always). None: as if the library offered no kernel. */
+    constexpr int kAnswers = 64;
+    std::vector<hipblasLtMatmulHeuristicResult_t> res(kAnswers);
+    int n = 0, take = -1;
+    hipblasStatus_t st = HIPBLAS_STATUS_SUCCESS;
+    for (int want = 1; take < 0 && st == HIPBLAS_STATUS_SUCCESS && want <= kAnswers; want *= kAnswers) {
+        n = 0;
+        st = hipblasLtMatmulAlgoGetHeuristic(g_handle, p.desc, p.a, p.b, p.c, p.c, pref, want, res.data(), &n);
+        for (int i = 0; st == HIPBLAS_STATUS_SUCCESS && take < 0 && i < n; i++)
+            if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= lib_ws_bytes) take = i;
+    }
     hipblasLtMatmulPreferenceDestroy(pref);
-    if (st != HIPBLAS_STATUS_SUCCESS || n == 0) return "the library offers no algorithm for this shape";
-    p.algo = res[0].algo;
+    if (take < 0) return "the library offers no algorithm for this shape";
+    p.algo = res[take].algo;
     p.ws_bytes = lib_ws_bytes;
     return nullptr;
 }

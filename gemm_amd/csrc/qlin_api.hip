@@ -814,7 +814,7 @@ int qlin_gemm_tokenmajor(float *Y, const void *W, uint32_t type, int n_cols, con
     if (g.prefill_bf16 && n_tok >= 8 && n_cols % 8 == 0) {
         /* opted in: activations rounded to bf16 on the device, then the matrix-core route of
          * qlin_gemm_bf16_any_dev with internal scratch */
-        const size_t ws_bytes = dense_gemm_weight_bytes(n_rows, n_cols) + ((size_t)32 << 20);
+        const size_t ws_bytes = dense_gemm_weight_bytes(n_rows, n_cols) + kDenseLibWorkspace;
         if (int rc = g.tmp[2].ensure((size_t)n_tok * n_cols * 2)) return rc;
         if (int rc = g.tmp[3].ensure(ws_bytes)) return rc;
         HIP_TRY(launch_dequant_bf16(T_F32, g.tmp[0].p, (uint16_t *)g.tmp[2].p, n_tok, n_cols, (size_t)n_cols * 4, g.stream));
@@ -832,9 +832,13 @@ int qlin_gemm_tokenmajor(float *Y, const void *W, uint32_t type, int n_cols, con
                 Wd = (const uint16_t *)g.tmp[3].p;
             }
             void *lib_ws = (char *)g.tmp[3].p + dense_gemm_weight_bytes(n_rows, n_cols);
-            if (const char *err = launch_gemm_dense_bf16(Wd, Xb, Yd, n_rows, n_cols, n_tok, n_cols, n_rows, lib_ws,
-                                                         (size_t)32 << 20, g.stream))
-                return fail(QLIN_ERR_DEVICE, "dense bf16 GEMM: %s", err);
+            if (launch_gemm_dense_bf16(Wd, Xb, Yd, n_rows, n_cols, n_tok, n_cols, n_rows, lib_ws, kDenseLibWorkspace, g.stream) != nullptr) {
+                /* a shape the library has no kernel for: this library's tile kernel or the vector-ALU kernel */
+                if (n_cols % 256 == 0 && aligned(Wd, 16))
+                    HIP_TRY(launch_gemm_dense_own(Wd, Xb, Yd, n_rows, n_cols, n_tok, n_cols, n_rows, g.stream));
+                else
+                    HIP_TRY(launch_gemm_f32(type, dW, (const float *)g.tmp[0].p, Yd, n_rows, n_cols, n_tok, n_cols, n_rows, g.stream));
+            }
         }
     } else if (n_tok >= kDenseMinTokens) {
         /* exact weights, fp32 activations, fp32 accumulation on the matrix cores: bands of rows are decoded
