@@ -55,6 +55,7 @@
 #include "qlin_internal.h"
 
 #include <algorithm>
+#include <climits>
 
 namespace qlin {
 
@@ -392,12 +393,32 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
  * the second launch costs 3.5 us. Measured, us, one piece (few-token kernel to 128 tokens, then tiles, or decode + library) / divided, Q4_K:
  * 4096 x 14336 with 77, 128, 160, 256, 384, 512, 768 tokens 31.8 / 26.4, 45 / 29.4, 67 / 39, 69 / 44, 71 / 63, 81 / 68, 121 / 97; 2560 x 6912
  * with 128, 160, 256 19.5 / 15.8, 28 / 18, 31 / 19.5; 2048 x 5632 18.6 / 14.2, 23.5 / 15.4, 25 / 17.3; Q6_K 4096 x 14336 with 256, 768 83 / 47, 133 /
- * 106. Not below 17 super-blocks: 4096 x 4096 gains nothing (160 tokens 18.9 / 17.9, 512 23.6 / 32), and K and V of 1024 rows, which would,
- * share a launch with Q that fills the chip as it is. The estimates, in us, are fitted to such figures;
- * they err by a tenth, so that a gain of less than 13 % is left alone. */
+ * 106. Not below 17 super-blocks: 4096 x 4096 gains nothing (160 tokens 18.9 / 17.9, 512 23.6 / 32).
+ * The estimates, in us, are fitted to such figures; they err by a tenth, so that a gain of less than 13 % is left alone.
+ * Not a tensor that may come with others (may_share): their one launch, in one piece, fills the chip together and costs less than a
+ * divided product and a join each, and a tensor's results are to be the same in a call of several and in one of its own. Q4_K Q, K and V
+ * of 5120 + 1024 + 1024 rows x 5120 shared / with K and V divided: 128 tokens 28 / 46, 256 28.5 / 51, 512 49 / 77; 4096 + 2048 + 2048 x
+ * 5376 at 256 32 / 60; three of 8192 x 8192 at 77 70 / 85. What that leaves on the table: 8192 x 8192 alone at 77 39 / 27.6, 1024 x 5120
+ * at 256 20.7 / 12.8. What it does not cover: K and V of 1536 rows and more in models 5632 wide and wider, whose shape is that of a
+ * down product of a small model (2048 x 5632 at 256 24.5 / 16.7): 8192 + 2048 + 2048 x 8192 at 256 72 / 85. */
+static bool may_share(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, FusedTile tile, bool few) {
+    if (n_rows > n_cols / 2) return true; /* Q (and what has its shape), gate, up */
+    /* K and V of a model 4352 to 5376 wide */
+    if (n_cols < 22 * 256) return true;
+    /* K and V of up to 1535 rows, where a Q of 0.75 to 1.6 times n_cols rows runs in the same kernel */
+    if (n_rows >= 1536) return false;
+    for (const long long q20 : {15, 20, 32}) {
+        const int q = (int)std::min(q20 * n_cols / 20, (long long)INT_MAX);
+        const bool q_few = fewtok_takes(type, q, n_cols, n_tok, ldx);
+        if (q_few == few && (few || choose_fused_tile(type, q, n_cols, n_tok, ldx, true) == tile)) return true;
+    }
+    return false;
+}
 FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, size_t workspace_bytes, FusedTile tile, bool few) {
     const int n_sb = n_cols / 256;
-    if (!gemm_kq_wave4_covers(type) || n_cols % 256 != 0 || n_sb < 17 || ldx >= (1 << 22) || n_tok < 65 || n_tok > 1024) return {tile, 1};
+    if (!gemm_kq_wave4_covers(type) || n_cols % 256 != 0 || n_sb < 17 || ldx >= (1 << 22) || n_tok < 65 || n_tok > 1024 ||
+        may_share(type, n_rows, n_cols, n_tok, ldx, tile, few))
+        return {tile, 1};
     double small = 1.0, large = 1.0, fewf = 1.0; /* the formats' times against Q4_K's */
     switch (type) {
     case T_Q5_K: small = 1.03; large = 1.02; break;
@@ -411,12 +432,12 @@ FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, 
     const double results = (double)n_rows * n_tok, weights = (double)n_rows * n_cols;
     const auto joined = [&](int parts) { return parts > 1 ? 3.5 + parts * results * 8.0 / 4e6 : 0.0; };
     const auto small_us = [&](int parts) {
-        const int items = (n_rows + 63) / 64 * ((n_tok + 127) / 128) * parts;
+        const long long items = ((long long)n_rows + 63) / 64 * ((n_tok + 127) / 128) * parts;
         const double rounds = parts > 1 ? (double)((items + 255) / 256) : std::max(1.0, items / 256.0);
         return 4.5 + (n_sb + parts - 1) / parts * rounds * small * (0.65 + 0.008 * n_sb + 0.3 * std::min(1.0, items / 256.0)) + joined(parts);
     };
     const auto large_us = [&](int parts) {
-        const int items = (n_rows + 127) / 128 * ((n_tok + 255) / 256) * parts;
+        const long long items = ((long long)n_rows + 127) / 128 * ((n_tok + 255) / 256) * parts;
         return 9.0 + (n_sb + parts - 1) / parts * ((items + 255) / 256) * large * (2.1 + 0.7 * std::min(1.0, items / 224.0)) + joined(parts);
     };
     double one; /* in one piece */

@@ -1227,46 +1227,49 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
     return QLIN_OK;
 }
 
+/* What several tensors of one format and row length share: a launch of one kernel of this library where each would take it by
+ * itself, or the widening of X for their matvecs; a tensor that divides K goes by itself (the parts' place holds one tensor's) */
+struct MultiPlan { bool together, matvecs, few; FusedTile tile; };
+static MultiPlan plan_multi(uint32_t type, int n_mat, const int *n_rows, int n_cols, int n_tok, int ldx, size_t x_span, size_t workspace_bytes) {
+    MultiPlan p = {true, true, false, kFusedNone};
+    for (int i = 0; i < n_mat && p.together; i++) {
+        const bool ws_ok = workspace_bytes >= qlin_gemm_bf16_any_workspace_bytes(n_rows[i], n_cols);
+        p.matvecs = p.matvecs && takes_matvec(type, n_rows[i], n_cols, n_tok, ws_ok) && x_fits(x_span, workspace_bytes);
+        if (p.matvecs) continue;
+        if (takes_split(type, n_rows[i], n_cols, n_tok, ldx, ws_ok, workspace_bytes).parts > 1) return {false, false, false, kFusedNone};
+        const bool few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
+        const FusedTile tile = few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        p.together = (few || tile != kFusedNone) && (i == 0 || (tile == p.tile && few == p.few));
+        p.tile = tile;
+        p.few = few;
+    }
+    return p;
+}
+
 int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, const uint16_t *X, float *const *Y,
                              const int *n_rows, int n_cols, int n_tok, int ldx, const int *ldy, void *workspace,
                              size_t workspace_bytes, void *stream) {
     if (n_mat < 1 || n_mat > 3) return fail(QLIN_ERR_ARG, "one to three tensors per call");
     if (!W || !Y || !n_rows || !ldy) return fail(QLIN_ERR_ARG, "null pointer");
-    /* one launch where every tensor on its own would take the same tile kernel; the checks are those of the
-     * single-tensor call, which a tensor that fails them goes through below to report it */
-    bool together = n_mat > 1 && n_tok > 0 && X && aligned(X, 16) && ldx % 8 == 0 && ldx >= n_cols;
-    FusedTile tile = kFusedNone;
-    bool few = false, matvecs = true; /* matvecs: widened once for all (IQ2_XXS 4096 + 1024 + 1024 rows x 4096, one token: 17.9 -> 13.8 us) */
+    /* the checks are those of the single-tensor call, which a tensor that fails them goes through below to report it
+     * (widened once for all: IQ2_XXS 4096 + 1024 + 1024 rows x 4096, one token: 17.9 -> 13.8 us) */
+    bool together = n_mat > 1 && n_tok > 0 && X && aligned(X, 16) && ldx % 8 == 0 && ldx >= n_cols && n_cols > 0;
+    for (int i = 0; i < n_mat && together; i++)
+        together = n_rows[i] > 0 && W[i] && Y[i] && aligned(W[i], 16) && aligned(Y[i], 4) && ldy[i] >= n_rows[i]; /* plan_multi checks the format */
     const size_t x_span = n_tok > 0 ? (size_t)(n_tok - 1) * ldx + n_cols : 0;
-    for (int i = 0; i < n_mat && together; i++) {
-        const bool ws_ok = workspace && aligned(workspace, 256) &&
-                           workspace_bytes >= qlin_gemm_bf16_any_workspace_bytes(n_rows[i], n_cols);
-        together = n_rows[i] > 0 && W[i] && Y[i] && aligned(W[i], 16) && aligned(Y[i], 4) && ldy[i] >= n_rows[i] &&
-                   n_cols > 0; /* the chooser checks format and row length */
-        if (!together) break;
-        matvecs = matvecs && takes_matvec(type, n_rows[i], n_cols, n_tok, ws_ok) && x_fits(x_span, workspace_bytes);
-        if (matvecs) continue;
-        if (takes_split(type, n_rows[i], n_cols, n_tok, ldx, ws_ok, workspace_bytes).parts > 1) { /* the parts' place holds one tensor's */
-            together = false;
-            break;
-        }
-        const bool mine_few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
-        /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
-        const FusedTile mine = mine_few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
-        together = (mine_few || mine != kFusedNone) && (i == 0 || (mine == tile && mine_few == few));
-        tile = mine;
-        few = mine_few;
-    }
-    if (together) {
+    MultiPlan plan = {false, false, false, kFusedNone};
+    if (together) plan = plan_multi(type, n_mat, n_rows, n_cols, n_tok, ldx, x_span, workspace && aligned(workspace, 256) ? workspace_bytes : 0);
+    if (plan.together) {
         {
             std::lock_guard<std::mutex> lk(g.mu);
             if (int rc = ensure_init_locked(0)) return rc;
         }
-        if (matvecs)
+        if (plan.matvecs)
             return matvec_tokens(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, x_span, (float *)workspace, (hipStream_t)stream);
-        if (few)
+        if (plan.few)
             HIP_TRY(launch_gemm_fewtok(type, {n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream}));
-        else if (tile == kFusedLarge)
+        else if (plan.tile == kFusedLarge)
             HIP_TRY(launch_gemm_kq_bf16_wave4_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
         else
             HIP_TRY(launch_gemm_kq_bf16_wave4s_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
@@ -1431,6 +1434,18 @@ int qlin_probe_gemm_route(uint32_t type, int n_rows, int n_cols, int n_tok, int 
     if (split.parts > 1) return (int)split.tile;
     if (takes_fewtok(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0)) return 3;
     return (int)takes_tile(type, n_rows, n_cols, n_tok, ldx, have_workspace != 0);
+}
+
+int qlin_probe_gemm_parts(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx) {
+    return takes_split(type, n_rows, n_cols, n_tok, ldx, true, qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols)).parts;
+}
+
+int qlin_probe_gemm_multi_route(uint32_t type, int n_mat, const int *n_rows, int n_cols, int n_tok, int ldx, int have_workspace) {
+    if (n_mat < 2 || n_mat > 3 || !n_rows || n_tok < 1) return 0;
+    size_t bytes = 0;
+    for (int i = 0; i < n_mat; i++) bytes = std::max(bytes, qlin_gemm_bf16_any_workspace_bytes(n_rows[i], n_cols));
+    const MultiPlan p = plan_multi(type, n_mat, n_rows, n_cols, n_tok, ldx, (size_t)(n_tok - 1) * ldx + n_cols, have_workspace ? bytes : 0);
+    return !p.together || p.matvecs ? 0 : p.few ? 3 : (int)p.tile;
 }
 
 int qlin_probe_gemm_f32_route(uint32_t type, int n_rows, int n_cols, int n_tok) {

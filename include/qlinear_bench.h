@@ -31,6 +31,10 @@ int qlin_probe_hbm_read(const void *buf, size_t n_bytes, void *stream);
 /* which kernel qlin_gemm_bf16_any_dev picks for a shape: 1 = the 256 x 128 tile kernel, 2 = the 128 x 64 one, 3 = the
  * few-token kernel, 0 = none of them (a matvec per token, or decode to bf16 + dense product) */
 int qlin_probe_gemm_route(uint32_t ggml_type, int n_rows, int n_cols, int n_tok, int ldx, int have_workspace);
+/* over how many workgroups a tile's K is divided, given a workspace of qlin_gemm_bf16_any_workspace_bytes bytes (1: it is not) */
+int qlin_probe_gemm_parts(uint32_t ggml_type, int n_rows, int n_cols, int n_tok, int ldx);
+/* the kernel whose one launch the tensors of a qlin_gemm_bf16_multi_dev call share, numbered as above (0: a call each) */
+int qlin_probe_gemm_multi_route(uint32_t ggml_type, int n_mat, const int *n_rows, int n_cols, int n_tok, int ldx, int have_workspace);
 /* whether qlin_gemm_f32_any_dev multiplies a shape's codes on the matrix cores (1) or decodes to fp32 for the library's
  * product, or takes the few-token fp32 kernel (0), given a workspace of qlin_gemm_f32_any_workspace_bytes bytes */
 int qlin_probe_gemm_f32_route(uint32_t ggml_type, int n_rows, int n_cols, int n_tok);

@@ -62,3 +62,15 @@ def test_several_tensors_are_one_call_each(tid):
     qlinear.sync()
     for dW, dY, r in zip(dWs, dYs, rows):
         assert np.array_equal(dY.to_numpy(np.float32, (n_tok, r)), product(tid, dW, dX, r, n_cols, n_tok, n_cols, r, ws))
+
+
+# every one of them divides: 16-byte stores of the sums (2000 rows) and single ones, a last tile of 2, 16, 18 and 93 rows, K in equal and in
+# unequal parts (56, 22 and 27 super-blocks), both tile kernels
+DIVIDED = [(77, 130, 14336, 133, SMALL), (150, 2000, 5632, 2000, SMALL), (200, 2002, 6912, 2005, SMALL), (400, 2000, 14336, 2004, LARGE)]
+
+
+@pytest.mark.parametrize("tid,n_tok,n_rows,n_cols,ldy,tile", [(t,) + s for t in FUSED for s in DIVIDED] + [(synth.GGML_Q4_K,) + BIG])
+def test_divided_products(oracle, tid, n_tok, n_rows, n_cols, ldy, tile):
+    assert qlinear.load().qlin_probe_gemm_parts(tid, n_rows, n_cols, n_tok, n_cols + 8) > 1
+    assert qlinear.load().qlin_probe_gemm_route(tid, n_rows, n_cols, n_tok, n_cols + 8, 1) == tile
+    test_against_rounded_weights(oracle, tid, n_tok, n_rows, n_cols, ldy, tile)

@@ -1,0 +1,55 @@
+"""Which calls of several tensors (qlin_gemm_bf16_multi_dev) share one launch, and which products divide K. CPU only: the choice is a
+function of format and shapes (qlin_probe_gemm_multi_route: 0 a call each, 1 and 2 the tile kernels, 3 few tokens;
+qlin_probe_gemm_parts: workgroups that a tile's K is divided over)."""
+import ctypes as C
+
+import pytest
+
+from gemm_amd import qlinear
+import synth
+from tests.test_routes import ALL, route
+
+NAMES = synth.TYPE_NAMES
+LARGE, SMALL, FEW = 1, 2, 3
+
+
+def shared(tid, rows, n_cols, n_tok, have_workspace=1):
+    return qlinear.load().qlin_probe_gemm_multi_route(tid, len(rows), (C.c_int * len(rows))(*rows), n_cols, n_tok, n_cols, have_workspace)
+
+
+def parts(tid, n_rows, n_cols, n_tok):
+    return qlinear.load().qlin_probe_gemm_parts(tid, n_rows, n_cols, n_tok, n_cols)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
+def test_q_k_and_v_share_a_launch(tid):
+    for rows, n_cols, n_tok, kernel in [
+            ((4096, 1024, 1024), 4096, 128, FEW), ((4096, 1024, 1024), 4096, 256, SMALL), ((5120, 1024, 1024), 5120, 128, FEW),
+            ((5120, 1024, 1024), 5120, 256, SMALL), ((8192, 1024, 1024), 8192, 256, SMALL), ((8192, 1024, 1024), 5120, 256, SMALL),
+            ((6144, 1024, 1024), 6144, 200, SMALL), ((4096, 2048, 2048), 5376, 256, SMALL), ((8192, 8192, 8192), 8192, 77, SMALL),
+            ((6656, 6656, 6656), 6656, 128, SMALL)]:
+        assert shared(tid, rows, n_cols, n_tok) == kernel, (rows, n_cols, n_tok)
+    if tid in (synth.GGML_Q4_K, synth.GGML_Q5_K, synth.GGML_Q3_K):
+        for rows, n_cols, n_tok in [((5120, 1024, 1024), 5120, 512), ((8192, 1024, 1024), 8192, 512)]:
+            assert shared(tid, rows, n_cols, n_tok) == SMALL, (rows, n_cols, n_tok)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
+def test_a_workspace_takes_no_launch_apart(tid):
+    """K and V of up to 1535 rows, whose kernels are Q's without a workspace: dividing their K must not part them from Q"""
+    for n_cols in range(1024, 16385, 1024):
+        for kv in (128, 1024, 1535):
+            for q in (n_cols * 3 // 4, n_cols, n_cols * 8 // 5):
+                for n_tok in range(65, 1025, 29):
+                    rows = (q, kv, kv)
+                    if shared(tid, rows, n_cols, n_tok, 0) and all(route(tid, r, n_cols, n_tok) for r in rows):
+                        assert shared(tid, rows, n_cols, n_tok), (rows, n_cols, n_tok)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
+def test_down_products_divide_k_and_what_may_share_a_launch_does_not(tid):
+    for n_rows, n_cols, n_tok in [(4096, 14336, 256), (2560, 6912, 256), (2048, 5632, 200), (3584, 9728, 200), (1536, 8960, 160)]:
+        assert parts(tid, n_rows, n_cols, n_tok) > 1, (n_rows, n_cols, n_tok)
+    for n_rows, n_cols, n_tok in [(8192, 8192, 77), (5120, 5120, 256), (1024, 5120, 256), (2048, 5376, 256), (1024, 8192, 256),
+                                  (1535, 8192, 256), (2048, 4096, 256), (4096, 14336, 64), (4096, 14336, 1025)]:
+        assert parts(tid, n_rows, n_cols, n_tok) == 1, (n_rows, n_cols, n_tok)
