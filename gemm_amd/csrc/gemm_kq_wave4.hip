@@ -363,10 +363,19 @@ bool gemm_kq_wave4_covers(uint32_t type) {
  * ones, and a small round costs 0.82 of a large one, its last part less the less there is of it (time of small tiles over large,
  * Q4_K ... Q6_K at 4096 columns: one round of large tiles, 512 small ones 0.82 - 0.89, 576 to 768 1.08 - 1.24, 1000 1.24 - 1.37;
  * two rounds, 792 to 960 small ones 0.71 - 0.81, 1160 0.92 - 0.98, 1400 1.06 - 1.14, 1840 1.31 - 1.46; three, 1560 0.81 - 0.87,
- * 2080 1.04 - 1.13, 2800 1.27 - 1.42; Q8_0's small tiles cost 1.2 times as much). */
+ * 2080 1.04 - 1.13, 2800 1.27 - 1.42; Q8_0's small tiles cost 1.2 times as much).
+ * Tensors share a launch only if each takes the same kernel by itself, so the rounds count for those that come with others only
+ * where they hold for the company too. Half to twice as many rows as columns (a Q, whose K and V take small tiles): large tiles from
+ * 200 on, as for tensors of any size before (Q4_K Q, K and V of 4096 + 1024 + 1024 rows x 4096 at 1280 tokens shared / Q apart in large
+ * tiles 80 / 99, 5120 + 1024 + 1024 x 5120 at 1024 97 / 119). More, below eight times (gate and up): by rounds where one tensor and the
+ * pair agree, else the same (2 x 10240 x 2560 Q2_K at 984 tokens large / small tiles 117 / 134, 2 x 5888 x 1536 Q4_K at 1440 76 / 81). */
+static bool small_by_rounds(uint32_t type, long long n_rows, int n_tok, int n_mat) {
+    const long long padded = ((n_rows + 127) / 128 * n_mat + 7) / 8 * 8 * ((n_tok + 255) / 256), rounds = (padded + 255) / 256;
+    return (n_rows + 63) / 64 * n_mat * ((n_tok + 127) / 128) <= (rounds == 1 || type == T_Q8_0 ? 512 : 650) * rounds;
+}
 FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool have_workspace) {
     if (!gemm_kq_wave4_covers(type) || n_cols % 256 != 0 || ldx >= (1 << 22)) return kFusedNone;
-    const long long large_tiles = ((long long)n_rows + 127) / 128 * ((n_tok + 255) / 256), small_tiles = ((long long)n_rows + 63) / 64 * ((n_tok + 127) / 128);
+    const long long large_tiles = ((long long)n_rows + 127) / 128 * ((n_tok + 255) / 256);
     /* token counts up to which the large-tile and the small-tile kernel measured faster than decode + dense */
     int large_max = 512, small_max = 256; /* Q8_0 */
     switch (type) {
@@ -380,8 +389,10 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     const bool large_ok = n_tok <= large_max || !have_workspace, small_ok = n_tok <= small_max || !have_workspace;
     if (large_tiles >= 200 && !large_ok) return kFusedNone;
     if (n_tok > 128 && large_ok && small_ok) {
-        const long long padded = (((long long)n_rows + 127) / 128 + 7) / 8 * 8 * ((n_tok + 255) / 256), rounds = (padded + 255) / 256;
-        return small_tiles > (rounds == 1 || type == T_Q8_0 ? 512 : 650) * rounds ? kFusedLarge : kFusedSmall;
+        bool small = small_by_rounds(type, n_rows, n_tok, 1);
+        const bool q = n_rows > n_cols / 2 && n_rows <= 2LL * n_cols, gate = n_rows > 2LL * n_cols && n_rows < 8LL * n_cols;
+        if (q || (gate && small != small_by_rounds(type, n_rows, n_tok, 2))) small = large_tiles < 200;
+        return small ? kFusedSmall : kFusedLarge;
     }
     if (large_tiles >= 200 && (n_tok > 128 || type == T_Q8_0)) return kFusedLarge;
     return small_ok ? kFusedSmall : kFusedNone;

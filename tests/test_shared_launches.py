@@ -30,7 +30,8 @@ def test_q_k_and_v_share_a_launch(tid):
             ((6656, 6656, 6656), 6656, 128, SMALL)]:
         assert shared(tid, rows, n_cols, n_tok) == kernel, (rows, n_cols, n_tok)
     if tid in (synth.GGML_Q4_K, synth.GGML_Q5_K, synth.GGML_Q3_K):
-        for rows, n_cols, n_tok in [((5120, 1024, 1024), 5120, 512), ((8192, 1024, 1024), 8192, 512)]:
+        for rows, n_cols, n_tok in [((5120, 1024, 1024), 5120, 512), ((8192, 1024, 1024), 8192, 512), ((5120, 1024, 1024), 5120, 1024),
+                                    ((6144, 1024, 1024), 6144, 1024)]:
             assert shared(tid, rows, n_cols, n_tok) == SMALL, (rows, n_cols, n_tok)
 
 
@@ -44,6 +45,16 @@ def test_a_workspace_takes_no_launch_apart(tid):
                     rows = (q, kv, kv)
                     if shared(tid, rows, n_cols, n_tok, 0) and all(route(tid, r, n_cols, n_tok) for r in rows):
                         assert shared(tid, rows, n_cols, n_tok), (rows, n_cols, n_tok)
+
+
+@pytest.mark.parametrize("tid", (synth.GGML_Q4_K, synth.GGML_Q5_K), ids=lambda t: NAMES[t])
+def test_gate_and_up_take_the_tiles_that_suit_the_pair(tid):
+    """9728 rows at 1024 tokens: 304 large tiles alone are two rounds of the chip, 1216 small ones take less; of the pair, 608 are three
+    and 2432 take more. 10880 rows at 200 tokens: 85 large tiles of one tensor and 170 of two are one round, 340 and 680 small ones are
+    one and two, and where the two disagree the kernel is the one of 200 large tiles and more"""
+    assert shared(tid, (9728, 9728), 2560, 1024) == LARGE and route(tid, 9728, 2560, 1024) == LARGE
+    assert shared(tid, (10880, 10880), 2048, 200) == SMALL
+    assert shared(tid, (13824, 13824), 5120, 512) == LARGE and shared(tid, (13824, 13824), 5120, 128) == SMALL
 
 
 @pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
