@@ -405,7 +405,8 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
  * 4096 x 14336 with 77, 128, 160, 256, 384, 512, 768 tokens 31.8 / 26.4, 45 / 29.4, 67 / 39, 69 / 44, 71 / 63, 81 / 68, 121 / 97; 2560 x 6912
  * with 128, 160, 256 19.5 / 15.8, 28 / 18, 31 / 19.5; 2048 x 5632 18.6 / 14.2, 23.5 / 15.4, 25 / 17.3; Q6_K 4096 x 14336 with 256, 768 83 / 47, 133 /
  * 106. Not below 17 super-blocks: 4096 x 4096 gains nothing (160 tokens 18.9 / 17.9, 512 23.6 / 32).
- * The estimates, in us, are fitted to such figures; they err by a tenth, so that a gain of less than 13 % is left alone.
+ * The estimates, in us, are fitted to such figures; they err by a tenth, so that a gain of less than 13 % is left alone. Over 500
+ * random products of 256 to 8192 rows x 5632 to 16384 columns that divide: 0.60 of the time in one piece in the geometric mean, two slower, by 3 %.
  * Not a tensor that may come with others (may_share): their one launch, in one piece, fills the chip together and costs less than a
  * divided product and a join each, and a tensor's results are to be the same in a call of several and in one of its own. Q4_K Q, K and V
  * of 5120 + 1024 + 1024 rows x 5120 shared / with K and V divided: 128 tokens 28 / 46, 256 28.5 / 51, 512 49 / 77; 4096 + 2048 + 2048 x
@@ -448,7 +449,7 @@ FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, 
         return 4.5 + (n_sb + parts - 1) / parts * rounds * small * (0.65 + 0.008 * n_sb + 0.3 * std::min(1.0, items / 256.0)) + joined(parts);
     };
     const auto large_us = [&](int parts) {
-        const long long items = ((long long)n_rows + 127) / 128 * ((n_tok + 255) / 256) * parts;
+        const long long items = (((long long)n_rows + 127) / 128 * parts + 7) / 8 * 8 * ((n_tok + 255) / 256); /* dealt to 8 XCDs of 32 units: 84 x 3 are two rounds */
         return 9.0 + (n_sb + parts - 1) / parts * ((items + 255) / 256) * large * (2.1 + 0.7 * std::min(1.0, items / 224.0)) + joined(parts);
     };
     double one; /* in one piece */

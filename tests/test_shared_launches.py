@@ -64,3 +64,8 @@ def test_down_products_divide_k_and_what_may_share_a_launch_does_not(tid):
     for n_rows, n_cols, n_tok in [(8192, 8192, 77), (5120, 5120, 256), (1024, 5120, 256), (2048, 5376, 256), (1024, 8192, 256),
                                   (1535, 8192, 256), (2048, 4096, 256), (4096, 14336, 64), (4096, 14336, 1025)]:
         assert parts(tid, n_rows, n_cols, n_tok) == 1, (n_rows, n_cols, n_tok)
+
+
+def test_large_parts_count_the_padding_of_their_row_tiles():
+    """21 row tiles in four parts are 84, which eight dies take as 88: times three token tiles two rounds of 256 compute units"""
+    assert parts(synth.GGML_IQ4_NL, 2624, 11520, 612) != 4 or route(synth.GGML_IQ4_NL, 2624, 11520, 612) != LARGE
