@@ -11,7 +11,7 @@
  *     vector and 6 LDS instructions, on operand-layout loads and an operand in LDS 150 and 20. This is what bounds the smaller formats.
  *   - The digits of x are made while the first blocks are on their way: requests complete in order and x is the first of them.
  *   - A pair's row group is eight rows of gate and eight of up, so 56 rows of either per compute unit are seven whole items.
- *   - Rows of up to 2048 elements start as many waves as they have super-blocks.
+ *   - Rows of up to 4096 elements start as many waves as they have super-blocks.
  * What bounds it now: at 4096 x 4096 and below the launch (3.5 us without work); in large tensors the load path, whose 1 KB requests
  * touch four blocks, that is twelve 128-byte lines instead of eight (Q6_K 14336 x 4096: 12.5 us, with the arithmetic removed
  * 12.4, with 16-byte aligned pieces, which cost more instructions than they save, 11.0; a bare read 8.6). Three images, eight
@@ -561,17 +561,23 @@ hipError_t dma_launch(const GemvJob &job, const float *x, int n_sb, int rows_per
 }
 
 /* Where this kernel measured faster than the one that would run instead (gemv_grid.hip, gemv_int.hip); us, that one / this, rows x
- * columns, 2 x: a gate and up pair.
+ * columns, 2 x: a gate and up pair. Over 512 to 32000 rows x 1024 to 14336 columns the choice costs 0.1 to 0.5 % of the better one's time in
+ * the geometric mean by format, 1.1 % with IQ2_XXS tensors alone.
  *   Q4_K, whose own kernels (gemv_q4k.hip) have this structure for one matrix and the same items: many rows of up to 2048 columns (32000 x
  *     1024 8.5 / 6.7, 2 x 14336 x 2048 9.2 / 8.3) and of 17 to 24 super-blocks (2 x 32000 x 5632 43.6 / 40.1; 9216 x 3072 5.3 / 5.9)
  *   Q6_K, Q5_K, Q3_K everywhere (256 to 151936 rows x 1024 to 14336: 1.21, 1.23 and 1.41 times faster in the mean, pairs 1.29, 1.34, 1.62)
- *   Q8_0 but for large tensors of 2304 to 4096 columns, which its own kernel streams row by row (2 x 9216 x 4096 15.7 / 18.8, 32000 x
- *     4096 24.7 / 25.8, 100000 x 2560 47 / 50, but 14336 x 4096 12.6 / 12.7)
- *   2304 to 3840 columns of a few rows: ten to fifteen waves with an item or two each do not make up for the start (2 x 4096 x 2560
- *     Q4_0 4.4 / 4.9, Q8_0 5.5 / 5.9; 6144 x 2560 Q4_0 4.1 / 4.5), and the 2- and 4-bit formats from 2048 on
- *   Q2_K, IQ4_XS: few rows of more than 12288 columns (1024 x 14336 7.2 / 7.7, 8.7 / 9.1)
- *   IQ3_S, IQ2_XXS, whose workgroups wait for their tables together: where rows are few (IQ3_S 6144 x 4096 7.4 / 7.8, IQ2_XXS 4096 x
- *     11008 7.2 / 8.7), but 32000 x 2048 14.2 / 10.4, 11.4 / 8.7, 2 x 14336 x 8192 43 / 28, 24 / 21 */
+ *   Nine to fifteen super-blocks: as many waves with an item or two each, which do not make up for the start, until a wave has several;
+ *     with one row group each it is even or better again
+ *       Q8_0 tensors of 3073 to 8192 rows (6144 x 2560 1.07 times the time), pairs of 1537 to 4096 (2 x 4096 x 2304 1.09; 2 x 512 x 2304 0.77)
+ *       Q4_0, IQ4_NL, IQ4_XS, Q2_K from eight on: tensors of up to 9216 rows (6144 x 2560 Q4_0 4.1 / 4.5, IQ4_XS 1.04 times the time), pairs of up
+ *         to 6144 (2 x 4096 x 2560 4.4 / 4.9, 1.12 times; IQ4_XS 2 x 2048 x 2048 1.07)
+ *   Q8_0 of twelve to sixteen super-blocks and many rows, which its own kernel streams row by row: 32000 x 4096 24.7 / 25.8; pairs of
+ *     eleven to sixteen from 8193 rows on (2 x 9216 x 4096 15.7 / 18.8, 2 x 14336 x 3072 1.06 times the time, 2 x 14336 x 4096 1.12)
+ *   Q2_K, IQ4_XS: few rows of more than 10240 and 12288 columns, whose blocks are small beside the x that every workgroup prepares (1024
+ *     x 14336 7.2 / 7.7, 8.7 / 9.1)
+ *   IQ3_S, IQ2_XXS, whose workgroups wait for their tables together, which rows must be many enough to cover: IQ3_S 6144 x 4096 7.4 / 7.8,
+ *     4096 x 6144 1.09 times the time, 2 x 512 x 4096 1.10, IQ2_XXS 4096 x 11008 7.2 / 8.7, 2 x 4096 x 4096 1.24, 2 x 4096 x 6144 1.21, but
+ *     32000 x 2048 14.2 / 10.4, 11.4 / 8.7, 2 x 14336 x 8192 43 / 28, 24 / 21 */
 bool dma_pays(uint32_t type, Kind kind, int n_rows, int n_sb) {
     const bool pair = kind == kPair, narrow = n_sb >= 9 && n_sb <= 15;
     switch (type) {
@@ -581,56 +587,70 @@ bool dma_pays(uint32_t type, Kind kind, int n_rows, int n_sb) {
     }
     case T_Q6_K: case T_Q5_K: case T_Q3_K: return true;
     case T_Q8_0:
-        if (pair && ((narrow && n_rows <= 4096) || (n_sb > 16 && n_sb <= 48 && n_rows > 2048 && n_rows <= 4096))) return false;
-        if (!pair && narrow && n_rows > 3072 && n_rows <= 8192) return false;
-        if (n_sb >= 9 && n_sb <= 16) return (pair ? 2 : 1) * (long long)n_rows <= (n_sb <= 10 ? 65536 : 16384);
-        return true;
+        if (pair) return !(narrow && n_rows > 1536 && n_rows <= 4096) && !(n_sb >= 11 && n_sb <= 16 && n_rows > 8192);
+        return !(narrow && n_rows > 3072 && n_rows <= 8192) && !(n_sb >= 12 && n_sb <= 16 && n_rows > 16384);
     case T_Q4_0: case T_IQ4_NL: case T_IQ4_XS: case T_Q2_K:
-        if (n_sb >= 8 && n_sb <= 15 && n_rows <= (pair ? 6144 : 9216)) return false;
-        if (type == T_Q4_0 && pair) return !(n_sb > 22 && n_sb <= 48 && n_rows > 2048 && n_rows <= 4096) && !(n_sb >= 11 && n_sb <= 15 && n_rows > 16384);
+        if ((narrow || n_sb == 8) && n_rows <= (pair ? 6144 : 9216)) return false;
         return pair || n_rows > 4096 || !((type == T_Q2_K && n_sb > 40) || (type == T_IQ4_XS && n_sb > 48));
-    case T_IQ3_S:
-        if (pair) return !(n_sb >= 9 && n_sb <= 16 && n_rows <= (n_sb <= 12 ? 4096 : 1024));
-        return !(n_sb >= 9 && n_sb <= (n_rows <= 4096 ? 32 : 24) && n_rows > 3072 && n_rows <= 8192);
+    case T_IQ3_S: return pair ? !(n_sb >= 9 && n_sb <= 16 && n_rows <= 4096) : !(n_sb >= 9 && n_sb <= 24 && n_rows > 3072 && n_rows <= 8192);
     case T_IQ2_XXS:
         if (n_sb < 8) return true;
         if (n_sb <= 12) return n_rows >= (pair ? 9216 : 14336);
-        return pair && n_sb > 16 && !(n_rows > 2048 && n_rows <= 4096 && n_sb <= 32);
+        return pair && n_sb > 16 && !(n_sb <= 24 && n_rows > 2048 && n_rows <= 4096);
     default: return false;
     }
+}
+
+/* how a call runs here: waves of a workgroup and its rows; waves 0: it does not */
+struct DmaPlan { int waves, rows_per_wg, rounds; bool lng; };
+
+template <uint32_t T> DmaPlan dma_plan(Kind kind, int n_mat, const int *n_rows_of, int n_cols, size_t pitch, int n_cu) {
+    using Short = DmaShape<DmaFmt<T>, 16, 2, false>;
+    using Long = DmaShape<DmaFmt<T>, 16, 2, true>;
+    const DmaPlan none = {0, 0, 0, false};
+    const int n_sb = n_cols / 256;
+    if (n_cols % 256 != 0 || n_sb < 1 || n_sb > 64 || pitch > (1u << 24)) return none;
+    int n_rows = n_rows_of[0];
+    if (kind == kSeveral)
+        for (int m = 1; m < n_mat; m++) {
+            if (n_rows_of[m - 1] % 16) return none; /* a row group would hold rows of two matrices */
+            n_rows += n_rows_of[m];
+        }
+    if (n_rows == 0 || !dma_pays(T, kind, n_rows, n_sb)) return none;
+    DmaPlan p;
+    p.waves = n_sb < kMaxWaves ? n_sb : kMaxWaves;
+    while (p.waves < n_sb && p.waves * Long::kWaveLds > Long::kBudget - 1024) p.waves--; /* Q8_0: 14 */
+    p.lng = p.waves < n_sb;
+    /* one workgroup per compute unit where its partial sums fit in LDS, else so many equal rounds of workgroups that they do */
+    const int unit = kind == kSeveral ? 16 : kind == kPair ? 8 : 1, group = kind == kPair ? 8 : 16;
+    const int max_rows = (Long::kBudget - p.waves * (p.lng ? Long::kWaveLds : Short::kWaveLds)) / (16 * p.waves * (int)sizeof(float)) * group;
+    const int per_cu = (n_rows + n_cu - 1) / n_cu;
+    p.rounds = (per_cu + max_rows - 1) / max_rows;
+    p.rows_per_wg = ((n_rows + n_cu * p.rounds - 1) / (n_cu * p.rounds) + unit - 1) / unit * unit;
+    return p;
 }
 
 template <uint32_t T>
 bool dma_typed(const GemvJob &job, const float *x, int n_cols, int n_cu, hipStream_t stream, hipError_t *err, size_t row_stride) {
     using F = DmaFmt<T>;
-    using Short = DmaShape<F, 16, 2, false>;
-    using Long = DmaShape<F, 16, 2, true>;
-    const int n_sb = n_cols / 256;
-    if (n_cols % 256 != 0 || n_sb < 1 || n_sb > 64 || ((uintptr_t)x & 15)) return false;
+    if ((uintptr_t)x & 15 || row_stride % F::kAlign) return false;
     for (int m = 0; m < job.n_mat; m++)
         if ((uintptr_t)job.W[m] % F::kAlign) return false;
-    if (row_stride % F::kAlign) return false;
     const Kind kind = job.mode == kSiluMul ? kPair : job.n_mat > 1 ? kSeveral : kOne;
-    const int n_rows = kind == kPair ? job.n_rows[0] : job.total_rows();
-    const size_t pitch = row_stride ? row_stride : (size_t)n_sb * F::kBlock;
-    if (n_rows == 0 || pitch > (1u << 24) || !dma_pays(T, kind, n_rows, n_sb)) return false;
-    if (kind == kSeveral)
-        for (int m = 0; m + 1 < job.n_mat; m++)
-            if (job.n_rows[m] % 16) return false;
-    int waves = n_sb < kMaxWaves ? n_sb : kMaxWaves;
-    while (waves < n_sb && waves * Long::kWaveLds > Long::kBudget - 1024) waves--; /* Q8_0: 14 */
-    const bool lng = waves < n_sb;
-    /* one workgroup per compute unit where its partial sums fit in LDS, else so many equal rounds of workgroups that they do */
-    const int unit = kind == kSeveral ? 16 : kind == kPair ? 8 : 1, group = kind == kPair ? 8 : 16;
-    const int max_rows = (Long::kBudget - waves * (lng ? Long::kWaveLds : Short::kWaveLds)) / (16 * waves * (int)sizeof(float)) * group;
-    const int per_cu = (n_rows + n_cu - 1) / n_cu, rounds = (per_cu + max_rows - 1) / max_rows;
-    const int rows_per_wg = ((n_rows + n_cu * rounds - 1) / (n_cu * rounds) + unit - 1) / unit * unit;
-    const auto go = [&](auto launch) { *err = launch(job, x, n_sb, rows_per_wg, waves, pitch, stream); };
-    if (kind == kPair) lng ? go(dma_launch<F, 16, 2, true, kPair>) : go(dma_launch<F, 16, 2, false, kPair>);
-    else if (kind == kSeveral) lng ? go(dma_launch<F, 16, 2, true, kSeveral>) : go(dma_launch<F, 16, 2, false, kSeveral>);
-    else if (rows_per_wg <= 8) lng ? go(dma_launch<F, 8, 2, true, kOne>) : go(dma_launch<F, 8, 2, false, kOne>);
-    else lng ? go(dma_launch<F, 16, 2, true, kOne>) : go(dma_launch<F, 16, 2, false, kOne>);
+    const size_t pitch = row_stride ? row_stride : (size_t)(n_cols / 256) * F::kBlock;
+    const DmaPlan p = dma_plan<T>(kind, job.n_mat, job.n_rows, n_cols, pitch, n_cu);
+    if (!p.waves) return false;
+    const auto go = [&](auto launch) { *err = launch(job, x, n_cols / 256, p.rows_per_wg, p.waves, pitch, stream); };
+    if (kind == kPair) p.lng ? go(dma_launch<F, 16, 2, true, kPair>) : go(dma_launch<F, 16, 2, false, kPair>);
+    else if (kind == kSeveral) p.lng ? go(dma_launch<F, 16, 2, true, kSeveral>) : go(dma_launch<F, 16, 2, false, kSeveral>);
+    else if (p.rows_per_wg <= 8) p.lng ? go(dma_launch<F, 8, 2, true, kOne>) : go(dma_launch<F, 8, 2, false, kOne>);
+    else p.lng ? go(dma_launch<F, 16, 2, true, kOne>) : go(dma_launch<F, 16, 2, false, kOne>);
     return true;
+}
+
+template <uint32_t T> int dma_probe(bool pair, int n_mat, const int *n_rows, int n_cols, int n_cu) {
+    const DmaPlan p = dma_plan<T>(pair ? kPair : n_mat > 1 ? kSeveral : kOne, n_mat, n_rows, n_cols, (size_t)(n_cols / 256) * DmaFmt<T>::kBlock, n_cu);
+    return p.waves + 100 * p.rounds;
 }
 
 }  // namespace
@@ -651,6 +671,23 @@ bool launch_gemv_dma(uint32_t type, const GemvJob &job, const float *x, int n_co
     case T_IQ2_XXS: return dma_typed<T_IQ2_XXS>(job, x, n_cols, n_cu, stream, err, row_stride);
     case T_IQ3_S: return dma_typed<T_IQ3_S>(job, x, n_cols, n_cu, stream, err, row_stride);
     default: return false;
+    }
+}
+
+int probe_gemv_dma(uint32_t type, bool pair, int n_mat, const int *n_rows, int n_cols, int n_cu) {
+    switch (type) {
+    case T_Q4_K: return dma_probe<T_Q4_K>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_Q6_K: return dma_probe<T_Q6_K>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_Q8_0: return dma_probe<T_Q8_0>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_Q5_K: return dma_probe<T_Q5_K>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_Q2_K: return dma_probe<T_Q2_K>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_Q3_K: return dma_probe<T_Q3_K>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_Q4_0: return dma_probe<T_Q4_0>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_IQ4_NL: return dma_probe<T_IQ4_NL>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_IQ4_XS: return dma_probe<T_IQ4_XS>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_IQ2_XXS: return dma_probe<T_IQ2_XXS>(pair, n_mat, n_rows, n_cols, n_cu);
+    case T_IQ3_S: return dma_probe<T_IQ3_S>(pair, n_mat, n_rows, n_cols, n_cu);
+    default: return 0;
     }
 }
 

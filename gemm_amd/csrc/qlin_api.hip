@@ -1456,6 +1456,13 @@ int qlin_probe_gemm_multi_route(uint32_t type, int n_mat, const int *n_rows, int
     return !p.together || p.matvecs ? 0 : p.few ? 3 : (int)p.tile;
 }
 
+int qlin_probe_gemv_lds(uint32_t type, int pair, int n_mat, const int *n_rows, int n_cols) {
+    if (n_mat < 1 || n_mat > 3 || !n_rows || n_cols < 0 || (pair && n_mat != 2)) return 0;
+    for (int m = 0; m < n_mat; m++)
+        if (n_rows[m] < 0) return 0;
+    return probe_gemv_dma(type, pair != 0, n_mat, n_rows, n_cols, g.n_cu);
+}
+
 int qlin_probe_gemm_f32_route(uint32_t type, int n_rows, int n_cols, int n_tok) {
     return n_tok >= kDenseMinTokens && f32_split_takes(type, n_rows, n_cols, n_tok, qlin_gemm_f32_any_workspace_bytes(n_rows, n_cols));
 }

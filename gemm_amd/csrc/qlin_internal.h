@@ -84,6 +84,8 @@ bool launch_gemv_grid(uint32_t type, const GemvJob &job, const float *x, int n_c
 /* matvec on blocks copied to LDS (gemv_dma.hip), where it measured faster than the others; same contract as launch_gemv_stream */
 bool launch_gemv_dma(uint32_t type, const GemvJob &job, const float *x, int n_cols, int n_cu, hipStream_t stream, hipError_t *err,
                      size_t row_stride = 0);
+/* for the tests: the waves of a workgroup + 100 x the rounds of workgroups that a call takes there (0: another kernel runs) */
+int probe_gemv_dma(uint32_t type, bool pair, int n_mat, const int *n_rows, int n_cols, int n_cu);
 bool gemv_grid_covers(uint32_t type); /* the formats it has an item for */
 /* A few tokens, each on its own, through their top_k experts as two matvec launches: gate + up + SiLU into h
  * (n_tok * top_k * n_ff floats, X [n_tok, n_embd] bf16), then down with the routing weights folded into h. Q4_K experts

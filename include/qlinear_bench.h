@@ -35,6 +35,9 @@ int qlin_probe_gemm_route(uint32_t ggml_type, int n_rows, int n_cols, int n_tok,
 int qlin_probe_gemm_parts(uint32_t ggml_type, int n_rows, int n_cols, int n_tok, int ldx);
 /* the kernel whose one launch the tensors of a qlin_gemm_bf16_multi_dev call share, numbered as above (0: a call each) */
 int qlin_probe_gemm_multi_route(uint32_t ggml_type, int n_mat, const int *n_rows, int n_cols, int n_tok, int ldx, int have_workspace);
+/* whether a matvec on aligned, unpadded operands copies its blocks to LDS (gemv_dma.hip), for one to three matrices or (pair) gate and
+ * up: 0, or the waves of a workgroup + 100 x the rounds of workgroups */
+int qlin_probe_gemv_lds(uint32_t ggml_type, int pair, int n_mat, const int *n_rows, int n_cols);
 /* whether qlin_gemm_f32_any_dev multiplies a shape's codes on the matrix cores (1) or decodes to fp32 for the library's
  * product, or takes the few-token fp32 kernel (0), given a workspace of qlin_gemm_f32_any_workspace_bytes bytes */
 int qlin_probe_gemm_f32_route(uint32_t ggml_type, int n_rows, int n_cols, int n_tok);

@@ -2,6 +2,8 @@
 groups of 8 and 16 and their remainders, one to sixteen waves, one to four passes over a row, an image slot used again, several
 rounds of workgroups, each call shape. Relative L2 <= 1e-5 like every fp32 matvec path; the error of the paths it replaces is 1e-7
 to 6e-7."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -27,7 +29,7 @@ def want_of(oracle, tid, W, x, n_cols):
     return np.resize(w, W.shape[0])
 
 
-# rows: 1 and 2043 (8 a workgroup, the last one short), 2049 (9), 9000 (36: a third group of 4), 40961 (161), 100003 (rounds)
+# rows: 1 and 2043 (8 a workgroup, the last one short), 2049 (9), 9000 (36: a third group of 4), 40961 (161), 100003 (391)
 # columns: 1, 5, 8 super-blocks; 17 and 22 (two passes, some waves one), 43 (three), 54 and 56 (four)
 @pytest.mark.parametrize("n_rows,n_cols", [(1, 256), (2043, 1280), (2049, 2048), (9000, 1024), (40961, 1536), (100003, 256), (13000, 5632),
                                            (14001, 4352), (517, 11008), (4100, 13824), (2111, 14336)])
@@ -88,3 +90,44 @@ def test_x_that_is_not_finite_and_zero(oracle, tid):
     qlinear.gemv_dev(tid, dW, qlinear.DevBuf.from_numpy(np.zeros(n_cols, np.float32)), dy, n_rows, n_cols)
     qlinear.sync()
     assert not dy.to_numpy(np.float32, (n_rows,)).any()
+
+
+# That the tests below reach this kernel: qlin_probe_gemv_lds gives waves + 100 x rounds of workgroups.
+EVERYWHERE = [synth.GGML_Q5_K, synth.GGML_Q6_K, synth.GGML_Q3_K]
+ALL_BUT_GRIDS = EVERYWHERE + [synth.GGML_Q8_0, synth.GGML_Q4_0, synth.GGML_IQ4_NL, synth.GGML_IQ4_XS, synth.GGML_Q2_K]
+
+
+def route(tid, rows, n_cols, pair=0):
+    return qlinear.load().qlin_probe_gemv_lds(tid, pair, len(rows), (C.c_int * len(rows))(*rows), n_cols)
+
+
+def cases(shapes):
+    """(format, shape..., route) of every shape's formats"""
+    return [pytest.param(t, *s[1:], id="%s-%s" % (synth.TYPE_NAMES[t], "-".join(map(str, s[1:-1])))) for s in shapes for t in s[0]]
+
+
+# one pass over a row with nine to sixteen waves: row groups of 8 (the last one short) and of 16; two rounds of workgroups
+@pytest.mark.parametrize("tid,n_rows,n_cols,want", cases([
+    (EVERYWHERE + [synth.GGML_Q8_0, synth.GGML_IQ3_S], 1030, 2304, 109), (EVERYWHERE + [synth.GGML_Q8_0, synth.GGML_IQ3_S], 2050, 2560, 110),
+    (ALL_BUT_GRIDS + [synth.GGML_IQ3_S], 10007, 3840, 115), (ALL_BUT_GRIDS + [synth.GGML_IQ3_S], 14341, 4096, 116),
+    ([synth.GGML_IQ2_XXS], 14341, 3072, 112), ([synth.GGML_Q6_K], 86503, 4096, 216)]))
+def test_one_matrix_nine_to_sixteen_waves(oracle, tid, n_rows, n_cols, want):
+    assert route(tid, [n_rows], n_cols) == want
+    test_one_matrix(oracle, tid, n_rows, n_cols)
+
+
+@pytest.mark.parametrize("tid,n_rows,n_cols,want", cases([
+    (EVERYWHERE + [synth.GGML_Q8_0], 1029, 2304, 109), (EVERYWHERE + [synth.GGML_Q8_0], 7001, 3840, 115),
+    (ALL_BUT_GRIDS, 2049, 4096, 116), ([synth.GGML_IQ3_S], 7001, 4096, 116), ([synth.GGML_IQ2_XXS], 10001, 2816, 111),
+    ([synth.GGML_Q4_K], 9001, 4352, 116), ([synth.GGML_Q6_K], 43507, 4096, 216), ([synth.GGML_Q8_0], 33003, 4352, 214)]))
+def test_gate_and_up_nine_to_sixteen_waves(oracle, tid, n_rows, n_cols, want):
+    assert route(tid, [n_rows] * 2, n_cols, pair=1) == want
+    test_gate_and_up(oracle, tid, n_rows, n_cols)
+
+
+@pytest.mark.parametrize("tid,rows,n_cols,want", cases([
+    (EVERYWHERE + [synth.GGML_Q8_0, synth.GGML_IQ3_S], (1024, 512, 519), 2304, 109), (ALL_BUT_GRIDS, (4096, 1024, 1025), 4096, 116),
+    (ALL_BUT_GRIDS + [synth.GGML_IQ3_S], (10240, 48, 17), 3840, 115)]))
+def test_several_matrices_nine_to_sixteen_waves(oracle, tid, rows, n_cols, want):
+    assert route(tid, rows, n_cols) == want
+    test_several_matrices(oracle, tid, rows, n_cols)
