@@ -573,7 +573,10 @@ def gemm_route(type_id, n_tok, n_rows, n_cols):
     if r == 3:
         return "few-token kernel, no workspace"
     if r:
-        return "decoded inside the product (%s tiles), no workspace" % ("256-token x 128-row" if r == 1 else "128-token x 64-row")
+        tiles = "256-token x 128-row" if r == 1 else "128-token x 64-row"
+        parts = qlinear.load().qlin_probe_gemm_parts(type_id, n_rows, n_cols, n_tok, n_cols)
+        return "decoded inside the product (%s tiles), %s" % (
+            tiles, "K in %d parts, their sums in the workspace" % parts if parts > 1 else "no workspace")
     return "dense library product" if type_id == synth.GGML_BF16 else "decode to bf16 + dense library product"
 
 
