@@ -529,12 +529,12 @@ struct TileSet { /* named members, not arrays: the kernels pick by comparisons o
     float *Y0, *Y1, *Y2;
     int n_rows0, n_rows1, n_rows2, ldy0, ldy1, ldy2, end0, end1, end2;
 };
-/* host: entries past n_mat repeat the last tensor and own no tile -> the number of row tiles */
+/* host: entries past n_mat repeat the last tensor and own no tile -> the number of row tiles (of items, KItems) */
 inline int fill_tile_set(TileSet &set, int n_mat, const void *const *W, float *const *Y, const int *n_rows, const int *ldy,
-                         int rows_per_tile) {
+                         int rows_per_tile, const KSplit &split = KSplit()) {
     int n_tiles = 0, end[3];
     for (int i = 0; i < 3; i++) {
-        if (i < n_mat) n_tiles += (n_rows[i] + rows_per_tile - 1) / rows_per_tile;
+        if (i < n_mat) n_tiles += (n_rows[i] + rows_per_tile - 1) / rows_per_tile * split.parts[i];
         end[i] = n_tiles;
     }
     const int j1 = n_mat > 1 ? 1 : 0, j2 = n_mat > 2 ? 2 : j1;
@@ -555,19 +555,35 @@ QLIN_INL TileOf tile_of(const TileSet &set, int tile_all) {
     return t;
 }
 
-/* A workgroup's share of K (KSplit, qlin_internal.h): every tile is `parts` items, and the ends of the TileSet count items */
+/* Where tensors of a launch divide K (KSplit, qlin_internal.h) a tile is its tensor's `parts` items, numbered one after another, and
+ * the ends of the TileSet count items. Launches that divide nothing have a kernel of their own: the choice costs each
+ * workgroup 0.2 to 0.4 us at its start (4096 x 4096 Q4_K at 256 tokens 18.2 -> 18.5 us). */
+template <bool DIVIDED> struct KItems {};
+template <> struct KItems<true> { float *buf0, *buf1, *buf2; int parts0, parts1, parts2; };
+inline KItems<true> k_items(const KSplit &s) { return {s.buf[0], s.buf[1], s.buf[2], s.parts[0], s.parts[1], s.parts[2]}; }
+
+/* a workgroup's share of K */
 struct KPart { const uint8_t *W; float *out; int n_rows, ld, tile, sb0, n_sb; };
-QLIN_INL KPart k_part(const TileSet &set, const KSplit &split, int item, int n_sb, int n_tok) {
+QLIN_INL KPart k_part(const TileSet &set, const KItems<false> &, int item, int n_sb, int) {
+    const TileOf t = tile_of(set, item);
+    return {t.W, t.Y, t.n_rows, t.ldy, t.tile, 0, n_sb};
+}
+QLIN_INL KPart k_part(const TileSet &set, const KItems<true> &split, int item, int n_sb, int n_tok) {
     const TileOf t = tile_of(set, item);
     KPart p = {t.W, t.Y, t.n_rows, t.ldy, t.tile, 0, n_sb};
-    if (split.parts > 1) {
+    int n_parts;
+    float *buf;
+    if (item < set.end0) { n_parts = split.parts0; buf = split.buf0; }
+    else if (item < set.end1) { n_parts = split.parts1; buf = split.buf1; }
+    else { n_parts = split.parts2; buf = split.buf2; }
+    if (n_parts > 1) {
         auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); }; /* (divisions run in vector registers) */
-        const unsigned parts = (unsigned)split.parts;
+        const unsigned parts = (unsigned)n_parts;
         p.tile = uniform((int)((unsigned)t.tile / parts));
-        const unsigned part = (unsigned)(t.tile - p.tile * split.parts);
+        const unsigned part = (unsigned)(t.tile - p.tile * n_parts);
         p.sb0 = uniform((int)((unsigned)n_sb * part / parts));
         p.n_sb = uniform((int)((unsigned)n_sb * (part + 1) / parts)) - p.sb0;
-        p.out = split.buf + (size_t)part * n_tok * t.n_rows;
+        p.out = buf + (size_t)part * n_tok * t.n_rows;
         p.ld = t.n_rows;
     }
     return p;

@@ -172,9 +172,10 @@ template <class F, int... J> QLIN_INL void load_cur_extra(Ctx<F> &c, std::intege
 
 }  // namespace
 
-template <class F>
+template <class F, bool DIVIDED>
 __global__ void __launch_bounds__(256)
-gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles, KSplit split) {
+gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles,
+                          const KItems<DIVIDED> split) {
     /* raw blocks of one super-block of each wave's 32 weight rows (32 x kPieces pieces, rounded up to whole requests) */
     __shared__ __attribute__((aligned(1024))) uint8_t w4_raw[4 * F::kReq * 1024];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -290,27 +291,40 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_
 
 namespace {
 
-/* adds the parts of K in order; a thread has R rows of a token */
+/* adds the parts of K in order; a thread has R rows of a token, blockIdx.z is the tensor */
+struct JoinOne { const float *buf; float *Y; int parts, n_rows, ldy; };
+struct JoinSet { JoinOne a, b, c; };
 template <int R>
 __global__ void __launch_bounds__(256)
-k_join_kernel(const float *__restrict__ buf, float *__restrict__ Y, int parts, int n_rows, int n_tok, int ldy) {
+k_join_kernel(const JoinSet set, int n_tok) {
     typedef float vec __attribute__((ext_vector_type(R)));
     const int row = (blockIdx.x * 256 + threadIdx.x) * R, t = blockIdx.y;
-    if (row >= n_rows) return;
-    const float *at = buf + (size_t)t * n_rows + row;
+    JoinOne j = set.a;
+    if (blockIdx.z == 1) j = set.b;
+    if (blockIdx.z == 2) j = set.c;
+    if (row >= j.n_rows) return;
+    const float *at = j.buf + (size_t)t * j.n_rows + row;
     vec sum = *reinterpret_cast<const vec *>(at);
 #pragma unroll 4
-    for (int p = 1; p < parts; p++) sum += *reinterpret_cast<const vec *>(at + (size_t)p * n_tok * n_rows);
-    *reinterpret_cast<vec *>(Y + (size_t)t * ldy + row) = sum;
+    for (int p = 1; p < j.parts; p++) sum += *reinterpret_cast<const vec *>(at + (size_t)p * n_tok * j.n_rows);
+    *reinterpret_cast<vec *>(j.Y + (size_t)t * j.ldy + row) = sum;
 }
 
 }  // namespace
 
-void launch_k_join(const KSplit &split, float *Y, int n_rows, int n_tok, int ldy, hipStream_t stream) {
-    const bool wide = n_rows % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0; /* (the workspace is 256-byte aligned) */
+void launch_k_join(const KSplit &split, int n_mat, float *const *Y, const int *n_rows, int n_tok, const int *ldy, hipStream_t stream) {
+    JoinSet set = {};
+    int n = 0, most = 0;
+    bool wide = true; /* (a tensor's place in the workspace is 256-byte aligned) */
+    for (int i = 0; i < n_mat; i++) {
+        if (split.parts[i] < 2) continue;
+        (n == 0 ? set.a : n == 1 ? set.b : set.c) = {split.buf[i], Y[i], split.parts[i], n_rows[i], ldy[i]};
+        wide = wide && n_rows[i] % 4 == 0 && ldy[i] % 4 == 0 && ((uintptr_t)Y[i] & 15) == 0;
+        most = std::max(most, n_rows[i]);
+        n++;
+    }
     const int per = 256 * (wide ? 4 : 1);
-    hipLaunchKernelGGL(wide ? k_join_kernel<4> : k_join_kernel<1>, dim3((n_rows + per - 1) / per, n_tok), dim3(256), 0, stream, split.buf, Y,
-                       split.parts, n_rows, n_tok, ldy);
+    hipLaunchKernelGGL(wide ? k_join_kernel<4> : k_join_kernel<1>, dim3((most + per - 1) / per, n_tok, n), dim3(256), 0, stream, set, n_tok);
 }
 
 namespace {
@@ -320,13 +334,16 @@ hipError_t launch_wave4(int n_mat, const void *const *W, const uint16_t *X, floa
     const int n_sb = n_cols / 256;
     const int m_tiles = (n_tok + kBM - 1) / kBM;
     TileSet set;
-    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN) * split.parts;
-    if (split.parts > 1) set.end0 = set.end1 = set.end2 = n_tiles; /* (one tensor) */
+    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN, split);
     /* ids are dealt to 8 XCDs; pad the n-tile count to a multiple of 8 (surplus groups exit) */
     const int n_tiles_pad = (n_tiles + 7) / 8 * 8;
-    hipLaunchKernelGGL(gemm_kq_bf16_wave4_kernel<F>, dim3(n_tiles_pad * m_tiles), dim3(256), 0, stream, set, X, n_sb,
-                       n_tok, ldx, m_tiles, split);
-    if (split.parts > 1) launch_k_join(split, Y[0], n_rows[0], n_tok, ldy[0], stream);
+    const dim3 grid(n_tiles_pad * m_tiles), block(256);
+    if (split.divides()) {
+        hipLaunchKernelGGL((gemm_kq_bf16_wave4_kernel<F, true>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, k_items(split));
+        launch_k_join(split, n_mat, Y, n_rows, n_tok, ldy, stream);
+    } else {
+        hipLaunchKernelGGL((gemm_kq_bf16_wave4_kernel<F, false>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, KItems<false>());
+    }
     return hipGetLastError();
 }
 template <class F>
@@ -411,8 +428,10 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
  * divided product and a join each, and a tensor's results are to be the same in a call of several and in one of its own. Q4_K Q, K and V
  * of 5120 + 1024 + 1024 rows x 5120 shared / with K and V divided: 128 tokens 28 / 46, 256 28.5 / 51, 512 49 / 77; 4096 + 2048 + 2048 x
  * 5376 at 256 32 / 60; three of 8192 x 8192 at 77 70 / 85. What that leaves on the table: 8192 x 8192 alone at 77 39 / 27.6, 1024 x 5120
- * at 256 20.7 / 12.8. What it does not cover: K and V of 1536 rows and more in models 5632 wide and wider, whose shape is that of a
- * down product of a small model (2048 x 5632 at 256 24.5 / 16.7): 8192 + 2048 + 2048 x 8192 at 256 72 / 85. */
+ * at 256 20.7 / 12.8. K and V of 1536 rows and more in models 5632 wide and wider do divide, since a down product of a small model has
+ * their shape (2048 x 5632 at 256 24.5 / 16.7). Divided tensors share a launch and a join as well, each in its own parts (undivided
+ * shared / a call each / divided shared): 8192 + 2048 + 2048 x 8192 at 256 tokens 73 / 86 / 69, at 512 118 / 138 / 123, 6144 + 1536 + 1536
+ * x 6144 at 256 54 / 64 / 46, at 354 56 / 86 / 63; Q6_K 8192 + 4096 + 4096 x 8192 at 256 100 / 126 / 121. */
 static bool may_share(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, FusedTile tile, bool few) {
     if (n_rows > n_cols / 2) return true; /* Q (and what has its shape), gate, up */
     /* K and V of a model 4352 to 5376 wide */
@@ -469,8 +488,8 @@ FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, 
 hipError_t launch_fused_split(FusedSplit s, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
                               int ldx, int ldy, void *workspace, hipStream_t stream) {
     KSplit split;
-    split.buf = (float *)workspace;
-    split.parts = s.parts;
+    split.buf[0] = (float *)workspace;
+    split.parts[0] = s.parts;
     return s.tile == kFusedLarge ? launch_gemm_kq_bf16_wave4_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split)
                                  : launch_gemm_kq_bf16_wave4s_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split);
 }

@@ -214,9 +214,10 @@ QLIN_INL void run_half(Ctx<F> &c, float *__restrict__ Y, int n_rows, int n_tok, 
 
 }  // namespace
 
-template <class F>
+template <class F, bool DIVIDED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles, KSplit split) {
+gemm_kq_bf16_wave4s_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles,
+                           const KItems<DIVIDED> split) {
     /* raw blocks of one super-block of the two row halves (32 x kPieces pieces each, rounded up to whole requests) */
     __shared__ __attribute__((aligned(1024))) uint8_t w4s_raw[2 * F::kReq * 1024];
     constexpr int nW = Ctx<F>::kMyReq;
@@ -311,12 +312,15 @@ hipError_t launch_wave4s(int n_mat, const void *const *W, const uint16_t *X, flo
     const int n_sb = n_cols / 256;
     const int m_tiles = (n_tok + kBM - 1) / kBM;
     TileSet set;
-    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN) * split.parts;
-    if (split.parts > 1) set.end0 = set.end1 = set.end2 = n_tiles; /* (one tensor) */
+    const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN, split);
     const int n_tiles_pad = (n_tiles + 7) / 8 * 8; /* ids are dealt to 8 XCDs; surplus groups exit */
-    hipLaunchKernelGGL(gemm_kq_bf16_wave4s_kernel<F>, dim3(n_tiles_pad * m_tiles), dim3(256), 0, stream, set, X, n_sb,
-                       n_tok, ldx, m_tiles, split);
-    if (split.parts > 1) launch_k_join(split, Y[0], n_rows[0], n_tok, ldy[0], stream);
+    const dim3 grid(n_tiles_pad * m_tiles), block(256);
+    if (split.divides()) {
+        hipLaunchKernelGGL((gemm_kq_bf16_wave4s_kernel<F, true>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, k_items(split));
+        launch_k_join(split, n_mat, Y, n_rows, n_tok, ldy, stream);
+    } else {
+        hipLaunchKernelGGL((gemm_kq_bf16_wave4s_kernel<F, false>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, KItems<false>());
+    }
     return hipGetLastError();
 }
 }  // namespace

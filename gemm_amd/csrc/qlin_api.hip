@@ -1236,19 +1236,24 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
 }
 
 /* What several tensors of one format and row length share: a launch of one kernel of this library where each would take it by
- * itself, or the widening of X for their matvecs; a tensor that divides K goes by itself (the parts' place holds one tensor's) */
-struct MultiPlan { bool together, matvecs, few; FusedTile tile; };
+ * itself, or the widening of X for their matvecs. Tensors that divide K share it too, each in its own parts; their places follow each
+ * other in the workspace, and where it does not hold them all the call is one per tensor. */
+struct MultiPlan { bool together, matvecs, few; FusedTile tile; int parts[3]; size_t at[3]; };
 static MultiPlan plan_multi(uint32_t type, int n_mat, const int *n_rows, int n_cols, int n_tok, int ldx, size_t x_span, size_t workspace_bytes) {
-    MultiPlan p = {true, true, false, kFusedNone};
+    MultiPlan p = {true, true, false, kFusedNone, {1, 1, 1}, {0, 0, 0}};
+    size_t used = 0;
     for (int i = 0; i < n_mat && p.together; i++) {
         const bool ws_ok = workspace_bytes >= qlin_gemm_bf16_any_workspace_bytes(n_rows[i], n_cols);
         p.matvecs = p.matvecs && takes_matvec(type, n_rows[i], n_cols, n_tok, ws_ok) && x_fits(x_span, workspace_bytes);
         if (p.matvecs) continue;
-        if (takes_split(type, n_rows[i], n_cols, n_tok, ldx, ws_ok, workspace_bytes).parts > 1) return {false, false, false, kFusedNone};
-        const bool few = takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        const FusedSplit split = takes_split(type, n_rows[i], n_cols, n_tok, ldx, ws_ok, workspace_bytes);
+        p.parts[i] = split.parts;
+        p.at[i] = used;
+        if (split.parts > 1) used += ((size_t)split.parts * n_rows[i] * n_tok * sizeof(float) + 255) & ~(size_t)255;
+        const bool few = split.parts == 1 && takes_fewtok(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
         /* (rows of X too far apart for the few-token kernel's offsets and few tokens: one call per tensor) */
-        const FusedTile tile = few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
-        p.together = (few || tile != kFusedNone) && (i == 0 || (tile == p.tile && few == p.few));
+        const FusedTile tile = split.parts > 1 ? split.tile : few || n_tok <= fewtok_unrounded(type) ? kFusedNone : takes_tile(type, n_rows[i], n_cols, n_tok, ldx, ws_ok);
+        p.together = (few || tile != kFusedNone) && (i == 0 || (tile == p.tile && few == p.few)) && used <= workspace_bytes;
         p.tile = tile;
         p.few = few;
     }
@@ -1266,7 +1271,7 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
     for (int i = 0; i < n_mat && together; i++)
         together = n_rows[i] > 0 && W[i] && Y[i] && aligned(W[i], 16) && aligned(Y[i], 4) && ldy[i] >= n_rows[i]; /* plan_multi checks the format */
     const size_t x_span = n_tok > 0 ? (size_t)(n_tok - 1) * ldx + n_cols : 0;
-    MultiPlan plan = {false, false, false, kFusedNone};
+    MultiPlan plan = {};
     if (together) plan = plan_multi(type, n_mat, n_rows, n_cols, n_tok, ldx, x_span, workspace && aligned(workspace, 256) ? workspace_bytes : 0);
     if (plan.together) {
         {
@@ -1275,12 +1280,19 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
         }
         if (plan.matvecs)
             return matvec_tokens(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, x_span, (float *)workspace, (hipStream_t)stream);
-        if (plan.few)
+        if (plan.few) {
             HIP_TRY(launch_gemm_fewtok(type, {n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream}));
-        else if (plan.tile == kFusedLarge)
-            HIP_TRY(launch_gemm_kq_bf16_wave4_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
+            return QLIN_OK;
+        }
+        KSplit split;
+        for (int i = 0; i < n_mat; i++) {
+            split.parts[i] = plan.parts[i];
+            if (plan.parts[i] > 1) split.buf[i] = (float *)((char *)workspace + plan.at[i]);
+        }
+        if (plan.tile == kFusedLarge)
+            HIP_TRY(launch_gemm_kq_bf16_wave4_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream, split));
         else
-            HIP_TRY(launch_gemm_kq_bf16_wave4s_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
+            HIP_TRY(launch_gemm_kq_bf16_wave4s_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream, split));
         return QLIN_OK;
     }
     for (int i = 0; i < n_mat; i++)

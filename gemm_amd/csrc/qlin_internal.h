@@ -188,10 +188,14 @@ bool gemm_kq_wave4_covers(uint32_t type);
 /* the same in 128-token x 64-row tiles, two workgroups per compute unit (gemm_kq_wave4s.hip) */
 hipError_t launch_gemm_kq_bf16_wave4s(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                                       int n_tok, int ldx, int ldy, hipStream_t stream);
-/* K divided over `parts` workgroups per tile of one tensor, which write their sums to buf, [part][token][row]; launch_k_join adds
- * them up. One part: the sums go to Y. */
-struct KSplit { float *buf = nullptr; int parts = 1; };
-void launch_k_join(const KSplit &split, float *Y, int n_rows, int n_tok, int ldy, hipStream_t stream);
+/* K of a tensor divided over parts[i] workgroups per tile, which write their sums to buf[i], [part][token][row]; launch_k_join adds
+ * them up, of all tensors that are divided. One part: the sums go to Y. */
+struct KSplit {
+    float *buf[3] = {nullptr, nullptr, nullptr};
+    int parts[3] = {1, 1, 1};
+    bool divides() const { return parts[0] > 1 || parts[1] > 1 || parts[2] > 1; }
+};
+void launch_k_join(const KSplit &split, int n_mat, float *const *Y, const int *n_rows, int n_tok, const int *ldy, hipStream_t stream);
 /* the same kernel over up to three tensors of one format and K in one launch (row tiles numbered through the tensors) */
 hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,

@@ -267,7 +267,8 @@ int qlin_gemm_bf16_any_dev(uint32_t ggml_type, const void *W, const uint16_t *X,
  * the Q, K and V projections of a prefill chunk, which the reference multiplies tensor by tensor
  * (tf_gemm_f16_mt_tokenmajor per projection, common/transformer.h:5256-5258). Y[i][t * ldy[i] + r] is tensor i's
  * product. Where every tensor on its own would take the same kernel of this library (few-token, small or large tiles)
- * they share one launch, their row tiles numbered through, with the results of one call per tensor bit for bit: a
+ * they share one launch, their row tiles numbered through, with the results of one call per tensor bit for bit (tensors that divide K
+ * do so in their own parts, whose sums one more launch adds, if the workspace holds them all): a
  * 1024-row K or V projection alone is 64 workgroups of 128 tokens x 64 rows at 512 tokens on 256 compute units (Q4_K
  * 4096 + 1024 + 1024 rows x 4096 at 512 tokens: 36 us in one launch against 24 + 22 + 22). Every other case is one
  * qlin_gemm_bf16_any_dev call per tensor (those that all go through the matvec share the widening of X), with its

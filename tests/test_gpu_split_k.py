@@ -1,6 +1,8 @@
 """GPU parity of bf16 products whose K is divided over workgroups (long rows on few tiles, given a workspace), through the C ABI:
 against the oracle's weights rounded once to bf16 (relative L2 <= 2e-5, the bar of the tile kernels, which compute the same sums in
 one piece), against the same call without a workspace, and several tensors against one call each, bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,38 @@ def test_divided_products(oracle, tid, n_tok, n_rows, n_cols, ldy, tile):
     assert qlinear.load().qlin_probe_gemm_parts(tid, n_rows, n_cols, n_tok, n_cols + 8) > 1
     assert qlinear.load().qlin_probe_gemm_route(tid, n_rows, n_cols, n_tok, n_cols + 8, 1) == tile
     test_against_rounded_weights(oracle, tid, n_tok, n_rows, n_cols, ldy, tile)
+
+
+# an undivided tensor among divided ones; rows that allow 16-byte stores of the sums and that do not; the large tiles; tensors whose
+# sums do not fit the workspace together (a call each)
+SEVERAL = [(t, (2900, 1601, 2000), 5632, 150, SMALL) for t in FUSED]
+SEVERAL += [(t, (2000, 1537), 14336, 400, LARGE) for t in FUSED if t != synth.GGML_Q8_0]
+SEVERAL += [(synth.GGML_Q4_K, (1600, 1600, 1604), 5632, 256, SMALL), (synth.GGML_Q4_K, (2048, 2048, 2048), 14336, 1000, 0)]
+
+
+@pytest.mark.parametrize("tid,rows,n_cols,n_tok,want", SEVERAL)
+def test_several_divided_tensors_share_a_launch(oracle, tid, rows, n_cols, n_tok, want):
+    lib, n = qlinear.load(), len(rows)
+    parts = [lib.qlin_probe_gemm_parts(tid, r, n_cols, n_tok, n_cols) for r in rows]
+    assert sum(p > 1 for p in parts) >= 2
+    assert lib.qlin_probe_gemm_multi_route(tid, n, (C.c_int * n)(*rows), n_cols, n_tok, n_cols, 1) == want
+    Ws = [synth.make_weights(tid, r, n_cols, seed=r + i) for i, r in enumerate(rows)]
+    Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=3, tokens=n_tok))
+    dWs, dX = [qlinear.DevBuf.from_numpy(W) for W in Ws], qlinear.DevBuf.from_numpy(Xb)
+    ws_bytes, behind = max(qlinear.gemm_bf16_any_workspace_bytes(r, n_cols) for r in rows), 1 << 20
+    ws = qlinear.DevBuf.from_numpy(np.full((ws_bytes + behind) // 4, np.nan, np.float32))
+    ldys = [r + 4 * i for i, r in enumerate(rows)]
+    dYs = [qlinear.DevBuf.from_numpy(np.full((n_tok, ld), -3.0, np.float32)) for ld in ldys]
+    P = C.c_void_p * n
+    qlinear.check(lib.qlin_gemm_bf16_multi_dev(tid, n, P(*[d.ptr for d in dWs]), dX.ptr, P(*[d.ptr for d in dYs]), (C.c_int * n)(*rows), n_cols,
+                                               n_tok, n_cols, (C.c_int * n)(*ldys), ws.ptr, ws_bytes, None))
+    qlinear.sync()
+    assert np.isnan(ws.to_numpy(np.float32, ((ws_bytes + behind) // 4,))[ws_bytes // 4:]).all()
+    for W, dW, dY, r, ld in zip(Ws, dWs, dYs, rows, ldys):
+        Y = dY.to_numpy(np.float32, (n_tok, ld))
+        assert np.array_equal(Y, product(tid, dW, dX, r, n_cols, n_tok, n_cols, ld, ws))
+        some = np.r_[0:40, r - 150:r]
+        _, designed = references(oracle, tid, W.reshape(r, -1)[some], Xb, n_cols)
+        assert rel_l2(Y[:, some], designed) <= 2e-5
+    for b in (*dWs, *dYs, dX, ws):
+        b.free()

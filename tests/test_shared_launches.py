@@ -36,6 +36,16 @@ def test_q_k_and_v_share_a_launch(tid):
 
 
 @pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
+def test_divided_tensors_share_a_launch(tid):
+    """beside an undivided one, and where the workspace holds the parts of all"""
+    for rows, n_cols, n_tok in [((8192, 2048, 2048), 8192, 256), ((6144, 1536, 1536), 6144, 200), ((2900, 1601, 2000), 5632, 150)]:
+        assert parts(tid, rows[0], n_cols, n_tok) == 1 and parts(tid, rows[1], n_cols, n_tok) > 1
+        assert shared(tid, rows, n_cols, n_tok) == SMALL, (rows, n_cols, n_tok)
+    if tid == synth.GGML_Q4_K:  # three times 33 MB of sums, 59 + 34 MB of workspace
+        assert parts(tid, 2048, 14336, 1000) == 4 and shared(tid, (2048,) * 3, 14336, 1000) == 0 and shared(tid, (2048,) * 2, 14336, 1000) == LARGE
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
 def test_a_workspace_takes_no_launch_apart(tid):
     """K and V of up to 1535 rows, whose kernels are Q's without a workspace: dividing their K must not part them from Q"""
     for n_cols in range(1024, 16385, 1024):
