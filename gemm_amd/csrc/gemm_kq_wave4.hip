@@ -424,31 +424,31 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
  * 106. Not below 17 super-blocks: 4096 x 4096 gains nothing (160 tokens 18.9 / 17.9, 512 23.6 / 32).
  * The estimates, in us, are fitted to such figures; they err by a tenth, so that a gain of less than 13 % is left alone. Over 500
  * random products of 256 to 8192 rows x 5632 to 16384 columns that divide: 0.60 of the time in one piece in the geometric mean, two slower, by 3 %.
- * Not a tensor that may come with others (may_share): their one launch, in one piece, fills the chip together and costs less than a
- * divided product and a join each, and a tensor's results are to be the same in a call of several and in one of its own. Q4_K Q, K and V
- * of 5120 + 1024 + 1024 rows x 5120 shared / with K and V divided: 128 tokens 28 / 46, 256 28.5 / 51, 512 49 / 77; 4096 + 2048 + 2048 x
- * 5376 at 256 32 / 60; three of 8192 x 8192 at 77 70 / 85. What that leaves on the table: 8192 x 8192 alone at 77 39 / 27.6, 1024 x 5120
- * at 256 20.7 / 12.8. K and V of 1536 rows and more in models 5632 wide and wider do divide, since a down product of a small model has
- * their shape (2048 x 5632 at 256 24.5 / 16.7). Divided tensors share a launch and a join as well, each in its own parts (undivided
- * shared / a call each / divided shared): 8192 + 2048 + 2048 x 8192 at 256 tokens 73 / 86 / 69, at 512 118 / 138 / 123, 6144 + 1536 + 1536
- * x 6144 at 256 54 / 64 / 46, at 354 56 / 86 / 63; Q6_K 8192 + 4096 + 4096 x 8192 at 256 100 / 126 / 121. */
-static bool may_share(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, FusedTile tile, bool few) {
-    if (n_rows > n_cols / 2) return true; /* Q (and what has its shape), gate, up */
-    /* K and V of a model 4352 to 5376 wide */
-    if (n_cols < 22 * 256) return true;
-    /* K and V of up to 1535 rows, where a Q of 0.75 to 1.6 times n_cols rows runs in the same kernel */
-    if (n_rows >= 1536) return false;
-    for (const long long q20 : {15, 20, 32}) {
-        const int q = (int)std::min(q20 * n_cols / 20, (long long)INT_MAX);
-        const bool q_few = fewtok_takes(type, q, n_cols, n_tok, ldx);
-        if (q_few == few && (few || choose_fused_tile(type, q, n_cols, n_tok, ldx, true) == tile)) return true;
-    }
+ * Not a tensor that may come with others (may_share) where their one launch, in one piece, costs less than a launch in parts
+ * and its join, or than one of them apart: a tensor's results are the same in a call of several and in one of its own. us, Q4_K unless said,
+ * undivided in one launch / divided and sharing what they can:
+ *   128 tokens: 5120 + 1024 + 1024 rows x 5120, Q in the few-token kernel, K and V not, 28 / 47; three of 5376 x 5376 IQ4_NL at 94 34 / 42;
+ *     but 8192 + 1024 + 1024 x 8192 at 77 68 / 42 (K and V alone are few-token products there), three of 8192 x 8192 at 77 69 / 69
+ *   more tokens: 5120 + 1024 + 1024 x 5120 at 256 29 / 36, 4096 + 2048 + 2048 x 5376 at 256 32 / 41, 6144 + 1024 + 1024 x 6144 at 512 61 / 71;
+ *     Q8_0 8192 + 512 + 512 x 8192 at 179, Q in large tiles then, 108 / 169
+ * That leaves on the table 8192 x 8192 Q6_K alone at 512 97 / 81, 1024 x 5120 alone at 256 20.6 / 13. K and V of 1536 rows and more in models
+ * 5632 wide and wider divide, since a down product of a small model has their shape (2048 x 5632 at 256 24.5 / 16.7): undivided
+ * in one launch / a call each / now 8192 + 2048 + 2048 x 8192 at 256 73 / 86 / 69, at 512 118 / 138 / 123, 6144 + 1536 + 1536 x 6144 at 256 54 /
+ * 64 / 46, at 354 56 / 86 / 63; Q5_K 6656 + 1664 + 1664 x 6656 at 268 60 / 89 / 70. */
+static bool may_share(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, FusedTile tile) {
+    if (n_tok <= 128) /* K and V beside a Q of n_cols rows in the few-token kernel; three tensors of this shape that the chip takes at once */
+        return fewtok_takes(type, n_cols, n_cols, n_tok, ldx) || (n_rows > n_cols / 2 && 3 * (((long long)n_rows + 63) / 64) <= 256);
+    if (n_rows > n_cols / 2) return true;  /* Q (and what has its shape), gate, up */
+    if (n_cols < 22 * 256) return true;    /* K and V of a model 4352 to 5376 wide */
+    if (n_rows >= 1536 && n_cols < 6LL * n_rows) return false;
+    for (const long long q20 : {15, 20, 32}) /* K and V of few rows, where a Q of 0.75 to 1.6 times n_cols rows takes the same tiles */
+        if (choose_fused_tile(type, (int)std::min(q20 * n_cols / 20, (long long)INT_MAX), n_cols, n_tok, ldx, true) == tile) return true;
     return false;
 }
 FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, size_t workspace_bytes, FusedTile tile, bool few) {
     const int n_sb = n_cols / 256;
     if (!gemm_kq_wave4_covers(type) || n_cols % 256 != 0 || n_sb < 17 || ldx >= (1 << 22) || n_tok < 65 || n_tok > 1024 ||
-        may_share(type, n_rows, n_cols, n_tok, ldx, tile, few))
+        may_share(type, n_rows, n_cols, n_tok, ldx, tile))
         return {tile, 1};
     double small = 1.0, large = 1.0, fewf = 1.0; /* the formats' times against Q4_K's */
     switch (type) {

@@ -233,8 +233,8 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * decoded inside the product by this library's tile kernels, with the same single rounding to bf16 and no workspace (it may be NULL
  * for them): 128-token x 64-row tiles up to 128 tokens (Q8_0: up to 25472 rows) and beyond where 512 of them or fewer hold the
  * product, 256-token x 128-row tiles above that wherever they take the chip fewer rounds; for tensors of half to twice as many rows as
- * columns wherever there are 200 of them. Given a workspace, rows of 5632 elements and more on few tiles (65 to 1024 tokens, at most half
- * as many rows as columns) divide K over workgroups, whose sums go through the workspace to a second
+ * columns wherever there are 200 of them. Given a workspace, rows of 5376 elements and more on few tiles (65 to 1024 tokens; above 128 at most
+ * half as many rows as columns) divide K over workgroups, whose sums go through the workspace to a second
  * launch (the order of the fp32 sums differs from a call without one).
  * Given a workspace, the decode + dense route still takes the shapes where decoding once measured
  * faster: large-tile shapes above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512 (Q6_K, Q8_0), small-tile

@@ -66,9 +66,9 @@ def test_several_tensors_are_one_call_each(tid):
         assert np.array_equal(dY.to_numpy(np.float32, (n_tok, r)), product(tid, dW, dX, r, n_cols, n_tok, n_cols, r, ws))
 
 
-# every one of them divides: 16-byte stores of the sums (2000 rows) and single ones, a last tile of 2, 16, 18 and 93 rows, K in equal and in
+# every one of them divides: 16-byte stores of the sums (2000 and 2400 rows) and single ones, a last tile of 2, 16, 18, 93 and 96 rows, K in equal and in
 # unequal parts (56, 22 and 27 super-blocks), both tile kernels
-DIVIDED = [(77, 130, 14336, 133, SMALL), (150, 2000, 5632, 2000, SMALL), (200, 2002, 6912, 2005, SMALL), (400, 2000, 14336, 2004, LARGE)]
+DIVIDED = [(77, 130, 14336, 133, SMALL), (150, 2000, 5632, 2000, SMALL), (200, 2002, 6912, 2005, SMALL), (400, 2400, 14336, 2404, LARGE)]
 
 
 @pytest.mark.parametrize("tid,n_tok,n_rows,n_cols,ldy,tile", [(t,) + s for t in FUSED for s in DIVIDED] + [(synth.GGML_Q4_K,) + BIG])
@@ -81,8 +81,8 @@ def test_divided_products(oracle, tid, n_tok, n_rows, n_cols, ldy, tile):
 # an undivided tensor among divided ones; rows that allow 16-byte stores of the sums and that do not; the large tiles; tensors whose
 # sums do not fit the workspace together (a call each)
 SEVERAL = [(t, (2900, 1601, 2000), 5632, 150, SMALL) for t in FUSED]
-SEVERAL += [(t, (2000, 1537), 14336, 400, LARGE) for t in FUSED if t != synth.GGML_Q8_0]
-SEVERAL += [(synth.GGML_Q4_K, (1600, 1600, 1604), 5632, 256, SMALL), (synth.GGML_Q4_K, (2048, 2048, 2048), 14336, 1000, 0)]
+SEVERAL += [(t, (2400, 2401), 14336, 400, LARGE) for t in FUSED if t != synth.GGML_Q8_0]
+SEVERAL += [(synth.GGML_Q4_K, (1600, 1600, 1604), 5632, 256, SMALL), (synth.GGML_Q4_K, (1536, 1536, 1536), 11776, 700, 0)]
 
 
 @pytest.mark.parametrize("tid,rows,n_cols,n_tok,want", SEVERAL)

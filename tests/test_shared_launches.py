@@ -27,7 +27,7 @@ def test_q_k_and_v_share_a_launch(tid):
             ((4096, 1024, 1024), 4096, 128, FEW), ((4096, 1024, 1024), 4096, 256, SMALL), ((5120, 1024, 1024), 5120, 128, FEW),
             ((5120, 1024, 1024), 5120, 256, SMALL), ((8192, 1024, 1024), 8192, 256, SMALL), ((8192, 1024, 1024), 5120, 256, SMALL),
             ((6144, 1024, 1024), 6144, 200, SMALL), ((4096, 2048, 2048), 5376, 256, SMALL), ((8192, 8192, 8192), 8192, 77, SMALL),
-            ((6656, 6656, 6656), 6656, 128, SMALL)]:
+            ((6656, 6656, 6656), 6656, 128, SMALL), ((8192, 1024, 1024), 8192, 100, SMALL), ((5376, 5376, 5376), 5376, 100, SMALL)]:
         assert shared(tid, rows, n_cols, n_tok) == kernel, (rows, n_cols, n_tok)
     if tid in (synth.GGML_Q4_K, synth.GGML_Q5_K, synth.GGML_Q3_K):
         for rows, n_cols, n_tok in [((5120, 1024, 1024), 5120, 512), ((8192, 1024, 1024), 8192, 512), ((5120, 1024, 1024), 5120, 1024),
@@ -41,18 +41,21 @@ def test_divided_tensors_share_a_launch(tid):
     for rows, n_cols, n_tok in [((8192, 2048, 2048), 8192, 256), ((6144, 1536, 1536), 6144, 200), ((2900, 1601, 2000), 5632, 150)]:
         assert parts(tid, rows[0], n_cols, n_tok) == 1 and parts(tid, rows[1], n_cols, n_tok) > 1
         assert shared(tid, rows, n_cols, n_tok) == SMALL, (rows, n_cols, n_tok)
-    if tid == synth.GGML_Q4_K:  # three times 33 MB of sums, 59 + 34 MB of workspace
-        assert parts(tid, 2048, 14336, 1000) == 4 and shared(tid, (2048,) * 3, 14336, 1000) == 0 and shared(tid, (2048,) * 2, 14336, 1000) == LARGE
+    if tid == synth.GGML_Q4_K:  # the sums of three do not fit the workspace
+        assert parts(tid, 1536, 11776, 700) == 6 and shared(tid, (1536,) * 3, 11776, 700) == 0 and shared(tid, (1536,) * 2, 11776, 700) == LARGE
 
 
 @pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
 def test_a_workspace_takes_no_launch_apart(tid):
-    """K and V of up to 1535 rows, whose kernels are Q's without a workspace: dividing their K must not part them from Q"""
+    """K and V of up to 1535 rows, whose kernels are Q's without a workspace: dividing their K must not part them from Q (in the few-token
+    kernel: from a Q of as many rows as columns)"""
     for n_cols in range(1024, 16385, 1024):
         for kv in (128, 1024, 1535):
             for q in (n_cols * 3 // 4, n_cols, n_cols * 8 // 5):
                 for n_tok in range(65, 1025, 29):
                     rows = (q, kv, kv)
+                    if q < n_cols and n_tok <= 128:
+                        continue
                     if shared(tid, rows, n_cols, n_tok, 0) and all(route(tid, r, n_cols, n_tok) for r in rows):
                         assert shared(tid, rows, n_cols, n_tok), (rows, n_cols, n_tok)
 
@@ -69,10 +72,11 @@ def test_gate_and_up_take_the_tiles_that_suit_the_pair(tid):
 
 @pytest.mark.parametrize("tid", ALL, ids=lambda t: NAMES[t])
 def test_down_products_divide_k_and_what_may_share_a_launch_does_not(tid):
-    for n_rows, n_cols, n_tok in [(4096, 14336, 256), (2560, 6912, 256), (2048, 5632, 200), (3584, 9728, 200), (1536, 8960, 160)]:
+    for n_rows, n_cols, n_tok in [(4096, 14336, 256), (2560, 6912, 256), (2048, 5632, 200), (3584, 9728, 200), (1536, 8960, 160), (8192, 8192, 77),
+                                  (1024, 8192, 100)]:
         assert parts(tid, n_rows, n_cols, n_tok) > 1, (n_rows, n_cols, n_tok)
-    for n_rows, n_cols, n_tok in [(8192, 8192, 77), (5120, 5120, 256), (1024, 5120, 256), (2048, 5376, 256), (1024, 8192, 256),
-                                  (1535, 8192, 256), (2048, 4096, 256), (4096, 14336, 64), (4096, 14336, 1025)]:
+    for n_rows, n_cols, n_tok in [(1024, 5120, 128), (5376, 5376, 100), (5440, 5632, 77), (5120, 5120, 256), (1024, 5120, 256), (2048, 5376, 256),
+                                  (1024, 8192, 256), (1535, 8192, 256), (1536, 12288, 200), (2048, 4096, 256), (4096, 14336, 64), (4096, 14336, 1025)]:
         assert parts(tid, n_rows, n_cols, n_tok) == 1, (n_rows, n_cols, n_tok)
 
 
