@@ -379,9 +379,11 @@ static int column_range(uint32_t type, int n_cols) {
     return range;
 }
 
-/* shape-based choice: tuned Q4_K kernel, else the matrix-instruction kernel for long rows of the codebook formats,
- * else the integer-dot kernel (formats with small integer codes), else the streaming float kernel, else - rows
- * too long for those - the same kernels over column ranges, else (ragged shapes, unaligned pointers) the plain kernel */
+/* shape-based choice (launch_gemv_tuned): the matvec on blocks copied to LDS where it measured faster (gemv_dma.hip, eleven formats), else
+ * the tuned Q4_K kernel, else the matrix-instruction kernel on operand-layout loads, else the integer-dot kernel (small integer codes; of
+ * Q6_K, Q5_K and Q3_K only several matrices that do not end on whole row groups, and Q5_K at 2-byte addresses), else the
+ * streaming float kernel, else - rows too long for those - the same kernels over column ranges, else (ragged shapes, unaligned
+ * pointers) the plain kernel */
 hipError_t dispatch_gemv_job(uint32_t type, const GemvJob &job, const float *x, int n_cols, hipStream_t s) {
     if ((job.mode == kSiluMul ? job.n_rows[0] : job.total_rows()) == 0) return hipSuccess;
     bool w_aligned = true;

@@ -99,8 +99,8 @@ def test_shapes(oracle, tid, n_tok, n_rows, n_cols, dense_kernel):
     (513, 8500, 1024),
 ])
 def test_fused_tile_kernel_shapes(oracle, tid, n_tok, n_rows, n_cols):
-    """200 or more 256-token x 128-row tiles: Q4_K, Q5_K, Q6_K and Q8_0 are decoded inside the product (no workspace is
-    read: none is passed); weights rounded once to bf16, as the decode + dense route rounds them"""
+    """hundreds of tiles and no workspace: every format with a tile kernel is decoded inside the product; weights rounded once to bf16,
+    as the decode + dense route rounds them"""
     W = synth.make_weights(tid, n_rows, n_cols, seed=n_rows + tid)
     Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_tok + tid, tokens=n_tok))
     ldx, ldy = n_cols + 8, n_rows + 3
