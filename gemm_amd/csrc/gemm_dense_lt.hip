@@ -17,6 +17,7 @@
  */
 #include <hipblaslt/hipblaslt.h>
 
+#include <algorithm>
 #include <array>
 #include <map>
 #include <mutex>
@@ -34,13 +35,15 @@ struct Plan {
     hipblasLtMatrixLayout_t a = nullptr, b = nullptr, c = nullptr;
     hipblasLtMatmulAlgo_t algo;
     size_t ws_bytes = 0; /* workspace the algorithm was chosen for */
+    bool none = false;   /* the library has no algorithm: kept too, so that it is not asked for its list again */
 };
 
 std::mutex g_mu;
 hipblasLtHandle_t g_handle = nullptr;
-std::map<std::array<long long, 6>, Plan> g_plans; /* (fp32?, n_rows, n_cols, n_tok, ldx, ldy) -> plan; at most kMaxPlans */
+std::map<std::array<long long, 7>, Plan> g_plans; /* (fp32?, n_rows, n_cols, n_tok, ldx, ldy, MiB of workspace) -> plan; at most kMaxPlans */
 
 constexpr size_t kMaxPlans = 512;
+const char kNoAlgorithm[] = "the library offers no algorithm for this shape";
 
 void destroy_plan(Plan &p) {
     if (p.a) hipblasLtMatrixLayoutDestroy(p.a);
@@ -51,7 +54,7 @@ void destroy_plan(Plan &p) {
 }
 
 const char *make_plan(Plan &p, bool fp32, long long n_rows, long long n_cols, long long n_tok, long long ldx,
-                      long long ldy, size_t lib_ws_bytes) {
+                      long long ldy, size_t room) {
     const hipDataType in = fp32 ? HIP_R_32F : HIP_R_16BF;
     if (hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F) != HIPBLAS_STATUS_SUCCESS)
         return "hipblasLtMatmulDescCreate failed";
@@ -68,13 +71,14 @@ const char *make_plan(Plan &p, bool fp32, long long n_rows, long long n_cols, lo
     /* The library's kernels that split K over workgroups and reduce through the workspace write a padded
      * output (ldy > n_rows) as if it were dense (measured: K = 8192 and up with few output tiles, relative
      * error 1.4). Kernels without a workspace write Y themselves. */
-    if (ldy != n_rows) lib_ws_bytes = 0;
+    if (ldy != n_rows) room = 0;
+    const size_t lib_ws_bytes = std::min(kDenseLibWorkspace, room);
     hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &lib_ws_bytes, sizeof(lib_ws_bytes));
     /* The limit above is no promise: the heuristic's first answer may need more (35536 x 2560 at 664 tokens 53 MiB, offered 32 or
      * nothing; 94 of 744 random products of 256 to 160000 rows and 65 to 4096 tokens, up to 64 MiB), and the product then runs
-     * and writes past the end. So an answer counts only if what it needs fits: the first one, else the first of a longer list (the
-     * second answer nearly always; more than one answer takes the library 24 ms where one takes 0.07, once per plan). None: as if the
-     * library offered no kernel. */
+     * and writes past the end. So an answer counts only if what it needs fits: the first one, for which a workspace sized for a larger
+     * tensor usually has room, else the first of a longer list (the second answer nearly always; more than one answer takes the
+     * library 24 ms where one takes 0.07, once per plan). None: as if the library offered no kernel. */
     constexpr int kAnswers = 64;
     std::vector<hipblasLtMatmulHeuristicResult_t> res(kAnswers);
     int n = 0, take = -1;
@@ -83,12 +87,12 @@ const char *make_plan(Plan &p, bool fp32, long long n_rows, long long n_cols, lo
         n = 0;
         st = hipblasLtMatmulAlgoGetHeuristic(g_handle, p.desc, p.a, p.b, p.c, p.c, pref, want, res.data(), &n);
         for (int i = 0; st == HIPBLAS_STATUS_SUCCESS && take < 0 && i < n; i++)
-            if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= lib_ws_bytes) take = i;
+            if (res[i].state == HIPBLAS_STATUS_SUCCESS && res[i].workspaceSize <= room) take = i;
     }
     hipblasLtMatmulPreferenceDestroy(pref);
-    if (take < 0) return "the library offers no algorithm for this shape";
+    if (take < 0) return kNoAlgorithm;
     p.algo = res[take].algo;
-    p.ws_bytes = lib_ws_bytes;
+    p.ws_bytes = std::max(lib_ws_bytes, res[take].workspaceSize);
     return nullptr;
 }
 
@@ -109,7 +113,8 @@ const char *launch_gemm_dense(bool fp32_operands, const void *Wd, const void *X,
         g_handle = nullptr;
         return "hipblasLtCreate failed";
     }
-    const std::array<long long, 6> key = {fp32_operands ? 1 : 0, n_rows, n_cols, n_tok, ldx, ldy};
+    const size_t room = lib_ws_bytes >= 2 * kDenseLibWorkspace ? 2 * kDenseLibWorkspace : lib_ws_bytes < kDenseLibWorkspace ? 0 : kDenseLibWorkspace;
+    const std::array<long long, 7> key = {fp32_operands ? 1 : 0, n_rows, n_cols, n_tok, ldx, ldy, (long long)(room >> 20)};
     auto it = g_plans.find(key);
     if (it == g_plans.end()) {
         if (g_plans.size() >= kMaxPlans) { /* a caller with ever-changing token counts: start over */
@@ -117,13 +122,15 @@ const char *launch_gemm_dense(bool fp32_operands, const void *Wd, const void *X,
             g_plans.clear();
         }
         Plan p;
-        if (const char *err = make_plan(p, fp32_operands, n_rows, n_cols, n_tok, ldx, ldy, lib_ws_bytes)) {
+        if (const char *err = make_plan(p, fp32_operands, n_rows, n_cols, n_tok, ldx, ldy, room)) {
             destroy_plan(p);
-            return err;
+            if (err != kNoAlgorithm) return err;
+            p.none = true;
         }
         it = g_plans.emplace(key, p).first;
     }
     const Plan &p = it->second;
+    if (p.none) return kNoAlgorithm;
     const float alpha = 1.0f, beta = 0.0f;
     if (hipblasLtMatmul(g_handle, p.desc, &alpha, Wd, p.a, X, p.b, &beta, Y, p.c, Y, p.c, &p.algo, p.ws_bytes ? lib_ws : nullptr,
                         p.ws_bytes, stream) != HIPBLAS_STATUS_SUCCESS)

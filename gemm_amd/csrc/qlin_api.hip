@@ -802,7 +802,6 @@ int qlin_matvec_expert(float *dst, const void *W, uint32_t type, int n_cols, int
     return qlin_matvec(dst, slice, type, n_cols, x, rows_per_expert);
 }
 
-static constexpr size_t kDenseLibWorkspace = (size_t)32 << 20; /* handed to the library GEMM */
 static constexpr int kDenseMinTokens = 8;                     /* below this the vector-ALU kernel is faster than decode + GEMM */
 
 int qlin_gemm_tokenmajor(float *Y, const void *W, uint32_t type, int n_cols, const float *X, int n_rows,
@@ -1217,7 +1216,7 @@ int qlin_gemm_bf16_any_dev(uint32_t type, const void *W, const uint16_t *X, floa
     }
     void *lib_ws = (char *)workspace + dense_gemm_weight_bytes(n_rows, n_cols);
     const char *err = mode == 2 ? "switched off" : launch_gemm_dense_bf16(Wd, X, Y, n_rows, n_cols, n_tok, ldx, ldy, lib_ws,
-                                                                          kDenseLibWorkspace, (hipStream_t)stream);
+                                                                          workspace_bytes - dense_gemm_weight_bytes(n_rows, n_cols), (hipStream_t)stream);
     if (!err) return QLIN_OK;
     if (own_ok && mode != 2) { /* a shape the library has no kernel for */
         HIP_TRY(launch_gemm_dense_own(Wd, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
@@ -1338,7 +1337,8 @@ int qlin_gemm_f32_any_dev(uint32_t type, const void *W, const float *X, float *Y
         Wd = (const float *)workspace;
     }
     void *lib_ws = (char *)workspace + dense_gemm_weight_bytes_f32(n_rows, n_cols);
-    if (launch_gemm_dense(true, Wd, X, Y, n_rows, n_cols, n_tok, ldx, ldy, lib_ws, kDenseLibWorkspace, (hipStream_t)stream) != nullptr)
+    if (launch_gemm_dense(true, Wd, X, Y, n_rows, n_cols, n_tok, ldx, ldy, lib_ws, workspace_bytes - dense_gemm_weight_bytes_f32(n_rows, n_cols),
+                          (hipStream_t)stream) != nullptr)
         HIP_TRY(launch_gemm_f32(type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream)); /* no library kernel for this shape */
     return QLIN_OK;
 }

@@ -111,6 +111,7 @@ hipError_t launch_gemm_f32(uint32_t type, const void *W, const float *X, float *
 /* any format: decode to bf16 (dequant.hip), then the dense library GEMM (gemm_dense_lt.hip) */
 hipError_t launch_dequant_bf16(uint32_t type, const void *W, uint16_t *out, int n_rows, int n_cols, size_t row_bytes,
                                hipStream_t stream);
+constexpr size_t kDenseLibWorkspace = (size_t)32 << 20; /* behind the decoded weights, for the library; up to twice that is used where there is room */
 size_t dense_gemm_weight_bytes(int n_rows, int n_cols);
 size_t dense_gemm_weight_bytes_f32(int n_rows, int n_cols);
 const char *launch_gemm_dense(bool fp32_operands, const void *Wd, const void *X, float *Y, int n_rows, int n_cols,

@@ -249,7 +249,8 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * IQ2_XXS tensor go one by one through the matvec kernels (exact weights, ~1e-6; the workspace holds their
  * activations as fp32, and when ldx is so wide that (n_tok - 1) * ldx + n_cols floats do not fit it they take the
  * decode + dense route). workspace: device memory, 256-byte aligned, at least
- * qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols) bytes (2 bytes per weight + 32 MiB for the library);
+ * qlin_gemm_bf16_any_workspace_bytes(n_rows, n_cols) bytes (2 bytes per weight + 32 MiB for the library, which has faster kernels for
+ * some products of many tiles where 64 MiB are there);
  * calls that share a workspace must be ordered on one stream. Relative L2 of Y against exact weights
  * <= 2e-3.
  * qlin_set_dense_gemm_own(1), or QLIN_DENSE_GEMM=own in the environment when the library initialises,

@@ -1,7 +1,7 @@
 """Products through decode and the vendor library's dense GEMM stay inside the workspace that the caller gives, through the C ABI.
 The shapes are ones for which the library's first choice of kernel can need more than the 32 MiB that the documented size holds for
-it (36 to 62 MiB, by its version): a region behind the workspace, of the same allocation, keeps its contents, and the result is right
-in every part of the tensor (relative L2 <= 2e-5 against weights rounded once to bf16, the bar of the dense route; 1e-5 in fp32).
+it (36 to 62 MiB, by its version), given that size and more: a region behind the workspace, of the same allocation, keeps its
+contents, and the result is right in every part of the tensor (relative L2 <= 2e-5 against weights rounded once to bf16, the bar of the dense route; 1e-5 in fp32).
 Run once with the library that this process has and once in a process that has loaded torch, whose own copy of the library takes the
 place of the system's."""
 import os
@@ -21,9 +21,9 @@ from tests.test_gpu_gemm_any import ALL, references
 
 pytestmark = pytest.mark.gpu
 BEHIND = 96 << 20
-BF16_SHAPES = [(t, r, c, n, pad) for t, r, c, n in (
+BF16_SHAPES = [(t, r, c, n, pad, more) for t, r, c, n in (
     (synth.GGML_Q8_0, 35536, 2560, 664), (synth.GGML_BF16, 20336, 1536, 1754), (synth.GGML_Q6_K, 6863, 3840, 2629),
-    (synth.GGML_IQ2_XS, 70000, 768, 300)) for pad in (0, 64)]
+    (synth.GGML_IQ2_XS, 70000, 768, 300)) for pad, more in ((0, 0), (64, 0), (0, 31 << 20), (0, 33 << 20), (64, 40 << 20))]
 
 
 def tall(tid, n_rows, n_cols, seed):
@@ -51,11 +51,11 @@ def run(call, tid, W, X, n_rows, n_cols, n_tok, ldy, ws_bytes):
     return Y
 
 
-def check_bf16(oracle, tid, n_rows, n_cols, n_tok, pad):
+def check_bf16(oracle, tid, n_rows, n_cols, n_tok, pad, more):
     W = tall(tid, n_rows, n_cols, seed=n_tok)
     Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_rows, tokens=n_tok))
     Y = run(qlinear.load().qlin_gemm_bf16_any_dev, tid, W, Xb, n_rows, n_cols, n_tok, n_rows + pad,
-            qlinear.gemm_bf16_any_workspace_bytes(n_rows, n_cols))
+            qlinear.gemm_bf16_any_workspace_bytes(n_rows, n_cols) + more)
     rows = sample(n_rows)
     _, designed = references(oracle, tid, W[rows], Xb, n_cols)
     got = Y[:, rows]
@@ -74,7 +74,7 @@ def check_fp32(oracle):
     assert rel_l2(Y[:, rows], exact) <= 1e-5
 
 
-@pytest.mark.parametrize("shape", BF16_SHAPES, ids=lambda s: "%s-%dx%d-%d+%d" % ((ALL[s[0]],) + s[1:]))
+@pytest.mark.parametrize("shape", BF16_SHAPES, ids=lambda s: "%s-%dx%d-%d+%d-%d" % ((ALL[s[0]],) + s[1:]))
 def test_bf16_product(oracle, shape):
     check_bf16(oracle, *shape)
 
