@@ -191,3 +191,52 @@ def test_fp32_product_in_a_graph(oracle):
         qlinear.sync()
     assert hip.hipGraphExecDestroy(gexec) == 0 and hip.hipGraphDestroy(graph) == 0
     assert hip.hipStreamDestroy(stream) == 0
+
+
+def test_divided_products_in_a_graph(oracle):
+    """A tensor that divides K, and three in one call of which two do, put their sums into the caller's workspace: four kernel nodes (the
+    products and the joins) and nothing else, replayed bit-identically over a workspace that holds something else in between."""
+    hip, lib, n = C.CDLL("libamdhip64.so"), qlinear.load(), 3
+    n_cols, n_tok, rows = 5632, 150, (2900, 1601, 2000)
+    parts = [lib.qlin_probe_gemm_parts(Q4K, r, n_cols, n_tok, n_cols) for r in rows]
+    assert parts[0] == 1 and parts[1] > 1 and parts[2] > 1
+    Ws = [synth.make_weights(Q4K, r, n_cols, seed=70 + r) for r in rows]
+    Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=71, tokens=n_tok))
+    dWs, dX = [qlinear.DevBuf.from_numpy(W) for W in Ws], qlinear.DevBuf.from_numpy(Xb)
+    dYs = [qlinear.DevBuf(n_tok * r * 4) for r in rows + (2000,)]
+    ws = qlinear.DevBuf(max(qlinear.gemm_bf16_any_workspace_bytes(r, n_cols) for r in rows))
+    Wp, Yp, rp = (C.c_void_p * n)(*[d.ptr for d in dWs]), (C.c_void_p * n)(*[d.ptr for d in dYs[:n]]), (C.c_int * n)(*rows)
+
+    def enqueue(s):
+        assert lib.qlin_gemm_bf16_multi_dev(Q4K, n, Wp, dX.ptr, Yp, rp, n_cols, n_tok, n_cols, rp, ws.ptr, ws.nbytes, s) == 0, lib.qlin_last_error()
+        assert lib.qlin_gemm_bf16_any_dev(Q4K, dWs[2].ptr, dX.ptr, dYs[3].ptr, 2000, n_cols, n_tok, n_cols, 2000, ws.ptr, ws.nbytes, s) == 0
+
+    enqueue(None)  # eager run: the reference for the replays, itself checked against the oracle
+    qlinear.sync()
+    want = [d.to_numpy(np.float32, (n_tok, r)) for d, r in zip(dYs, rows + (2000,))]
+    Xf = synth.bf16_bits_to_f32(Xb).astype(np.float64)
+    for W, got in zip(Ws, want):
+        dec = synth.bf16_bits_to_f32(synth.to_bf16_bits(oracle.dequant_matrix(Q4K, W, n_cols)))
+        assert rel_l2(got, Xf @ dec.astype(np.float64).T) <= 2e-5
+    assert np.array_equal(want[2], want[3])
+    stream, graph, gexec, n_nodes = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_size_t(0)
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+    assert hip.hipStreamBeginCapture(stream, 0) == 0  # hipStreamCaptureModeGlobal
+    enqueue(stream)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, C.c_size_t(0)) == 0
+    assert hip.hipGraphGetNodes(graph, None, C.byref(n_nodes)) == 0 and n_nodes.value == 4
+    junk = np.full(ws.nbytes // 4, np.nan, np.float32)
+    for replay in range(3):
+        for d in [ws] + dYs:
+            assert lib.qlin_dev_upload(d.ptr, junk.ctypes.data, d.nbytes) == 0
+        assert hip.hipGraphLaunch(gexec, stream) == 0
+        assert hip.hipStreamSynchronize(stream) == 0
+        for d, w in zip(dYs, want):
+            assert np.array_equal(d.to_numpy(np.float32, w.shape), w), replay
+        enqueue(None)  # eager work between replays
+        qlinear.sync()
+    assert hip.hipGraphExecDestroy(gexec) == 0 and hip.hipGraphDestroy(graph) == 0
+    assert hip.hipStreamDestroy(stream) == 0
+    for b in dWs + dYs + [dX, ws]:
+        b.free()
