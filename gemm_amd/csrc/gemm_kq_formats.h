@@ -59,24 +59,29 @@ template <int N> QLIN_INL void wait_vmcnt() {
 /* where a lane finds vector J of its raw data in its row's image: byte offset, and what the upper lane half adds */
 struct VecAt { int off; int by_half; };
 
-/* scratch of the decode that all formats share */
-struct Temps {
+/* scratch of the decode that all formats share; of a code word, the words with an odd and an even number apart, so that the
+ * pieces of two words can take turns (tile_piece_at) */
+struct WordTemps {
     uint32_t cm, hb, lo, hi;
     float2v cp0, cp1;
     float f0, f1, f2, f3, w0, w1, w2, w3;
+};
+struct Temps {
+    WordTemps word[2];
+    uint32_t lo, hi;
     float s_a, s_b, m_a, m_b, dl_a, dl_b, nml_a, nml_b; /* of the two sub-blocks (scale groups) of the tile in work */
 };
 
 /* four bytes cm -> four weights f * dl + off as two bf16 pairs of `out` (HALF 0: x, y; 1: z, w), in the pieces 2..6 of
  * a code word's seven */
 template <int PH, int HALF, class C> QLIN_INL void bytes4_piece(C &c, float dl, float off, u32x4 &out) {
-    Temps &t = c.t;
-    if constexpr (PH == 2) { t.f0 = ubyte_f32<0>(t.cm); t.f1 = ubyte_f32<1>(t.cm); }
-    else if constexpr (PH == 3) { t.f2 = ubyte_f32<2>(t.cm); t.f3 = ubyte_f32<3>(t.cm); }
-    else if constexpr (PH == 4) { t.w0 = fmaf(t.f0, dl, off); t.w1 = fmaf(t.f1, dl, off); }
-    else if constexpr (PH == 5) { t.w2 = fmaf(t.f2, dl, off); t.w3 = fmaf(t.f3, dl, off); }
-    else if constexpr (HALF == 0) { out.x = pack_bf16(t.w0, t.w1); out.y = pack_bf16(t.w2, t.w3); }
-    else { out.z = pack_bf16(t.w0, t.w1); out.w = pack_bf16(t.w2, t.w3); }
+    WordTemps &w = c.t.word[HALF];
+    if constexpr (PH == 2) { w.f0 = ubyte_f32<0>(w.cm); w.f1 = ubyte_f32<1>(w.cm); }
+    else if constexpr (PH == 3) { w.f2 = ubyte_f32<2>(w.cm); w.f3 = ubyte_f32<3>(w.cm); }
+    else if constexpr (PH == 4) { w.w0 = fmaf(w.f0, dl, off); w.w1 = fmaf(w.f1, dl, off); }
+    else if constexpr (PH == 5) { w.w2 = fmaf(w.f2, dl, off); w.w3 = fmaf(w.f3, dl, off); }
+    else if constexpr (HALF == 0) { out.x = pack_bf16(w.w0, w.w1); out.y = pack_bf16(w.w2, w.w3); }
+    else { out.z = pack_bf16(w.w0, w.w1); out.w = pack_bf16(w.w2, w.w3); }
 }
 
 /* d, dmin and the 6-bit scales and mins of a Q4_K / Q5_K super-block from its 16-byte header (get_scale_min_k4,
@@ -108,7 +113,7 @@ template <int TC, int P, class C> QLIN_INL void k4_tile_scales(C &c) {
  * takes the header and code bytes 16 kg .. + 15 of every quarter. k-step s of a tile: low (s < 2) or high nibbles of
  * the lane's bytes 8 (s & 1) .. + 7. */
 struct FQ4K {
-    static constexpr int kBlockBytes = 144, kPieces = 9, kReq = 5, kLaneVec = 5, kPrepPieces = 4, kTilePieces = 44;
+    static constexpr int kBlockBytes = 144, kPieces = 9, kReq = 5, kLaneVec = 5, kPrepPieces = 4, kTilePieces = 44, kWordPieces = 5;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     static constexpr int frag_xor(int s) { return ((s & 1) << 4) | ((s >> 1) << 6); }
@@ -124,14 +129,15 @@ struct FQ4K {
         if constexpr (P < 4) k4_tile_scales<TC, P>(c);
         else {
             constexpr int dw = (P - 4) / 5, ph = (P - 4) % 5; /* code word 0..3: low nibbles of the lane's dwords, 4..7: high */
+            WordTemps &w = t.word[dw & 1];
             const uint32_t word = raw[1 + TC][dw & 3];
             const float dl = dw < 4 ? t.dl_a : t.dl_b, nml = dw < 4 ? t.nml_a : t.nml_b;
-            if constexpr (ph == 0) t.cm = (dw < 4 ? word : word >> 4) & 0x0F0F0F0Fu;
-            else if constexpr (ph == 1) { t.cp0 = fp8_pair_lo(t.cm); t.cp1 = fp8_pair_hi(t.cm); }
-            else if constexpr (ph == 2) { t.w0 = fmaf(t.cp0.x, dl, nml); t.w1 = fmaf(t.cp0.y, dl, nml); }
-            else if constexpr (ph == 3) { t.w2 = fmaf(t.cp1.x, dl, nml); t.w3 = fmaf(t.cp1.y, dl, nml); }
-            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].y = pack_bf16(t.w2, t.w3); }
-            else { c.wa[WB][dw >> 1].z = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].w = pack_bf16(t.w2, t.w3); }
+            if constexpr (ph == 0) w.cm = (dw < 4 ? word : word >> 4) & 0x0F0F0F0Fu;
+            else if constexpr (ph == 1) { w.cp0 = fp8_pair_lo(w.cm); w.cp1 = fp8_pair_hi(w.cm); }
+            else if constexpr (ph == 2) { w.w0 = fmaf(w.cp0.x, dl, nml); w.w1 = fmaf(w.cp0.y, dl, nml); }
+            else if constexpr (ph == 3) { w.w2 = fmaf(w.cp1.x, dl, nml); w.w3 = fmaf(w.cp1.y, dl, nml); }
+            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].y = pack_bf16(w.w2, w.w3); }
+            else { c.wa[WB][dw >> 1].z = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].w = pack_bf16(w.w2, w.w3); }
         }
     }
 };
@@ -140,7 +146,7 @@ struct FQ4K {
  * bytes as Q4_K. A lane takes the header, fifth-bit bytes 16 kg .. + 15 and its code bytes of every quarter; the 5-bit
  * code goes through the byte-to-float conversion (the fp8 reading is linear up to 15 only). */
 struct FQ5K {
-    static constexpr int kBlockBytes = 176, kPieces = 11, kReq = 6, kLaneVec = 6, kPrepPieces = 4, kTilePieces = 60;
+    static constexpr int kBlockBytes = 176, kPieces = 11, kReq = 6, kLaneVec = 6, kPrepPieces = 4, kTilePieces = 60, kWordPieces = 7;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     static constexpr int frag_xor(int s) { return ((s & 1) << 4) | ((s >> 1) << 6); }
@@ -156,9 +162,10 @@ struct FQ5K {
         if constexpr (P < 4) k4_tile_scales<TC, P>(c);
         else {
             constexpr int dw = (P - 4) / 7, ph = (P - 4) % 7, hi = dw >> 2;
+            WordTemps &w = t.word[dw & 1];
             const float dl = hi ? t.dl_b : t.dl_a, nml = hi ? t.nml_b : t.nml_a;
-            if constexpr (ph == 0) t.cm = (hi ? raw[2 + TC][dw & 3] >> 4 : raw[2 + TC][dw & 3]) & 0x0F0F0F0Fu;
-            else if constexpr (ph == 1) { t.hb = (raw[1][dw & 3] >> (2 * TC + hi)) & 0x01010101u; t.cm |= t.hb << 4; }
+            if constexpr (ph == 0) w.cm = (hi ? raw[2 + TC][dw & 3] >> 4 : raw[2 + TC][dw & 3]) & 0x0F0F0F0Fu;
+            else if constexpr (ph == 1) { w.hb = (raw[1][dw & 3] >> (2 * TC + hi)) & 0x01010101u; w.cm |= w.hb << 4; }
             else bytes4_piece<ph, dw & 1>(c, dl, nml, c.wa[WB][dw >> 1]);
         }
     }
@@ -171,7 +178,7 @@ struct FQ5K {
  * they come, bytes 194..209 (d in its last two) as the 14th, and one of padding (15: an odd stride). */
 struct Q6Scales { float d; };
 struct FQ6K {
-    static constexpr int kBlockBytes = 210, kPieces = 15, kReq = 8, kLaneVec = 8, kPrepPieces = 1, kTilePieces = 60;
+    static constexpr int kBlockBytes = 210, kPieces = 15, kReq = 8, kLaneVec = 8, kPrepPieces = 1, kTilePieces = 60, kWordPieces = 7;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     static constexpr int frag_xor(int s) { return ((s & 1) << 4) | ((s >> 1) << 6); }
@@ -197,9 +204,10 @@ struct FQ6K {
             else { t.dl_b = c.sc.d * t.s_b; t.nml_b = -32.0f * t.dl_b; }
         } else {
             constexpr int dw = (P - 4) / 7, ph = (P - 4) % 7, jj = dw >> 2;
+            WordTemps &w = t.word[dw & 1];
             const float dl = jj ? t.dl_b : t.dl_a, off = jj ? t.nml_b : t.nml_a;
-            if constexpr (ph == 0) t.cm = (p ? raw[2 * half + jj][dw & 3] >> 4 : raw[2 * half + jj][dw & 3]) & 0x0F0F0F0Fu;
-            else if constexpr (ph == 1) { t.hb = (raw[4 + half][dw & 3] >> (4 * p + 2 * jj)) & 0x03030303u; t.cm |= t.hb << 4; }
+            if constexpr (ph == 0) w.cm = (p ? raw[2 * half + jj][dw & 3] >> 4 : raw[2 * half + jj][dw & 3]) & 0x0F0F0F0Fu;
+            else if constexpr (ph == 1) { w.hb = (raw[4 + half][dw & 3] >> (4 * p + 2 * jj)) & 0x03030303u; w.cm |= w.hb << 4; }
             else bytes4_piece<ph, dw & 1>(c, dl, off, c.wa[WB][dw >> 1]);
         }
     }
@@ -212,7 +220,7 @@ struct FQ6K {
  * four suffice, the k order inside a tile differs from the K-quants': lane half kg takes ALL codes of block 2 c + kg of
  * tile c, k-step s its codes 8 s .. 8 s + 7, and the activation fragment of that lane half is chunk 4 kg + s. */
 struct FQ8_0 {
-    static constexpr int kBlockBytes = 272, kPieces = 16, kReq = 8, kLaneVec = 8, kPrepPieces = 0, kTilePieces = 49;
+    static constexpr int kBlockBytes = 272, kPieces = 16, kReq = 8, kLaneVec = 8, kPrepPieces = 0, kTilePieces = 49, kWordPieces = 6;
     static constexpr int kExtraVec = 1, kExtraLoads = 4, kKgChunk = 4;
     /* a row's image is 256 bytes, a whole turn of the LDS banks: piece p of row r sits at position p ^ (r % 16) of the
      * row, so that 16 rows reading the same piece hit 16 different bank groups */
@@ -235,7 +243,8 @@ struct FQ8_0 {
         else {
             /* the int8 code with its sign bit flipped is code + 128 as an unsigned byte */
             constexpr int dw = (P - 1) / 6, ph = (P - 1) % 6;
-            if constexpr (ph == 0) t.cm = raw[2 * TC + (dw >> 2)][dw & 3] ^ 0x80808080u;
+            WordTemps &w = t.word[dw & 1];
+            if constexpr (ph == 0) w.cm = raw[2 * TC + (dw >> 2)][dw & 3] ^ 0x80808080u;
             else bytes4_piece<ph + 1, dw & 1>(c, t.dl_a, t.nml_a, c.wa[WB][dw >> 1]);
         }
     }
@@ -250,7 +259,7 @@ struct FQ8_0 {
  * bit 3 of the index: about 5 vector instructions per weight, more than one wave per SIMD can issue beside the matrix
  * instructions, but far fewer than the decode to bf16 in memory costs. */
 struct FIQ4NL {
-    static constexpr int kBlockBytes = 144, kPieces = 9, kReq = 5, kLaneVec = 9, kPrepPieces = 0, kTilePieces = 82;
+    static constexpr int kBlockBytes = 144, kPieces = 9, kReq = 5, kLaneVec = 9, kPrepPieces = 0, kTilePieces = 82, kWordPieces = 10;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     struct Scales {};
@@ -273,23 +282,24 @@ struct FIQ4NL {
             else { t.dl_b = d; t.nml_b = -128.0f * d; }
         } else {
             constexpr int dw = (P - 2) / 10, ph = (P - 2) % 10, b = 2 * TC + (dw >> 2), at = 18 * b + 2 + 4 * (dw & 3);
+            WordTemps &w = t.word[dw & 1];
             const float dl = (dw >> 2) ? t.dl_b : t.dl_a, off = (dw >> 2) ? t.nml_b : t.nml_a;
             if constexpr (ph == 0) {
                 uint32_t src;
                 if constexpr ((at & 3) == 0) src = image_dword<(at >> 2)>(raw);
                 else src = __builtin_amdgcn_alignbyte(image_dword<(at >> 2) + 1>(raw), image_dword<(at >> 2)>(raw), at & 3);
-                t.hb = src >> (4u * (uint32_t)c.kg); /* the lane half's nibble of every byte */
+                w.hb = src >> (4u * (uint32_t)c.kg); /* the lane half's nibble of every byte */
             } else if constexpr (ph == 1) {
-                t.cm = t.hb & 0x0F0F0F0Fu;
-                t.hb = t.cm & 0x07070707u;
+                w.cm = w.hb & 0x0F0F0F0Fu;
+                w.hb = w.cm & 0x07070707u;
             } else if constexpr (ph == 2) {
-                t.lo = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, t.hb); /* table entries 0..7, + 128 */
-                t.hi = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, t.hb); /* entries 8..15 */
+                w.lo = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, w.hb); /* table entries 0..7, + 128 */
+                w.hi = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, w.hb); /* entries 8..15 */
             } else if constexpr (ph == 3) {
-                t.hb = (t.cm >> 3) & 0x01010101u;
+                w.hb = (w.cm >> 3) & 0x01010101u;
             } else if constexpr (ph == 4) {
-                t.hb *= 255u; /* 0xFF in the bytes whose index is 8 or more */
-                t.cm = (t.hb & t.hi) | (~t.hb & t.lo);
+                w.hb *= 255u; /* 0xFF in the bytes whose index is 8 or more */
+                w.cm = (w.hb & w.hi) | (~w.hb & w.lo);
             } else {
                 bytes4_piece<ph - 3, dw & 1>(c, dl, off, c.wa[WB][dw >> 1]);
             }
@@ -301,7 +311,7 @@ struct FIQ4NL {
  * (common/ggml_dequant.h:2850-2862). The layout and the lane roles of IQ4_NL with the arithmetic of Q4_K: the nibbles
  * go through the fp8 reading. */
 struct FQ4_0 {
-    static constexpr int kBlockBytes = 144, kPieces = 9, kReq = 5, kLaneVec = 9, kPrepPieces = 0, kTilePieces = 50;
+    static constexpr int kBlockBytes = 144, kPieces = 9, kReq = 5, kLaneVec = 9, kPrepPieces = 0, kTilePieces = 50, kWordPieces = 6;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     struct Scales {};
@@ -321,18 +331,19 @@ struct FQ4_0 {
             else { t.dl_b = d * c.unit; t.nml_b = -8.0f * d; }
         } else {
             constexpr int dw = (P - 2) / 6, ph = (P - 2) % 6, b = 2 * TC + (dw >> 2), at = 18 * b + 2 + 4 * (dw & 3);
+            WordTemps &w = t.word[dw & 1];
             const float dl = (dw >> 2) ? t.dl_b : t.dl_a, off = (dw >> 2) ? t.nml_b : t.nml_a;
             if constexpr (ph == 0) {
                 uint32_t src;
                 if constexpr ((at & 3) == 0) src = FIQ4NL::image_dword<(at >> 2)>(raw);
                 else src = __builtin_amdgcn_alignbyte(FIQ4NL::image_dword<(at >> 2) + 1>(raw), FIQ4NL::image_dword<(at >> 2)>(raw), at & 3);
-                t.hb = src >> (4u * (uint32_t)c.kg);
-            } else if constexpr (ph == 1) t.cm = t.hb & 0x0F0F0F0Fu;
-            else if constexpr (ph == 2) { t.cp0 = fp8_pair_lo(t.cm); t.cp1 = fp8_pair_hi(t.cm); }
-            else if constexpr (ph == 3) { t.w0 = fmaf(t.cp0.x, dl, off); t.w1 = fmaf(t.cp0.y, dl, off); }
-            else if constexpr (ph == 4) { t.w2 = fmaf(t.cp1.x, dl, off); t.w3 = fmaf(t.cp1.y, dl, off); }
-            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].y = pack_bf16(t.w2, t.w3); }
-            else { c.wa[WB][dw >> 1].z = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].w = pack_bf16(t.w2, t.w3); }
+                w.hb = src >> (4u * (uint32_t)c.kg);
+            } else if constexpr (ph == 1) w.cm = w.hb & 0x0F0F0F0Fu;
+            else if constexpr (ph == 2) { w.cp0 = fp8_pair_lo(w.cm); w.cp1 = fp8_pair_hi(w.cm); }
+            else if constexpr (ph == 3) { w.w0 = fmaf(w.cp0.x, dl, off); w.w1 = fmaf(w.cp0.y, dl, off); }
+            else if constexpr (ph == 4) { w.w2 = fmaf(w.cp1.x, dl, off); w.w3 = fmaf(w.cp1.y, dl, off); }
+            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].y = pack_bf16(w.w2, w.w3); }
+            else { c.wa[WB][dw >> 1].z = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].w = pack_bf16(w.w2, w.w3); }
         }
     }
 };
@@ -343,7 +354,7 @@ struct FQ4_0 {
  * super-block); the code dwords are aligned. */
 struct XsScales { float d; };
 struct FIQ4XS {
-    static constexpr int kBlockBytes = 136, kPieces = 9, kReq = 5, kLaneVec = 9, kPrepPieces = 1, kTilePieces = 88;
+    static constexpr int kBlockBytes = 136, kPieces = 9, kReq = 5, kLaneVec = 9, kPrepPieces = 1, kTilePieces = 88, kWordPieces = 10;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     typedef XsScales Scales;
@@ -368,20 +379,21 @@ struct FIQ4XS {
             else nml = -128.0f * dl;
         } else {
             constexpr int dw = (P - 8) / 10, ph = (P - 8) % 10, g = 2 * TC + (dw >> 2);
+            WordTemps &w = t.word[dw & 1];
             const float dl = (dw >> 2) ? t.dl_b : t.dl_a, off = (dw >> 2) ? t.nml_b : t.nml_a;
             if constexpr (ph == 0) {
-                t.hb = FIQ4NL::image_dword<2 + 4 * g + (dw & 3)>(raw) >> (4u * (uint32_t)c.kg);
+                w.hb = FIQ4NL::image_dword<2 + 4 * g + (dw & 3)>(raw) >> (4u * (uint32_t)c.kg);
             } else if constexpr (ph == 1) {
-                t.cm = t.hb & 0x0F0F0F0Fu;
-                t.hb = t.cm & 0x07070707u;
+                w.cm = w.hb & 0x0F0F0F0Fu;
+                w.hb = w.cm & 0x07070707u;
             } else if constexpr (ph == 2) {
-                t.lo = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, t.hb);
-                t.hi = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, t.hb);
+                w.lo = __builtin_amdgcn_perm(0x766A5D4Fu, 0x3F2D1801u, w.hb);
+                w.hi = __builtin_amdgcn_perm(0xF1D9C5B5u, 0xA6998D81u, w.hb);
             } else if constexpr (ph == 3) {
-                t.hb = (t.cm >> 3) & 0x01010101u;
+                w.hb = (w.cm >> 3) & 0x01010101u;
             } else if constexpr (ph == 4) {
-                t.hb *= 255u;
-                t.cm = (t.hb & t.hi) | (~t.hb & t.lo);
+                w.hb *= 255u;
+                w.cm = (w.hb & w.hi) | (~w.hb & w.lo);
             } else {
                 bytes4_piece<ph - 3, dw & 1>(c, dl, off, c.wa[WB][dw >> 1]);
             }
@@ -402,7 +414,7 @@ template <int TC, int DW> struct K23 { static constexpr int half = TC >> 1, j = 
  * bytes 80..95 would leave the row, and the buffer at its last row). */
 struct Q2Scales { float d, dmin; };
 struct FQ2K {
-    static constexpr int kBlockBytes = 84, kPieces = 6, kReq = 3, kLaneVec = 4, kPrepPieces = 1, kTilePieces = 44;
+    static constexpr int kBlockBytes = 84, kPieces = 6, kReq = 3, kLaneVec = 4, kPrepPieces = 1, kTilePieces = 44, kWordPieces = 5;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     typedef Q2Scales Scales;
@@ -427,14 +439,15 @@ struct FQ2K {
             else { t.nml_a = -(c.sc.dmin * t.m_a); t.nml_b = -(c.sc.dmin * t.m_b); }
         } else {
             constexpr int dw = (P - 4) / 5, ph = (P - 4) % 5;
+            WordTemps &w = t.word[dw & 1];
             typedef K23<TC, dw> G;
             const float dl = dw < 4 ? t.dl_a : t.dl_b, nml = dw < 4 ? t.nml_a : t.nml_b;
-            if constexpr (ph == 0) t.cm = (raw[1 + G::half][dw & 3] >> (2 * G::j)) & 0x03030303u;
-            else if constexpr (ph == 1) { t.cp0 = fp8_pair_lo(t.cm); t.cp1 = fp8_pair_hi(t.cm); }
-            else if constexpr (ph == 2) { t.w0 = fmaf(t.cp0.x, dl, nml); t.w1 = fmaf(t.cp0.y, dl, nml); }
-            else if constexpr (ph == 3) { t.w2 = fmaf(t.cp1.x, dl, nml); t.w3 = fmaf(t.cp1.y, dl, nml); }
-            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].y = pack_bf16(t.w2, t.w3); }
-            else { c.wa[WB][dw >> 1].z = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].w = pack_bf16(t.w2, t.w3); }
+            if constexpr (ph == 0) w.cm = (raw[1 + G::half][dw & 3] >> (2 * G::j)) & 0x03030303u;
+            else if constexpr (ph == 1) { w.cp0 = fp8_pair_lo(w.cm); w.cp1 = fp8_pair_hi(w.cm); }
+            else if constexpr (ph == 2) { w.w0 = fmaf(w.cp0.x, dl, nml); w.w1 = fmaf(w.cp0.y, dl, nml); }
+            else if constexpr (ph == 3) { w.w2 = fmaf(w.cp1.x, dl, nml); w.w3 = fmaf(w.cp1.y, dl, nml); }
+            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].y = pack_bf16(w.w2, w.w3); }
+            else { c.wa[WB][dw >> 1].z = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].w = pack_bf16(w.w2, w.w3); }
         }
     }
 };
@@ -445,7 +458,7 @@ struct FQ2K {
  * packed scales start two bytes into that piece; once per super-block they are cut out and spread to sixteen bytes. */
 struct Q3Scales { float d, dm4; uint32_t a0, a1, hi, sc[4]; }; /* d with the fp8 reading's factor, dm4 = -4 d without */
 struct FQ3K {
-    static constexpr int kBlockBytes = 110, kPieces = 7, kReq = 4, kLaneVec = 4, kPrepPieces = 4, kTilePieces = 52;
+    static constexpr int kBlockBytes = 110, kPieces = 7, kReq = 4, kLaneVec = 4, kPrepPieces = 4, kTilePieces = 52, kWordPieces = 6;
     static constexpr int kExtraVec = 0, kExtraLoads = 0, kKgChunk = 2;
     static constexpr bool kSwizzle = false;
     typedef Q3Scales Scales;
@@ -482,18 +495,29 @@ struct FQ3K {
             else { t.nml_a = c.sc.dm4 * t.s_a; t.nml_b = c.sc.dm4 * t.s_b; }
         } else {
             constexpr int dw = (P - 4) / 6, ph = (P - 4) % 6;
+            WordTemps &w = t.word[dw & 1];
             typedef K23<TC, dw> G;
             const float dl = dw < 4 ? t.dl_a : t.dl_b, nml = dw < 4 ? t.nml_a : t.nml_b;
-            if constexpr (ph == 0) t.cm = (raw[1 + G::half][dw & 3] >> (2 * G::j)) & 0x03030303u;
-            else if constexpr (ph == 1) { t.hb = (raw[0][dw & 3] >> (4 * G::half + G::j)) & 0x01010101u; t.cm |= t.hb << 2; }
-            else if constexpr (ph == 2) { t.cp0 = fp8_pair_lo(t.cm); t.cp1 = fp8_pair_hi(t.cm); }
-            else if constexpr (ph == 3) { t.w0 = fmaf(t.cp0.x, dl, nml); t.w1 = fmaf(t.cp0.y, dl, nml); }
-            else if constexpr (ph == 4) { t.w2 = fmaf(t.cp1.x, dl, nml); t.w3 = fmaf(t.cp1.y, dl, nml); }
-            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].y = pack_bf16(t.w2, t.w3); }
-            else { c.wa[WB][dw >> 1].z = pack_bf16(t.w0, t.w1); c.wa[WB][dw >> 1].w = pack_bf16(t.w2, t.w3); }
+            if constexpr (ph == 0) w.cm = (raw[1 + G::half][dw & 3] >> (2 * G::j)) & 0x03030303u;
+            else if constexpr (ph == 1) { w.hb = (raw[0][dw & 3] >> (4 * G::half + G::j)) & 0x01010101u; w.cm |= w.hb << 2; }
+            else if constexpr (ph == 2) { w.cp0 = fp8_pair_lo(w.cm); w.cp1 = fp8_pair_hi(w.cm); }
+            else if constexpr (ph == 3) { w.w0 = fmaf(w.cp0.x, dl, nml); w.w1 = fmaf(w.cp0.y, dl, nml); }
+            else if constexpr (ph == 4) { w.w2 = fmaf(w.cp1.x, dl, nml); w.w3 = fmaf(w.cp1.y, dl, nml); }
+            else if constexpr ((dw & 1) == 0) { c.wa[WB][dw >> 1].x = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].y = pack_bf16(w.w2, w.w3); }
+            else { c.wa[WB][dw >> 1].z = pack_bf16(w.w0, w.w1); c.wa[WB][dw >> 1].w = pack_bf16(w.w2, w.w3); }
         }
     }
 };
+
+/* The number of the piece that a tile takes p-th: scales first, then the pieces of the eight code words, those of words 2 i and
+ * 2 i + 1 in turns. The pieces of one word depend on each other, and a wave that is alone on its SIMD issues a vector instruction
+ * that needs the last one's result only every eight cycles. */
+template <class F> constexpr int tile_piece_at(int p) {
+    constexpr int n0 = F::kTilePieces - 8 * F::kWordPieces;
+    if (p < n0) return p;
+    const int pair = (p - n0) / (2 * F::kWordPieces), r = (p - n0) % (2 * F::kWordPieces);
+    return n0 + (2 * pair + (r & 1)) * F::kWordPieces + (r >> 1);
+}
 
 /* Does a wave that takes half WK of a tile's k-steps (2 WK and 2 WK + 1) run tile piece q of format F? */
 template <class F, int WK> constexpr bool owns_piece(int q) {
@@ -505,7 +529,7 @@ template <class F, int WK> constexpr bool owns_piece(int q) {
 template <class F, int WK, int NPREP> struct Owned {
     static constexpr int count() {
         int n = NPREP;
-        for (int q = 0; q < F::kTilePieces; q++) n += owns_piece<F, WK>(q) ? 1 : 0;
+        for (int q = 0; q < F::kTilePieces; q++) n += owns_piece<F, WK>(tile_piece_at<F>(q)) ? 1 : 0;
         return n;
     }
     /* the i-th of them: below NPREP a prep piece, else NPREP + the tile piece's number */
@@ -513,8 +537,8 @@ template <class F, int WK, int NPREP> struct Owned {
         if (i < NPREP) return i;
         int n = NPREP;
         for (int q = 0; q < F::kTilePieces; q++)
-            if (owns_piece<F, WK>(q)) {
-                if (n == i) return NPREP + q;
+            if (owns_piece<F, WK>(tile_piece_at<F>(q))) {
+                if (n == i) return NPREP + tile_piece_at<F>(q);
                 n++;
             }
         return -1;

@@ -1,6 +1,6 @@
 /*
  * gemm_kq_wave4.hip - the fused block-format x bf16 prefill GEMM (Q2_K ... Q6_K, Q8_0, IQ4_NL, IQ4_XS, Q4_0: the formats of
- * gemm_kq_formats.h) in 256-token x 128-row tiles: four waves per workgroup, one per SIMD.
+ * gemm_kq_formats.h) in tiles of 128 rows x 256 tokens, or 192, 160, 128, 96: four waves per workgroup, one per SIMD.
  *
  *   Y[t*ldy + r] = sum_k X[t*ldx + k] * decode(W)[r][k]      X bf16, Y fp32, fp32 accumulate
  *
@@ -20,9 +20,9 @@
  *                                          would need)
  *     buffer_load_dwordx4 ... lds          the same 64 B per clock, no register or LDS-store cost
  * So nothing is stored to LDS by a wave:
- *   - activations go from global memory to LDS by the load-to-LDS path, 256 tokens x 64 k per tile, whole 128-byte
+ *   - activations go from global memory to LDS by the load-to-LDS path, 32 NB tokens x 64 k per tile, whole 128-byte
  *     row segments per 8 lanes, four stages deep;
- *   - decoded weights never touch LDS: wave w owns rows 32 w .. 32 w + 31 of the workgroup's 128 and all 256 tokens,
+ *   - decoded weights never touch LDS: wave w owns rows 32 w .. 32 w + 31 of the workgroup's 128 and all its tokens,
  *     its lane (row i, half kg) takes 16 of the 32 code bytes of a quarter super-block of its row and decodes them
  *     straight into the matrix instruction's first-operand layout (8 consecutive k of one row per lane): no decode
  *     is done twice in the workgroup, and there is nothing to exchange. The raw blocks of a wave's rows come the same
@@ -40,13 +40,25 @@
  * the low (s < 2) or high nibbles of code bytes 16 kg + 8 (s & 1) .. + 7, i.e. tile k 32 (s >> 1) + 16 kg + 8 (s & 1) ..;
  * the activation fragment of that lane half is chunk 4 (s >> 1) + 2 kg + (s & 1) of the token's 128-byte row segment.
  *
- * LDS: four stages of [256 tokens][64 k] bf16 = 32 KB; 16-byte chunk c of token row r sits at chunk position
+ * LDS: four stages of [32 NB tokens][64 k] bf16 = 4 NB KB; 16-byte chunk c of token row r sits at chunk position
  * c ^ f(r), f = bits 1 and 2 of (r >> 1) & 7 swapped, so that the 16 rows of a fragment fetch hit 16 different
- * 16-byte bank groups. One tile = 32 slots of [matrix instruction, fragment fetch for the next k-step, side work],
+ * 16-byte bank groups. One tile = 4 NB slots of [matrix instruction, fragment fetch for the next k-step, side work],
  * nothing moves between slots; side work = the load-to-LDS requests of the tile three ahead and of the raw blocks
- * two super-blocks ahead, and the decode of the next tile in 44 pieces of at most two vector instructions. Before the last
+ * two super-blocks ahead, and the decode of the next tile in 44 to 88 pieces of at most two vector instructions. Before the last
  * k-step: wait for this wave's requests of the next tile, barrier (the next tile is complete; nobody reads the
  * stage that is requested next, its last fragments were fetched a k-step earlier).
+ *
+ * Fewer token blocks: a tile's decode costs the same whatever its tokens, about as much vector time as six blocks' matrix
+ * instructions (Q4_K, one tile of 64 k on a chip of 224 workgroups: 0.41 us + 0.10 per block), so that eight blocks cost least per
+ * token, and fewer win where eight would be padding or leave a second round of the chip nearly empty. Against the better one of
+ * 256 x 128 and 128 x 64 tiles, us (choose_token_blocks picks): Q4_K x 4096, 77 tokens 28672 rows 37.4 -> 31.8 (three), 128 tokens 41.3 -> 38.3
+ * (four), 180 tokens 55 -> 48.6 (six), 300 tokens 12288 rows 51 -> 37.9 (five), 512 tokens 6144 rows 36.6 -> 32.9 (four). Q6_K 48.6 ->
+ * 42.8, 53.5 -> 48.1, 65 -> 60.4, 57 -> 46.6, 46.6 -> 41.7. 128 x 128 tiles on eight waves, four row groups x two halves of K, were built and
+ * are slower than four blocks here: 36.7 for 6144 rows at 512 tokens, a third of the waves' time at the barriers.
+ *
+ * Every wave keeps two sums per result, of k-steps 0 and 1 of the tiles and of 2 and 3, and adds them at the end: the 128 x 64 kernel's
+ * two halves of K. So all tile shapes give the same bits, and which one a launch takes is free - the one that suits its tensors together.
+ * (Where K is divided over workgroups the shape is a tensor's own choice, and one sum is kept: the second costs a launch 1 us.)
  */
 #include <climits>
 #include <utility>
@@ -63,27 +75,21 @@ using namespace kq;
 
 namespace {
 
-constexpr int kBM = 256, kBN = 128;
-constexpr int kXStage = kBM * 128; /* bytes of one stage */
+constexpr int kBN = 128, kLargeBlocks = 8;
 
-/* the four stages are separate objects: a fetch from one stage then never has to wait for a request into another */
-__shared__ __attribute__((aligned(1024))) uint8_t w4_stage0[kXStage];
-__shared__ __attribute__((aligned(1024))) uint8_t w4_stage1[kXStage];
-__shared__ __attribute__((aligned(1024))) uint8_t w4_stage2[kXStage];
-__shared__ __attribute__((aligned(1024))) uint8_t w4_stage3[kXStage];
-
-
-template <int ST> QLIN_INL uint8_t *stage_ptr() {
-    if constexpr (ST == 0) return w4_stage0;
-    else if constexpr (ST == 1) return w4_stage1;
-    else if constexpr (ST == 2) return w4_stage2;
-    else return w4_stage3;
+/* The four stages, 32 NB tokens x 64 k each, are separate objects: a fetch from one stage then never has to wait for a request into
+ * another */
+template <int NB, int ST> QLIN_INL uint8_t *stage_ptr() {
+    __shared__ __attribute__((aligned(1024))) uint8_t w4_stage[NB * 4096];
+    return w4_stage;
 }
 
 /* everything a slot touches; every member ends up in registers (all indices are constants after inlining) */
-template <class F> struct Ctx {
-    floatx16 acc[8];         /* [token block]: 32 rows x 32 tokens each */
-    bf16x8 xf[2][8];         /* activation fragments of the k-step in use and of the next: [k-step & 1][token block] */
+template <class Fmt, int NBLOCKS, int SUMS> struct Ctx {
+    using F = Fmt;
+    static constexpr int NB = NBLOCKS, S = 4 * NB, kSums = SUMS; /* token blocks; slots of a tile */
+    floatx16 acc[SUMS][NB];  /* [SUMS 2: k-steps 0 and 1 of the tiles, 2 and 3][token block]: 32 rows x 32 tokens each */
+    bf16x8 xf[2][NB];         /* activation fragments of the k-step in use and of the next: [k-step & 1][token block] */
     u32x4 wa[2][4];          /* decoded weights of the tile in use and of the next: [tile & 1][k-step] */
     u32x4 cur[F::kLaneVec + F::kExtraVec], nxt[F::kLaneVec + F::kExtraVec]; /* raw data of the super-block of the tile being
                                 decoded, and of the next: kLaneVec vectors out of the LDS image, kExtraVec straight from memory */
@@ -91,7 +97,7 @@ template <class F> struct Ctx {
     Temps t;
     uint32_t xrd;            /* byte offset of this lane's fragment fetches in a stage: k-step 0, token block 0 */
     __amdgpu_buffer_rsrc_t w_rsrc, x_rsrc;
-    uint32_t w_off[F::kReq], w_rd, w_swz, w_own, x_off[8]; /* w_swz: see kSwizzle; w_own: byte offset of the lane's own
+    uint32_t w_off[F::kReq], w_rd, w_swz, w_own, x_off[NB]; /* w_swz: see kSwizzle; w_own: byte offset of the lane's own
                                                                row in the weight tile */
     uint8_t *raw;            /* the workgroup's raw-block area in LDS */
     int wv, kg;              /* wave of the workgroup; lane half */
@@ -102,77 +108,101 @@ template <class F> struct Ctx {
 
 /* request Q (0 .. kReq - 1) of this wave for the raw blocks of super-block `sb` of its 32 rows (past the end of K: a
  * harmless re-read) */
-template <class F, int Q> QLIN_INL void request_w(Ctx<F> &c, int sb) {
-    dma16(c.w_rsrc, c.raw + (c.wv * F::kReq + Q) * 1024, c.w_off[Q], min(sb, c.n_sb - 1) * F::kBlockBytes);
+template <int Q, class C> QLIN_INL void request_w(C &c, int sb) {
+    dma16(c.w_rsrc, c.raw + (c.wv * C::F::kReq + Q) * 1024, c.w_off[Q], min(sb, c.n_sb - 1) * C::F::kBlockBytes);
 }
 /* vector J of this lane's raw data out of its row's image */
-template <class F, int J> QLIN_INL u32x4 load_raw(Ctx<F> &c) {
-    constexpr VecAt at = F::vec_at(J);
+template <int J, class C> QLIN_INL u32x4 load_raw(C &c) {
+    constexpr VecAt at = C::F::vec_at(J);
     return *reinterpret_cast<const u32x4 *>(c.raw + c.w_rd + ((uint32_t)(at.off + at.by_half * c.kg) ^ c.w_swz));
 }
 
-/* request I (0..7) of this wave for 64-k tile `tile` into stage ST: token rows 64 wv + 8 I .. + 7, 128 bytes each */
-template <class F, int ST, int I> QLIN_INL void request_x(Ctx<F> &c, int tile) {
-    dma16(c.x_rsrc, stage_ptr<ST>() + (8 * c.wv + I) * 1024, c.x_off[I], min(tile, 4 * c.n_sb - 1) * 128);
+/* request I (below NB) of this wave for 64-k tile `tile` into stage ST: token rows 8 (NB wv + I) .. + 7, 128 bytes each */
+template <int ST, int I, class C> QLIN_INL void request_x(C &c, int tile) {
+    dma16(c.x_rsrc, stage_ptr<C::NB, ST>() + (C::NB * c.wv + I) * 1024, c.x_off[I], min(tile, 4 * c.n_sb - 1) * 128);
 }
 
 /* activation fragment of token block BJ, k-step S of stage ST */
-template <class F, int ST, int S, int BJ> QLIN_INL bf16x8 load_frag(Ctx<F> &c) {
-    return *reinterpret_cast<const bf16x8 *>(stage_ptr<ST>() + (c.xrd ^ (uint32_t)F::frag_xor(S)) + BJ * 4096);
+template <int ST, int S, int BJ, class C> QLIN_INL bf16x8 load_frag(C &c) {
+    return *reinterpret_cast<const bf16x8 *>(stage_ptr<C::NB, ST>() + (c.xrd ^ (uint32_t)C::F::frag_xor(S)) + BJ * 4096);
 }
 
-/* slot T (0..31) of tile 4 sb + U */
-template <class F, int U, int T> QLIN_INL void slot(Ctx<F> &c) {
-    constexpr int s = T / 8, bj = T % 8;
-    if constexpr (T == 24) {
-        /* this wave's requests of the next tile have landed: younger are the 8 of the tile after it, 6 of the one
-         * after that, the weight requests of a tile with U = 1 and the scale loads of one with U = 0 (all of them if
-         * that was the tile before, those of its first 24 slots if it is this one) */
-        constexpr int w_now = F::kReq < 6 ? F::kReq : 6, x_now = F::kExtraLoads < 6 ? F::kExtraLoads : 6;
-        wait_vmcnt<14 + (U == 0 ? x_now : 0) + (U == 1 ? w_now + F::kExtraLoads : 0) + (U == 2 ? F::kReq : 0)>();
+/* n items of side work over the first `slots` slots of a tile: those of slot T are first(T) .. first(T + 1) - 1 */
+constexpr int first_of(int T, int n, int slots) { return T >= slots ? n : (T * n + slots - 1) / slots; }
+
+/* slot T (0 .. 4 NB - 1) of tile 4 sb + U */
+template <int U, int T, class C> QLIN_INL void slot(C &c) {
+    using F = typename C::F;
+    constexpr int NB = C::NB, S = C::S, s = T / NB, bj = T % NB;
+    if constexpr (T == 3 * NB) {
+        /* this wave's requests of the next tile have landed: younger are the NB of the tile after it, three quarters of those of the
+         * one after that, the weight requests of a tile with U = 1 and the scale loads of one with U = 0 (all of them if
+         * that was the tile before, those of its slots so far if it is this one) */
+        constexpr int w_now = first_of(T, F::kReq, S), x_now = first_of(T, F::kExtraLoads, S);
+        wait_vmcnt<NB + (3 * NB + 1) / 4 + (U == 0 ? x_now : 0) + (U == 1 ? w_now + F::kExtraLoads : 0) + (U == 2 ? F::kReq : 0)>();
         __builtin_amdgcn_s_barrier();
     }
-    c.acc[bj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, c.wa[U & 1][s]), c.xf[s & 1][bj], c.acc[bj], 0, 0, 0);
-    c.xf[(s + 1) & 1][bj] = load_frag<F, (s == 3 ? (U + 1) & 3 : U), (s + 1) & 3, bj>(c);
-    if constexpr (T % 4 == 2) request_x<F, (U + 3) & 3, T / 4>(c, 4 * c.sb + U + 3);
+    floatx16 &acc = c.acc[C::kSums == 2 ? s >> 1 : 0][bj];
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, c.wa[U & 1][s]), c.xf[s & 1][bj], acc, 0, 0, 0);
+    c.xf[(s + 1) & 1][bj] = load_frag<(s == 3 ? (U + 1) & 3 : U), (s + 1) & 3, bj>(c);
+    if constexpr (T % 4 == 2) request_x<(U + 3) & 3, T / 4>(c, 4 * c.sb + U + 3);
     /* U = 0: the raw data of the next super-block (requested three tiles ago) into registers; U = 1: request the
      * one after it into the same place; U = 3: the tile being decoded is the first of the next super-block, which
      * then becomes the one in work */
-    if constexpr (U == 0 && T % 3 == 1 && T / 3 < F::kLaneVec) c.nxt[T / 3] = load_raw<F, T / 3>(c);
-    if constexpr (U == 0 && T % 4 == 1 && T / 4 < F::kExtraLoads) F::template extra_load<T / 4>(c, c.nxt, min(c.sb + 1, c.n_sb - 1));
-    if constexpr (U == 1 && T % 4 == 1 && T / 4 < F::kReq) request_w<F, T / 4>(c, c.sb + 2);
-    if constexpr (U == 3 && T % 3 == 2 && T / 3 < F::kLaneVec + F::kExtraVec) c.cur[T / 3] = c.nxt[T / 3];
+    auto some = [&](auto n, auto slots, auto fn) { /* (at most four per slot) */
+        constexpr int N = decltype(n)::value, SL = decltype(slots)::value, i0 = first_of(T, N, SL), i1 = first_of(T + 1, N, SL);
+        static_assert(i1 - i0 <= 4, "items of a slot");
+        if constexpr (i0 < i1) fn(std::integral_constant<int, i0>{});
+        if constexpr (i0 + 1 < i1) fn(std::integral_constant<int, i0 + 1>{});
+        if constexpr (i0 + 2 < i1) fn(std::integral_constant<int, i0 + 2>{});
+        if constexpr (i0 + 3 < i1) fn(std::integral_constant<int, i0 + 3>{});
+    };
+    using std::integral_constant;
+    if constexpr (U == 0) {
+        some(integral_constant<int, F::kLaneVec>{}, integral_constant<int, 3 * NB>{}, [&](auto i) { c.nxt[decltype(i)::value] = load_raw<decltype(i)::value>(c); });
+        some(integral_constant<int, F::kExtraLoads>{}, integral_constant<int, S>{}, [&](auto i) { F::template extra_load<decltype(i)::value>(c, c.nxt, min(c.sb + 1, c.n_sb - 1)); });
+    }
+    if constexpr (U == 1) some(integral_constant<int, F::kReq>{}, integral_constant<int, S>{}, [&](auto i) { request_w<decltype(i)::value>(c, c.sb + 2); });
+    if constexpr (U == 3) some(integral_constant<int, F::kLaneVec + F::kExtraVec>{}, integral_constant<int, S>{}, [&](auto i) { c.cur[decltype(i)::value] = c.nxt[decltype(i)::value]; });
     constexpr int n_pieces = F::kTilePieces + (U == 3 ? F::kPrepPieces : 0);
-    constexpr int p0 = (T * n_pieces + 31) / 32, p1 = ((T + 1) * n_pieces + 31) / 32; /* pieces p with p * 32 / n_pieces == T */
+    constexpr int p0 = first_of(T, n_pieces, S), p1 = first_of(T + 1, n_pieces, S);
+    /* (beside eight blocks there are fewer than two per slot, and a word's own order is as good) */
+    constexpr auto nth = [](int p) constexpr { return NB == 8 ? p : tile_piece_at<F>(p); };
     auto piece = [&](auto pc) {
         constexpr int p = decltype(pc)::value;
         if constexpr (p < p1) {
             if constexpr (U == 3) {
                 if constexpr (p < F::kPrepPieces) F::template prep<p>(c, c.nxt);
-                else F::template tile_piece<0, 0, p - F::kPrepPieces>(c, c.nxt);
+                else F::template tile_piece<0, 0, nth(p - F::kPrepPieces)>(c, c.nxt);
             } else {
-                F::template tile_piece<U + 1, (U + 1) & 1, p>(c, c.cur);
+                F::template tile_piece<U + 1, (U + 1) & 1, nth(p)>(c, c.cur);
             }
         }
     };
-    piece(std::integral_constant<int, p0>{});
-    piece(std::integral_constant<int, p0 + 1>{});
-    piece(std::integral_constant<int, p0 + 2>{});
-    static_assert(p1 - p0 <= 3, "at most three pieces per slot");
+    piece(integral_constant<int, p0>{});
+    piece(integral_constant<int, p0 + 1>{});
+    piece(integral_constant<int, p0 + 2>{});
+    piece(integral_constant<int, p0 + 3>{});
+    piece(integral_constant<int, p0 + 4>{});
+    piece(integral_constant<int, p0 + 5>{});
+    piece(integral_constant<int, p0 + 6>{});
+    piece(integral_constant<int, p0 + 7>{});
+    static_assert(p1 - p0 <= 8, "at most eight pieces per slot");
     __builtin_amdgcn_sched_barrier(0);
 }
 
-template <class F, int U, int... T> QLIN_INL void run_tile(Ctx<F> &c, std::integer_sequence<int, T...>) { (slot<F, U, T>(c), ...); }
-template <class F, int... P> QLIN_INL void prep_first(Ctx<F> &c, std::integer_sequence<int, P...>) { (F::template prep<P>(c, c.cur), ...); }
-template <class F, int... P> QLIN_INL void decode_first(Ctx<F> &c, std::integer_sequence<int, P...>) { (F::template tile_piece<0, 0, P>(c, c.cur), ...); }
-template <class F, int ST, int... I> QLIN_INL void request_tile(Ctx<F> &c, int tile, std::integer_sequence<int, I...>) { (request_x<F, ST, I>(c, tile), ...); }
-template <class F, int... Q> QLIN_INL void request_raw(Ctx<F> &c, int sb, std::integer_sequence<int, Q...>) { (request_w<F, Q>(c, sb), ...); }
-template <class F, int... J> QLIN_INL void load_cur(Ctx<F> &c, std::integer_sequence<int, J...>) { ((c.cur[J] = load_raw<F, J>(c)), ...); }
-template <class F, int... J> QLIN_INL void load_cur_extra(Ctx<F> &c, std::integer_sequence<int, J...>) { (F::template extra_load<J>(c, c.cur, 0), ...); }
+template <int U, class C, int... T> QLIN_INL void run_tile(C &c, std::integer_sequence<int, T...>) { (slot<U, T>(c), ...); }
+template <class C, int... P> QLIN_INL void prep_first(C &c, std::integer_sequence<int, P...>) { (C::F::template prep<P>(c, c.cur), ...); }
+template <class C, int... P> QLIN_INL void decode_first(C &c, std::integer_sequence<int, P...>) { (C::F::template tile_piece<0, 0, P>(c, c.cur), ...); }
+template <int ST, class C, int... I> QLIN_INL void request_tile(C &c, int tile, std::integer_sequence<int, I...>) { (request_x<ST, I>(c, tile), ...); }
+template <class C, int... Q> QLIN_INL void request_raw(C &c, int sb, std::integer_sequence<int, Q...>) { (request_w<Q>(c, sb), ...); }
+template <class C, int... J> QLIN_INL void load_cur(C &c, std::integer_sequence<int, J...>) { ((c.cur[J] = load_raw<J>(c)), ...); }
+template <class C, int... J> QLIN_INL void load_cur_extra(C &c, std::integer_sequence<int, J...>) { (C::F::template extra_load<J>(c, c.cur, 0), ...); }
+template <class C, int... B> QLIN_INL void load_first(C &c, std::integer_sequence<int, B...>) { ((c.xf[0][B] = load_frag<0, 0, B>(c)), ...); }
 
 }  // namespace
 
-template <class F, bool DIVIDED>
+template <class F, int NB, bool DIVIDED>
 __global__ void __launch_bounds__(256)
 gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles,
                           const KItems<DIVIDED> split) {
@@ -193,7 +223,8 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_
     float *Y = part.out;
     X += part.sb0 * 256;
 
-    Ctx<F> c;
+    Ctx<F, NB, DIVIDED ? 1 : 2> c;
+    constexpr int kBM = 32 * NB;
     c.raw = w4_raw;
     c.wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     c.n_sb = n_sb;
@@ -218,51 +249,52 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_
     c.w_swz = F::kSwizzle ? (uint32_t)(li & 15) << 4 : 0u;
     c.w_own = (uint32_t)min(32 * c.wv + li, w_rows - 1) * row_bytes;
     /* Activation requests: request I of this wave fills 1 KB of a stage, lane l the 16 bytes at chunk position l % 8 of
-     * token row 64 wv + 8 I + l / 8, i.e. chunk (l % 8) ^ f(row) of that token's 128 bytes; tokens past the end
+     * token row 8 (NB wv + I) + l / 8, i.e. chunk (l % 8) ^ f(row) of that token's 128 bytes; tokens past the end
      * re-read the last one (never stored) */
     const int x_rows = min(kBM, n_tok - tile_m * kBM);
     c.x_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(X) + (size_t)tile_m * kBM * ldx, 0,
                                                  ((x_rows - 1) * ldx + n_sb * 256) * 2, 0x00020000);
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int row = 64 * c.wv + 8 * i + (lane >> 3);
+    for (int i = 0; i < NB; i++) {
+        const int row = 8 * (NB * c.wv + i) + (lane >> 3);
         c.x_off[i] = (uint32_t)min(row, x_rows - 1) * (uint32_t)(2 * ldx) + (uint32_t)((((lane & 7) ^ fsw(row))) << 4);
     }
     /* fragment fetches: token li of each block of 32; chunk 4 (s >> 1) + 2 kg + (s & 1) for the K-quants */
     c.xrd = (uint32_t)(li * 128 + (((F::kKgChunk * kg) ^ fsw(li)) << 4));
 
 #pragma unroll
-    for (int i = 0; i < 8; i++)
+    for (int i = 0; i < NB; i++)
 #pragma unroll
-        for (int v = 0; v < 16; v++) c.acc[i][v] = 0.0f;
+        for (int v = 0; v < 16; v++) {
+            c.acc[0][i][v] = 0.0f;
+            if constexpr (!DIVIDED) c.acc[1][i][v] = 0.0f;
+        }
 
     /* ---- prologue: raw blocks of super-block 0 fetched and read back, those of super-block 1 and tiles 0..2
      * requested; tile 0 decoded; fragments of its k-step 0 fetched */
     c.sb = 0;
-    load_cur_extra<F>(c, std::make_integer_sequence<int, F::kExtraLoads>{});
-    request_raw<F>(c, 0, std::make_integer_sequence<int, F::kReq>{});
-    request_tile<F, 0>(c, 0, std::make_integer_sequence<int, 8>{});
-    wait_vmcnt<8>();
-    load_cur<F>(c, std::make_integer_sequence<int, F::kLaneVec>{});
+    load_cur_extra(c, std::make_integer_sequence<int, F::kExtraLoads>{});
+    request_raw(c, 0, std::make_integer_sequence<int, F::kReq>{});
+    request_tile<0>(c, 0, std::make_integer_sequence<int, NB>{});
+    wait_vmcnt<NB>();
+    load_cur(c, std::make_integer_sequence<int, F::kLaneVec>{});
     __builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0): the registers hold super-block 0 before its place is requested again */
-    request_raw<F>(c, 1, std::make_integer_sequence<int, F::kReq>{});
-    request_tile<F, 1>(c, 1, std::make_integer_sequence<int, 8>{});
-    request_tile<F, 2>(c, 2, std::make_integer_sequence<int, 8>{});
-    prep_first<F>(c, std::make_integer_sequence<int, F::kPrepPieces>{});
-    decode_first<F>(c, std::make_integer_sequence<int, F::kTilePieces>{});
-    wait_vmcnt<16>(); /* tile 0 and the raw blocks of super-block 1 are in LDS as far as this wave's requests go */
+    request_raw(c, 1, std::make_integer_sequence<int, F::kReq>{});
+    request_tile<1>(c, 1, std::make_integer_sequence<int, NB>{});
+    request_tile<2>(c, 2, std::make_integer_sequence<int, NB>{});
+    prep_first(c, std::make_integer_sequence<int, F::kPrepPieces>{});
+    decode_first(c, std::make_integer_sequence<int, F::kTilePieces>{});
+    wait_vmcnt<2 * NB>(); /* tile 0 and the raw blocks of super-block 1 are in LDS as far as this wave's requests go */
     __builtin_amdgcn_s_barrier();
-    c.xf[0][0] = load_frag<F, 0, 0, 0>(c); c.xf[0][1] = load_frag<F, 0, 0, 1>(c); c.xf[0][2] = load_frag<F, 0, 0, 2>(c);
-    c.xf[0][3] = load_frag<F, 0, 0, 3>(c); c.xf[0][4] = load_frag<F, 0, 0, 4>(c); c.xf[0][5] = load_frag<F, 0, 0, 5>(c);
-    c.xf[0][6] = load_frag<F, 0, 0, 6>(c); c.xf[0][7] = load_frag<F, 0, 0, 7>(c);
+    load_first(c, std::make_integer_sequence<int, NB>{});
 
 #pragma unroll 1
     for (int sb = 0; sb < n_sb; sb++) { /* one super-block of K = four tiles per pass */
         c.sb = sb;
-        run_tile<F, 0>(c, std::make_integer_sequence<int, 32>{});
-        run_tile<F, 1>(c, std::make_integer_sequence<int, 32>{});
-        run_tile<F, 2>(c, std::make_integer_sequence<int, 32>{});
-        run_tile<F, 3>(c, std::make_integer_sequence<int, 32>{});
+        run_tile<0>(c, std::make_integer_sequence<int, 4 * NB>{});
+        run_tile<1>(c, std::make_integer_sequence<int, 4 * NB>{});
+        run_tile<2>(c, std::make_integer_sequence<int, 4 * NB>{});
+        run_tile<3>(c, std::make_integer_sequence<int, 4 * NB>{});
     }
     wait_vmcnt<0>(); /* requests past the end of K are still on their way into LDS */
 
@@ -270,14 +302,19 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_
      * l % 32 (a token): four runs of four consecutive floats of one token's output row per lane */
     const bool vec_ok = (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
 #pragma unroll
-    for (int bj = 0; bj < 8; bj++) {
+    for (int bj = 0; bj < NB; bj++) {
         const int m = tile_m * kBM + 32 * bj + li;
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             const int n = tile_n * kBN + 32 * c.wv + 8 * g + 4 * kg;
             if (m >= n_tok) continue;
             float *y = Y + (size_t)m * ldy + n;
-            const floatx4 a = {c.acc[bj][4 * g], c.acc[bj][4 * g + 1], c.acc[bj][4 * g + 2], c.acc[bj][4 * g + 3]};
+            floatx4 a;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                a[v] = c.acc[0][bj][4 * g + v];
+                if constexpr (!DIVIDED) a[v] += c.acc[1][bj][4 * g + v];
+            }
             if (vec_ok && n + 3 < n_rows) {
                 *reinterpret_cast<floatx4 *>(y) = a;
             } else {
@@ -328,28 +365,37 @@ void launch_k_join(const KSplit &split, int n_mat, float *const *Y, const int *n
 }
 
 namespace {
-template <class F>
-hipError_t launch_wave4(int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows, int n_cols,
+template <class F, int NB>
+hipError_t launch_wave4_blocks(int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows, int n_cols,
                         int n_tok, int ldx, const int *ldy, KSplit split, hipStream_t stream) {
     const int n_sb = n_cols / 256;
-    const int m_tiles = (n_tok + kBM - 1) / kBM;
+    const int m_tiles = (n_tok + 32 * NB - 1) / (32 * NB);
     TileSet set;
     const int n_tiles = fill_tile_set(set, n_mat, W, Y, n_rows, ldy, kBN, split);
     /* ids are dealt to 8 XCDs; pad the n-tile count to a multiple of 8 (surplus groups exit) */
     const int n_tiles_pad = (n_tiles + 7) / 8 * 8;
     const dim3 grid(n_tiles_pad * m_tiles), block(256);
     if (split.divides()) {
-        hipLaunchKernelGGL((gemm_kq_bf16_wave4_kernel<F, true>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, k_items(split));
-        launch_k_join(split, n_mat, Y, n_rows, n_tok, ldy, stream);
+        if constexpr (NB == kLargeBlocks) {
+            hipLaunchKernelGGL((gemm_kq_bf16_wave4_kernel<F, NB, true>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, k_items(split));
+            launch_k_join(split, n_mat, Y, n_rows, n_tok, ldy, stream);
+        } else return hipErrorInvalidValue;
     } else {
-        hipLaunchKernelGGL((gemm_kq_bf16_wave4_kernel<F, false>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, KItems<false>());
+        hipLaunchKernelGGL((gemm_kq_bf16_wave4_kernel<F, NB, false>), grid, block, 0, stream, set, X, n_sb, n_tok, ldx, m_tiles, KItems<false>());
     }
     return hipGetLastError();
 }
 template <class F>
-hipError_t launch_wave4(const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok, int ldx, int ldy,
-                        hipStream_t stream) {
-    return launch_wave4<F>(1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, KSplit(), stream);
+hipError_t launch_wave4(int blocks, int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows, int n_cols,
+                        int n_tok, int ldx, const int *ldy, KSplit split, hipStream_t stream) {
+    switch (blocks) {
+    case 3: return launch_wave4_blocks<F, 3>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case 4: return launch_wave4_blocks<F, 4>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case 5: return launch_wave4_blocks<F, 5>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case 6: return launch_wave4_blocks<F, 6>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case kLargeBlocks: return launch_wave4_blocks<F, kLargeBlocks>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    default: return hipErrorInvalidValue;
+    }
 }
 }  // namespace
 
@@ -490,43 +536,90 @@ hipError_t launch_fused_split(FusedSplit s, uint32_t type, const void *W, const 
     KSplit split;
     split.buf[0] = (float *)workspace;
     split.parts[0] = s.parts;
-    return s.tile == kFusedLarge ? launch_gemm_kq_bf16_wave4_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split)
+    return s.tile == kFusedLarge ? launch_gemm_kq_bf16_wave4_multi(type, kLargeBlocks, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split)
                                  : launch_gemm_kq_bf16_wave4s_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split);
+}
+
+/* How many token blocks the tiles of a launch have (0: the 128-token x 64-row kernel), of tensors that take `tile` each by itself. All
+ * shapes give the same bits, so the tensors of a launch are looked at together. Estimates in us: a super-block costs a full round of
+ * 256 workgroups what the table says (measured at 224 workgroups; the 128 x 64 kernel's at up to 256 workgroups and at 512), a round
+ * that leaves compute units idle less - the clock is higher then, the more so the more blocks; three blocks fit a compute unit's
+ * LDS twice. Row tiles are dealt to 8 XCDs of 32 compute units. Over 198 products of nine formats (2048 to 28672 rows x 2048 to 4096 and
+ * 14336 columns, 77 to 1024 tokens) the choice costs 1.0 % of the best kernel's time and takes 0.90 of what `tile` does (one tensor). A gain of less
+ * than 4 % is left alone. */
+int choose_token_blocks(uint32_t type, FusedTile tile, int n_mat, const int *n_rows, int n_cols, int n_tok) {
+    struct Cost { float b3, b4, b5, b6, b8, small_256, small_512; };
+    Cost c;
+    switch (type) { /* the measurements: 3.5 us + 16 super-blocks times this, 4096 columns */
+    case T_Q4_K: c = {1.77f, 2.15f, 2.45f, 2.82f, 3.53f, 1.37f, 2.42f}; break;
+    case T_Q5_K: c = {1.86f, 2.28f, 2.65f, 3.04f, 3.67f, 1.51f, 2.50f}; break;
+    case T_Q6_K: c = {2.46f, 2.79f, 3.05f, 3.56f, 4.00f, 1.79f, 2.95f}; break;
+    case T_Q8_0: c = {2.61f, 3.23f, 3.75f, 3.92f, 4.67f, 2.19f, 3.80f}; break;
+    case T_IQ4_NL: c = {1.99f, 2.50f, 2.75f, 3.29f, 3.73f, 1.48f, 2.62f}; break;
+    case T_IQ4_XS: c = {2.04f, 2.50f, 2.78f, 3.23f, 3.74f, 1.53f, 2.68f}; break;
+    case T_Q4_0: c = {1.76f, 2.17f, 2.50f, 2.88f, 3.49f, 1.40f, 2.39f}; break;
+    case T_Q2_K: c = {1.64f, 2.09f, 2.37f, 2.72f, 3.48f, 1.31f, 2.30f}; break;
+    default: c = {1.85f, 2.26f, 2.57f, 3.04f, 3.56f, 1.38f, 2.54f}; break; /* Q3_K */
+    }
+    long long rows128 = 0, rows64 = 0;
+    for (int i = 0; i < n_mat; i++) { rows128 += ((long long)n_rows[i] + 127) / 128; rows64 += ((long long)n_rows[i] + 63) / 64; }
+    const auto workgroups = [&](long long row_tiles, int tokens) { return (row_tiles + 7) / 8 * 8 * ((n_tok + tokens - 1) / tokens); };
+    /* the part of a full round's time that n workgroups take on the chip: `low` up to 112 of them */
+    const auto round = [](double low, double n) {
+        const double x = std::min(1.0, std::max(0.0, (n - 112) / 112));
+        return low + (1 - low) * x * x * x;
+    };
+    const auto blocks_us = [&](int nb, double full, double low) {
+        const long long n = workgroups(rows128, 32 * nb), per = nb == 3 ? 512 : 256, rest = n % per;
+        double rounds = (double)(n / per) * (nb == 3 ? 1.85 : 1.0);
+        if (rest > 256) rounds += 1.0 + 0.85 * (0.6 + 0.4 * (rest - 256) / 256);
+        else if (rest > 0) rounds += round(low, (double)rest);
+        return 3.5 + n_cols / 256 * full * rounds;
+    };
+    const long long n_small = workgroups(rows64, 128), rest = n_small % 512;
+    double small = (double)(n_small / 512) * c.small_512;
+    if (rest > 256) small += c.small_256 + (c.small_512 - c.small_256) * (0.55 + 0.45 * (rest - 256) / 256);
+    else if (rest > 0) small += c.small_256 * (0.9 + 0.1 * rest / 256);
+    small = 3.5 + n_cols / 256 * small;
+    const double us[5] = {blocks_us(3, c.b3, 0.92), blocks_us(4, c.b4, 0.80), blocks_us(5, c.b5, 0.78), blocks_us(6, c.b6, 0.75), blocks_us(8, c.b8, 0.71)};
+    const int blocks[5] = {3, 4, 5, 6, kLargeBlocks};
+    int best = tile == kFusedLarge ? kLargeBlocks : 0;
+    double best_us = 0.96 * (tile == kFusedLarge ? us[4] : small);
+    if (small < best_us) { best = 0; best_us = small; }
+    for (int i = 0; i < 5; i++)
+        if (us[i] < best_us) { best = blocks[i]; best_us = us[i]; }
+    return best;
+}
+
+hipError_t launch_fused_tiles(FusedTile tile, uint32_t type, int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows,
+                              int n_cols, int n_tok, int ldx, const int *ldy, hipStream_t stream) {
+    if (tile == kFusedNone) return hipErrorInvalidValue;
+    const int blocks = choose_token_blocks(type, tile, n_mat, n_rows, n_cols, n_tok);
+    return blocks ? launch_gemm_kq_bf16_wave4_multi(type, blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream)
+                  : launch_gemm_kq_bf16_wave4s_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
 }
 
 hipError_t launch_fused_tile(FusedTile tile, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows,
                              int n_cols, int n_tok, int ldx, int ldy, hipStream_t stream) {
-    if (tile == kFusedLarge) return launch_gemm_kq_bf16_wave4(type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    if (tile == kFusedSmall) return launch_gemm_kq_bf16_wave4s(type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
-    return hipErrorInvalidValue;
+    return launch_fused_tiles(tile, type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream);
 }
 
-hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
+hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int blocks, int n_mat, const void *const *W, const uint16_t *X,
                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
                                            const int *ldy, hipStream_t stream, KSplit split) {
     if (n_mat < 1 || n_mat > 3) return hipErrorInvalidValue;
     switch (type) {
-    case T_Q4_K: return launch_wave4<FQ4K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_Q5_K: return launch_wave4<FQ5K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_Q6_K: return launch_wave4<FQ6K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_Q8_0: return launch_wave4<FQ8_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_IQ4_NL: return launch_wave4<FIQ4NL>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_IQ4_XS: return launch_wave4<FIQ4XS>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_Q4_0: return launch_wave4<FQ4_0>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_Q2_K: return launch_wave4<FQ2K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
-    case T_Q3_K: return launch_wave4<FQ3K>(n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q4_K: return launch_wave4<FQ4K>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q5_K: return launch_wave4<FQ5K>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q6_K: return launch_wave4<FQ6K>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q8_0: return launch_wave4<FQ8_0>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_IQ4_NL: return launch_wave4<FIQ4NL>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_IQ4_XS: return launch_wave4<FIQ4XS>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q4_0: return launch_wave4<FQ4_0>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q2_K: return launch_wave4<FQ2K>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
+    case T_Q3_K: return launch_wave4<FQ3K>(blocks, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, split, stream);
     default: return hipErrorInvalidValue;
     }
-}
-
-hipError_t launch_gemm_kq_bf16_wave4(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
-                                     int n_tok, int ldx, int ldy, hipStream_t stream) {
-    return launch_gemm_kq_bf16_wave4_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream);
-}
-
-hipError_t launch_gemm_q4k_bf16_wave4(const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
-                                      int ldx, int ldy, hipStream_t stream) {
-    return launch_wave4<FQ4K>(W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, stream);
 }
 
 }  // namespace qlin

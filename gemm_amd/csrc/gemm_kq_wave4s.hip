@@ -343,9 +343,4 @@ hipError_t launch_gemm_kq_bf16_wave4s_multi(uint32_t type, int n_mat, const void
     }
 }
 
-hipError_t launch_gemm_kq_bf16_wave4s(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
-                                      int n_tok, int ldx, int ldy, hipStream_t stream) {
-    return launch_gemm_kq_bf16_wave4s_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream);
-}
-
 }  // namespace qlin

@@ -1290,8 +1290,10 @@ int qlin_gemm_bf16_multi_dev(uint32_t type, int n_mat, const void *const *W, con
             split.parts[i] = plan.parts[i];
             if (plan.parts[i] > 1) split.buf[i] = (float *)((char *)workspace + plan.at[i]);
         }
-        if (plan.tile == kFusedLarge)
-            HIP_TRY(launch_gemm_kq_bf16_wave4_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream, split));
+        if (!split.divides())
+            HIP_TRY(launch_fused_tiles(plan.tile, type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream));
+        else if (plan.tile == kFusedLarge)
+            HIP_TRY(launch_gemm_kq_bf16_wave4_multi(type, 8, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream, split));
         else
             HIP_TRY(launch_gemm_kq_bf16_wave4s_multi(type, n_mat, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy, (hipStream_t)stream, split));
         return QLIN_OK;
@@ -1483,7 +1485,7 @@ int qlin_probe_gemm_f32_route(uint32_t type, int n_rows, int n_cols, int n_tok) 
 
 int qlin_probe_gemm_tile(int tile, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                          int n_tok, int ldx, int ldy, void *stream) {
-    if (tile < 0 || tile > 1) return fail(QLIN_ERR_ARG, "tile: 0 (256 x 128) or 1 (128 x 64)");
+    if (tile != 0 && tile != 1 && (tile < 3 || tile > 6)) return fail(QLIN_ERR_ARG, "tile: 0 (256 x 128), 1 (128 x 64) or 3 to 6 (32 times as many tokens x 128)");
     if (!gemm_kq_wave4_covers(type)) return fail(QLIN_ERR_TYPE, "no fused tile kernel for type %u", type);
     if (int rc = check_linear_shape(type, n_rows, n_cols)) return rc;
     if (n_tok < 0 || ldx < n_cols || ldy < n_rows || n_cols % 256 || ldx >= (1 << 22))
@@ -1493,8 +1495,8 @@ int qlin_probe_gemm_tile(int tile, uint32_t type, const void *W, const uint16_t 
     if (!aligned(W, 16) || !aligned(X, 16) || !aligned(Y, 4) || ldx % 8)
         return fail(QLIN_ERR_ARG, "W and X need 16-byte alignment, Y 4-byte, ldx %% 8 == 0");
     if (int rc = init_once()) return rc;
-    HIP_TRY(launch_fused_tile(tile == 0 ? kFusedLarge : kFusedSmall, type, W, X, Y, n_rows, n_cols, n_tok, ldx, ldy,
-                              (hipStream_t)stream));
+    if (tile == 1) HIP_TRY(launch_gemm_kq_bf16_wave4s_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, (hipStream_t)stream));
+    else HIP_TRY(launch_gemm_kq_bf16_wave4_multi(type, tile ? tile : 8, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, (hipStream_t)stream));
     return QLIN_OK;
 }
 

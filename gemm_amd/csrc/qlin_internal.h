@@ -183,12 +183,9 @@ hipError_t f32_split_iq4xs(const F32SplitCall &c);
 hipError_t f32_split_iq3s(const F32SplitCall &c);
 hipError_t f32_split_iq2xxs(const F32SplitCall &c);
 constexpr int kMatvecTokens = 4; /* qlin_gemm_bf16_any_dev: up to this many tokens of a format without a few-token kernel go through the matvec */
-/* 256-token x 128-row tiles on four waves, one per SIMD, weights decoded from their blocks into the matrix operand
+/* Tiles of 128 rows on four waves, one per SIMD, weights decoded from their blocks into the matrix operand
  * (gemm_kq_wave4.hip): the formats of gemm_kq_wave4_covers, n_cols % 256 == 0, ldx < 2^22 */
 bool gemm_kq_wave4_covers(uint32_t type);
-/* the same in 128-token x 64-row tiles, two workgroups per compute unit (gemm_kq_wave4s.hip) */
-hipError_t launch_gemm_kq_bf16_wave4s(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
-                                      int n_tok, int ldx, int ldy, hipStream_t stream);
 /* K of a tensor divided over parts[i] workgroups per tile, which write their sums to buf[i], [part][token][row]; launch_k_join adds
  * them up, of all tensors that are divided. One part: the sums go to Y. */
 struct KSplit {
@@ -197,8 +194,10 @@ struct KSplit {
     bool divides() const { return parts[0] > 1 || parts[1] > 1 || parts[2] > 1; }
 };
 void launch_k_join(const KSplit &split, int n_mat, float *const *Y, const int *n_rows, int n_tok, const int *ldy, hipStream_t stream);
-/* the same kernel over up to three tensors of one format and K in one launch (row tiles numbered through the tensors) */
-hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
+/* up to three tensors of one format and K in one launch (row tiles numbered through the tensors): tiles of 128 rows x 32 `blocks`
+ * tokens, blocks 3, 4, 5, 6 or 8 (8 where K is divided), or of 64 rows x 128 tokens, two workgroups per compute unit (gemm_kq_wave4s.hip).
+ * Every shape gives the same bits */
+hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int blocks, int n_mat, const void *const *W, const uint16_t *X,
                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
                                            const int *ldy, hipStream_t stream, KSplit split = {});
 hipError_t launch_gemm_kq_bf16_wave4s_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
@@ -213,12 +212,12 @@ struct FusedSplit { FusedTile tile; int parts; };
 FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, size_t workspace_bytes, FusedTile tile, bool few);
 hipError_t launch_fused_split(FusedSplit s, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
                               int ldx, int ldy, void *workspace, hipStream_t stream);
+/* tensors that take a tile kernel each by itself, undivided, in one launch of the tile shape that suits them together */
+int choose_token_blocks(uint32_t type, FusedTile tile, int n_mat, const int *n_rows, int n_cols, int n_tok);
+hipError_t launch_fused_tiles(FusedTile tile, uint32_t type, int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows,
+                              int n_cols, int n_tok, int ldx, const int *ldy, hipStream_t stream);
 hipError_t launch_fused_tile(FusedTile tile, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows,
                              int n_cols, int n_tok, int ldx, int ldy, hipStream_t stream);
-hipError_t launch_gemm_kq_bf16_wave4(uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
-                                     int n_tok, int ldx, int ldy, hipStream_t stream);
-hipError_t launch_gemm_q4k_bf16_wave4(const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,
-                                      int ldx, int ldy, hipStream_t stream);
 hipError_t launch_gemm_q4k_bf16(const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols,
                                 int n_tok, int ldx, int ldy, hipStream_t stream);
 

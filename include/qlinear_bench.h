@@ -25,11 +25,12 @@ int qlin_probe_clocks(void *stream, double *shader_mhz);
 int qlin_probe_hbm_read(const void *buf, size_t n_bytes, void *stream);
 
 /* One tile kernel of the fused prefill GEMM by name, whatever the shape-based choice of qlin_gemm_bf16_any_dev would be:
- * tile 0 = 256 tokens x 128 rows, 1 = 128 tokens x 64 rows. Arguments and result as qlin_gemm_bf16_any_dev without a
+ * tile 0 = 256 tokens x 128 rows, 1 = 128 tokens x 64 rows, 3 to 6 = that many times 32 tokens x 128 rows. Arguments and result as qlin_gemm_bf16_any_dev without a
  * workspace; Q4_K, Q5_K, Q6_K, Q8_0, IQ4_NL, IQ4_XS, Q4_0; n_cols % 256 == 0. For timing one against the other and for the parity tests of
  * each on small shapes. */
-/* which kernel qlin_gemm_bf16_any_dev picks for a shape: 1 = the 256 x 128 tile kernel, 2 = the 128 x 64 one, 3 = the
- * few-token kernel, 0 = none of them (a matvec per token, or decode to bf16 + dense product) */
+/* which kernel qlin_gemm_bf16_any_dev picks for a shape: 1 = 256 x 128 tiles, 2 = 128 x 64 ones (1 and 2: unless another tile shape,
+ * with the same results, suits the launch better), 3 = the few-token kernel, 0 = none of them (a matvec per token, or decode to bf16 +
+ * dense product) */
 int qlin_probe_gemm_route(uint32_t ggml_type, int n_rows, int n_cols, int n_tok, int ldx, int have_workspace);
 /* over how many workgroups a tile's K is divided, given a workspace of qlin_gemm_bf16_any_workspace_bytes bytes (1: it is not) */
 int qlin_probe_gemm_parts(uint32_t ggml_type, int n_rows, int n_cols, int n_tok, int ldx);

@@ -149,6 +149,28 @@ def test_each_tile_kernel_on_small_and_ragged_shapes(oracle, tile, tid, n_tok, n
         assert rel_l2(Y[:, :n_rows], exact) <= 3e-3
 
 
+@pytest.mark.parametrize("tid", FUSED, ids=lambda t: ALL[t])
+@pytest.mark.parametrize("n_tok,n_rows,n_cols", [(1, 3, 256), (96, 128, 512), (97, 129, 1280), (161, 127, 768), (193, 260, 256)])
+def test_tile_shapes_give_the_same_bits(oracle, tid, n_tok, n_rows, n_cols):
+    """tiles of three to eight token blocks x 128 rows against the 128 x 64 kernel: edges of a tile in tokens and rows, one super-block, odd
+    counts of them; the values against the oracle's weights rounded once (the other kernels' bar)"""
+    W = synth.make_weights(tid, n_rows, n_cols, seed=5 * n_rows + tid)
+    Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=n_tok + tid, tokens=n_tok))
+    dW, dX, ldy = qlinear.DevBuf.from_numpy(W), qlinear.DevBuf.from_numpy(Xb), n_rows + 1
+    got = {}
+    for tile in (1, 3, 4, 5, 6, 0):
+        dY = qlinear.DevBuf.from_numpy(np.full((n_tok, ldy), -3.0, np.float32))
+        qlinear.probe_gemm_tile(tile, tid, dW, dX, dY, n_rows, n_cols, n_tok, n_cols, ldy)
+        qlinear.sync()
+        got[tile] = dY.to_numpy(np.float32, (n_tok, ldy))
+        dY.free()
+    dW.free()
+    dX.free()
+    assert all(np.array_equal(got[1], y) for y in got.values())
+    assert np.all(got[1][:, n_rows:] == -3.0)
+    assert rel_l2(got[1][:, :n_rows], references(oracle, tid, W, Xb, n_cols)[1]) <= 2e-5
+
+
 def multi_case(tid, rows, n_cols, n_tok, seed):
     Ws = [synth.make_weights(tid, r, n_cols, seed=seed + i) for i, r in enumerate(rows)]
     Xb = synth.to_bf16_bits(synth.make_activation(n_cols, seed=seed + 9, tokens=n_tok))
