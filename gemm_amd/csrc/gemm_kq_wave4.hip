@@ -404,6 +404,53 @@ bool gemm_kq_wave4_covers(uint32_t type) {
            type == T_Q4_0 || type == T_Q2_K || type == T_Q3_K;
 }
 
+/* Estimates, in us, for the tensors of a launch in each shape of tile. A super-block costs a full round of 256 workgroups what the
+ * table says (the 128 x 64 kernel's: up to 256 workgroups, and 512), a round that leaves compute units idle less - the clock is higher
+ * then, the more so the more blocks; three blocks fit a compute unit's LDS twice. Row tiles are dealt to 8 XCDs of 32 compute units.
+ * The results go to memory at 3.3 TB/s beside that. Fitted to 3700 measured products of nine formats (640 to 28672 rows x 1024 to
+ * 14336 columns, 77 to 4096 tokens, runs long enough that the power limit counts); an estimate errs by 3.8 % in the mean. */
+static constexpr int kTokenBlocks[6] = {0, 3, 4, 5, 6, kLargeBlocks};
+static void tile_us(uint32_t type, int n_mat, const int *n_rows, int n_cols, int n_tok, double us[6]) {
+    struct Cost { float small_256, small_512, b[5]; };
+    Cost c;
+    switch (type) {
+    case T_Q4_K: c = {1.18f, 2.07f, {1.45f, 1.83f, 2.10f, 2.44f, 3.10f}}; break;
+    case T_Q5_K: c = {1.25f, 2.20f, {1.61f, 2.02f, 2.28f, 2.67f, 3.20f}}; break;
+    case T_Q6_K: c = {1.55f, 2.69f, {2.01f, 2.37f, 2.70f, 3.09f, 3.61f}}; break;
+    case T_Q8_0: c = {2.03f, 3.52f, {2.42f, 2.83f, 3.07f, 3.44f, 3.95f}}; break;
+    case T_IQ4_NL: c = {1.36f, 2.30f, {1.83f, 2.18f, 2.40f, 2.82f, 3.33f}}; break;
+    case T_IQ4_XS: c = {1.46f, 2.33f, {1.85f, 2.22f, 2.47f, 2.89f, 3.42f}}; break;
+    case T_Q4_0: c = {1.18f, 2.09f, {1.47f, 1.86f, 2.13f, 2.51f, 3.10f}}; break;
+    case T_Q2_K: c = {1.13f, 1.96f, {1.37f, 1.74f, 2.05f, 2.35f, 3.05f}}; break;
+    default: c = {1.28f, 2.21f, {1.59f, 1.93f, 2.21f, 2.59f, 3.18f}}; break; /* Q3_K */
+    }
+    constexpr float kIdle[5] = {0.97f, 0.90f, 0.865f, 0.85f, 0.825f}; /* of a round's time, where at most 112 workgroups run */
+    long long rows = 0, rows128 = 0, rows64 = 0;
+    for (int i = 0; i < n_mat; i++) {
+        rows += n_rows[i];
+        rows128 += ((long long)n_rows[i] + 127) / 128;
+        rows64 += ((long long)n_rows[i] + 63) / 64;
+    }
+    const auto workgroups = [&](long long row_tiles, int tokens) { return (row_tiles + 7) / 8 * 8 * ((n_tok + tokens - 1) / tokens); };
+    const double fixed = 3.3 + 1.2e-6 * rows * n_tok;
+    const long long n_small = workgroups(rows64, 128), rest_small = n_small % 512;
+    double rounds = (double)(n_small / 512) * c.small_512;
+    if (rest_small > 256) rounds += c.small_256 + (c.small_512 - c.small_256) * (0.64 + 0.36 * (rest_small - 256) / 256);
+    else if (rest_small > 0) rounds += c.small_256 * (0.73 + 0.27 * rest_small / 507.0);
+    us[0] = fixed + n_cols / 256 * rounds;
+    for (int i = 0; i < 5; i++) {
+        const int nb = kTokenBlocks[i + 1];
+        const long long n = workgroups(rows128, 32 * nb), per = nb == 3 ? 512 : 256, rest = n % per;
+        rounds = (double)(n / per) * (nb == 3 ? 1.98 : 1.0);
+        if (rest > 256) rounds += 1.0 + 0.98 * (0.6 + 0.4 * (rest - 256) / 256);
+        else if (rest > 0) {
+            const double x = std::min(1.0, std::max(0.0, (rest - 112) / 112.0));
+            rounds += kIdle[i] + (1 - kIdle[i]) * x * x * x;
+        }
+        us[i + 1] = fixed + n_cols / 256 * c.b[i] * rounds;
+    }
+}
+
 /* Which kernel takes a prefill GEMM of a format with a fused kernel, beyond the token counts of the few-token kernels.
  * 200 or more 256-token x 128-row tiles fill the chip: the large-tile kernel - up to a token count, because it decodes
  * the weights again every 256 tokens, which costs more the more there is to decode, while decoding once into a workspace
@@ -419,6 +466,13 @@ bool gemm_kq_wave4_covers(uint32_t type) {
  * IQ4_NL 27 / 45, 80 / 108, 46 / 55, 148 / 161, 63 / 63, 44 / 88; IQ4_XS 27 / 45, 82 / 110, 47 / 55, 154 / 162, 64 / 63,
  * 45 / 80; Q4_0 24 / 41, 72 / 91, 41 / 50, 133 / 144, 57 / 56, 39 / 72; Q2_K 24 / 42, 70 / 94, 41 / 52, 132 / 149, 55 / 58,
  * 38 / 74; Q3_K 26 / 45, 75 / 102, 44 / 54, 144 / 160, 61 / 61, 42 / 82).
+ * Those lines are for tensors of any size; smaller ones, whose tiles end in fewer or fuller rounds, gain beyond them. There the
+ * estimates decide (tile_us; decode + library: 10.7 us, the decode 0.53 us per million weights, the product 1.48 PFLOP/s and its
+ * results). The library's errs by a tenth, so that 10 % are asked for, of Q8_0 14: at 7 % Q6_K 1024 x 3584 at 1139 tokens and at 10 %
+ * Q8_0 2048 x 2048 at 863 lost 2 us. us, decode + library / tiles: Q6_K 2048 x 2048 at 640 tokens 23.7 / 15.8, 2560 x 6912 at 640
+ * 48 / 39, 2048 x 4096 at 1024 36 / 28; Q8_0 11008 x 1024 at 328 29.5 / 21.2; IQ4_NL 2048 x 2048 at 1300 28 / 22; Q4_K 4096 x 14336 at
+ * 2048 235 / 201; Q2_K 4096 x 5120 at 3904 134 / 158, left alone. Of 837 random products past the lines 110 take tiles, in 0.84 of the
+ * time (one is slower by more than 3 %); their error against 64 bits is 0.7 of that of the library's product.
  * Without a workspace there is no decode + dense route to prefer.
  * Up to 128 tokens half of a large tile is empty: small tiles whatever their number (77 tokens 28672 x 4096 large / small: Q4_K
  * 51 / 38, Q5_K 52 / 41, Q6_K 57 / 48; 128 tokens 65536 x 1024 Q4_K 1.26 times, IQ4_XS 1.27, Q3_K 1.30; Q8_0 even). Past 128
@@ -449,7 +503,16 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     case T_Q6_K: small_max = 512; break;
     default: break;
     }
-    const bool large_ok = n_tok <= large_max || !have_workspace, small_ok = n_tok <= small_max || !have_workspace;
+    bool large_ok = n_tok <= large_max || !have_workspace, small_ok = n_tok <= small_max || !have_workspace;
+    /* beyond: the estimates, in the range they were measured over (256 rows x 2304 IQ4_NL at 1860 tokens would lose 2 us; Q8_0's K
+     * and V of a model wider than 11008 divide K at such token counts, and would part from a Q in tiles) */
+    if ((!large_ok || !small_ok) && n_rows >= 640 && n_cols <= (type == T_Q8_0 ? 11008 : 14336)) {
+        double us[6];
+        tile_us(type, 1, &n_rows, n_cols, n_tok, us);
+        const double weights = (double)n_rows * n_cols, results = (double)n_rows * n_tok;
+        if (*std::min_element(us, us + 6) < (type == T_Q8_0 ? 0.86 : 0.9) * (10.7 + 0.53e-6 * weights + 1.352e-9 * weights * n_tok + 1.41e-3 * n_cols + 0.773e-6 * results))
+            large_ok = small_ok = true;
+    }
     if (large_tiles >= 200 && !large_ok) return kFusedNone;
     if (n_tok > 128 && large_ok && small_ok) {
         bool small = small_by_rounds(type, n_rows, n_tok, 1);
@@ -540,55 +603,19 @@ hipError_t launch_fused_split(FusedSplit s, uint32_t type, const void *W, const 
                                  : launch_gemm_kq_bf16_wave4s_multi(type, 1, &W, X, &Y, &n_rows, n_cols, n_tok, ldx, &ldy, stream, split);
 }
 
-/* How many token blocks the tiles of a launch have (0: the 128-token x 64-row kernel), of tensors that take `tile` each by itself. All
- * shapes give the same bits, so the tensors of a launch are looked at together. Estimates in us: a super-block costs a full round of
- * 256 workgroups what the table says (measured at 224 workgroups; the 128 x 64 kernel's at up to 256 workgroups and at 512), a round
- * that leaves compute units idle less - the clock is higher then, the more so the more blocks; three blocks fit a compute unit's
- * LDS twice. Row tiles are dealt to 8 XCDs of 32 compute units. Over 198 products of nine formats (2048 to 28672 rows x 2048 to 4096 and
- * 14336 columns, 77 to 1024 tokens) the choice costs 1.0 % of the best kernel's time and takes 0.90 of what `tile` does (one tensor). A gain of less
- * than 4 % is left alone. */
+/* How many token blocks the tiles of a launch have (0: the 128-token x 64-row kernel), of tensors that take `tile` each by itself: the
+ * least of tile_us. All shapes give the same bits, so the tensors of a launch are looked at together. Over 198 products of nine formats
+ * (2048 to 28672 rows x 2048 to 4096 and 14336 columns, 77 to 1024 tokens) the choice costs 0.3 % of the best kernel's time and takes
+ * 0.94 of what `tile` does (one tensor). A gain of less than 4 % is left alone: at 2 % pairs of 5632 x 1536 IQ4_XS at
+ * 557 tokens lost 1 %. */
 int choose_token_blocks(uint32_t type, FusedTile tile, int n_mat, const int *n_rows, int n_cols, int n_tok) {
-    struct Cost { float b3, b4, b5, b6, b8, small_256, small_512; };
-    Cost c;
-    switch (type) { /* the measurements: 3.5 us + 16 super-blocks times this, 4096 columns */
-    case T_Q4_K: c = {1.77f, 2.15f, 2.45f, 2.82f, 3.53f, 1.37f, 2.42f}; break;
-    case T_Q5_K: c = {1.86f, 2.28f, 2.65f, 3.04f, 3.67f, 1.51f, 2.50f}; break;
-    case T_Q6_K: c = {2.46f, 2.79f, 3.05f, 3.56f, 4.00f, 1.79f, 2.95f}; break;
-    case T_Q8_0: c = {2.61f, 3.23f, 3.75f, 3.92f, 4.67f, 2.19f, 3.80f}; break;
-    case T_IQ4_NL: c = {1.99f, 2.50f, 2.75f, 3.29f, 3.73f, 1.48f, 2.62f}; break;
-    case T_IQ4_XS: c = {2.04f, 2.50f, 2.78f, 3.23f, 3.74f, 1.53f, 2.68f}; break;
-    case T_Q4_0: c = {1.76f, 2.17f, 2.50f, 2.88f, 3.49f, 1.40f, 2.39f}; break;
-    case T_Q2_K: c = {1.64f, 2.09f, 2.37f, 2.72f, 3.48f, 1.31f, 2.30f}; break;
-    default: c = {1.85f, 2.26f, 2.57f, 3.04f, 3.56f, 1.38f, 2.54f}; break; /* Q3_K */
-    }
-    long long rows128 = 0, rows64 = 0;
-    for (int i = 0; i < n_mat; i++) { rows128 += ((long long)n_rows[i] + 127) / 128; rows64 += ((long long)n_rows[i] + 63) / 64; }
-    const auto workgroups = [&](long long row_tiles, int tokens) { return (row_tiles + 7) / 8 * 8 * ((n_tok + tokens - 1) / tokens); };
-    /* the part of a full round's time that n workgroups take on the chip: `low` up to 112 of them */
-    const auto round = [](double low, double n) {
-        const double x = std::min(1.0, std::max(0.0, (n - 112) / 112));
-        return low + (1 - low) * x * x * x;
-    };
-    const auto blocks_us = [&](int nb, double full, double low) {
-        const long long n = workgroups(rows128, 32 * nb), per = nb == 3 ? 512 : 256, rest = n % per;
-        double rounds = (double)(n / per) * (nb == 3 ? 1.85 : 1.0);
-        if (rest > 256) rounds += 1.0 + 0.85 * (0.6 + 0.4 * (rest - 256) / 256);
-        else if (rest > 0) rounds += round(low, (double)rest);
-        return 3.5 + n_cols / 256 * full * rounds;
-    };
-    const long long n_small = workgroups(rows64, 128), rest = n_small % 512;
-    double small = (double)(n_small / 512) * c.small_512;
-    if (rest > 256) small += c.small_256 + (c.small_512 - c.small_256) * (0.55 + 0.45 * (rest - 256) / 256);
-    else if (rest > 0) small += c.small_256 * (0.9 + 0.1 * rest / 256);
-    small = 3.5 + n_cols / 256 * small;
-    const double us[5] = {blocks_us(3, c.b3, 0.92), blocks_us(4, c.b4, 0.80), blocks_us(5, c.b5, 0.78), blocks_us(6, c.b6, 0.75), blocks_us(8, c.b8, 0.71)};
-    const int blocks[5] = {3, 4, 5, 6, kLargeBlocks};
-    int best = tile == kFusedLarge ? kLargeBlocks : 0;
-    double best_us = 0.96 * (tile == kFusedLarge ? us[4] : small);
-    if (small < best_us) { best = 0; best_us = small; }
-    for (int i = 0; i < 5; i++)
-        if (us[i] < best_us) { best = blocks[i]; best_us = us[i]; }
-    return best;
+    double us[6];
+    tile_us(type, n_mat, n_rows, n_cols, n_tok, us);
+    int best = tile == kFusedLarge ? 5 : 0;
+    double best_us = 0.96 * us[best];
+    for (int i = 0; i < 6; i++)
+        if (us[i] < best_us) { best = i; best_us = us[i]; }
+    return kTokenBlocks[best];
 }
 
 hipError_t launch_fused_tiles(FusedTile tile, uint32_t type, int n_mat, const void *const *W, const uint16_t *X, float *const *Y, const int *n_rows,

@@ -231,14 +231,14 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * W is decoded once to bf16 (nearest even) into `workspace` and multiplied by the dense matrix-core GEMM of
  * the vendor library. Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, IQ4_NL, IQ4_XS and Q4_0 tensors (n_cols % 256 == 0) are instead
  * decoded inside the product by this library's tile kernels, with the same single rounding to bf16 and no workspace (it may be NULL
- * for them): 128-token x 64-row tiles up to 128 tokens (Q8_0: up to 25472 rows) and beyond where 512 of them or fewer hold the
- * product, 256-token x 128-row tiles above that wherever they take the chip fewer rounds; for tensors of half to twice as many rows as
- * columns wherever there are 200 of them. Given a workspace, rows of 5376 elements and more on few tiles (65 to 1024 tokens; above 128 at most
+ * for them), in tiles of 128 tokens x 64 rows or of 96, 128, 160, 192 or 256 tokens x 128 rows, whichever should take the tensors of the
+ * launch the least time (every shape gives the same bits). Given a workspace, rows of 5376 elements and more on few tiles (65 to 1024 tokens; above 128 at most
  * half as many rows as columns) divide K over workgroups, whose sums go through the workspace to a second
  * launch (the order of the fp32 sums differs from a call without one).
  * Given a workspace, the decode + dense route still takes the shapes where decoding once measured
- * faster: large-tile shapes above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512 (Q6_K, Q8_0), small-tile
- * shapes of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024.
+ * faster: tensors that fill the chip with 256-token tiles above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512
+ * (Q6_K, Q8_0), smaller ones of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024, except where an estimate of
+ * both says that the tiles take less than 0.9 of the time (Q8_0: 0.86) (tensors of 640 rows and more).
  * A few tokens of these formats (and, given a workspace, up to 64 of IQ3_S and IQ2_XXS) run in the few-token kernel
  * (n_cols % 256 == 0, no workspace used), which streams the blocks once: with unrounded codes (~1e-6) up to 32 tokens of
  * Q4_K, 24 of Q5_K, Q6_K, Q2_K, Q3_K and Q8_0 and 4 of the others; beyond that, with the same single rounding to bf16, up

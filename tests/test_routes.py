@@ -78,3 +78,17 @@ def test_the_lines_between_the_kernels_past_48_tokens(tid):
             (16384, 2048, 256, small), (16385, 2048, 256, large), (16384, 2048, 129, small), (16385, 2048, 130, large),
             (10880, 2048, 200, small), (41984, 2048, 256, large), (32896, 2048, 256, large if q8 else small)]:
         assert route(tid, n_rows, n_cols, n_tok) == want, (n_rows, n_cols, n_tok)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: synth.TYPE_NAMES[t])
+def test_tensors_that_fill_few_rounds_stay_in_tiles_beyond_the_lines_for_large_ones(tid):
+    """2048 x 2048 at 640 tokens costs less in tiles than to decode (Q8_0: 11008 x 1024 at 328); 28672 x 4096 at 4096 does not, and neither does
+    what is wider, or has fewer rows, than the estimates were measured for; without a workspace there is no choice"""
+    small, large, dense = 2, 1, 0
+    assert route(tid, 2048, 2048, 640) == small if tid != synth.GGML_Q8_0 else route(tid, 11008, 1024, 328) == large
+    for n_rows, n_cols, n_tok, want in [(4096, 4096, 2048, dense if tid in (synth.GGML_Q8_0, synth.GGML_Q6_K) else large),
+                                        (14336, 4096, 4096, dense), (28672, 4096, 4096, dense), (4096, 14592, 2048, dense)]:
+        assert route(tid, n_rows, n_cols, n_tok) == want, (n_rows, n_cols, n_tok)
+    assert route(tid, 28672, 4096, 4096, 0) == large
+    if tid in (synth.GGML_Q6_K, synth.GGML_Q8_0, synth.GGML_IQ4_NL, synth.GGML_IQ4_XS):
+        assert route(tid, 639, 1024, 1860) == dense and route(tid, 640, 1024, 1860) == small
