@@ -573,7 +573,7 @@ def gemm_route(type_id, n_tok, n_rows, n_cols):
     if r == 3:
         return "few-token kernel, no workspace"
     if r:
-        tiles = "256-token x 128-row" if r == 1 else "128-token x 64-row"
+        tiles = "128-row" if r == 1 else "64- or 128-row"
         parts = qlinear.load().qlin_probe_gemm_parts(type_id, n_rows, n_cols, n_tok, n_cols)
         return "decoded inside the product (%s tiles), %s" % (
             tiles, "K in %d parts, their sums in the workspace" % parts if parts > 1 else "no workspace")
