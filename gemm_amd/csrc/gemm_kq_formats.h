@@ -587,20 +587,20 @@ template <> struct KItems<true> { float *buf0, *buf1, *buf2; int parts0, parts1,
 inline KItems<true> k_items(const KSplit &s) { return {s.buf[0], s.buf[1], s.buf[2], s.parts[0], s.parts[1], s.parts[2]}; }
 
 /* a workgroup's share of K */
-struct KPart { const uint8_t *W; float *out; int n_rows, ld, tile, sb0, n_sb; };
+struct KPart { const uint8_t *W; float *out; int n_rows, ld, tile, sb0, n_sb; bool divided; };
 QLIN_INL KPart k_part(const TileSet &set, const KItems<false> &, int item, int n_sb, int) {
     const TileOf t = tile_of(set, item);
-    return {t.W, t.Y, t.n_rows, t.ldy, t.tile, 0, n_sb};
+    return {t.W, t.Y, t.n_rows, t.ldy, t.tile, 0, n_sb, false};
 }
 QLIN_INL KPart k_part(const TileSet &set, const KItems<true> &split, int item, int n_sb, int n_tok) {
     const TileOf t = tile_of(set, item);
-    KPart p = {t.W, t.Y, t.n_rows, t.ldy, t.tile, 0, n_sb};
     int n_parts;
     float *buf;
     if (item < set.end0) { n_parts = split.parts0; buf = split.buf0; }
     else if (item < set.end1) { n_parts = split.parts1; buf = split.buf1; }
     else { n_parts = split.parts2; buf = split.buf2; }
-    if (n_parts > 1) {
+    KPart p = {t.W, t.Y, t.n_rows, t.ldy, t.tile, 0, n_sb, n_parts > 1};
+    if (p.divided) {
         auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); }; /* (divisions run in vector registers) */
         const unsigned parts = (unsigned)n_parts;
         p.tile = uniform((int)((unsigned)t.tile / parts));

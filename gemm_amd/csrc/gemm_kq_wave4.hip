@@ -58,7 +58,8 @@
  *
  * Every wave keeps two sums per result, of k-steps 0 and 1 of the tiles and of 2 and 3, and adds them at the end: the 128 x 64 kernel's
  * two halves of K. So all tile shapes give the same bits, and which one a launch takes is free - the one that suits its tensors together.
- * (Where K is divided over workgroups the shape is a tensor's own choice, and one sum is kept: the second costs a launch 1 us.)
+ * (Where K is divided over workgroups the shape is a tensor's own choice, and one sum is kept: the second costs a launch 1 us. A
+ * tensor that shares such a launch with its K whole keeps two.)
  */
 #include <climits>
 #include <utility>
@@ -200,32 +201,23 @@ template <class C, int... J> QLIN_INL void load_cur(C &c, std::integer_sequence<
 template <class C, int... J> QLIN_INL void load_cur_extra(C &c, std::integer_sequence<int, J...>) { (C::F::template extra_load<J>(c, c.cur, 0), ...); }
 template <class C, int... B> QLIN_INL void load_first(C &c, std::integer_sequence<int, B...>) { ((c.xf[0][B] = load_frag<0, 0, B>(c)), ...); }
 
-}  // namespace
-
-template <class F, int NB, bool DIVIDED>
-__global__ void __launch_bounds__(256)
-gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles,
-                          const KItems<DIVIDED> split) {
-    /* raw blocks of one super-block of each wave's 32 weight rows (32 x kPieces pieces, rounded up to whole requests) */
+/* raw blocks of one super-block of each wave's 32 weight rows (32 x kPieces pieces, rounded up to whole requests) */
+template <class F> QLIN_INL uint8_t *raw_ptr() {
     __shared__ __attribute__((aligned(1024))) uint8_t w4_raw[4 * F::kReq * 1024];
-    const int tid = threadIdx.x, lane = tid & 63;
+    return w4_raw;
+}
 
-    /* consecutive workgroup ids land on different XCDs (id % 8), each with its own L2; the token tiles
-     * that share one weight tile get ids 8 apart and meet in the same L2 */
-    const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
-    const int tile_m = slot_id % m_tiles;
-    const int item = (slot_id / m_tiles) * 8 + xcd;
-    if (item >= set.end2) return;
-    /* this workgroup's super-blocks, and where its sums go */
-    const KPart part = k_part(set, split, item, n_sb_all, n_tok);
+/* one tile: this workgroup's super-blocks (`part`, of rows of n_sb_all) of token tile tile_m, in SUMS sums per result; `tid` = threadIdx.x */
+template <class F, int NB, int SUMS> QLIN_INL void run_part(const KPart &part, const uint16_t *X, int n_sb_all, int n_tok, int ldx, int tile_m, int tid) {
+    const int lane = tid & 63;
     const int n_sb = part.n_sb, n_rows = part.n_rows, ldy = part.ld, tile_n = part.tile;
     const uint8_t *W = part.W + (size_t)part.sb0 * F::kBlockBytes;
     float *Y = part.out;
     X += part.sb0 * 256;
 
-    Ctx<F, NB, DIVIDED ? 1 : 2> c;
+    Ctx<F, NB, SUMS> c;
     constexpr int kBM = 32 * NB;
-    c.raw = w4_raw;
+    c.raw = raw_ptr<F>();
     c.wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     c.n_sb = n_sb;
     c.unit = 1.0f / fp8_pair_lo(1u).x;
@@ -267,7 +259,7 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             c.acc[0][i][v] = 0.0f;
-            if constexpr (!DIVIDED) c.acc[1][i][v] = 0.0f;
+            if constexpr (SUMS == 2) c.acc[1][i][v] = 0.0f;
         }
 
     /* ---- prologue: raw blocks of super-block 0 fetched and read back, those of super-block 1 and tiles 0..2
@@ -313,7 +305,7 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 a[v] = c.acc[0][bj][4 * g + v];
-                if constexpr (!DIVIDED) a[v] += c.acc[1][bj][4 * g + v];
+                if constexpr (SUMS == 2) a[v] += c.acc[1][bj][4 * g + v];
             }
             if (vec_ok && n + 3 < n_rows) {
                 *reinterpret_cast<floatx4 *>(y) = a;
@@ -324,6 +316,35 @@ gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_
             }
         }
     }
+}
+
+}  // namespace
+
+template <class F, int NB, bool DIVIDED>
+__global__ void __launch_bounds__(256)
+gemm_kq_bf16_wave4_kernel(TileSet set, const uint16_t *__restrict__ X, int n_sb_all, int n_tok, int ldx, int m_tiles,
+                          const KItems<DIVIDED> split) {
+    /* consecutive workgroup ids land on different XCDs (id % 8), each with its own L2; the token tiles
+     * that share one weight tile get ids 8 apart and meet in the same L2 */
+    const int xcd = blockIdx.x & 7, slot_id = blockIdx.x >> 3;
+    const int tile_m = slot_id % m_tiles;
+    const int item = (slot_id / m_tiles) * 8 + xcd;
+    if (item >= set.end2) return;
+    /* this workgroup's super-blocks, and where its sums go */
+    const KPart part = k_part(set, split, item, n_sb_all, n_tok);
+    int tid = threadIdx.x;
+    if constexpr (DIVIDED) {
+        /* One branch per workgroup: a tensor that keeps its K whole beside divided ones has two sums here as well, as in a call of its own.
+         * That costs such a launch 1 % (Q5_K 13568 + 3392 + 3392 rows x 13568 at 1009 tokens 563 -> 571 us), a launch for each kind 3.5 % in
+         * the mean and up to 13 (Q5_K 10240 + 1100 + 1100 x 10240 at 899 282 -> 297, IQ4_NL 12032 + 1705 + 1705 x 12032 at 737 333 -> 379);
+         * launches with divided tensors only take what they did. (The lane's number is opaque to the compiler in one branch, which
+         * else computes both branches' offsets ahead of them and spills some.) */
+        if (part.divided) run_part<F, NB, 1>(part, X, n_sb_all, n_tok, ldx, tile_m, tid);
+        else {
+            asm volatile("" : "+v"(tid));
+            run_part<F, NB, 2>(part, X, n_sb_all, n_tok, ldx, tile_m, tid);
+        }
+    } else run_part<F, NB, 2>(part, X, n_sb_all, n_tok, ldx, tile_m, tid);
 }
 
 namespace {

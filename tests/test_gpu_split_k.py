@@ -83,6 +83,9 @@ def test_divided_products(oracle, tid, n_tok, n_rows, n_cols, ldy, tile):
 SEVERAL = [(t, (2900, 1601, 2000), 5632, 150, SMALL) for t in FUSED]
 SEVERAL += [(t, (2400, 2401), 14336, 400, LARGE) for t in FUSED if t != synth.GGML_Q8_0]
 SEVERAL += [(synth.GGML_Q4_K, (1600, 1600, 1604), 5632, 256, SMALL), (synth.GGML_Q4_K, (1536, 1536, 1536), 11776, 700, 0)]
+# an undivided tensor among divided ones in large tiles, first and in the middle, a last tile of 26 rows
+MIXED_LARGE = {synth.GGML_Q6_K: ((1930, 7680, 1920), 9216, 968), synth.GGML_Q8_0: ((12693, 3815, 3815), 7936, 369)}
+SEVERAL += [(t, *MIXED_LARGE.get(t, ((4250, 690, 690), 11520, 915)), LARGE) for t in FUSED]
 
 
 @pytest.mark.parametrize("tid,rows,n_cols,n_tok,want", SEVERAL)

@@ -41,6 +41,9 @@ def test_divided_tensors_share_a_launch(tid):
     for rows, n_cols, n_tok in [((8192, 2048, 2048), 8192, 256), ((6144, 1536, 1536), 6144, 200), ((2900, 1601, 2000), 5632, 150)]:
         assert parts(tid, rows[0], n_cols, n_tok) == 1 and parts(tid, rows[1], n_cols, n_tok) > 1
         assert shared(tid, rows, n_cols, n_tok) == SMALL, (rows, n_cols, n_tok)
+    rows, n_cols, n_tok = {synth.GGML_Q6_K: ((7680, 1930, 1920), 9216, 968), synth.GGML_Q8_0: ((12693, 3815, 3815), 7936, 369)}.get(
+        tid, ((4250, 690, 690), 11520, 915))
+    assert [parts(tid, r, n_cols, n_tok) > 1 for r in rows] == [False, True, True] and shared(tid, rows, n_cols, n_tok) == LARGE
     if tid == synth.GGML_Q4_K:  # the sums of three do not fit the workspace
         assert parts(tid, 1536, 11776, 700) == 6 and shared(tid, (1536,) * 3, 11776, 700) == 0 and shared(tid, (1536,) * 2, 11776, 700) == LARGE
 
