@@ -292,7 +292,6 @@ template <class F, int NB, int SUMS> QLIN_INL void run_part(const KPart &part, c
 
     /* C layout of the 32x32 MFMA: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4 (a weight row), column
      * l % 32 (a token): four runs of four consecutive floats of one token's output row per lane */
-    const bool vec_ok = (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
 #pragma unroll
     for (int bj = 0; bj < NB; bj++) {
         const int m = tile_m * kBM + 32 * bj + li;
@@ -307,13 +306,7 @@ template <class F, int NB, int SUMS> QLIN_INL void run_part(const KPart &part, c
                 a[v] = c.acc[0][bj][4 * g + v];
                 if constexpr (SUMS == 2) a[v] += c.acc[1][bj][4 * g + v];
             }
-            if (vec_ok && n + 3 < n_rows) {
-                *reinterpret_cast<floatx4 *>(y) = a;
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    if (n + v < n_rows) y[v] = a[v];
-            }
+            store4(y, a, n_rows - n);
         }
     }
 }

@@ -186,7 +186,6 @@ QLIN_INL void run_half(Ctx<F> &c, float *__restrict__ Y, int n_rows, int n_tok, 
 
     /* C layout of the 32x32 MFMA: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4 (a weight row), column
      * l % 32 (a token): four runs of four consecutive floats of one token's output row per lane */
-    const bool vec_ok = (ldy & 3) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;
     const int kg = lane >> 5;
 #pragma unroll
     for (int b = 0; b < 2; b++) {
@@ -201,13 +200,7 @@ QLIN_INL void run_half(Ctx<F> &c, float *__restrict__ Y, int n_rows, int n_tok, 
             a = WK == 0 ? a + other : other + a;
             if (m >= n_tok) continue;
             float *y = Y + (size_t)m * ldy + n;
-            if (vec_ok && n + 3 < n_rows) {
-                *reinterpret_cast<floatx4 *>(y) = a;
-            } else {
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    if (n + v < n_rows) y[v] = a[v];
-            }
+            store4(y, a, n_rows - n);
         }
     }
 }
