@@ -1,5 +1,5 @@
 /*
- * gemm_kq_formats.h - what the fused prefill GEMM kernels (gemm_kq_wave4.hip, gemm_kq_wave4s.hip) share: the format
+ * gemm_kq_formats.h - what the fused prefill GEMM kernels (gemm_kq_wave4.h, gemm_kq_wave4s.hip) share: the format
  * descriptions (what a lane takes from its row's block and the arithmetic that turns it into bf16 matrix operands) and
  * a few device helpers. A kernel hands a format description its context `c`: the members it reads and writes are
  * wa[2][4] (decoded operands), t (scratch), sc (the super-block's scales), kg (lane half), unit (the fp8 reading's

@@ -184,7 +184,7 @@ hipError_t f32_split_iq3s(const F32SplitCall &c);
 hipError_t f32_split_iq2xxs(const F32SplitCall &c);
 constexpr int kMatvecTokens = 4; /* qlin_gemm_bf16_any_dev: up to this many tokens of a format without a few-token kernel go through the matvec */
 /* Tiles of 128 rows on four waves, one per SIMD, weights decoded from their blocks into the matrix operand
- * (gemm_kq_wave4.hip): the formats of gemm_kq_wave4_covers, n_cols % 256 == 0, ldx < 2^22 */
+ * (gemm_kq_wave4.h): the formats of gemm_kq_wave4_covers, n_cols % 256 == 0, ldx < 2^22 */
 bool gemm_kq_wave4_covers(uint32_t type);
 /* K of a tensor divided over parts[i] workgroups per tile, which write their sums to buf[i], [part][token][row]; launch_k_join adds
  * them up, of all tensors that are divided. One part: the sums go to Y. */
@@ -200,6 +200,17 @@ void launch_k_join(const KSplit &split, int n_mat, float *const *Y, const int *n
 hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int blocks, int n_mat, const void *const *W, const uint16_t *X,
                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
                                            const int *ldy, hipStream_t stream, KSplit split = {});
+constexpr int kLargeBlocks = 8;
+struct Wave4Call { int blocks, n_mat; const void *const *W; const uint16_t *X; float *const *Y; const int *n_rows; int n_cols, n_tok, ldx; const int *ldy; KSplit split; hipStream_t stream; };
+hipError_t wave4_q4k(const Wave4Call &c);
+hipError_t wave4_q5k(const Wave4Call &c);
+hipError_t wave4_q2k(const Wave4Call &c);
+hipError_t wave4_q6k(const Wave4Call &c);
+hipError_t wave4_q3k(const Wave4Call &c);
+hipError_t wave4_q8_0(const Wave4Call &c);
+hipError_t wave4_q4_0(const Wave4Call &c);
+hipError_t wave4_iq4nl(const Wave4Call &c);
+hipError_t wave4_iq4xs(const Wave4Call &c);
 hipError_t launch_gemm_kq_bf16_wave4s_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
                                             float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
                                             const int *ldy, hipStream_t stream, KSplit split = {});
