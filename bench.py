@@ -573,7 +573,8 @@ def gemm_route(type_id, n_tok, n_rows, n_cols):
     if r == 3:
         return "few-token kernel, no workspace"
     if r:
-        tiles = "128-row" if r == 1 else "64- or 128-row"
+        blocks = qlinear.load().qlin_probe_gemm_blocks(type_id, 1, (ctypes.c_int * 1)(n_rows), n_cols, n_tok, n_cols, 1)
+        tiles = "128-token x 64-row" if blocks == 1 else "%d-token x 128-row" % (32 * blocks)
         parts = qlinear.load().qlin_probe_gemm_parts(type_id, n_rows, n_cols, n_tok, n_cols)
         return "decoded inside the product (%s tiles), %s" % (
             tiles, "K in %d parts, their sums in the workspace" % parts if parts > 1 else "no workspace")

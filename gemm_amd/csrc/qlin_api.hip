@@ -1472,6 +1472,20 @@ int qlin_probe_gemm_multi_route(uint32_t type, int n_mat, const int *n_rows, int
     return !p.together || p.matvecs ? 0 : p.few ? 3 : (int)p.tile;
 }
 
+int qlin_probe_gemm_blocks(uint32_t type, int n_mat, const int *n_rows, int n_cols, int n_tok, int ldx, int have_workspace) {
+    if (n_mat < 1 || n_mat > 3 || !n_rows || n_tok < 1) return 0;
+    for (int i = 0; i < n_mat; i++)
+        if (n_rows[i] < 1) return 0;
+    const int route = n_mat > 1 ? qlin_probe_gemm_multi_route(type, n_mat, n_rows, n_cols, n_tok, ldx, have_workspace)
+                                : qlin_probe_gemm_route(type, n_rows[0], n_cols, n_tok, ldx, have_workspace);
+    if (route != kFusedLarge && route != kFusedSmall) return 0;
+    bool divided = false;
+    for (int i = 0; i < n_mat; i++) divided = divided || (have_workspace && qlin_probe_gemm_parts(type, n_rows[i], n_cols, n_tok, ldx) > 1);
+    if (divided) return route == kFusedLarge ? kLargeBlocks : 1;
+    const int blocks = choose_token_blocks(type, (FusedTile)route, n_mat, n_rows, n_cols, n_tok);
+    return blocks ? blocks : 1;
+}
+
 int qlin_probe_gemv_lds(uint32_t type, int pair, int n_mat, const int *n_rows, int n_cols) {
     if (n_mat < 1 || n_mat > 3 || !n_rows || n_cols < 0 || (pair && n_mat != 2)) return 0;
     for (int m = 0; m < n_mat; m++)

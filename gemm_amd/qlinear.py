@@ -123,6 +123,7 @@ SIGNATURES = {
     "qlin_probe_gemm_parts": (C.c_int, [C.c_uint32, C.c_int, C.c_int, C.c_int, C.c_int]),
     "qlin_probe_gemm_multi_route": (C.c_int, [C.c_uint32, C.c_int, C.POINTER(C.c_int), C.c_int, C.c_int, C.c_int, C.c_int]),
     "qlin_probe_gemv_lds": (C.c_int, [C.c_uint32, C.c_int, C.c_int, C.POINTER(C.c_int), C.c_int]),
+    "qlin_probe_gemm_blocks": (C.c_int, [C.c_uint32, C.c_int, C.POINTER(C.c_int), C.c_int, C.c_int, C.c_int, C.c_int]),
     "qlin_probe_gemm_f32_route": (C.c_int, [C.c_uint32, C.c_int, C.c_int, C.c_int]),
     "qlin_probe_gemm_tile": (C.c_int, [C.c_int, C.c_uint32, _vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _vp]),
     "qlin_timer_begin": (C.c_int, [_vp]),
