@@ -53,10 +53,16 @@ bool gemm_kq_wave4_covers(uint32_t type) {
 }
 
 /* Estimates, in us, for the tensors of a launch in each shape of tile. A super-block costs a full round of 256 workgroups what the
- * table says (the 128 x 64 kernel's: up to 256 workgroups, and 512), a round that leaves compute units idle less - the clock is higher
- * then, the more so the more blocks; three blocks fit a compute unit's LDS twice. Row tiles are dealt to 8 XCDs of 32 compute units.
+ * table says (the 128 x 64 kernel's: 256 workgroups beside more, and 512), a round that leaves compute units idle less - the clock is
+ * higher then, the more so the more blocks; three blocks fit a compute unit's LDS twice. Row tiles are dealt to 8 XCDs of 32 compute units.
  * The results go to memory at 3.3 TB/s beside that. Fitted to 3700 measured products of nine formats (640 to 28672 rows x 1024 to
- * 14336 columns, 77 to 4096 tokens, runs long enough that the power limit counts); an estimate errs by 3.8 % in the mean. */
+ * 14336 columns, 77 to 4096 tokens, few of them past 2048, runs long enough that the power limit counts), fractions of a round
+ * included: 0.73 + 0.27 of 507ths of one (of up to 256 workgroups; of 256ths it would be 7 % off from 130 on). On another card and in short
+ * runs, where the power limit does not count, 1250 products of that range err by 7 % in the mean.
+ * The 128 x 64 kernel reads X twice as often, and past 2048 tokens the workgroups of an XCD no longer meet in its L2 as they do below:
+ * measured over estimated without the factor 1.15 (up to 1.8) at 2049 to 2560 tokens, 1.4 to 3072, 1.55 to 4096, 1.6 from there to 16384;
+ * with 1024 to 1792 columns 1.09, 1.22, 1.5 and 1.5, with fewer 0.92 to 1.18. Beyond what it was fitted to an estimate errs by more: rows of 256 to 768 elements
+ * 0.75 to 1.05 of the time, 28676 to 160000 rows 0.91 to 0.99, past 4096 tokens 0.83 to 0.98, 14592 to 28672 columns 0.97 to 1.15. */
 static constexpr int kTokenBlocks[6] = {0, 3, 4, 5, 6, kLargeBlocks};
 static void tile_us(uint32_t type, int n_mat, const int *n_rows, int n_cols, int n_tok, double us[6]) {
     struct Cost { float small_256, small_512, b[5]; };
@@ -85,7 +91,8 @@ static void tile_us(uint32_t type, int n_mat, const int *n_rows, int n_cols, int
     double rounds = (double)(n_small / 512) * c.small_512;
     if (rest_small > 256) rounds += c.small_256 + (c.small_512 - c.small_256) * (0.64 + 0.36 * (rest_small - 256) / 256);
     else if (rest_small > 0) rounds += c.small_256 * (0.73 + 0.27 * rest_small / 507.0);
-    us[0] = fixed + n_cols / 256 * rounds;
+    const double past = n_cols < 1024 ? 0.0 : std::min(1.0, std::max(0.0, (n_tok - (n_cols < 2048 ? 2304 : 2048)) / 1280.0));
+    us[0] = (fixed + n_cols / 256 * rounds) * (1.0 + 0.6 * past);
     for (int i = 0; i < 5; i++) {
         const int nb = kTokenBlocks[i + 1];
         const long long n = workgroups(rows128, 32 * nb), per = nb == 3 ? 512 : 256, rest = n % per;
@@ -153,8 +160,13 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     }
     bool large_ok = n_tok <= large_max || !have_workspace, small_ok = n_tok <= small_max || !have_workspace;
     /* beyond: the estimates, in the range they were measured over (256 rows x 2304 IQ4_NL at 1860 tokens would lose 2 us; Q8_0's K
-     * and V of a model wider than 11008 divide K at such token counts, and would part from a Q in tiles) */
-    if ((!large_ok || !small_ok) && n_rows >= 640 && n_cols <= (type == T_Q8_0 ? 11008 : 14336)) {
+     * and V of a model wider than 11008 divide K at such token counts, and would part from a Q in tiles; past 4096 tokens Q2_K 819 x 1024
+     * at 7370 took 42 us in tiles, decode + library 28). Rows below 1024 elements, which they were not fitted to, go by them only from
+     * decode + library to tiles (Q6_K 1697 x 512 at 1700, the mean of 2400: 0.65 of the time), not between tiles (Q2_K 3048 x 512 at 1816
+     * 14.1 -> 16.4). */
+    const bool tiles = large_tiles >= 200 ? large_ok : small_ok;
+    if ((!large_ok || !small_ok) && (n_cols >= 1024 || !tiles) && n_rows >= 640 && n_rows <= 28672 && n_cols <= (type == T_Q8_0 ? 11008 : 14336) &&
+        n_tok <= 4096) {
         double us[6];
         tile_us(type, 1, &n_rows, n_cols, n_tok, us);
         const double weights = (double)n_rows * n_cols, results = (double)n_rows * n_tok;
@@ -255,12 +267,17 @@ hipError_t launch_fused_split(FusedSplit s, uint32_t type, const void *W, const 
  * least of tile_us. All shapes give the same bits, so the tensors of a launch are looked at together. Over 198 products of nine formats
  * (2048 to 28672 rows x 2048 to 4096 and 14336 columns, 77 to 1024 tokens) the choice costs 0.3 % of the best kernel's time and takes
  * 0.94 of what `tile` does (one tensor). A gain of less than 4 % is left alone: at 2 % pairs of 5632 x 1536 IQ4_XS at
- * 557 tokens lost 1 %. */
+ * 557 tokens lost 1 %. Beyond what the estimates were fitted to 8 % are asked for: of 2460 random products there 44 lost more than 3 % and up
+ * to 33 with 4 % (Q2_K 2320 x 1536 at 8568 tokens 116 -> 154 us, Q4_K 14892 x 512 at 1540 50 -> 61, Q2_K 85460 x 1280 at 104 42.0 -> 44.8), nine
+ * and up to 8 with 8, two with 10, which leaves more alone. */
 int choose_token_blocks(uint32_t type, FusedTile tile, int n_mat, const int *n_rows, int n_cols, int n_tok) {
     double us[6];
     tile_us(type, n_mat, n_rows, n_cols, n_tok, us);
+    long long rows = 0;
+    for (int i = 0; i < n_mat; i++) rows += n_rows[i];
+    const bool fitted = n_cols >= 1024 && n_tok <= 4096 && rows <= 28672;
     int best = tile == kFusedLarge ? 5 : 0;
-    double best_us = 0.96 * us[best];
+    double best_us = (fitted ? 0.96 : 0.92) * us[best];
     for (int i = 0; i < 6; i++)
         if (us[i] < best_us) { best = i; best_us = us[i]; }
     return kTokenBlocks[best];

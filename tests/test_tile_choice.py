@@ -6,7 +6,7 @@ import pytest
 
 from gemm_amd import qlinear
 import synth
-from tests.test_routes import ALL
+from tests.test_routes import ALL, route
 
 SMALL = 1
 
@@ -27,6 +27,19 @@ def test_tiles_of_the_tokens_and_rounds_that_there_are(tid):
             ((14336,), 4096, 512, 8), ((4096,), 4096, 512, SMALL), ((8192,), 2048, 192, SMALL), ((8192, 8192), 2048, 192, 3),
             ((10240,), 4096, 150, 3), ((2048, 256, 256), 2048, 320, SMALL)]:
         assert blocks(tid, rows, n_cols, n_tok) == want, (rows, n_cols, n_tok)
+
+
+@pytest.mark.parametrize("tid", ALL, ids=lambda t: synth.TYPE_NAMES[t])
+def test_beyond_what_the_estimates_were_fitted_to(tid):
+    """many tokens: 64-row tiles read X twice as often, so that large tiles stay (Q2_K 2320 x 1536 at 8568 116 us, in small ones 154), and
+    decode + library is not left for tiles (819 x 1024 at 7370 28 us / 42); short rows and very many rows: the tiles of the class, if others
+    are estimated to gain less than 8 % (Q4_K 14892 x 512 at 1540 50 us, in five blocks 61; Q2_K 85460 x 1280 at 104 42.0, in four 44.8)"""
+    for rows, n_cols, n_tok in [((2320,), 1536, 8568), ((1188,), 2048, 13199), ((14892,), 512, 1540)]:
+        assert blocks(tid, rows, n_cols, n_tok) == 8, (rows, n_cols, n_tok)
+    assert route(tid, 819, 1024, 7370) == 0
+    if tid in (synth.GGML_Q4_K, synth.GGML_Q2_K, synth.GGML_Q4_0):
+        assert blocks(tid, (85460,), 1280, 104) == SMALL
+        assert route(tid, 3048, 512, 1816) == 2  # 128 x 64 tiles, as by the lines (Q2_K 14.1 us, in large ones 16.4)
 
 
 @pytest.mark.parametrize("tid", ALL, ids=lambda t: synth.TYPE_NAMES[t])
