@@ -161,11 +161,12 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
     bool large_ok = n_tok <= large_max || !have_workspace, small_ok = n_tok <= small_max || !have_workspace;
     /* beyond: the estimates, in the range they were measured over (256 rows x 2304 IQ4_NL at 1860 tokens would lose 2 us; Q8_0's K
      * and V of a model wider than 11008 divide K at such token counts, and would part from a Q in tiles; past 4096 tokens Q2_K 819 x 1024
-     * at 7370 took 42 us in tiles, decode + library 28). Rows below 1024 elements, which they were not fitted to, go by them only from
+     * at 7370 took 42 us in tiles, decode + library 28), and for more rows, where the library's product can be far slower than estimated (24
+     * products of 29572 to 44444 rows x 8448 to 14336 at 555 to 1768 tokens: tiles take 0.50 to 0.92 of its time). Rows below 1024 elements, which they were not fitted to, go by them only from
      * decode + library to tiles (Q6_K 1697 x 512 at 1700, the mean of 2400: 0.65 of the time), not between tiles (Q2_K 3048 x 512 at 1816
      * 14.1 -> 16.4). */
     const bool tiles = large_tiles >= 200 ? large_ok : small_ok;
-    if ((!large_ok || !small_ok) && (n_cols >= 1024 || !tiles) && n_rows >= 640 && n_rows <= 28672 && n_cols <= (type == T_Q8_0 ? 11008 : 14336) &&
+    if ((!large_ok || !small_ok) && (n_cols >= 1024 || !tiles) && n_rows >= 640 && n_cols <= (type == T_Q8_0 ? 11008 : 14336) &&
         n_tok <= 4096) {
         double us[6];
         tile_us(type, 1, &n_rows, n_cols, n_tok, us);

@@ -37,6 +37,8 @@ def test_beyond_what_the_estimates_were_fitted_to(tid):
     for rows, n_cols, n_tok in [((2320,), 1536, 8568), ((1188,), 2048, 13199), ((14892,), 512, 1540)]:
         assert blocks(tid, rows, n_cols, n_tok) == 8, (rows, n_cols, n_tok)
     assert route(tid, 819, 1024, 7370) == 0
+    if tid in (synth.GGML_Q2_K, synth.GGML_Q3_K, synth.GGML_Q4_0):
+        assert route(tid, 30544, 14336, 1236) == 1  # more rows than fitted: decode + library takes 1.9 times as long
     if tid in (synth.GGML_Q4_K, synth.GGML_Q2_K, synth.GGML_Q4_0):
         assert blocks(tid, (85460,), 1280, 104) == SMALL
         assert route(tid, 3048, 512, 1816) == 2  # 128 x 64 tiles, as by the lines (Q2_K 14.1 us, in large ones 16.4)
