@@ -145,7 +145,7 @@ static bool small_by_rounds(uint32_t type, long long n_rows, int n_tok, int n_ma
     const long long padded = ((n_rows + 127) / 128 * n_mat + 7) / 8 * 8 * ((n_tok + 255) / 256), rounds = (padded + 255) / 256;
     return (n_rows + 63) / 64 * n_mat * ((n_tok + 127) / 128) <= (rounds == 1 || type == T_Q8_0 ? 512 : 650) * rounds;
 }
-FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool have_workspace) {
+FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool have_workspace, bool estimates) {
     if (!gemm_kq_wave4_covers(type) || n_cols % 256 != 0 || ldx >= (1 << 22)) return kFusedNone;
     const long long large_tiles = ((long long)n_rows + 127) / 128 * ((n_tok + 255) / 256);
     /* token counts up to which the large-tile and the small-tile kernel measured faster than decode + dense */
@@ -166,7 +166,7 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
      * decode + library to tiles (Q6_K 1697 x 512 at 1700, the mean of 2400: 0.65 of the time), not between tiles (Q2_K 3048 x 512 at 1816
      * 14.1 -> 16.4). */
     const bool tiles = large_tiles >= 200 ? large_ok : small_ok;
-    if ((!large_ok || !small_ok) && (n_cols >= 1024 || !tiles) && n_rows >= 640 && n_cols <= (type == T_Q8_0 ? 11008 : 14336) &&
+    if (estimates && (!large_ok || !small_ok) && (n_cols >= 1024 || !tiles) && n_rows >= 640 && n_cols <= (type == T_Q8_0 ? 11008 : 14336) &&
         n_tok <= 4096) {
         double us[6];
         tile_us(type, 1, &n_rows, n_cols, n_tok, us);
@@ -192,6 +192,9 @@ FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, in
  * 4096 x 14336 with 77, 128, 160, 256, 384, 512, 768 tokens 31.8 / 26.4, 45 / 29.4, 67 / 39, 69 / 44, 71 / 63, 81 / 68, 121 / 97; 2560 x 6912
  * with 128, 160, 256 19.5 / 15.8, 28 / 18, 31 / 19.5; 2048 x 5632 18.6 / 14.2, 23.5 / 15.4, 25 / 17.3; Q6_K 4096 x 14336 with 256, 768 83 / 47, 133 /
  * 106. Not below 17 super-blocks: 4096 x 4096 gains nothing (160 tokens 18.9 / 17.9, 512 23.6 / 32).
+ * What a product takes in one piece is what the lines of choose_fused_tile say, without the estimates beyond them: there Q6_K divides where
+ * parts gain 13 % on decode + library, and if tiles come close to that, parts are as good or better still (2560 x 10240 at 753 tokens 54.9 /
+ * in tiles 60.9, 2916 x 12800 at 616 70 / 74, 2944 x 11776 at 612 66 / 66).
  * The estimates, in us, are fitted to such figures; they err by a tenth, so that a gain of less than 13 % is left alone. Over 500
  * random products of 256 to 8192 rows x 5632 to 16384 columns that divide: 0.60 of the time in one piece in the geometric mean, two slower, by 3 %.
  * Not a tensor that may come with others (may_share) where their one launch, in one piece, costs less than a launch in parts
@@ -212,7 +215,7 @@ static bool may_share(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx,
     if (n_cols < 22 * 256) return true;    /* K and V of a model 4352 to 5376 wide */
     if (n_rows >= 1536 && n_cols < 6LL * n_rows) return false;
     for (const long long q20 : {15, 20, 32}) /* K and V of few rows, where a Q of 0.75 to 1.6 times n_cols rows takes the same tiles */
-        if (choose_fused_tile(type, (int)std::min(q20 * n_cols / 20, (long long)INT_MAX), n_cols, n_tok, ldx, true) == tile) return true;
+        if (choose_fused_tile(type, (int)std::min(q20 * n_cols / 20, (long long)INT_MAX), n_cols, n_tok, ldx, true, false) == tile) return true;
     return false;
 }
 FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, size_t workspace_bytes, FusedTile tile, bool few) {

@@ -1139,14 +1139,14 @@ static bool takes_fewtok(uint32_t type, int n_rows, int n_cols, int n_tok, int l
     return fewtok_takes(type, n_rows, n_cols, n_tok, ldx) && (gemm_kq_wave4_covers(type) || (ws_ok && g.dense_gemm_mode == 0)) &&
            !takes_matvec(type, n_rows, n_cols, n_tok, ws_ok);
 }
-static FusedTile takes_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool ws_ok) {
-    return takes_matvec(type, n_rows, n_cols, n_tok, ws_ok) ? kFusedNone : choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok);
+static FusedTile takes_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool ws_ok, bool estimates = true) {
+    return takes_matvec(type, n_rows, n_cols, n_tok, ws_ok) ? kFusedNone : choose_fused_tile(type, n_rows, n_cols, n_tok, ldx, ws_ok, estimates);
 }
 
 /* long rows on few tiles: K over several workgroups (parts of 1: not this shape) */
 static FusedSplit takes_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool ws_ok, size_t workspace_bytes) {
     if (!ws_ok) return {kFusedNone, 1};
-    return choose_fused_split(type, n_rows, n_cols, n_tok, ldx, workspace_bytes, takes_tile(type, n_rows, n_cols, n_tok, ldx, true),
+    return choose_fused_split(type, n_rows, n_cols, n_tok, ldx, workspace_bytes, takes_tile(type, n_rows, n_cols, n_tok, ldx, true, false),
                               takes_fewtok(type, n_rows, n_cols, n_tok, ldx, true));
 }
 

@@ -214,11 +214,12 @@ hipError_t wave4_iq4xs(const Wave4Call &c);
 hipError_t launch_gemm_kq_bf16_wave4s_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
                                             float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
                                             const int *ldy, hipStream_t stream, KSplit split = {});
-/* the fused kernel for a shape (kFusedNone: decode + dense product, or the format has none) and its launch */
+/* the fused kernel for a shape (kFusedNone: decode + dense product, or the format has none), by the lines between token counts and the
+ * estimates of what lies beyond them, or by the lines alone */
 enum FusedTile { kFusedNone = 0, kFusedLarge, kFusedSmall };
-FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool have_workspace);
-/* whether K is divided, and over how many workgroups a tile (1: it is not), given what would take the product whole; the parts
- * lie at the start of the workspace */
+FusedTile choose_fused_tile(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, bool have_workspace, bool estimates = true);
+/* whether K is divided, and over how many workgroups a tile (1: it is not), given what would take the product whole by the lines alone;
+ * the parts lie at the start of the workspace */
 struct FusedSplit { FusedTile tile; int parts; };
 FusedSplit choose_fused_split(uint32_t type, int n_rows, int n_cols, int n_tok, int ldx, size_t workspace_bytes, FusedTile tile, bool few);
 hipError_t launch_fused_split(FusedSplit s, uint32_t type, const void *W, const uint16_t *X, float *Y, int n_rows, int n_cols, int n_tok,

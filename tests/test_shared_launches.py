@@ -83,6 +83,12 @@ def test_down_products_divide_k_and_what_may_share_a_launch_does_not(tid):
         assert parts(tid, n_rows, n_cols, n_tok) == 1, (n_rows, n_cols, n_tok)
 
 
+def test_the_estimates_of_tiles_take_no_division_away():
+    """Q6_K past 512 tokens: decode + library by the lines, tiles by the estimates, and faster than either in parts"""
+    for n_rows, n_cols, n_tok, n in [(3008, 12032, 630, 3), (2560, 10240, 753, 4), (2432, 9728, 765, 4), (2933, 12288, 599, 3)]:
+        assert parts(synth.GGML_Q6_K, n_rows, n_cols, n_tok) == n and route(synth.GGML_Q6_K, n_rows, n_cols, n_tok) == LARGE
+
+
 def test_large_parts_count_the_padding_of_their_row_tiles():
     """21 row tiles in four parts are 84, which eight dies take as 88: times three token tiles two rounds of 256 compute units"""
     assert parts(synth.GGML_IQ4_NL, 2624, 11520, 612) != 4 or route(synth.GGML_IQ4_NL, 2624, 11520, 612) != LARGE
