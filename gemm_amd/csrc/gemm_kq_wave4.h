@@ -49,9 +49,12 @@
  * k-step: wait for this wave's requests of the next tile, barrier (the next tile is complete; nobody reads the
  * stage that is requested next, its last fragments were fetched a k-step earlier).
  *
- * Fewer token blocks: a tile's decode costs the same whatever its tokens, about as much vector time as six blocks' matrix
- * instructions (Q4_K, one tile of 64 k on a chip of 224 workgroups: 0.41 us + 0.10 per block), so that eight blocks cost least per
- * token, and fewer win where eight would be padding or leave a second round of the chip nearly empty. Against the better one of
+ * Fewer token blocks: a tile's decode costs the same whatever its tokens (9.0 vector instructions per matrix instruction, itself
+ * included, at three blocks, 6.0 at five, 4.0 at eight, Q4_K), so that eight blocks cost least per token - a tile of 64 k in a full round of 256 workgroups takes 0.46 us
+ * with four, 0.53, 0.61 and 0.78 with five, six and eight - and fewer win where eight would be padding or leave a second round of the chip
+ * nearly empty. Three blocks fit a compute unit twice (at most 80 KB of LDS, 256 registers): 448 workgroups run at once, two waves
+ * per SIMD. What bounds fewer blocks is the vector ALU, and start and drain: the matrix pipe is busy 28 and 37 % of a kernel of three blocks
+ * (Q6_K, Q4_K), 26 and 32 of five. Against the better one of
  * 256 x 128 and 128 x 64 tiles, us (choose_token_blocks picks): Q4_K x 4096, 77 tokens 28672 rows 37.4 -> 31.8 (three), 128 tokens 41.3 -> 38.3
  * (four), 180 tokens 55 -> 48.6 (six), 300 tokens 12288 rows 51 -> 37.9 (five), 512 tokens 6144 rows 36.6 -> 32.9 (four). Q6_K 48.6 ->
  * 42.8, 53.5 -> 48.1, 65 -> 60.4, 57 -> 46.6, 46.6 -> 41.7. 128 x 128 tiles on eight waves, four row groups x two halves of K, were built and

@@ -106,15 +106,19 @@ static void tile_us(uint32_t type, int n_mat, const int *n_rows, int n_cols, int
     }
 }
 
-/* Which kernel takes a prefill GEMM of a format with a fused kernel, beyond the token counts of the few-token kernels.
- * 200 or more 256-token x 128-row tiles fill the chip: the large-tile kernel - up to a token count, because it decodes
+/* What takes a prefill GEMM of a format with a fused kernel, beyond the token counts of the few-token kernels: decode + library, given a
+ * workspace, or tiles, and of those the class, large or small. A class is no kernel any more: every shape of tile gives the same bits,
+ * and choose_token_blocks picks one for the tensors of a launch. It says which tensors may share a launch (those of one class by themselves),
+ * which kernel divides K, and which shape stays where no other is estimated to gain enough. The figures below are of 256-token x 128-row
+ * (large) and 128-token x 64-row tiles (small).
+ * 200 or more large tiles fill the chip: the large class - up to a token count, because it decodes
  * the weights again every 256 tokens, which costs more the more there is to decode, while decoding once into a workspace
  * costs 27 - 38 us whatever the token count (14336 x 4096, large tiles against decode + the vendor library's product, us:
  * at 512 tokens Q4_K 61 / 86, Q5_K 62 / 92, Q6_K 66 / 84, Q8_0 71 / 83, IQ4_NL 62 / 95, IQ4_XS 68 / 99, Q4_0 62 / 81,
  * Q2_K 59 / 82, Q3_K 62 / 91; at 1024 118 / 125, 121 / 135, 131 / 126, 139 / 121, 123 / 132, 133 / 139, 122 / 120,
  * 117 / 120, 127 / 128; at 1536 Q4_K 181 / 190, Q5_K 185 / 195, Q6_K 206 / 184, Q8_0 216 / 177; at 2048 267 / 244,
  * 262 / 260, 273 / 240, 311 / 224, 279 / 254, 305 / 270, 272 / 241, 251 / 222, 261 / 253).
- * Fewer large tiles: the small-tile kernel, up to a token count per format (small tiles / decode + library, us, at
+ * Fewer large tiles: the small class, up to a token count per format (small tiles / decode + library, us, at
  * 4096 x 4096 and 4096 x 14336 with 512 tokens, the same two with 1024, 6144 x 4096 with 768, 14336 x 4096 with 256:
  * Q4_K 24 / 43, 72 / 97, 42 / 52, 133 / 153, 57 / 59, 39 / 75; Q5_K 25 / 44, 74 / 104, 43 / 54, 139 / 158, 59 / 61, 41 / 80;
  * Q6_K 29 / 40, 85 / 96, 49 / 51, 163 / 154, 68 / 57, 47 / 71; Q8_0 35 / 38, 109 / 97, 64 / 49, 216 / 152, 91 / 55, 62 / 75;
@@ -129,15 +133,15 @@ static void tile_us(uint32_t type, int n_mat, const int *n_rows, int n_cols, int
  * 2048 235 / 201; Q2_K 4096 x 5120 at 3904 134 / 158, left alone. Of 837 random products past the lines 110 take tiles, in 0.84 of the
  * time (one is slower by more than 3 %); their error against 64 bits is 0.7 of that of the library's product.
  * Without a workspace there is no decode + dense route to prefer.
- * Up to 128 tokens half of a large tile is empty: small tiles whatever their number (77 tokens 28672 x 4096 large / small: Q4_K
+ * The class up to 128 tokens, where half of a 256-token tile is empty: small, whatever the number of tiles (77 tokens 28672 x 4096 large / small: Q4_K
  * 51 / 38, Q5_K 52 / 41, Q6_K 57 / 48; 128 tokens 65536 x 1024 Q4_K 1.26 times, IQ4_XS 1.27, Q3_K 1.30; Q8_0 even). Past 128
- * tokens by how often the chip has to go round: 256 large tiles (their row tiles are padded to eights) run at a time, 512 small
+ * tokens the class goes by how often the chip has to go round: 256 large tiles (their row tiles are padded to eights) run at a time, 512 small
  * ones, and a small round costs 0.82 of a large one, its last part less the less there is of it (time of small tiles over large,
  * Q4_K ... Q6_K at 4096 columns: one round of large tiles, 512 small ones 0.82 - 0.89, 576 to 768 1.08 - 1.24, 1000 1.24 - 1.37;
  * two rounds, 792 to 960 small ones 0.71 - 0.81, 1160 0.92 - 0.98, 1400 1.06 - 1.14, 1840 1.31 - 1.46; three, 1560 0.81 - 0.87,
  * 2080 1.04 - 1.13, 2800 1.27 - 1.42; Q8_0's small tiles cost 1.2 times as much).
- * Tensors share a launch only if each takes the same kernel by itself, so the rounds count for those that come with others only
- * where they hold for the company too. Half to twice as many rows as columns (a Q, whose K and V take small tiles): large tiles from
+ * Tensors share a launch only if each is of the same class by itself, so the rounds count for those that come with others only
+ * where they hold for the company too. Half to twice as many rows as columns (a Q, whose K and V are of the small class): large from
  * 200 on, as for tensors of any size before (Q4_K Q, K and V of 4096 + 1024 + 1024 rows x 4096 at 1280 tokens shared / Q apart in large
  * tiles 80 / 99, 5120 + 1024 + 1024 x 5120 at 1024 97 / 119). More, below eight times (gate and up): by rounds where one tensor and the
  * pair agree, else the same (2 x 10240 x 2560 Q2_K at 984 tokens large / small tiles 117 / 134, 2 x 5888 x 1536 Q4_K at 1440 76 / 81). */

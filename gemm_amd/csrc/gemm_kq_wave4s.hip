@@ -1,7 +1,7 @@
 /*
  * gemm_kq_wave4s.hip - the fused block-format x bf16 prefill GEMM (the formats of gemm_kq_formats.h) in 128-token x 64-row
- * tiles, for the shapes whose 256-token x 128-row tiles (gemm_kq_wave4.h) would leave most of the chip idle: 4096-row projections
- * at 512 tokens (64 large tiles, 256 small ones), 14336 rows at 129..256 tokens.
+ * tiles, for the shapes whose tiles of 128 rows (gemm_kq_wave4.h) would leave most of the chip idle: 4096-row projections
+ * at 512 tokens (128 tiles of 128 x 128, 256 of these), narrow models up to a few hundred tokens.
  *
  *   Y[t*ldy + r] = sum_k X[t*ldx + k] * decode(W)[r][k]      X bf16, Y fp32, fp32 accumulate
  *

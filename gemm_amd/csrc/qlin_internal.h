@@ -200,8 +200,22 @@ void launch_k_join(const KSplit &split, int n_mat, float *const *Y, const int *n
 hipError_t launch_gemm_kq_bf16_wave4_multi(uint32_t type, int blocks, int n_mat, const void *const *W, const uint16_t *X,
                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
                                            const int *ldy, hipStream_t stream, KSplit split = {});
+hipError_t launch_gemm_kq_bf16_wave4s_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
+                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
+                                            const int *ldy, hipStream_t stream, KSplit split = {});
+/* the 128-row kernel by format (gemm_kq_wave4_*.hip) */
 constexpr int kLargeBlocks = 8;
-struct Wave4Call { int blocks, n_mat; const void *const *W; const uint16_t *X; float *const *Y; const int *n_rows; int n_cols, n_tok, ldx; const int *ldy; KSplit split; hipStream_t stream; };
+struct Wave4Call {
+    int blocks, n_mat;
+    const void *const *W;
+    const uint16_t *X;
+    float *const *Y;
+    const int *n_rows;
+    int n_cols, n_tok, ldx;
+    const int *ldy;
+    KSplit split;
+    hipStream_t stream;
+};
 hipError_t wave4_q4k(const Wave4Call &c);
 hipError_t wave4_q5k(const Wave4Call &c);
 hipError_t wave4_q2k(const Wave4Call &c);
@@ -211,9 +225,6 @@ hipError_t wave4_q8_0(const Wave4Call &c);
 hipError_t wave4_q4_0(const Wave4Call &c);
 hipError_t wave4_iq4nl(const Wave4Call &c);
 hipError_t wave4_iq4xs(const Wave4Call &c);
-hipError_t launch_gemm_kq_bf16_wave4s_multi(uint32_t type, int n_mat, const void *const *W, const uint16_t *X,
-                                            float *const *Y, const int *n_rows, int n_cols, int n_tok, int ldx,
-                                            const int *ldy, hipStream_t stream, KSplit split = {});
 /* the fused kernel for a shape (kFusedNone: decode + dense product, or the format has none), by the lines between token counts and the
  * estimates of what lies beyond them, or by the lines alone */
 enum FusedTile { kFusedNone = 0, kFusedLarge, kFusedSmall };

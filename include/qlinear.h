@@ -232,13 +232,13 @@ int qlin_gemm_bf16_dev(uint32_t ggml_type, const void *W, const uint16_t *X, flo
  * the vendor library. Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, IQ4_NL, IQ4_XS and Q4_0 tensors (n_cols % 256 == 0) are instead
  * decoded inside the product by this library's tile kernels, with the same single rounding to bf16 and no workspace (it may be NULL
  * for them), in tiles of 128 tokens x 64 rows or of 96, 128, 160, 192 or 256 tokens x 128 rows, whichever should take the tensors of the
- * launch the least time (every shape gives the same bits). Given a workspace, rows of 5376 elements and more on few tiles (65 to 1024 tokens; above 128 at most
- * half as many rows as columns) divide K over workgroups, whose sums go through the workspace to a second
+ * launch the least time (every shape gives the same bits). Given a workspace, rows of 5376 elements and more on few tiles (65 to
+ * 1024 tokens; above 128 at most half as many rows as columns) divide K over workgroups, whose sums go through the workspace to a second
  * launch (the order of the fp32 sums differs from a call without one).
  * Given a workspace, the decode + dense route still takes the shapes where decoding once measured
  * faster: tensors that fill the chip with 256-token tiles above 1536 tokens (Q4_K, Q5_K, IQ4_NL), 1024 (Q2_K, Q3_K, IQ4_XS, Q4_0) or 512
  * (Q6_K, Q8_0), smaller ones of Q8_0 above 256 tokens, of Q6_K above 512, of IQ4_NL and IQ4_XS above 1024, except where an estimate of
- * both says that the tiles take less than 0.9 of the time (Q8_0: 0.86) (tensors of 640 rows and more).
+ * both says that the tiles take less than 0.9 of the time (Q8_0: 0.86) (tensors of 640 rows and more, up to 4096 tokens).
  * A few tokens of these formats (and, given a workspace, up to 64 of IQ3_S and IQ2_XXS) run in the few-token kernel
  * (n_cols % 256 == 0, no workspace used), which streams the blocks once: with unrounded codes (~1e-6) up to 32 tokens of
  * Q4_K, 24 of Q5_K, Q6_K, Q2_K, Q3_K and Q8_0 and 4 of the others; beyond that, with the same single rounding to bf16, up
@@ -267,13 +267,14 @@ int qlin_gemm_bf16_any_dev(uint32_t ggml_type, const void *W, const uint16_t *X,
 /* qlin_gemm_bf16_any_dev for one to three weight tensors of ONE format and row length against the same activations:
  * the Q, K and V projections of a prefill chunk, which the reference multiplies tensor by tensor
  * (tf_gemm_f16_mt_tokenmajor per projection, common/transformer.h:5256-5258). Y[i][t * ldy[i] + r] is tensor i's
- * product. Where every tensor on its own would take the same kernel of this library (few-token, small or large tiles)
- * they share one launch, their row tiles numbered through, with the results of one call per tensor bit for bit (tensors that divide K
+ * product. Where every tensor on its own would go to the few-token kernel, or to tiles of one class (256-token tiles or 128 x 64 ones, as
+ * far as the class goes; the launch then takes the shape of tile that suits them together), they share one launch, their row tiles numbered through, with the results of one call per tensor bit for bit (tensors that divide K
  * do so in their own parts, whose sums one more launch adds, if the workspace holds them all): a
  * 1024-row K or V projection alone is 64 workgroups of 128 tokens x 64 rows at 512 tokens on 256 compute units (Q4_K
  * 4096 + 1024 + 1024 rows x 4096 at 512 tokens: 36 us in one launch against 24 + 22 + 22). Every other case is one
  * qlin_gemm_bf16_any_dev call per tensor (those that all go through the matvec share the widening of X), with its
- * argument checks and its use of the workspace (sized for the largest tensor). The arrays W, Y, n_rows and ldy are host memory and are read before the call returns. */
+ * argument checks and its use of the workspace (sized for the largest tensor). The arrays W, Y, n_rows and ldy are host memory and are
+ * read before the call returns. */
 int qlin_gemm_bf16_multi_dev(uint32_t ggml_type, int n_mat, const void *const *W, const uint16_t *X, float *const *Y,
                              const int *n_rows, int n_cols, int n_tok, int ldx, const int *ldy, void *workspace,
                              size_t workspace_bytes, void *stream);
