@@ -59,10 +59,13 @@ bool gemm_kq_wave4_covers(uint32_t type) {
  * 14336 columns, 77 to 4096 tokens, few of them past 2048, runs long enough that the power limit counts), fractions of a round
  * included: 0.73 + 0.27 of 507ths of one (of up to 256 workgroups; of 256ths it would be 7 % off from 130 on). On another card and in short
  * runs, where the power limit does not count, 1250 products of that range err by 7 % in the mean.
- * The 128 x 64 kernel reads X twice as often, and past 2048 tokens the workgroups of an XCD no longer meet in its L2 as they do below:
- * measured over estimated without the factor 1.15 (up to 1.8) at 2049 to 2560 tokens, 1.4 to 3072, 1.55 to 4096, 1.6 from there to 16384;
- * with 1024 to 1792 columns 1.09, 1.22, 1.5 and 1.5, with fewer 0.92 to 1.18. Beyond what it was fitted to an estimate errs by more: rows of 256 to 768 elements
- * 0.75 to 1.05 of the time, 28676 to 160000 rows 0.91 to 0.99, past 4096 tokens 0.83 to 0.98, 14592 to 28672 columns 0.97 to 1.15. */
+ * The 128 x 64 kernel reads X twice as often for a result, and past 2048 tokens the 64 workgroups that an XCD runs at a time no longer
+ * meet on the same tokens in its L2, four row tiles on each: measured over estimated without the factor 1.15 (up to 1.8) at 2049 to 2560
+ * tokens, 1.4 to 3072, 1.55 to 4096, 1.6 from there to 16384; with 1024 to 1792 columns 1.09, 1.22, 1.5 and 1.5, with fewer 0.92 to 1.18.
+ * Not of fewer than 640 rows: there it is 1.1 to 1.6, but the other shapes are as far off where it counts, and with the factor two tensors
+ * of 188 rows x 6400 Q8_0 at 3359 tokens went to large tiles, 54 -> 77 us. Beyond what it was fitted to an estimate errs by more: rows of
+ * 256 to 768 elements 0.75 to 1.05 of the time, 28676 to 160000 rows 0.91 to 0.99, past 4096 tokens 0.83 to 0.98, 14592 to 28672 columns
+ * 0.97 to 1.15. */
 static constexpr int kTokenBlocks[6] = {0, 3, 4, 5, 6, kLargeBlocks};
 static void tile_us(uint32_t type, int n_mat, const int *n_rows, int n_cols, int n_tok, double us[6]) {
     struct Cost { float small_256, small_512, b[5]; };
@@ -91,7 +94,7 @@ static void tile_us(uint32_t type, int n_mat, const int *n_rows, int n_cols, int
     double rounds = (double)(n_small / 512) * c.small_512;
     if (rest_small > 256) rounds += c.small_256 + (c.small_512 - c.small_256) * (0.64 + 0.36 * (rest_small - 256) / 256);
     else if (rest_small > 0) rounds += c.small_256 * (0.73 + 0.27 * rest_small / 507.0);
-    const double past = n_cols < 1024 ? 0.0 : std::min(1.0, std::max(0.0, (n_tok - (n_cols < 2048 ? 2304 : 2048)) / 1280.0));
+    const double past = n_cols < 1024 || rows < 640 ? 0.0 : std::min(1.0, std::max(0.0, (n_tok - (n_cols < 2048 ? 2304 : 2048)) / 1280.0));
     us[0] = (fixed + n_cols / 256 * rounds) * (1.0 + 0.6 * past);
     for (int i = 0; i < 5; i++) {
         const int nb = kTokenBlocks[i + 1];

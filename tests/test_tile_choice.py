@@ -36,6 +36,8 @@ def test_beyond_what_the_estimates_were_fitted_to(tid):
     are estimated to gain less than 8 % (Q4_K 14892 x 512 at 1540 50 us, in five blocks 61; Q2_K 85460 x 1280 at 104 42.0, in four 44.8)"""
     for rows, n_cols, n_tok in [((2320,), 1536, 8568), ((1188,), 2048, 13199), ((14892,), 512, 1540)]:
         assert blocks(tid, rows, n_cols, n_tok) == 8, (rows, n_cols, n_tok)
+    for rows, n_cols, n_tok in [((53, 53), 3072, 3034), ((188, 188), 6400, 3359), ((344,), 1024, 3977)]:  # us: 22 / 24, 54 / 77, 13.4 / 16.6 in large ones
+        assert blocks(tid, rows, n_cols, n_tok) == SMALL, (rows, n_cols, n_tok)
     assert route(tid, 819, 1024, 7370) == 0
     if tid in (synth.GGML_Q2_K, synth.GGML_Q3_K, synth.GGML_Q4_0):
         assert route(tid, 30544, 14336, 1236) == 1  # more rows than fitted: decode + library takes 1.9 times as long
